@@ -1784,8 +1784,6 @@ struct bh_mlp {
     int terms = kLearnTerms;  // basis terms of the loss and of the walk's correction (3 or 7)
     float *X = nullptr, *T = nullptr;  // data set
     uint32_t cap = 0, n = 0;
-    float* S = nullptr;  // training scratch
-    size_t S_cap = 0;
     float* partials = nullptr;
     size_t part_cap = 0;
     double* loss_part = nullptr;
@@ -1968,12 +1966,10 @@ bh_status bh_mlp_forward(bh_mlp* m, const float* X, uint32_t n, float* Y, int bf
 
 static bh_status mlp_grad_device(bh_mlp* m, const float* dX, const float* dT, const uint32_t* order,
                                  uint32_t B) {
-    bh_status st = ensure_m(m, &m->S, &m->S_cap, mlp_scratch_floats(B));
-    if (st == BH_OK) st = ensure_m(m, &m->partials, &m->part_cap, (size_t)mlp_grad_chunks(B) * kMlpParams);
+    bh_status st = ensure_m(m, &m->partials, &m->part_cap, (size_t)mlp_grad_chunks(B) * kMlpParams);
     if (st == BH_OK) st = ensure_m(m, &m->loss_part, &m->loss_cap, mlp_loss_blocks(B));
     if (st != BH_OK) return st;
-    launch_mlp_grad(m->stream, dX, dT, order, B, m->params, m->S, m->loss_part, m->partials,
-                    m->terms);
+    launch_mlp_grad(m->stream, dX, dT, order, B, m->params, m->loss_part, m->partials, m->terms);
     return mcheck(m, hipGetLastError(), "gradient");
 }
 
@@ -1990,7 +1986,7 @@ bh_status bh_mlp_loss_grad(bh_mlp* m, const float* X, const float* T, uint32_t n
                         dG, 0);
         st = mcheck(m, hipGetLastError(), "gradient sum");
     }
-    std::vector<double> lp(mlp_loss_blocks(n));
+    std::vector<double> lp(mlp_grad_chunks(n));
     if (st == BH_OK && grads)
         st = mcheck(m, hipMemcpyAsync(grads, dG, kMlpParams * 4, hipMemcpyDeviceToHost, m->stream), "grads");
     if (st == BH_OK)
@@ -2091,19 +2087,19 @@ bh_status bh_mlp_train(bh_mlp* m, int epochs, uint32_t batch, float lr, uint64_t
         st = mcheck(m, hipGetLastError(), "prep");
     }
     if (st == BH_OK && final_loss) {
-        // loss over the whole data set in chunks (forward + backward kernels, loss partials only)
+        // loss over the whole data set (forward only)
         double tot = 0.0;
-        const uint32_t C = 65536;
-        for (uint32_t o = 0; o < n && st == BH_OK; o += C) {
-            const uint32_t b = std::min(C, n - o);
-            st = mlp_grad_device(m, m->X + (size_t)o * kLearnSample, m->T + (size_t)o * 2, nullptr, b);
-            std::vector<double> lp(mlp_loss_blocks(b));
-            if (st == BH_OK)
-                st = mcheck(m, hipMemcpyAsync(lp.data(), m->loss_part, lp.size() * 8,
-                                              hipMemcpyDeviceToHost, m->stream), "loss");
-            if (st == BH_OK) st = mcheck(m, hipStreamSynchronize(m->stream), "loss");
-            for (double v : lp) tot += v;
+        st = ensure_m(m, &m->loss_part, &m->loss_cap, mlp_loss_blocks(n));
+        std::vector<double> lp(mlp_loss_blocks(n));
+        if (st == BH_OK) {
+            launch_mlp_loss(m->stream, m->X, m->T, n, m->params, m->loss_part, m->terms);
+            st = mcheck(m, hipGetLastError(), "loss");
         }
+        if (st == BH_OK)
+            st = mcheck(m, hipMemcpyAsync(lp.data(), m->loss_part, lp.size() * 8,
+                                          hipMemcpyDeviceToHost, m->stream), "loss");
+        if (st == BH_OK) st = mcheck(m, hipStreamSynchronize(m->stream), "loss");
+        for (double v : lp) tot += v;
         *final_loss = tot / (2.0 * n);
     }
     if (st == BH_OK) st = mcheck(m, hipStreamSynchronize(m->stream), "train");

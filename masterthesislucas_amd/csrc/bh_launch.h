@@ -198,13 +198,15 @@ struct MlpBf16;
 void launch_mlp_prep(hipStream_t s, const float* params, MlpBf16* w);
 void launch_mlp_infer_bf16(hipStream_t s, const float* X, uint32_t n, const MlpBf16* w, float* Y);
 void launch_mlp_forward_f32(hipStream_t s, const float* X, uint32_t n, const float* p, float* Y);
-size_t mlp_scratch_floats(uint32_t B);
+// gradient of a batch: mlp_grad_chunks(B) partials of every parameter and of the squared error
+// (terms: basis terms the loss uses, 3 or 7); launch_mlp_loss: the squared error alone, in
+// mlp_loss_blocks(B) >= mlp_grad_chunks(B) partials
 uint32_t mlp_grad_chunks(uint32_t B);
 uint32_t mlp_loss_blocks(uint32_t B);
-// (terms: basis terms the loss uses, 3 or 7)
 void launch_mlp_grad(hipStream_t s, const float* X, const float* T, const uint32_t* order,
-                     uint32_t B, const float* p, float* S, double* loss_part, float* partials,
-                     int terms);
+                     uint32_t B, const float* p, double* loss_part, float* partials, int terms);
+void launch_mlp_loss(hipStream_t s, const float* X, const float* T, uint32_t B, const float* p,
+                     double* loss_part, int terms);
 void launch_mlp_adam(hipStream_t s, float* p, const float* partials, uint32_t nchunks, float* m1,
                      float* m2, float lr, int step, float* grad_out, int apply);
 void launch_mlp_adam_grad(hipStream_t s, float* p, const float* g, float* m1, float* m2, float lr,

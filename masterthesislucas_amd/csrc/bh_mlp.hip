@@ -191,156 +191,280 @@ __device__ __forceinline__ void learned_basis_f(float ux, float uy, float q, flo
 }
 
 // ---------------------------------------------------------------------------------------------
-// training: per-sample forward + backward to the pre-activation gradients, written
-// feature-major to scratch S (rows of length B): A1[64] DZ1[64] A2[64] DZ2[64] DY[14] X[10].
+// training: forward, backward and weight gradients of a batch in one kernel.
 // A sample is a row of kLearnSample floats (10 cell features, w_x, w_y, q) and a label
 // T[2]; its prediction is p = sum_j c_j b_j (complex) with c = the network's 14 outputs and b
 // the basis of (w, q); loss = sum |p - T|^2 / (2 B).
+//
+// A block of four waves takes tiles of kTrainTile samples. Every product (three forward, two
+// backward, three weight gradients) runs on the FP32 matrix instruction
+// v_mfma_f32_16x16x4_f32, wave w owning the hidden units [16 w, 16 w + 16): its columns of W1,
+// W2, W2^T and W3^T stay in registers, activations pass between the waves through LDS, and the
+// weight gradients accumulate in registers over the block's tiles and are written once, as the
+// block's partial (k_mlp_adam adds the partials in block order: deterministic).
+//   D = A B of 16x16x4: A[row l % 16][k l / 16], B[k l / 16][col l % 16],
+//   D[row 4 (l / 16) + e][col l % 16] in element e of lane l.
+// Bound by latency (a 4,096-sample batch is 133 MFLOP, 0.9 us of matrix work on the whole chip):
+// 128 blocks of 32 samples, no scratch in memory. Before: one thread per sample on 16 blocks
+// (79 us) with the activations in memory, and a thread per parameter reading 1,024 samples one
+// after the other (189 us).
 // ---------------------------------------------------------------------------------------------
-constexpr int kRowA1 = 0, kRowDZ1 = 64, kRowA2 = 128, kRowDZ2 = 192, kRowDY = 256;
-constexpr int kRowX = kRowDY + kMlpOut;
-constexpr int kScratchRows = kRowX + kMlpIn;
+constexpr int kTrainTile = 32;            // samples per tile
+constexpr uint32_t kTrainBlocks = 256;    // most blocks (and gradient partials) of a launch
+constexpr int kActStride = kMlpH + 4;     // LDS row stride of activations (bank spread)
+constexpr int kTrainX = 12;               // inputs padded to a multiple of 4; slot 10 holds 1
 
-__global__ __launch_bounds__(kBlock) void k_mlp_fwdbwd(const float* __restrict__ X,
-                                                       const float* __restrict__ T,
-                                                       const uint32_t* __restrict__ order,
-                                                       uint32_t B, const float* __restrict__ p,
-                                                       float* __restrict__ S,
-                                                       double* __restrict__ loss_part, int terms) {
-    __shared__ double red[kWavesPerBlock];
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    double sq = 0.0;
-    if (i < B) {
-        const uint32_t src = order ? order[i] : i;
-        const float* row = X + (size_t)src * kLearnSample;
-        float x[kMlpIn];
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+template <bool GRAD>
+__global__ __launch_bounds__(kBlock) void k_mlp_train(const float* __restrict__ X,
+                                                      const float* __restrict__ T,
+                                                      const uint32_t* __restrict__ order,
+                                                      uint32_t B, const float* __restrict__ p,
+                                                      double* __restrict__ loss_part,
+                                                      float* __restrict__ partials, int terms) {
+    constexpr int ST = kTrainTile / 16;  // sample blocks of a tile
+    __shared__ float s_x[kTrainTile][16 + 1];
+    __shared__ float s_off[kTrainTile][5];  // w_x, w_y, q, label
+    __shared__ float s_a1[kTrainTile][kActStride], s_a2[kTrainTile][kActStride];
+    __shared__ float s_dz[kTrainTile][kActStride];
+    __shared__ float s_y[kTrainTile][17];   // outputs, then their gradients
+    __shared__ double s_sq[kTrainTile];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r = lane & 15, q4 = lane >> 4;
+    const int unit = 16 * w + r;
+    // this wave's weights as B operands
+    float w1[kTrainX / 4], w2[kMlpH / 4], w2t[kMlpH / 4], w3t[4];
 #pragma unroll
-        for (int c = 0; c < kMlpIn; ++c) {
-            x[c] = row[c];
-            S[(size_t)(kRowX + c) * B + i] = x[c];
-        }
-        float a1[kMlpH];
-#pragma unroll
-        for (int j = 0; j < kMlpH; ++j) {
-            float z = p[kMlpOffB1 + j];
-#pragma unroll
-            for (int c = 0; c < kMlpIn; ++c) z = fmaf(x[c], p[kMlpOffW1 + c * kMlpH + j], z);
-            a1[j] = silu_f(z);
-            S[(size_t)(kRowA1 + j) * B + i] = a1[j];
-            S[(size_t)(kRowDZ1 + j) * B + i] = dsilu_f(z);  // silu'(z1), scaled below
-        }
-        float y[kMlpOut];
-#pragma unroll
-        for (int o = 0; o < kMlpOut; ++o) y[o] = p[kMlpOffB3 + o];
-        for (int j = 0; j < kMlpH; ++j) {
-            float z = p[kMlpOffB2 + j];
-#pragma unroll
-            for (int k = 0; k < kMlpH; ++k) z = fmaf(a1[k], p[kMlpOffW2 + k * kMlpH + j], z);
-            const float a2 = silu_f(z);
-            S[(size_t)(kRowA2 + j) * B + i] = a2;
-            S[(size_t)(kRowDZ2 + j) * B + i] = dsilu_f(z);  // silu'(z2), scaled below
-#pragma unroll
-            for (int o = 0; o < kMlpOut; ++o) y[o] = fmaf(a2, p[kMlpOffW3 + j * kMlpOut + o], y[o]);
-        }
-        float bas[kMlpOut];
-        learned_basis_f(row[kMlpIn], row[kMlpIn + 1], row[kMlpIn + 2], bas);
-        // a network trained with fewer terms: the basis beyond them is zero (no prediction, no
-        // gradient)
-#pragma unroll
-        for (int o = 0; o < kMlpOut; ++o)
-            if (o >= 2 * terms) bas[o] = 0.f;
-        float pr = 0.f, pi = 0.f;
-#pragma unroll
-        for (int j = 0; j < kLearnTerms; ++j) {
-            pr = fmaf(y[2 * j], bas[2 * j], fmaf(-y[2 * j + 1], bas[2 * j + 1], pr));
-            pi = fmaf(y[2 * j], bas[2 * j + 1], fmaf(y[2 * j + 1], bas[2 * j], pi));
-        }
-        const float ex = pr - T[(size_t)src * 2], ey = pi - T[(size_t)src * 2 + 1];
-        sq = (double)ex * ex + (double)ey * ey;
-        // loss = sum |e|^2 / (2 B): dL/dRe c_j = Re(conj(e) b_j) / B, dL/dIm c_j = Im(conj(b_j) e)/B
-        const float inv_b = 1.0f / (float)B;
-        float dy[kMlpOut];
-#pragma unroll
-        for (int j = 0; j < kLearnTerms; ++j) {
-            const float br = bas[2 * j], bi = bas[2 * j + 1];
-            dy[2 * j] = fmaf(ex, br, ey * bi) * inv_b;
-            dy[2 * j + 1] = fmaf(ey, br, -ex * bi) * inv_b;
-            S[(size_t)(kRowDY + 2 * j) * B + i] = dy[2 * j];
-            S[(size_t)(kRowDY + 2 * j + 1) * B + i] = dy[2 * j + 1];
-        }
-        float dz2[kMlpH];
-#pragma unroll
-        for (int j = 0; j < kMlpH; ++j) {
-            float da2 = 0.f;
-#pragma unroll
-            for (int o = 0; o < kMlpOut; ++o) da2 = fmaf(dy[o], p[kMlpOffW3 + j * kMlpOut + o], da2);
-            dz2[j] = da2 * S[(size_t)(kRowDZ2 + j) * B + i];
-            S[(size_t)(kRowDZ2 + j) * B + i] = dz2[j];
-        }
-        for (int k = 0; k < kMlpH; ++k) {
-            float da1 = 0.f;
-#pragma unroll
-            for (int j = 0; j < kMlpH; ++j) da1 = fmaf(dz2[j], p[kMlpOffW2 + k * kMlpH + j], da1);
-            S[(size_t)(kRowDZ1 + k) * B + i] *= da1;
-        }
+    for (int k = 0; k < kTrainX / 4; ++k) {
+        const int in = 4 * k + q4;
+        w1[k] = in < kMlpIn ? p[kMlpOffW1 + in * kMlpH + unit]
+                            : (in == kMlpIn ? p[kMlpOffB1 + unit] : 0.f);
     }
-    if (loss_part) {
-        for (int o = 32; o > 0; o >>= 1) sq += __shfl_xor(sq, o, 64);
-        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = sq;
+#pragma unroll
+    for (int k = 0; k < kMlpH / 4; ++k) {
+        w2[k] = p[kMlpOffW2 + (4 * k + q4) * kMlpH + unit];
+        if (GRAD) w2t[k] = p[kMlpOffW2 + unit * kMlpH + 4 * k + q4];
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const int o = 4 * k + q4;
+        w3t[k] = GRAD && o < kMlpOut ? p[kMlpOffW3 + unit * kMlpOut + o] : 0.f;
+    }
+    float w3[kMlpH / 4];  // layer 3: output r, all units (waves 0 .. ST - 1 use it)
+#pragma unroll
+    for (int k = 0; k < kMlpH / 4; ++k)
+        w3[k] = w < ST && r < kMlpOut ? p[kMlpOffW3 + (4 * k + q4) * kMlpOut + r] : 0.f;
+    const float b2 = p[kMlpOffB2 + unit];
+    const float b3 = r < kMlpOut ? p[kMlpOffB3 + r] : 0.f;
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 g1 = zero, g3 = zero, g2[4] = {zero, zero, zero, zero};
+    float gb2 = 0.f, gb3 = 0.f;
+    double sq = 0.0;  // threads < kTrainTile: squared errors of their samples
+    const float inv_b = 1.0f / (float)B;
+    const uint32_t ntiles = (B + kTrainTile - 1) / kTrainTile;
+    for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        // stage the tile: 8 threads per sample, features (bias input 1 in slot 10) and offsets
+        {
+            const int smp = tid >> 3, part = tid & 7;
+            const uint32_t i = tile * kTrainTile + smp;
+            const bool live = i < B;
+            const uint32_t src = live ? (order ? order[i] : i) : 0u;
+            const float* row = X + (size_t)src * kLearnSample;
+#pragma unroll
+            for (int c = part; c < 16; c += 8)
+                s_x[smp][c] = c < kMlpIn ? (live ? row[c] : 0.f) : (c == kMlpIn && live ? 1.f : 0.f);
+            if (part < 5)
+                s_off[smp][part] = !live ? 0.f
+                                 : part < 3 ? row[kMlpIn + part] : T[(size_t)src * 2 + part - 3];
+        }
         __syncthreads();
-        if (threadIdx.x == 0) {
-            double b = 0.0;
-            for (int k = 0; k < kWavesPerBlock; ++k) b += red[k];
-            loss_part[blockIdx.x] = b;
+        // layer 1
+        float d1[ST][4], d2[ST][4];
+#pragma unroll
+        for (int st = 0; st < ST; ++st) {
+            f32x4 z = zero;
+#pragma unroll
+            for (int k = 0; k < kTrainX / 4; ++k) z = mfma4(s_x[16 * st + r][4 * k + q4], w1[k], z);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                s_a1[16 * st + 4 * q4 + e][unit] = silu_f(z[e]);
+                d1[st][e] = GRAD ? dsilu_f(z[e]) : 0.f;
+            }
         }
+        __syncthreads();
+        // layer 2
+        f32x4 z2[ST];
+#pragma unroll
+        for (int st = 0; st < ST; ++st) z2[st] = f32x4{b2, b2, b2, b2};
+#pragma unroll
+        for (int k = 0; k < kMlpH / 4; ++k)
+#pragma unroll
+            for (int st = 0; st < ST; ++st)
+                z2[st] = mfma4(s_a1[16 * st + r][4 * k + q4], w2[k], z2[st]);
+#pragma unroll
+        for (int st = 0; st < ST; ++st)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                s_a2[16 * st + 4 * q4 + e][unit] = silu_f(z2[st][e]);
+                d2[st][e] = GRAD ? dsilu_f(z2[st][e]) : 0.f;
+            }
+        __syncthreads();
+        // layer 3: one sample block per wave
+        if (w < ST) {
+            f32x4 y0 = {b3, b3, b3, b3}, y1 = zero;
+#pragma unroll
+            for (int k = 0; k < kMlpH / 4; k += 2) {
+                y0 = mfma4(s_a2[16 * w + r][4 * k + q4], w3[k], y0);
+                y1 = mfma4(s_a2[16 * w + r][4 * k + 4 + q4], w3[k + 1], y1);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s_y[16 * w + 4 * q4 + e][r] = y0[e] + y1[e];
+        }
+        __syncthreads();
+        // prediction, error and output gradients of one sample per thread
+        if (tid < kTrainTile) {
+            float bas[kMlpOut];
+            learned_basis_f(s_off[tid][0], s_off[tid][1], s_off[tid][2], bas);
+            // a network trained with fewer terms: the basis beyond them is zero (no prediction,
+            // no gradient)
+#pragma unroll
+            for (int o = 0; o < kMlpOut; ++o)
+                if (o >= 2 * terms) bas[o] = 0.f;
+            float pr = 0.f, pi = 0.f;
+#pragma unroll
+            for (int j = 0; j < kLearnTerms; ++j) {
+                const float yr = s_y[tid][2 * j], yi = s_y[tid][2 * j + 1];
+                pr = fmaf(yr, bas[2 * j], fmaf(-yi, bas[2 * j + 1], pr));
+                pi = fmaf(yr, bas[2 * j + 1], fmaf(yi, bas[2 * j], pi));
+            }
+            const bool live = tile * kTrainTile + tid < B;
+            const float ex = live ? pr - s_off[tid][3] : 0.f;
+            const float ey = live ? pi - s_off[tid][4] : 0.f;
+            sq += (double)ex * ex + (double)ey * ey;
+            if (GRAD) {
+                // dL/dRe c_j = Re(conj(e) b_j) / B, dL/dIm c_j = Im(conj(b_j) e) / B
+#pragma unroll
+                for (int j = 0; j < kLearnTerms; ++j) {
+                    const float br = bas[2 * j], bi = bas[2 * j + 1];
+                    s_y[tid][2 * j] = fmaf(ex, br, ey * bi) * inv_b;
+                    s_y[tid][2 * j + 1] = fmaf(ey, br, -ex * bi) * inv_b;
+                }
+                s_y[tid][14] = s_y[tid][15] = 0.f;
+            }
+        }
+        __syncthreads();
+        if constexpr (GRAD) {
+            // dz2 = (dy W3^T) * silu'(z2)
+#pragma unroll
+            for (int st = 0; st < ST; ++st) {
+                f32x4 da = zero;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) da = mfma4(s_y[16 * st + r][4 * k + q4], w3t[k], da);
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    s_dz[16 * st + 4 * q4 + e][unit] = da[e] * d2[st][e];
+            }
+            __syncthreads();
+            // dz1 = (dz2 W2^T) * silu'(z1), kept until the reads of dz2 below are done
+            f32x4 da[ST];
+#pragma unroll
+            for (int st = 0; st < ST; ++st) da[st] = zero;
+#pragma unroll
+            for (int k = 0; k < kMlpH / 4; ++k)
+#pragma unroll
+                for (int st = 0; st < ST; ++st)
+                    da[st] = mfma4(s_dz[16 * st + r][4 * k + q4], w2t[k], da[st]);
+            // dW2 (rows a1 units, columns this wave's units), dW3 (rows this wave's units), biases
+#pragma unroll
+            for (int k = 0; k < kTrainTile / 4; ++k) {
+                const float bz = s_dz[4 * k + q4][unit];
+#pragma unroll
+                for (int t = 0; t < 4; ++t) g2[t] = mfma4(s_a1[4 * k + q4][16 * t + r], bz, g2[t]);
+                g3 = mfma4(s_a2[4 * k + q4][unit], s_y[4 * k + q4][r], g3);
+            }
+            if (tid < kMlpH) {
+#pragma unroll
+                for (int s = 0; s < kTrainTile; ++s) gb2 += s_dz[s][tid];
+            } else if (tid < kMlpH + kMlpOut) {
+#pragma unroll
+                for (int s = 0; s < kTrainTile; ++s) gb3 += s_y[s][tid - kMlpH];
+            }
+            __syncthreads();
+#pragma unroll
+            for (int st = 0; st < ST; ++st)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    s_dz[16 * st + 4 * q4 + e][unit] = da[st][e] * d1[st][e];
+            // dW1 and, in row 10, db1: this wave reads only the columns it wrote
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+            for (int k = 0; k < kTrainTile / 4; ++k)
+                g1 = mfma4(s_x[4 * k + q4][r], s_dz[4 * k + q4][unit], g1);
+        }
+        __syncthreads();  // the next tile overwrites the staged samples
+    }
+    if (tid < kTrainTile) s_sq[tid] = sq;
+    __syncthreads();
+    if (tid == 0 && loss_part) {
+        double s = 0.0;
+        for (int k = 0; k < kTrainTile; ++k) s += s_sq[k];
+        loss_part[blockIdx.x] = s;
+    }
+    if constexpr (GRAD) {
+        float* out = partials + (size_t)blockIdx.x * kMlpParams;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int row = 4 * q4 + e;
+            if (row < kMlpIn) out[kMlpOffW1 + row * kMlpH + unit] = g1[e];
+            if (row == kMlpIn) out[kMlpOffB1 + unit] = g1[e];
+            if (r < kMlpOut) out[kMlpOffW3 + (16 * w + row) * kMlpOut + r] = g3[e];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) out[kMlpOffW2 + (16 * t + row) * kMlpH + unit] = g2[t][e];
+        }
+        if (tid < kMlpH) out[kMlpOffB2 + tid] = gb2;
+        else if (tid < kMlpH + kMlpOut) out[kMlpOffB3 + tid - kMlpH] = gb3;
     }
 }
 
-// gradient partials: block (param group g, sample chunk c); each thread owns parameters and
-// sums row products over the chunk
-constexpr int kGradChunk = 1024;
-
-__device__ __forceinline__ void param_rows(int q, int& ra, int& rb) {
-    // returns the scratch rows whose product summed over samples is dL/dparam q (rb = -1: bias)
-    if (q < kMlpOffB1) { ra = kRowX + q / kMlpH; rb = kRowDZ1 + q % kMlpH; return; }
-    if (q < kMlpOffW2) { ra = -1; rb = kRowDZ1 + (q - kMlpOffB1); return; }
-    if (q < kMlpOffB2) { const int r = q - kMlpOffW2; ra = kRowA1 + r / kMlpH; rb = kRowDZ2 + r % kMlpH; return; }
-    if (q < kMlpOffW3) { ra = -1; rb = kRowDZ2 + (q - kMlpOffB2); return; }
-    if (q < kMlpOffB3) { const int r = q - kMlpOffW3; ra = kRowA2 + r / kMlpOut; rb = kRowDY + r % kMlpOut; return; }
-    ra = -1;
-    rb = kRowDY + (q - kMlpOffB3);
-}
-
-__global__ __launch_bounds__(kBlock) void k_mlp_wgrad(const float* __restrict__ S, uint32_t B,
-                                                      float* __restrict__ partials) {
-    const int q = blockIdx.x * kBlock + threadIdx.x;
-    const uint32_t c = blockIdx.y;
-    if (q >= kMlpParams) return;
-    int ra, rb;
-    param_rows(q, ra, rb);
-    const uint32_t s0 = c * kGradChunk, s1 = min(B, s0 + kGradChunk);
-    const float* pb = S + (size_t)rb * B;
-    float acc = 0.f;
-    if (ra < 0) {
-        for (uint32_t s = s0; s < s1; ++s) acc += pb[s];
-    } else {
-        const float* pa = S + (size_t)ra * B;
-        for (uint32_t s = s0; s < s1; ++s) acc = fmaf(pa[s], pb[s], acc);
-    }
-    partials[(size_t)c * kMlpParams + q] = acc;
-}
-
-// sum the chunk partials in order; optionally export the gradient; Adam update
-__global__ __launch_bounds__(kBlock) void k_mlp_adam(float* __restrict__ p,
+// Sum the block partials in order (kAdamGroups threads per parameter take every kAdamGroups-th
+// partial, several loads in flight, and their sums are added in order); optionally export the
+// gradient; Adam update. Latency bound: 128 partials of 5,774 parameters (3 MB).
+constexpr int kAdamGroups = 16;
+__global__ __launch_bounds__(64 * kAdamGroups) void k_mlp_adam(float* __restrict__ p,
                                                      const float* __restrict__ partials,
                                                      uint32_t nchunks, float* __restrict__ m1,
                                                      float* __restrict__ m2, float lr, float beta1,
                                                      float beta2, float eps, int step,
                                                      float* __restrict__ grad_out, int apply) {
-    const int q = blockIdx.x * kBlock + threadIdx.x;
-    if (q >= kMlpParams) return;
+    __shared__ float s_g[kAdamGroups][64];
+    const int lane = threadIdx.x & 63, grp = threadIdx.x >> 6;
+    const int q = blockIdx.x * 64 + lane;
+    float s = 0.f;
+    if (q < kMlpParams) {
+        constexpr uint32_t kUnroll = 8;
+        for (uint32_t c0 = grp; c0 < nchunks; c0 += kUnroll * kAdamGroups) {
+            float v[kUnroll];
+#pragma unroll
+            for (uint32_t u = 0; u < kUnroll; ++u) {
+                const uint32_t c = c0 + u * kAdamGroups;
+                v[u] = c < nchunks ? partials[(size_t)c * kMlpParams + q] : 0.f;
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < kUnroll; ++u) s += v[u];
+        }
+    }
+    s_g[grp][lane] = s;
+    __syncthreads();
+    if (grp != 0 || q >= kMlpParams) return;
     float g = 0.f;
-    for (uint32_t c = 0; c < nchunks; ++c) g += partials[(size_t)c * kMlpParams + q];
+#pragma unroll
+    for (int k = 0; k < kAdamGroups; ++k) g += s_g[k][lane];
     if (grad_out) grad_out[q] = g;
     if (!apply) return;
     const float a = m1[q] = beta1 * m1[q] + (1.f - beta1) * g;
@@ -639,21 +763,28 @@ void launch_mlp_infer_bf16(hipStream_t s, const float* X, uint32_t n, const MlpB
 void launch_mlp_forward_f32(hipStream_t s, const float* X, uint32_t n, const float* p, float* Y) {
     k_mlp_forward_f32<<<div_up_u(n, kBlock), kBlock, 0, s>>>(X, n, p, Y);
 }
-size_t mlp_scratch_floats(uint32_t B) { return (size_t)kScratchRows * B; }
-uint32_t mlp_grad_chunks(uint32_t B) { return div_up_u(B, kGradChunk); }
-uint32_t mlp_loss_blocks(uint32_t B) { return div_up_u(B, kBlock); }
+uint32_t mlp_grad_chunks(uint32_t B) {
+    const uint32_t g = div_up_u(B, kTrainTile);
+    return g < kTrainBlocks ? g : kTrainBlocks;
+}
+uint32_t mlp_loss_blocks(uint32_t B) {
+    const uint32_t g = div_up_u(B, kTrainTile);
+    return g < 4 * kTrainBlocks ? g : 4 * kTrainBlocks;
+}
 void launch_mlp_grad(hipStream_t s, const float* X, const float* T, const uint32_t* order,
-                     uint32_t B, const float* p, float* S, double* loss_part, float* partials,
-                     int terms) {
-    k_mlp_fwdbwd<<<div_up_u(B, kBlock), kBlock, 0, s>>>(X, T, order, B, p, S, loss_part, terms);
-    dim3 g(div_up_u(kMlpParams, kBlock), mlp_grad_chunks(B));
-    k_mlp_wgrad<<<g, kBlock, 0, s>>>(S, B, partials);
+                     uint32_t B, const float* p, double* loss_part, float* partials, int terms) {
+    k_mlp_train<true><<<mlp_grad_chunks(B), kBlock, 0, s>>>(X, T, order, B, p, loss_part,
+                                                            partials, terms);
+}
+void launch_mlp_loss(hipStream_t s, const float* X, const float* T, uint32_t B, const float* p,
+                     double* loss_part, int terms) {
+    k_mlp_train<false><<<mlp_loss_blocks(B), kBlock, 0, s>>>(X, T, nullptr, B, p, loss_part,
+                                                             nullptr, terms);
 }
 void launch_mlp_adam(hipStream_t s, float* p, const float* partials, uint32_t nchunks, float* m1,
                      float* m2, float lr, int step, float* grad_out, int apply) {
-    k_mlp_adam<<<div_up_u(kMlpParams, kBlock), kBlock, 0, s>>>(p, partials, nchunks, m1, m2, lr,
-                                                               0.9f, 0.999f, 1e-8f, step, grad_out,
-                                                               apply);
+    k_mlp_adam<<<div_up_u(kMlpParams, 64), 64 * kAdamGroups, 0, s>>>(
+        p, partials, nchunks, m1, m2, lr, 0.9f, 0.999f, 1e-8f, step, grad_out, apply);
 }
 void launch_mlp_adam_grad(hipStream_t s, float* p, const float* g, float* m1, float* m2, float lr,
                           int step) {
