@@ -108,7 +108,6 @@ struct bh_ctx {
     double* tz = nullptr;
     double* kl_part = nullptr;
     double* kl_out = nullptr;
-    uint32_t* iota_dev = nullptr;
 
     bool learned = false;  // second moments in builds, learned correction available
     float* lfeat = nullptr;   // cell features of the last build (kMlpIn per node)
@@ -619,10 +618,8 @@ static bh_status create_impl(bh_ctx** out, const bh_config* cfg, uint32_t extra_
         TRY(hip_check(c, hipEventCreateWithFlags(&c->ev_att, hipEventDisableTiming),
                       "hipEventCreate"));
         TRY(dalloc(c, &c->tz, 2));
-        TRY(dalloc(c, &c->kl_part, kMaxReduceBlocks));
+        TRY(dalloc(c, &c->kl_part, std::max(kMaxReduceBlocks, tsne_z_blocks(N))));
         TRY(dalloc(c, &c->kl_out, 2));
-        TRY(dalloc(c, &c->iota_dev, N));
-        launch_iota(c->stream, c->iota_dev, N);
     }
     if (!c->wide) {
         TRY(dalloc(c, &c->slot_a, c->slot_cap));
@@ -1361,33 +1358,9 @@ bh_status bh_tsne_kl(bh_ctx* c, double* kl, double* z_exact) {
     if (st == BH_OK) st = tsne_stage_build(c);
     if (st != BH_OK) return st;
     const uint32_t n = c->p_n;
-    // exact Z: FP64 direct sum over all sinks (their totals), then the KL sum over P
-    const uint32_t S = direct_splits(n, n);
-    const uint64_t need_s = 2ull * n, need_p = (uint64_t)(3ull * S + 3ull) * n;
-    if (need_s > c->dsink_cap) {
-        if (c->dsinks) (void)hipFree(c->dsinks);
-        c->dsinks = nullptr;
-        c->dsink_cap = 0;
-        st = hip_check(c, hipMalloc((void**)&c->dsinks, need_s * 4), "hipMalloc sinks");
-        if (st != BH_OK) return st;
-        c->dsink_cap = need_s;
-    }
-    if (need_p > c->dpart_cap) {
-        if (c->dpart) (void)hipFree(c->dpart);
-        c->dpart = nullptr;
-        c->dpart_cap = 0;
-        st = hip_check(c, hipMalloc((void**)&c->dpart, need_p * 8), "hipMalloc partials");
-        if (st != BH_OK) return st;
-        c->dpart_cap = need_p;
-    }
+    // exact Z over all pairs (FP64), then the KL sum over P
     hipStream_t s = c->stream;
-    st = hip_check(c, hipMemcpyAsync(c->dsinks, c->iota_dev, (size_t)n * 4, hipMemcpyDeviceToDevice, s),
-                   "sinks");
-    if (st != BH_OK) return st;
-    double* out = c->dpart + (uint64_t)3 * S * n;
-    launch_direct_f64(s, kKernelTsne, c->pos4, c->id[c->cur], n, c->dsinks, n, 1.0, 0.0, c->where,
-                      c->dsinks + n, c->dpart, S, out, out + n, out + 2ull * n);
-    launch_sum_f64(s, out + 2ull * n, n, c->tz);
+    launch_tsne_z(s, c->pos4, n, c->kl_part, c->tz);
     launch_tsne_kl(s, c->p_row, c->p_col, c->p_val, n, c->ty_x[c->ty_cur], c->ty_y[c->ty_cur],
                    c->tz, c->kl_part, c->kl_out);
     st = launch_status(c, "KL");

@@ -191,7 +191,9 @@ uint32_t tsne_kl_blocks(uint32_t n);
 void launch_tsne_kl(hipStream_t s, const uint32_t* row_ptr, const uint32_t* col, const float* val,
                     uint32_t n, const float* yx, const float* yy, const double* z,
                     double* partials, double* out);
-void launch_sum_f64(hipStream_t s, const double* v, uint32_t nv, double* out);
+// exact Z of n unit-mass points: tsne_z_blocks(n) partials, summed into z
+uint32_t tsne_z_blocks(uint32_t n);
+void launch_tsne_z(hipStream_t s, const float4* pos4, uint32_t n, double* partials, double* z);
 
 // learned far-field correction (bh_mlp.hip)
 struct MlpBf16;

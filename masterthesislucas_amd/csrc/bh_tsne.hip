@@ -93,6 +93,86 @@ __global__ __launch_bounds__(kBlock) void k_tsne_combine(uint32_t n, const float
     }
 }
 
+// ------------------------------------------------------------------------------------------
+// Exact Z of an embedding (unit masses): sum over ordered pairs of 1 / (1 + |y_i - y_j|^2), FP64.
+// Every unordered pair of tiles of kZTile points is one item of work, counted twice (a diagonal
+// tile once); within it a thread holds two rows and runs over the columns in LDS. The two terms
+// of a column share one reciprocal, 1/a + 1/b = (a + b) / (a b): a and b are at least 1 and at
+// most 1e78 for FP32 positions, so the product neither under- nor overflows. The reciprocal
+// estimate (relative error 4.6e-8) takes two Newton steps, which leave rounding only. Diagonal
+// tiles and the ragged last one take each term by itself, masked.
+// FP64 VALU bound: 15 full-rate FP64 operations and one estimate per two pairs, each pair once.
+// 70,000 points: the whole cost call 5.48 -> 1.00 ms.
+// Before: every ordered pair with an IEEE division, through per-sink sums of forces too.
+// ------------------------------------------------------------------------------------------
+constexpr int kZTile = 256;
+constexpr int kZThreads = kZTile / 2;
+constexpr uint32_t kZMaxBlocks = 4096;
+
+__device__ __forceinline__ double rcp_newton2(double v) {
+    double r = __builtin_amdgcn_rcp(v);
+    r = fma(r, fma(-v, r, 1.0), r);
+    return fma(r, fma(-v, r, 1.0), r);
+}
+
+__global__ __launch_bounds__(kZThreads) void k_tsne_z(const float4* __restrict__ pos4, uint32_t n,
+                                                      double* __restrict__ partials) {
+    __shared__ double2 s_q[kZTile];
+    __shared__ double red[kZThreads / kWave];
+    const int tid = threadIdx.x;
+    const uint64_t nt = (n + kZTile - 1) / kZTile, items = nt * (nt + 1) / 2;
+    double acc = 0.0;
+    for (uint64_t it = blockIdx.x; it < items; it += gridDim.x) {
+        // item -> (I, J), I <= J: column J starts at item J (J + 1) / 2
+        uint64_t J = (uint64_t)((sqrt(8.0 * (double)it + 1.0) - 1.0) * 0.5);
+        while (J * (J + 1) / 2 > it) --J;
+        while ((J + 1) * (J + 2) / 2 <= it) ++J;
+        const uint64_t I = it - J * (J + 1) / 2;
+        const uint32_t i0 = (uint32_t)I * kZTile + tid, i1 = i0 + kZThreads;
+        const uint32_t j0 = (uint32_t)J * kZTile;
+        __syncthreads();  // the previous item's columns are read
+        for (int c = tid; c < kZTile; c += kZThreads) {
+            const float4 q = pos4[min(j0 + c, n - 1)];
+            s_q[c] = make_double2(q.x, q.y);
+        }
+        const float4 f0 = pos4[min(i0, n - 1)], f1 = pos4[min(i1, n - 1)];
+        const double x0 = f0.x, y0 = f0.y, x1 = f1.x, y1 = f1.y;
+        __syncthreads();
+        double s = 0.0;
+        if (I != J && j0 + kZTile <= n) {  // block-uniform
+#pragma unroll 4
+            for (int c = 0; c < kZTile; ++c) {
+                const double2 q = s_q[c];
+                const double dx0 = q.x - x0, dy0 = q.y - y0, dx1 = q.x - x1, dy1 = q.y - y1;
+                const double a = fma(dx0, dx0, fma(dy0, dy0, 1.0));
+                const double b = fma(dx1, dx1, fma(dy1, dy1, 1.0));
+                s = fma(a + b, rcp_newton2(a * b), s);
+            }
+            s *= 2.0;
+        } else {
+            const uint32_t cols = min((uint32_t)kZTile, n - j0);
+            for (uint32_t c = 0; c < cols; ++c) {
+                const double2 q = s_q[c];
+                const double dx0 = q.x - x0, dy0 = q.y - y0, dx1 = q.x - x1, dy1 = q.y - y1;
+                const double a = fma(dx0, dx0, fma(dy0, dy0, 1.0));
+                const double b = fma(dx1, dx1, fma(dy1, dy1, 1.0));
+                if (i0 < n && j0 + c != i0) s += rcp_newton2(a);
+                if (i1 < n && j0 + c != i1) s += rcp_newton2(b);
+            }
+            if (I != J) s *= 2.0;
+        }
+        acc += s;
+    }
+    acc = wave_sum_d(acc);
+    if ((tid & 63) == 0) red[tid >> 6] = acc;
+    __syncthreads();
+    if (tid == 0) {
+        double b = 0.0;
+        for (int k = 0; k < kZThreads / kWave; ++k) b += red[k];
+        partials[blockIdx.x] = b;
+    }
+}
+
 // KL divergence sum_{i != j} P_ij log2(P_ij / Q_ij), Q_ij = w_ij / Z, in FP64
 // (costFunction, tsne.h:383-460); block partials, summed in order by k_tsne_kl_final.
 __global__ __launch_bounds__(kBlock) void k_tsne_kl(const uint32_t* __restrict__ row_ptr,
@@ -112,9 +192,8 @@ __global__ __launch_bounds__(kBlock) void k_tsne_kl(const uint32_t* __restrict__
             const uint32_t c = col[e];
             if (c == r) continue;
             const double ddx = (double)yx[c] - xi, ddy = (double)yy[c] - yi;
-            const double q = (1.0 / (1.0 + (ddx * ddx + ddy * ddy))) / Z;
-            const double p = val[e];
-            acc += p * log2(p / q);
+            const double p = val[e];  // P / Q = P Z (1 + |y_i - y_j|^2)
+            acc += p * log2(p * Z * (1.0 + (ddx * ddx + ddy * ddy)));
         }
     }
     acc = wave_sum_d(acc);
@@ -179,8 +258,15 @@ void launch_tsne_kl(hipStream_t s, const uint32_t* row_ptr, const uint32_t* col,
     k_sum_f64<<<1, kBlock, 0, s>>>(partials, g, out);
 }
 
-void launch_sum_f64(hipStream_t s, const double* v, uint32_t nv, double* out) {
-    k_sum_f64<<<1, kBlock, 0, s>>>(v, nv, out);
+uint32_t tsne_z_blocks(uint32_t n) {
+    const uint64_t nt = div_up(n, kZTile), items = nt * (nt + 1) / 2;
+    return items < kZMaxBlocks ? (uint32_t)items : kZMaxBlocks;
+}
+
+void launch_tsne_z(hipStream_t s, const float4* pos4, uint32_t n, double* partials, double* z) {
+    const uint32_t g = tsne_z_blocks(n);
+    k_tsne_z<<<g, kZThreads, 0, s>>>(pos4, n, partials);
+    k_sum_f64<<<1, kBlock, 0, s>>>(partials, g, z);
 }
 
 }  // namespace bh

@@ -42,3 +42,35 @@ def test_training_gradient_edges(gpu, n, terms):
     net.set_dataset(X, T)
     assert abs(net.train(0) - ref_loss) < 1e-5 * ref_loss
     net.close()
+
+
+@pytest.mark.parametrize("n", [2, 3, 255, 256, 257, 513, 1500])
+def test_exact_z_edges(gpu, n):
+    """Z over tiles of 256 x 256 pairs: less than a tile, exact tiles, ragged last tiles, with
+    coincident and far points; Z and KL to 1e-12 (each of the n^2 FP64 terms carries a few units
+    of 1e-16)."""
+    rng = np.random.default_rng(n)
+    y = rng.normal(0, 3, (n, 2)).astype(np.float32)
+    y[-1] = y[0]
+    if n > 2:
+        y[1] = (3e4, -2e4)
+    rows = np.repeat(np.arange(n), min(n - 1, 4))
+    cols = (rows + 1 + np.tile(np.arange(min(n - 1, 4)), n)) % n
+    o = np.lexsort((cols, rows))
+    rows, cols = rows[o], cols[o]
+    val = rng.uniform(0.1, 1.0, rows.size)
+    val = (val / val.sum()).astype(np.float32)
+    rp = np.zeros(n + 1, np.uint32)
+    rp[1:] = np.cumsum(np.bincount(rows, minlength=n))
+    t = tsne.TSNE(rp, cols.astype(np.uint32), val, (y[:, 0].copy(), y[:, 1].copy()))
+    kl, z = t.costFunction()
+    t.close()
+    d = y.astype(np.float64)
+    d2 = ((d[:, None, :] - d[None, :, :]) ** 2).sum(2)
+    w = 1.0 / (1.0 + d2)
+    np.fill_diagonal(w, 0.0)
+    want_z = w.sum()
+    p = val.astype(np.float64)
+    want_kl = (p * np.log2(p * want_z * (1.0 + d2[rows, cols]))).sum()
+    assert abs(z - want_z) <= 1e-12 * want_z
+    assert abs(kl - want_kl) <= 1e-12 * np.abs(p * np.log2(p * want_z)).sum()
