@@ -27,12 +27,14 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 __host__ __device__ static inline uint32_t div_up_a(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 
-constexpr int kAffCols = 64;                  // candidate columns per tile
-constexpr int kAffKC = 128;                   // K halfs per staged chunk
-constexpr int kAffPad = 8;                    // LDS row padding (conflict-free 16-byte reads)
-constexpr uint32_t kAffCap = 256;             // candidate slots per row
-constexpr uint32_t kAffKeep = kAffCap - kAffCols;  // compact above this many (a tile adds <= 64)
-constexpr int kAffMaxDimPad = 1024;           // dim <= 1024 (8 chunks of operands in registers)
+constexpr int kAffRows = 128;                 // query rows per workgroup
+constexpr int kAffCols = 256;                 // candidate columns per tile
+constexpr int kAffKC = 64;                    // K halfs per staged chunk
+constexpr int kAffPad = 8;                    // LDS row padding (bank spread of 16-byte reads)
+constexpr uint32_t kAffCap = 512;             // candidate slots per row and column range
+constexpr uint32_t kAffHold = kAffCap - kAffCols;  // compact above this many (a tile adds <= 256)
+constexpr uint32_t kAffKeep = 192;            // most candidates of a row over all columns
+constexpr uint32_t kAffMaxSplits = 4;         // most column ranges
 
 // ---------------------------------------------------------------------------------------------
 // scaled FP16 copy, squared norms and rounding bounds (one wave per point)
@@ -65,250 +67,396 @@ __global__ __launch_bounds__(kBlock) void k_aff_pack(const float* __restrict__ X
 }
 
 // ---------------------------------------------------------------------------------------------
-// candidates: a workgroup owns 64 query rows (their FP16 block resident in LDS) and streams all
-// columns in tiles of 64; per tile each wave computes a 16 x 64 block of Gram products
+// candidates: a workgroup owns kAffRows query rows and streams the columns of its range in tiles
+// of kAffCols; the range is all columns, or one of `splits` equal ranges where the row blocks
+// alone leave compute units idle (k_aff_refine merges a row's lists)
 // ---------------------------------------------------------------------------------------------
-// compact row r's candidate buffer (one wave): T = min(T, k-th smallest upper bound), keep the
-// entries whose lower bound is at most T, in order
-__device__ __forceinline__ void aff_compact(uint32_t* __restrict__ cj, float* __restrict__ clo,
-                                            float* __restrict__ chi, uint32_t* cnt, float* T,
-                                            uint32_t* over, uint32_t k) {
+// one wave, PER entries per lane: a bit pattern t with #(hb <= t among valid) >= k, found in at
+// most `steps` halvings of the range of the entries; 32 steps give the smallest one (upper bounds
+// are >= 0, so their bits order them). At least k entries are valid.
+template <int PER>
+__device__ __forceinline__ uint32_t aff_kth(const uint32_t (&hb)[PER], const bool (&v)[PER],
+                                            uint32_t k, int steps) {
+    uint32_t a = 0xFFFFFFFFu, b = 0u;
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        a = min(a, v[u] ? hb[u] : 0xFFFFFFFFu);
+        b = max(b, v[u] ? hb[u] : 0u);
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        a = min(a, (uint32_t)__shfl_xor((int)a, o, kWave));
+        b = max(b, (uint32_t)__shfl_xor((int)b, o, kWave));
+    }
+    a = (uint32_t)__builtin_amdgcn_readfirstlane((int)a);
+    b = (uint32_t)__builtin_amdgcn_readfirstlane((int)b);
+    for (int it = 0; it < steps && a < b; ++it) {
+        const uint32_t mid = a + ((b - a) >> 1);
+        uint32_t m = 0;
+#pragma unroll
+        for (int u = 0; u < PER; ++u) m += (uint32_t)__popcll(__ballot(v[u] && hb[u] <= mid));
+        if (m >= k) b = mid; else a = mid + 1;
+    }
+    return b;
+}
+
+// Bounds [lo, hi] of the exact distance of a pair from its Gram value g (header comment):
+// ni, ai, ei and nj, aj, ej are |x^|^2, |x^| (rounded up) and the rounding bound of its points.
+__device__ __forceinline__ void aff_bounds(float g, float kdelta, float ni, float ai, float ei,
+                                           float nj, float aj, float ej, float& lo, float& hi) {
+    const float sn = ni + nj, d = sn - 2.0f * g;
+    const float delta = (kdelta * ai * aj + 0x1p-22f * sn) * (1.0f + 0x1p-20f);
+    const float e2 = (ei + ej) * (1.0f + 0x1p-20f);
+    lo = sqrtf(fmaxf(d - delta, 0.f)) * (1.0f - 0x1p-20f) - e2;
+    lo -= fabsf(lo) * 0x1p-22f;
+    hi = (sqrtf(fmaxf(d + delta, 0.f)) * (1.0f + 0x1p-20f) + e2) * (1.0f + 0x1p-22f);
+}
+
+// Per point |x^|^2, |x^| and the rounding bound (k_aff_pack)
+struct AffPoints {
+    const float *nh, *ah, *eb;
+};
+__device__ __forceinline__ float aff_kdelta(uint32_t dp) { return 0x1p-24f * (float)(2 * dp + 4); }
+
+// Compact row i's candidate list (one wave), its entries (column, Gram value) already in `en`:
+// T = min(T, about the k-th smallest upper bound), keep the entries whose lower bound is at most
+// T, in order. T comes from ten halvings (a wave needs no more to thin the list); a window that
+// does not fit is settled with the exact k-th.
+constexpr int kAffPer = kAffCap / kWave;
+__device__ __forceinline__ void aff_load(const uint2* __restrict__ list, uint32_t c, uint32_t i,
+                                         uint2 (&en)[kAffPer]) {
+#pragma unroll
+    for (int u = 0; u < kAffPer; ++u) {
+        const uint32_t q = (threadIdx.x & 63) + 64u * u;
+        en[u] = q < c ? list[q] : make_uint2(i, 0u);
+    }
+}
+__device__ __forceinline__ void aff_compact(uint2* __restrict__ list, AffPoints P, uint32_t dp,
+                                            uint32_t i, const uint2 (&en)[kAffPer], uint32_t* cnt,
+                                            float* T, uint32_t* over, uint32_t k) {
     const int lane = threadIdx.x & 63;
     const uint32_t c = *cnt;
-    uint32_t j[4];
-    float lo[4];
-    uint32_t hb[4];
-    bool v[4];
+    const float kd = aff_kdelta(dp), ni = P.nh[i], ai = P.ah[i], ei = P.eb[i];
+    uint32_t hb[kAffPer];
+    float lo[kAffPer];
+    bool v[kAffPer];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        const uint32_t q = lane + 64u * u;
-        v[u] = q < c;
-        j[u] = v[u] ? cj[q] : 0u;
-        lo[u] = v[u] ? clo[q] : 0.f;
-        hb[u] = v[u] ? __float_as_uint(chi[q]) : 0u;  // upper bounds are >= 0: bits order them
+    for (int u = 0; u < kAffPer; ++u) {
+        v[u] = lane + 64u * u < c;
+        float hi;
+        aff_bounds(__uint_as_float(en[u].y), kd, ni, ai, ei, P.nh[en[u].x], P.ah[en[u].x],
+                   P.eb[en[u].x], lo[u], hi);
+        hb[u] = __float_as_uint(hi);
     }
-    float t = *T;
-    if (c >= k) {
-        uint32_t a = 0u, b = 0x7F800000u;  // smallest pattern with #(hi <= pattern) >= k
-        while (a < b) {
-            const uint32_t mid = a + ((b - a) >> 1);
-            uint32_t m = 0;
-#pragma unroll
-            for (int u = 0; u < 4; ++u) m += (uint32_t)__popcll(__ballot(v[u] && hb[u] <= mid));
-            if (m >= k) b = mid; else a = mid + 1;
-        }
-        t = fminf(t, __uint_as_float(a));
-    }
+    const float t0 = *T;
+    float t = t0;
     uint32_t base = 0;
-    uint32_t pos[4];
-    bool keep[4];
+    uint64_t keep[kAffPer];
+    for (int steps = 10;; steps = 32) {
+        if (c >= k) t = fminf(t0, __uint_as_float(aff_kth<kAffPer>(hb, v, k, steps)));
+        base = 0;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-        keep[u] = v[u] && lo[u] <= t;
-        const uint64_t bm = __ballot(keep[u]);
-        pos[u] = base + (uint32_t)__popcll(bm & lane_mask_lt());
-        base += (uint32_t)__popcll(bm);
-    }
-    __builtin_amdgcn_wave_barrier();
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-        if (keep[u] && pos[u] < kAffKeep) {
-            cj[pos[u]] = j[u];
-            clo[pos[u]] = lo[u];
-            chi[pos[u]] = __uint_as_float(hb[u]);
+        for (int u = 0; u < kAffPer; ++u) {
+            keep[u] = __ballot(v[u] && lo[u] <= t);
+            base += (uint32_t)__popcll(keep[u]);
         }
-    __builtin_amdgcn_wave_barrier();
+        if (base <= kAffHold || steps == 32) break;
+    }
+    uint32_t at = 0;
+#pragma unroll
+    for (int u = 0; u < kAffPer; ++u) {
+        const uint32_t pos = at + (uint32_t)__popcll(keep[u] & lane_mask_lt());
+        if (((keep[u] >> lane) & 1ull) && pos < kAffHold) list[pos] = en[u];
+        at += (uint32_t)__popcll(keep[u]);
+    }
     if (lane == 0) {
         *T = t;
-        if (base > kAffKeep) *over = 1u;  // the window outgrew the buffer: reported, not used
-        *cnt = min(base, kAffKeep);
+        if (base > kAffHold) *over = 1u;  // the window outgrew the buffer: reported, not used
+        *cnt = min(base, kAffHold);
     }
 }
 
-// Workgroup: kAffWaves waves, 16 query rows each, whose FP16 operands for the whole K stay in
-// registers (NCH chunks of 128 halfs: 16 NCH VGPRs); the columns stream through LDS in tiles of
-// 64 x 128 halfs, double-buffered: the next chunk's global loads are in flight while the
-// current one feeds the MFMAs.
-constexpr int kAffWaves = 8;
-constexpr int kAffThreads = kAffWaves * kWave;
-constexpr int kAffRowsWG = 16 * kAffWaves;
-constexpr int kAffChunkLoads = kAffCols * (kAffKC / 8) / kAffThreads;  // 16-byte loads per thread
-static_assert(kAffChunkLoads * kAffThreads == kAffCols * (kAffKC / 8), "chunk loads");
+// lane 0 of each row of 16 lanes to the whole row (DPP row_newbcast:0)
+__device__ __forceinline__ uint32_t row_first(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x150, 0xF, 0xF, false);
+}
 
-template <int NCH>
+// Workgroup: 8 waves as 2 x 4 over a 128 x 256 tile of Gram products, 64 x 64 per wave (16
+// v_mfma_f32_16x16x32_f16 tiles from 4 + 4 operand reads per K step of 32). Rows and columns
+// stream through LDS in chunks of 64 halfs, double-buffered: the next chunk's global loads are
+// in flight while the current one feeds the MFMAs. Bound by the matrix cores and the LDS reads
+// that feed them (8 reads of 1 KB per 16 MFMAs; the earlier 16 x 64 tile per wave read LDS once
+// per MFMA and left the matrix cores three quarters idle). The epilogue tests a pair against the
+// row's threshold without square roots, conservatively (a few percent of the pairs pass, so in
+// nearly every wave some lane does), and appends (column, Gram value); the bounds themselves are
+// taken when a row's list is compacted, 64 entries at a time. One LDS atomic per row and 64
+// columns reserves its slots. 20,000 points in 784-D: 4.68 -> 2.45 ms.
+constexpr int kAffThreads = 512;
+constexpr int kAffLd = kAffKC + kAffPad;
+constexpr int kAffLoads = (kAffRows + kAffCols) * (kAffKC / 8) / kAffThreads;  // 16 B per thread
+static_assert(kAffLoads * kAffThreads == (kAffRows + kAffCols) * (kAffKC / 8), "chunk loads");
+
 __global__ __launch_bounds__(kAffThreads) void k_aff_candidates(const _Float16* __restrict__ Xh,
                                                                 const float* __restrict__ nh,
                                                                 const float* __restrict__ ah,
                                                                 const float* __restrict__ eb,
-                                                                uint32_t n, uint32_t k,
-                                                                uint32_t* __restrict__ cj,
-                                                                float* __restrict__ clo,
-                                                                float* __restrict__ chi,
+                                                                uint32_t n, uint32_t dp,
+                                                                uint32_t k,
+                                                                uint2* __restrict__ cand,
                                                                 uint32_t* __restrict__ ccount,
                                                                 uint32_t* __restrict__ overflow) {
-    constexpr uint32_t dp = NCH * kAffKC;
-    constexpr uint32_t ldb = kAffKC + kAffPad;
-    __shared__ __attribute__((aligned(16))) _Float16 Bs[2][kAffCols * ldb];
-    __shared__ uint32_t s_cnt[kAffRowsWG], s_over[kAffRowsWG];
-    __shared__ float s_T[kAffRowsWG], s_nh[kAffRowsWG], s_ah[kAffRowsWG], s_eb[kAffRowsWG];
+    __shared__ __attribute__((aligned(16))) _Float16 s_t[2][(kAffRows + kAffCols) * kAffLd];
+    __shared__ uint32_t s_cnt[kAffRows], s_over[kAffRows];
+    __shared__ float s_T[kAffRows], s_nh[kAffRows], s_ka[kAffRows], s_eb[kAffRows];
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wr = w >> 2, wc = w & 3;
     const int r16 = lane & 15, q4 = lane >> 4;
-    const uint32_t row0 = blockIdx.x * kAffRowsWG;
-    // this lane's A operands: row 16 w + r16, k = 32 s + 8 q4 .. + 7 for every step s
-    half8 A[NCH * (kAffKC / 32)];
-    {
-        const uint32_t ar = row0 + 16 * w + r16;
-#pragma unroll
-        for (int s = 0; s < NCH * (kAffKC / 32); ++s)
-            A[s] = ar < n ? *(const half8*)(Xh + (size_t)ar * dp + 32 * s + 8 * q4) : half8{};
-    }
-    if (tid < kAffRowsWG) {
+    const uint32_t row0 = blockIdx.x * kAffRows;
+    const uint32_t ntiles = div_up_a(n, kAffCols);
+    const uint32_t t0 = (uint32_t)((uint64_t)ntiles * blockIdx.y / gridDim.y);
+    const uint32_t t1 = (uint32_t)((uint64_t)ntiles * (blockIdx.y + 1) / gridDim.y);
+    const size_t lists = (size_t)blockIdx.y * n;  // this column range's lists: row i at lists + i
+    const AffPoints P{nh, ah, eb};
+    // the test's factors: delta's and the threshold's a little larger than aff_bounds takes them
+    constexpr float kUp = 1.0f + 0x1p-17f;
+    if (tid < kAffRows) {
         const uint32_t i = row0 + tid;
         s_cnt[tid] = 0u;
         s_over[tid] = 0u;
         s_T[tid] = __uint_as_float(0x7F800000u);
         s_nh[tid] = i < n ? nh[i] : 0.f;
-        s_ah[tid] = i < n ? ah[i] : 0.f;
-        s_eb[tid] = i < n ? eb[i] : 0.f;
+        s_ka[tid] = i < n ? aff_kdelta(dp) * ah[i] * kUp : 0.f;
+        s_eb[tid] = i < n ? eb[i] * kUp : 0.f;
     }
-    const float kdelta = 0x1p-24f * (float)(2 * dp + 4);
-    const uint32_t ntiles = div_up_a(n, kAffCols);
-    const uint32_t nchunks = ntiles * NCH;  // (tile, chunk) in order
-    // chunk c = (tile c / NCH, K chunk c % NCH): 64 columns x 16 loads of 16 bytes
-    half8 pre[kAffChunkLoads];
-    auto fetch = [&](uint32_t c) {
-        const uint32_t c0 = (c / NCH) * kAffCols, ch = c % NCH;
+    const uint32_t nch = dp / kAffKC, nchunks = (t1 - t0) * nch;  // (tile, K chunk) in order
+    half8 pre[kAffLoads];
+    auto fetch = [&](uint32_t tile, uint32_t ch) {
 #pragma unroll
-        for (int u = 0; u < kAffChunkLoads; ++u) {
+        for (int u = 0; u < kAffLoads; ++u) {
             const int e = tid + u * kAffThreads;
-            const int col = e >> 4, q = e & 15;
-            pre[u] = c0 + col < n
-                         ? *(const half8*)(Xh + (size_t)(c0 + col) * dp + ch * kAffKC + q * 8)
-                         : half8{};
+            const int q = e & (kAffKC / 8 - 1), rc = e / (kAffKC / 8);
+            const uint32_t g = rc < kAffRows ? row0 + rc : tile * kAffCols + (rc - kAffRows);
+            pre[u] = g < n ? *(const half8*)(Xh + (size_t)g * dp + ch * kAffKC + q * 8) : half8{};
         }
     };
     auto stage = [&](int buf) {
 #pragma unroll
-        for (int u = 0; u < kAffChunkLoads; ++u) {
+        for (int u = 0; u < kAffLoads; ++u) {
             const int e = tid + u * kAffThreads;
-            *(half8*)(&Bs[buf][(e >> 4) * ldb + (e & 15) * 8]) = pre[u];
+            const int q = e & (kAffKC / 8 - 1), rc = e / (kAffKC / 8);
+            *(half8*)(&s_t[buf][rc * kAffLd + q * 8]) = pre[u];
         }
     };
-    fetch(0);
-    stage(0);
+    if (nchunks) {
+        fetch(t0, 0);
+        stage(0);
+    }
     __syncthreads();
-    f32x4 acc[4];
-    for (uint32_t t = 0; t < ntiles; ++t) {
+    uint32_t c = 0;
+    for (uint32_t t = t0; t < t1; ++t) {
+        // the epilogue's column constants, in flight during the products
+        const uint32_t c0 = t * kAffCols;
+        float nj[4], aj[4], ej[4];
+        bool jv[4];
 #pragma unroll
-        for (int cb = 0; cb < 4; ++cb) acc[cb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int b = 0; b < 4; ++b) {
+            const uint32_t j = c0 + 64 * wc + 16 * b + r16;
+            jv[b] = j < n;
+            nj[b] = jv[b] ? nh[j] : 0.f;
+            aj[b] = jv[b] ? ah[j] : 0.f;
+            ej[b] = jv[b] ? eb[j] * kUp : 0.f;
+        }
+        f32x4 acc[4][4];
 #pragma unroll
-        for (int ch = 0; ch < NCH; ++ch) {
-            const uint32_t c = t * NCH + ch;
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+            for (int b = 0; b < 4; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (uint32_t ch = 0; ch < nch; ++ch, ++c) {
             const int buf = c & 1;
-            if (c + 1 < nchunks) fetch(c + 1);  // in flight during the MFMAs below
+            const bool more = c + 1 < nchunks;
+            if (more) fetch(ch + 1 < nch ? t : t + 1, ch + 1 < nch ? ch + 1 : 0);
+            const _Float16* A = &s_t[buf][(64 * wr + r16) * kAffLd + 8 * q4];
+            const _Float16* Bp = &s_t[buf][(kAffRows + 64 * wc + r16) * kAffLd + 8 * q4];
 #pragma unroll
             for (int s = 0; s < kAffKC / 32; ++s) {
-                const half8 a = A[ch * (kAffKC / 32) + s];
+                half8 av[4], bv[4];
 #pragma unroll
-                for (int cb = 0; cb < 4; ++cb) {
-                    const half8 b =
-                        *(const half8*)(&Bs[buf][(16 * cb + r16) * ldb + s * 32 + 8 * q4]);
-                    acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, acc[cb], 0, 0, 0);
-                }
+                for (int a = 0; a < 4; ++a) av[a] = *(const half8*)(A + 16 * a * kAffLd + 32 * s);
+#pragma unroll
+                for (int b = 0; b < 4; ++b) bv[b] = *(const half8*)(Bp + 16 * b * kAffLd + 32 * s);
+#pragma unroll
+                for (int a = 0; a < 4; ++a)
+#pragma unroll
+                    for (int b = 0; b < 4; ++b)
+                        acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(av[a], bv[b], acc[a][b],
+                                                                           0, 0, 0);
             }
             // the other buffer was last read in the previous chunk, before its barrier
-            if (c + 1 < nchunks) stage(buf ^ 1);
+            if (more) stage(buf ^ 1);
             __syncthreads();
         }
-        // tile done: acc[cb][e] = x^_i . x^_j, i = row0 + 16 w + 4 q4 + e, j = c0 + 16 cb + r16
-        const uint32_t c0 = t * kAffCols;
+        // acc[a][b][e] = x^_i . x^_j, i = row0 + 64 wr + 16 a + 4 q4 + e, j = c0 + 64 wc + 16 b + r16
+        // tiles off the diagonal and inside both ranges need no per-pair checks
+        const bool edge = (c0 < row0 + kAffRows && row0 < c0 + kAffCols) || c0 + kAffCols > n ||
+                          row0 + kAffRows > n;
 #pragma unroll
-        for (int cb = 0; cb < 4; ++cb) {
-            const uint32_t j = c0 + 16 * cb + r16;
-            const bool jv = j < n;
-            const float nj = jv ? nh[j] : 0.f, aj = jv ? ah[j] : 0.f, ej = jv ? eb[j] : 0.f;
+        for (int a = 0; a < 4; ++a) {
+            uint32_t hits[4][4], base[4];  // hits: the row's 16 lanes' ballot, per row e and block b
+            uint32_t any = 0;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int il = 16 * w + 4 * q4 + e;
-                const uint32_t i = row0 + il;
-                const float sn = s_nh[il] + nj;
-                const float d = sn - 2.0f * acc[cb][e];
-                const float delta = (kdelta * s_ah[il] * aj + 0x1p-22f * sn) * (1.0f + 0x1p-20f);
-                const float e2 = (s_eb[il] + ej) * (1.0f + 0x1p-20f);
-                float lo = sqrtf(fmaxf(d - delta, 0.f)) * (1.0f - 0x1p-20f) - e2;
-                lo -= fabsf(lo) * 0x1p-22f;
-                const float hi =
-                    (sqrtf(fmaxf(d + delta, 0.f)) * (1.0f + 0x1p-20f) + e2) * (1.0f + 0x1p-22f);
-                if (jv && i < n && j != i && lo <= s_T[il]) {
-                    const uint32_t p = atomicAdd(&s_cnt[il], 1u);  // < kAffCap: see kAffKeep
-                    const size_t o = (size_t)i * kAffCap + p;
-                    cj[o] = j;
-                    clo[o] = lo;
-                    chi[o] = hi;
+                const int il = 64 * wr + 16 * a + 4 * q4 + e;
+                const float ni = s_nh[il], kai = s_ka[il], Te = fmaf(s_T[il], kUp, s_eb[il]);
+                uint32_t tot = 0;
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    const float sn = ni + nj[b];
+                    const float d = sn - 2.0f * acc[a][b][e];
+                    const float te = Te + ej[b];
+                    const float dm = fmaf(-kai, aj[b], fmaf(-0x1p-21f, sn, d));
+                    bool hit = !(dm > te * te);
+                    if (edge) {
+                        const uint32_t i = row0 + il, j = c0 + 64 * wc + 16 * b + r16;
+                        hit = hit && jv[b] && i < n && j != i;
+                    }
+                    const uint64_t m = __ballot(hit);
+                    const uint32_t half = lane & 32 ? (uint32_t)(m >> 32) : (uint32_t)m;
+                    hits[e][b] = (half >> (lane & 16)) & 0xFFFFu;
+                    tot += (uint32_t)__popc(hits[e][b]);
+                }
+                base[e] = 0;
+                if (r16 == 0 && tot) base[e] = atomicAdd(&s_cnt[il], tot);
+                any |= tot;
+            }
+            if (!__ballot(any != 0u)) continue;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const uint32_t i = row0 + 64 * wr + 16 * a + 4 * q4 + e;
+                uint32_t at = row_first(base[e]);  // < kAffCap with the ranks below: kAffHold
+                uint2* list = cand + (lists + i) * kAffCap;
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    if ((hits[e][b] >> r16) & 1u)
+                        list[at + (uint32_t)__popc(hits[e][b] & ((1u << r16) - 1u))] = make_uint2(
+                            c0 + 64 * wc + 16 * b + r16, __float_as_uint(acc[a][b][e]));
+                    at += (uint32_t)__popc(hits[e][b]);
                 }
             }
         }
         __syncthreads();
         // rows whose buffer could overflow with the next tile are compacted, a wave per row
-        for (int r = w; r < kAffRowsWG; r += kAffWaves) {
-            const uint32_t i = row0 + r;
-            if (i < n && s_cnt[r] > kAffKeep)
-                aff_compact(cj + (size_t)i * kAffCap, clo + (size_t)i * kAffCap,
-                            chi + (size_t)i * kAffCap, &s_cnt[r], &s_T[r], &s_over[r], k);
+        uint64_t need = __ballot(lane < kAffRows / 8 && s_cnt[w * (kAffRows / 8) + (lane & 15)] > kAffHold);
+        uint2 en[kAffPer], nx[kAffPer];
+        int r = w * (kAffRows / 8) + (need ? __builtin_ctzll(need) : 0);
+        if (need) aff_load(cand + (lists + row0 + r) * kAffCap, s_cnt[r], row0 + r, en);
+        while (need) {
+            need &= need - 1;
+            const int rn = w * (kAffRows / 8) + (need ? __builtin_ctzll(need) : 0);
+            if (need)  // the next row's entries are in flight during this row's selection
+                aff_load(cand + (lists + row0 + rn) * kAffCap, s_cnt[rn], row0 + rn, nx);
+            aff_compact(cand + (lists + row0 + r) * kAffCap, P, dp, row0 + r, en, &s_cnt[r],
+                        &s_T[r], &s_over[r], k);
+            r = rn;
+#pragma unroll
+            for (int u = 0; u < kAffPer; ++u) en[u] = nx[u];
         }
         __syncthreads();
     }
-    for (int r = w; r < kAffRowsWG; r += kAffWaves) {
-        const uint32_t i = row0 + r;
-        if (i >= n) continue;
-        aff_compact(cj + (size_t)i * kAffCap, clo + (size_t)i * kAffCap, chi + (size_t)i * kAffCap,
-                    &s_cnt[r], &s_T[r], &s_over[r], k);
-        if (lane == 0) {
-            ccount[i] = s_cnt[r];
-            if (s_over[r] || s_cnt[r] < k) atomicAdd(overflow, 1u);
-        }
+    // the lists as they stand (at most kAffHold entries each): the refinement merges and thins them
+    if (tid < kAffRows && row0 + tid < n) {
+        ccount[lists + row0 + tid] = s_cnt[tid];
+        if (s_over[tid]) atomicAdd(overflow, 1u);
     }
 }
 
 // ---------------------------------------------------------------------------------------------
-// exact selection: FP64 distances of the candidates from the FP32 inputs, the k smallest by
-// (distance, index), ascending (one wave per row)
+// exact selection (one wave per row): the row's lists over the column ranges merged to the
+// columns whose lower bound is at most the k-th smallest upper bound of them all, then FP64
+// distances of those from the FP32 inputs and the k smallest by (distance, index), ascending.
+// Bound by the reads of the candidates' rows (n k dim 4 bytes from the caches); four candidates
+// at a time keep their loads in flight and share the reduction across the lanes (20,000 points in
+// 784-D, k = 90: 1.81 -> 1.13 ms).
 // ---------------------------------------------------------------------------------------------
+constexpr int kAffBatch = 4;
 __global__ __launch_bounds__(kBlock) void k_aff_refine(const float* __restrict__ X, uint32_t n,
-                                                       uint32_t dim, uint32_t k,
-                                                       const uint32_t* __restrict__ cj,
+                                                       uint32_t dim, uint32_t dp, uint32_t k,
+                                                       uint32_t splits, AffPoints P,
+                                                       const uint2* __restrict__ cand,
                                                        const uint32_t* __restrict__ ccount,
                                                        uint32_t* __restrict__ idx,
-                                                       double* __restrict__ d2) {
+                                                       double* __restrict__ d2,
+                                                       uint32_t* __restrict__ overflow) {
     __shared__ double s_d[kWavesPerBlock][kAffKeep];
     __shared__ uint32_t s_j[kWavesPerBlock][kAffKeep];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const uint32_t i = blockIdx.x * kWavesPerBlock + w;
     if (i >= n) return;
-    const uint32_t c = min(ccount[i], kAffKeep);
-    float xi[kAffMaxDimPad / kWave];
+    uint32_t c = 0;
+    {
+        constexpr int kPer = kAffHold / kWave;  // entries per lane and list
+        const float kd = aff_kdelta(dp), ni = P.nh[i], ai = P.ah[i], ei = P.eb[i];
+        uint32_t j[kAffMaxSplits * kPer], hb[kAffMaxSplits * kPer];
+        float lo[kAffMaxSplits * kPer];
+        bool v[kAffMaxSplits * kPer];
 #pragma unroll
-    for (int t = 0; t < kAffMaxDimPad / kWave; ++t) {
-        const uint32_t e = lane + kWave * t;
-        xi[t] = e < dim ? X[(size_t)i * dim + e] : 0.f;
-    }
-    for (uint32_t q = 0; q < c; ++q) {
-        const uint32_t j = cj[(size_t)i * kAffCap + q];
-        double s = 0.0;
+        for (int s = 0; s < (int)kAffMaxSplits; ++s) {
+            const uint32_t cs = s < (int)splits ? ccount[(size_t)s * n + i] : 0u;
 #pragma unroll
-        for (int t = 0; t < kAffMaxDimPad / kWave; ++t) {
-            const uint32_t e = lane + kWave * t;
-            if (e < dim) {
-                const double df = (double)xi[t] - (double)X[(size_t)j * dim + e];
-                s = fma(df, df, s);
+            for (int u = 0; u < kPer; ++u) {
+                const size_t o = ((size_t)s * n + i) * kAffCap + lane + 64 * u;
+                const int x = s * kPer + u;
+                v[x] = (uint32_t)(lane + 64 * u) < cs;
+                const uint2 en = v[x] ? cand[o] : make_uint2(i, 0u);
+                float hi;
+                aff_bounds(__uint_as_float(en.y), kd, ni, ai, ei, P.nh[en.x], P.ah[en.x],
+                           P.eb[en.x], lo[x], hi);
+                j[x] = en.x;
+                hb[x] = __float_as_uint(hi);
             }
         }
-        s = wave_sum_d(s);
-        if (lane == 0) {
-            s_d[w][q] = s;
-            s_j[w][q] = j;
+        const float t = __uint_as_float(aff_kth<kAffMaxSplits * kPer>(hb, v, k, 32));
+#pragma unroll
+        for (int x = 0; x < (int)kAffMaxSplits * kPer; ++x) {
+            const bool keep = v[x] && lo[x] <= t;
+            const uint64_t bm = __ballot(keep);
+            const uint32_t p = c + (uint32_t)__popcll(bm & lane_mask_lt());
+            if (keep && p < kAffKeep) s_j[w][p] = j[x];
+            c += (uint32_t)__popcll(bm);
         }
+        if (lane == 0 && (c > kAffKeep || c < k)) atomicAdd(overflow, 1u);
+        c = min(c, kAffKeep);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    const float* xi = X + (size_t)i * dim;
+    for (uint32_t q = 0; q < c; q += kAffBatch) {
+        const float* xj[kAffBatch];
+        double s[kAffBatch];
+#pragma unroll
+        for (int u = 0; u < kAffBatch; ++u) {
+            xj[u] = X + (size_t)s_j[w][min(q + u, c - 1)] * dim;
+            s[u] = 0.0;
+        }
+#pragma unroll 4
+        for (uint32_t e = lane; e < dim; e += kWave) {
+            const double a = xi[e];
+#pragma unroll
+            for (int u = 0; u < kAffBatch; ++u) {
+                const double df = a - (double)xj[u][e];
+                s[u] = fma(df, df, s[u]);
+            }
+        }
+        // sums over the lanes: halves and quarters of the wave take over one candidate each
+        static_assert(kAffBatch == 4, "two exchange steps");
+        const bool h = lane & 32, qd = lane & 16;
+        const double a0 = h ? s[2] : s[0], a1 = h ? s[3] : s[1];
+        const double b0 = h ? s[0] : s[2], b1 = h ? s[1] : s[3];
+        const double p0 = a0 + __shfl_xor(b0, 32, kWave), p1 = a1 + __shfl_xor(b1, 32, kWave);
+        double r = (qd ? p1 : p0) + __shfl_xor(qd ? p0 : p1, 16, kWave);
+        for (int o = 8; o > 0; o >>= 1) r += __shfl_xor(r, o, kWave);
+        const uint32_t at = q + (h ? 2u : 0u) + (qd ? 1u : 0u);
+        if ((lane & 15) == 0 && at < c) s_d[w][at] = r;
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -437,6 +585,18 @@ __global__ __launch_bounds__(kBlock) void k_sym_reduce(const uint64_t* __restric
 // ---------------------------------------------------------------------------------------------
 uint32_t aff_dim_padded(uint32_t dim) { return div_up_a(dim, kAffKC) * kAffKC; }
 uint32_t aff_cap() { return kAffCap; }
+uint32_t aff_keep() { return kAffKeep; }
+
+// Column ranges: one where the row blocks fill the 256 compute units about twice, else as many
+// (up to kAffMaxSplits, at least two tiles each) as bring them there: 20,000 points are 157 row
+// blocks, one per compute unit, so a single range would leave 99 units idle.
+uint32_t aff_splits(uint32_t n) {
+    const uint32_t rb = div_up_a(n, kAffRows), tiles = div_up_a(n, kAffCols);
+    uint32_t s = 512u / rb;
+    if (s > kAffMaxSplits) s = kAffMaxSplits;
+    if (s > tiles / 2) s = tiles / 2;
+    return s ? s : 1u;
+}
 
 void launch_aff_pack(hipStream_t s, const float* X, uint32_t n, uint32_t dim, float scale,
                      _Float16* Xh, float* nh, float* ah, float* eb) {
@@ -444,25 +604,19 @@ void launch_aff_pack(hipStream_t s, const float* X, uint32_t n, uint32_t dim, fl
                                                               scale, Xh, nh, ah, eb);
 }
 void launch_aff_candidates(hipStream_t s, const _Float16* Xh, const float* nh, const float* ah,
-                           const float* eb, uint32_t n, uint32_t dim, uint32_t k, uint32_t* cj,
-                           float* clo, float* chi, uint32_t* ccount, uint32_t* overflow) {
-    const uint32_t g = div_up_a(n, kAffRowsWG);
-    switch (aff_dim_padded(dim) / kAffKC) {
-#define BH_AFFC(C)                                                                                \
-    case C:                                                                                       \
-        k_aff_candidates<C><<<g, kAffThreads, 0, s>>>(Xh, nh, ah, eb, n, k, cj, clo, chi, ccount,  \
-                                                      overflow);                                  \
-        break
-        BH_AFFC(1); BH_AFFC(2); BH_AFFC(3); BH_AFFC(4);
-        BH_AFFC(5); BH_AFFC(6); BH_AFFC(7); BH_AFFC(8);
-#undef BH_AFFC
-        default: break;  // dim > 1024 is rejected by the caller
-    }
+                           const float* eb, uint32_t n, uint32_t dim, uint32_t k, uint32_t splits,
+                           uint2* cand, uint32_t* ccount, uint32_t* overflow) {
+    const dim3 g(div_up_a(n, kAffRows), splits);
+    k_aff_candidates<<<g, kAffThreads, 0, s>>>(Xh, nh, ah, eb, n, aff_dim_padded(dim), k, cand,
+                                               ccount, overflow);
 }
-void launch_aff_refine(hipStream_t s, const float* X, uint32_t n, uint32_t dim, uint32_t k,
-                       const uint32_t* cj, const uint32_t* ccount, uint32_t* idx, double* d2) {
-    k_aff_refine<<<div_up_a(n, kWavesPerBlock), kBlock, 0, s>>>(X, n, dim, k, cj, ccount, idx,
-                                                                d2);
+void launch_aff_refine(hipStream_t s, const float* X, const float* nh, const float* ah,
+                       const float* eb, uint32_t n, uint32_t dim, uint32_t k, uint32_t splits,
+                       const uint2* cand, const uint32_t* ccount, uint32_t* idx, double* d2,
+                       uint32_t* overflow) {
+    k_aff_refine<<<div_up_a(n, kWavesPerBlock), kBlock, 0, s>>>(
+        X, n, dim, aff_dim_padded(dim), k, splits, AffPoints{nh, ah, eb}, cand, ccount, idx, d2,
+        overflow);
 }
 void launch_aff_bandwidth(hipStream_t s, const double* d2, uint32_t n, uint32_t k, double target,
                           double tol, int max_iter, double* P, double* beta) {

@@ -1260,6 +1260,7 @@ bh_status bh_tsne_affinities(bh_ctx* c, const float* X, uint32_t n, uint32_t dim
     if (maxabs > 0.0) (void)std::frexp(maxabs, &ex);
     const float scale = maxabs > 0.0 ? std::ldexp(1.0f, 14 - ex) : 1.0f;
     const uint32_t dp = aff_dim_padded(dim), cap = aff_cap();
+    uint32_t splits = aff_splits(n);
     hipStream_t s = c->stream;
     std::vector<void*> tmp;
     auto alloc = [&](void** p, size_t bytes) -> bh_status {
@@ -1269,10 +1270,11 @@ bh_status bh_tsne_affinities(bh_ctx* c, const float* X, uint32_t n, uint32_t dim
         tmp.push_back(*p);
         return BH_OK;
     };
-    float *dX = nullptr, *nh = nullptr, *ah = nullptr, *eb = nullptr, *clo = nullptr, *chi = nullptr;
+    float *dX = nullptr, *nh = nullptr, *ah = nullptr, *eb = nullptr;
+    uint2* cand = nullptr;
     float* dval = nullptr;
     _Float16* Xh = nullptr;
-    uint32_t *cj = nullptr, *ccount = nullptr, *flags = nullptr, *idx = nullptr, *vals_a = nullptr,
+    uint32_t *ccount = nullptr, *flags = nullptr, *idx = nullptr, *vals_a = nullptr,
              *vals_b = nullptr, *head = nullptr, *pos = nullptr, *spart = nullptr,
              *scratch = nullptr, *dcol = nullptr, *drp = nullptr;
     uint64_t *keys_a = nullptr, *keys_b = nullptr;
@@ -1284,10 +1286,8 @@ bh_status bh_tsne_affinities(bh_ctx* c, const float* X, uint32_t n, uint32_t dim
     if (st == BH_OK) st = alloc((void**)&nh, (size_t)n * 4);
     if (st == BH_OK) st = alloc((void**)&ah, (size_t)n * 4);
     if (st == BH_OK) st = alloc((void**)&eb, (size_t)n * 4);
-    if (st == BH_OK) st = alloc((void**)&cj, (size_t)n * cap * 4);
-    if (st == BH_OK) st = alloc((void**)&clo, (size_t)n * cap * 4);
-    if (st == BH_OK) st = alloc((void**)&chi, (size_t)n * cap * 4);
-    if (st == BH_OK) st = alloc((void**)&ccount, (size_t)n * 4);
+    if (st == BH_OK) st = alloc((void**)&cand, (size_t)splits * n * cap * 8);
+    if (st == BH_OK) st = alloc((void**)&ccount, (size_t)splits * n * 4);
     if (st == BH_OK) st = alloc((void**)&flags, 4 * 4);  // [0] rows over capacity, [1] sort error, [2] nnz
     if (st == BH_OK) st = alloc((void**)&idx, nk * 4);
     if (st == BH_OK) st = alloc((void**)&d2, nk * 8);
@@ -1308,32 +1308,37 @@ bh_status bh_tsne_affinities(bh_ctx* c, const float* X, uint32_t n, uint32_t dim
     if (st == BH_OK) {
         st = hip_check(c, hipMemcpyAsync(dX, X, (size_t)n * dim * 4, hipMemcpyHostToDevice, s), "X");
     }
-    if (st == BH_OK) {
-        launch_fill_u32(s, flags, 4, 0u);
-        launch_aff_pack(s, dX, n, dim, scale, Xh, nh, ah, eb);
-        launch_aff_candidates(s, Xh, nh, ah, eb, n, dim, k, cj, clo, chi, ccount, flags);
-        launch_aff_refine(s, dX, n, dim, k, cj, ccount, idx, d2);
-        launch_aff_bandwidth(s, d2, n, k, std::log(perplexity), 1e-5, 200, P, dbeta);
-        launch_sym_entries(s, idx, n, k, keys_a, vals_a);
-        int key_bits = 1;
-        while (key_bits < 64 && ((uint64_t)n * n - 1) >> key_bits) ++key_bits;
-        bool in_b = false;
-        launch_radix_sort(s, keys_a, vals_a, keys_b, vals_b, m, key_bits, true, scratch, flags + 1,
-                          kSortSpinLimit, &in_b);
-        const uint64_t* ks = in_b ? keys_b : keys_a;
-        const uint32_t* vs = in_b ? vals_b : vals_a;
-        launch_sym_heads(s, ks, m, head);
-        launch_exclusive_scan(s, head, pos, m, spart, flags + 2);
-        launch_sym_reduce(s, ks, vs, pos, m, n, (uint32_t)nk, P, dcol, dval, drp, flags + 2);
-        st = launch_status(c, "affinities launch");
+    // Column ranges keep thresholds of their own, so a range's list can overflow where one list
+    // over all columns would not: such a call is repeated with one range.
+    for (;; splits = 1) {
+        if (st == BH_OK) {
+            launch_fill_u32(s, flags, 4, 0u);
+            launch_aff_pack(s, dX, n, dim, scale, Xh, nh, ah, eb);
+            launch_aff_candidates(s, Xh, nh, ah, eb, n, dim, k, splits, cand, ccount, flags);
+            launch_aff_refine(s, dX, nh, ah, eb, n, dim, k, splits, cand, ccount, idx, d2, flags);
+            launch_aff_bandwidth(s, d2, n, k, std::log(perplexity), 1e-5, 200, P, dbeta);
+            launch_sym_entries(s, idx, n, k, keys_a, vals_a);
+            int key_bits = 1;
+            while (key_bits < 64 && ((uint64_t)n * n - 1) >> key_bits) ++key_bits;
+            bool in_b = false;
+            launch_radix_sort(s, keys_a, vals_a, keys_b, vals_b, m, key_bits, true, scratch,
+                              flags + 1, kSortSpinLimit, &in_b);
+            const uint64_t* ks = in_b ? keys_b : keys_a;
+            const uint32_t* vs = in_b ? vals_b : vals_a;
+            launch_sym_heads(s, ks, m, head);
+            launch_exclusive_scan(s, head, pos, m, spart, flags + 2);
+            launch_sym_reduce(s, ks, vs, pos, m, n, (uint32_t)nk, P, dcol, dval, drp, flags + 2);
+            st = launch_status(c, "affinities launch");
+        }
+        if (st == BH_OK)
+            st = hip_check(c, hipMemcpyAsync(h_flags, flags, sizeof(h_flags), hipMemcpyDeviceToHost, s), "flags");
+        if (st == BH_OK) st = hip_check(c, hipStreamSynchronize(s), "affinities");
+        if (st != BH_OK || !h_flags[0] || splits == 1) break;
     }
-    if (st == BH_OK)
-        st = hip_check(c, hipMemcpyAsync(h_flags, flags, sizeof(h_flags), hipMemcpyDeviceToHost, s), "flags");
-    if (st == BH_OK) st = hip_check(c, hipStreamSynchronize(s), "affinities");
     if (st == BH_OK && h_flags[0])
         st = fail(c, BH_ERR_CAPACITY,
                   "%u points have more than %u candidates within the FP16 error bound of their "
-                  "k-th neighbour (many exact or near duplicates)", h_flags[0], cap - 64);
+                  "k-th neighbour (many exact or near duplicates)", h_flags[0], aff_keep());
     if (st == BH_OK && h_flags[1]) st = fail(c, BH_ERR_HIP, "the radix sort gave up waiting");
     const uint32_t nz = h_flags[2];
     if (st == BH_OK && (nz == 0 || nz > m)) st = fail(c, BH_ERR_HIP, "bad nonzero count %u", nz);

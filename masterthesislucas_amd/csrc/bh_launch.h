@@ -247,13 +247,17 @@ void launch_cell_coefs(hipStream_t s, const float* feat, const Node* nodes,
 // bandwidths by bisection, symmetrisation keyed by row * n + column
 uint32_t aff_dim_padded(uint32_t dim);
 uint32_t aff_cap();
+uint32_t aff_keep();  // most candidates of a row after the merge (more: counted in overflow)
+uint32_t aff_splits(uint32_t n);  // column ranges (lists per row) of the candidate search
 void launch_aff_pack(hipStream_t s, const float* X, uint32_t n, uint32_t dim, float scale,
                      _Float16* Xh, float* nh, float* ah, float* eb);
 void launch_aff_candidates(hipStream_t s, const _Float16* Xh, const float* nh, const float* ah,
-                           const float* eb, uint32_t n, uint32_t dim, uint32_t k, uint32_t* cj,
-                           float* clo, float* chi, uint32_t* ccount, uint32_t* overflow);
-void launch_aff_refine(hipStream_t s, const float* X, uint32_t n, uint32_t dim, uint32_t k,
-                       const uint32_t* cj, const uint32_t* ccount, uint32_t* idx, double* d2);
+                           const float* eb, uint32_t n, uint32_t dim, uint32_t k, uint32_t splits,
+                           uint2* cand, uint32_t* ccount, uint32_t* overflow);
+void launch_aff_refine(hipStream_t s, const float* X, const float* nh, const float* ah,
+                       const float* eb, uint32_t n, uint32_t dim, uint32_t k, uint32_t splits,
+                       const uint2* cand, const uint32_t* ccount, uint32_t* idx, double* d2,
+                       uint32_t* overflow);
 void launch_aff_bandwidth(hipStream_t s, const double* d2, uint32_t n, uint32_t k, double target,
                           double tol, int max_iter, double* P, double* beta);
 void launch_sym_entries(hipStream_t s, const uint32_t* idx, uint32_t n, uint32_t k,

@@ -74,3 +74,27 @@ def test_exact_z_edges(gpu, n):
     want_kl = (p * np.log2(p * want_z * (1.0 + d2[rows, cols]))).sum()
     assert abs(z - want_z) <= 1e-12 * want_z
     assert abs(kl - want_kl) <= 1e-12 * np.abs(p * np.log2(p * want_z)).sum()
+
+
+@pytest.mark.parametrize("n,dim,k", [(2, 1, 1), (129, 63, 5), (257, 64, 90), (513, 65, 128),
+                                     (1100, 20, 30), (2600, 130, 15)])
+def test_affinity_tile_edges(gpu, n, dim, k):
+    """Row blocks of 128, column tiles of 256 in one or several ranges, K chunks of 64: the exact
+    neighbours and distances against FP64 brute force (distances to 1e-12, as FP64 sums in another
+    order allow; ties by index)."""
+    rng = np.random.default_rng(n + dim)
+    X = (rng.normal(0, 1, (n, dim)) + 3.0 * rng.integers(0, 4, (n, 1))).astype(np.float32)
+    X[-1] = X[0]  # a duplicate pair
+    a = tsne.affinities(X, perplexity=max(1.0, k / 3.0), k=k)
+    d = X.astype(np.float64)
+    d2 = ((d[:, None, :] - d[None, :, :]) ** 2).sum(2) if n * n * dim < 4e7 else None
+    if d2 is None:
+        d2 = np.stack([((d - row) ** 2).sum(1) for row in d])
+    np.fill_diagonal(d2, np.inf)
+    idx = np.argsort(d2, axis=1, kind="stable")[:, :k]
+    want = np.take_along_axis(d2, idx, 1)
+    assert np.allclose(a["d2"], want, rtol=1e-12, atol=0)
+    differ = a["idx"] != idx  # only where two distances agree to rounding
+    gap = np.abs(np.take_along_axis(d2, a["idx"].astype(np.int64), 1) - want)
+    assert np.all(gap[differ] <= 1e-12 * want[differ])
+    assert abs(a["val"].astype(np.float64).sum() - 1.0) < 1e-6
