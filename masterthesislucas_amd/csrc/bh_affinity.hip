@@ -36,6 +36,24 @@ constexpr uint32_t kAffHold = kAffCap - kAffCols;  // compact above this many (a
 constexpr uint32_t kAffKeep = 192;            // most candidates of a row over all columns
 constexpr uint32_t kAffMaxSplits = 4;         // most column ranges
 
+// largest magnitude bits of the inputs (order = |x|; infinities and NaN above every finite one),
+// into *out (cleared by the caller); one integer atomic per block
+__global__ __launch_bounds__(kBlock) void k_aff_maxbits(const uint32_t* __restrict__ x, uint64_t n,
+                                                        uint32_t* __restrict__ out) {
+    __shared__ uint32_t red[kWavesPerBlock];
+    uint32_t m = 0;
+    for (uint64_t e = (uint64_t)blockIdx.x * kBlock + threadIdx.x; e < n;
+         e += (uint64_t)gridDim.x * kBlock)
+        m = max(m, x[e] & 0x7FFFFFFFu);
+    for (int o = 32; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o, kWave));
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kWavesPerBlock; ++w) m = max(m, red[w]);
+        atomicMax(out, m);
+    }
+}
+
 // ---------------------------------------------------------------------------------------------
 // scaled FP16 copy, squared norms and rounding bounds (one wave per point)
 // ---------------------------------------------------------------------------------------------
@@ -598,6 +616,10 @@ uint32_t aff_splits(uint32_t n) {
     return s ? s : 1u;
 }
 
+void launch_aff_maxbits(hipStream_t s, const float* x, uint64_t n, uint32_t* out) {
+    const uint32_t g = div_up_a(n, 8 * kBlock);
+    k_aff_maxbits<<<g < 2048 ? g : 2048, kBlock, 0, s>>>((const uint32_t*)x, n, out);
+}
 void launch_aff_pack(hipStream_t s, const float* X, uint32_t n, uint32_t dim, float scale,
                      _Float16* Xh, float* nh, float* ah, float* eb) {
     k_aff_pack<<<div_up_a(n, kWavesPerBlock), kBlock, 0, s>>>(X, n, dim, aff_dim_padded(dim),

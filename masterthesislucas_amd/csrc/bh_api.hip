@@ -107,6 +107,8 @@ struct bh_ctx {
     hipEvent_t ev_staged = nullptr, ev_att = nullptr;
     double* tz = nullptr;
     double* kl_part = nullptr;
+    void* aff_buf = nullptr;   // workspace of bh_tsne_affinities (grow-only until bh_tsne_set_p)
+    size_t aff_bytes = 0;
     double* kl_out = nullptr;
 
     bool learned = false;  // second moments in builds, learned correction available
@@ -458,6 +460,7 @@ bh_status bh_config_default(bh_config* cfg) {
 const char* bh_last_error(const bh_ctx* ctx) { return ctx ? ctx->err.c_str() : "null context"; }
 
 static void graph_reset(bh_ctx* c);
+static void aff_release(bh_ctx* c);
 
 void bh_destroy(bh_ctx* c) {
     if (!c) return;
@@ -478,6 +481,7 @@ void bh_destroy(bh_ctx* c) {
     if (c->part) (void)hipFree(c->part);
     if (c->fmm_buf) (void)hipFree(c->fmm_buf);
     if (c->side) (void)hipFree(c->side);
+    aff_release(c);
     if (c->h_status) (void)hipHostFree(c->h_status);
     if (c->h_prm) (void)hipHostFree(c->h_prm);
     if (c->h_dsum) (void)hipHostFree(c->h_dsum);
@@ -1108,6 +1112,7 @@ bh_status bh_tsne_set_p(bh_ctx* c, uint32_t n, const uint32_t* row_ptr, const ui
         if (row_ptr[r] > row_ptr[r + 1]) return fail(c, BH_ERR_ARG, "row_ptr decreases at %u", r);
     for (uint32_t e = 0; e < nnz; ++e)
         if (col[e] >= n) return fail(c, BH_ERR_ARG, "column %u out of range at %u", col[e], e);
+    aff_release(c);  // the descent begins: the affinities' workspace is given back
     if (c->p_row) (void)hipFree(c->p_row);
     if (c->p_col) (void)hipFree(c->p_col);
     if (c->p_val) (void)hipFree(c->p_val);
@@ -1231,6 +1236,12 @@ bh_status bh_tsne_run(bh_ctx* c, const bh_tsne_params* p, int32_t first, int32_t
     return finish_build_call(c, "t-SNE run");
 }
 
+static void aff_release(bh_ctx* c) {
+    if (c->aff_buf) (void)hipFree(c->aff_buf);
+    c->aff_buf = nullptr;
+    c->aff_bytes = 0;
+}
+
 bh_status bh_tsne_affinities(bh_ctx* c, const float* X, uint32_t n, uint32_t dim,
                              double perplexity, uint32_t k, uint32_t* row_ptr, uint32_t* col,
                              float* val, uint32_t* nnz, uint32_t* knn_idx, double* knn_d2,
@@ -1244,32 +1255,9 @@ bh_status bh_tsne_affinities(bh_ctx* c, const float* X, uint32_t n, uint32_t dim
     if (m64 >= (1ull << 31) || (uint64_t)n * n >= (1ull << 62))
         return fail(c, BH_ERR_ARG, "%u points x %u neighbours is too large", n, k);
     const uint32_t m = (uint32_t)m64;
-    // scale by a power of two so that the largest |x| lands in [2^13, 2^14): no FP16 overflow.
-    // The magnitude bits of a float order its |x|; infinities and NaN have all exponent bits set
-    uint32_t maxbits = 0;
-    {
-        const uint32_t* xb = reinterpret_cast<const uint32_t*>(X);
-        const uint64_t cnt = (uint64_t)n * dim;
-        for (uint64_t e = 0; e < cnt; ++e) maxbits = std::max(maxbits, xb[e] & 0x7FFFFFFFu);
-    }
-    if (maxbits >= 0x7F800000u) return fail(c, BH_ERR_ARG, "an input coordinate is not finite");
-    float maxf;
-    std::memcpy(&maxf, &maxbits, 4);
-    const double maxabs = maxf;
-    int ex = 0;
-    if (maxabs > 0.0) (void)std::frexp(maxabs, &ex);
-    const float scale = maxabs > 0.0 ? std::ldexp(1.0f, 14 - ex) : 1.0f;
     const uint32_t dp = aff_dim_padded(dim), cap = aff_cap();
     uint32_t splits = aff_splits(n);
     hipStream_t s = c->stream;
-    std::vector<void*> tmp;
-    auto alloc = [&](void** p, size_t bytes) -> bh_status {
-        *p = nullptr;
-        hipError_t e = hipMalloc(p, bytes ? bytes : 16);
-        if (e != hipSuccess) return hip_check(c, e, "hipMalloc (affinities)");
-        tmp.push_back(*p);
-        return BH_OK;
-    };
     float *dX = nullptr, *nh = nullptr, *ah = nullptr, *eb = nullptr;
     uint2* cand = nullptr;
     float* dval = nullptr;
@@ -1280,33 +1268,70 @@ bh_status bh_tsne_affinities(bh_ctx* c, const float* X, uint32_t n, uint32_t dim
     uint64_t *keys_a = nullptr, *keys_b = nullptr;
     double *d2 = nullptr, *P = nullptr, *dbeta = nullptr;
     const size_t nsp = scan_partials_size(m);
-    bh_status st = BH_OK;
-    st = alloc((void**)&dX, (size_t)n * dim * 4);
-    if (st == BH_OK) st = alloc((void**)&Xh, (size_t)n * dp * 2);
-    if (st == BH_OK) st = alloc((void**)&nh, (size_t)n * 4);
-    if (st == BH_OK) st = alloc((void**)&ah, (size_t)n * 4);
-    if (st == BH_OK) st = alloc((void**)&eb, (size_t)n * 4);
-    if (st == BH_OK) st = alloc((void**)&cand, (size_t)splits * n * cap * 8);
-    if (st == BH_OK) st = alloc((void**)&ccount, (size_t)splits * n * 4);
-    if (st == BH_OK) st = alloc((void**)&flags, 4 * 4);  // [0] rows over capacity, [1] sort error, [2] nnz
-    if (st == BH_OK) st = alloc((void**)&idx, nk * 4);
-    if (st == BH_OK) st = alloc((void**)&d2, nk * 8);
-    if (st == BH_OK) st = alloc((void**)&P, nk * 8);
-    if (st == BH_OK) st = alloc((void**)&dbeta, (size_t)n * 8);
-    if (st == BH_OK) st = alloc((void**)&keys_a, (size_t)m * 8);
-    if (st == BH_OK) st = alloc((void**)&keys_b, (size_t)m * 8);
-    if (st == BH_OK) st = alloc((void**)&vals_a, (size_t)m * 4);
-    if (st == BH_OK) st = alloc((void**)&vals_b, (size_t)m * 4);
-    if (st == BH_OK) st = alloc((void**)&head, (size_t)m * 4);
-    if (st == BH_OK) st = alloc((void**)&pos, (size_t)m * 4);
-    if (st == BH_OK) st = alloc((void**)&spart, (nsp + 1) * 4);
-    if (st == BH_OK) st = alloc((void**)&scratch, sort_scratch_words(m) * 4);
-    if (st == BH_OK) st = alloc((void**)&dcol, (size_t)m * 4);
-    if (st == BH_OK) st = alloc((void**)&dval, (size_t)m * 4);
-    if (st == BH_OK) st = alloc((void**)&drp, ((size_t)n + 1) * 4);
-    uint32_t h_flags[4] = {0, 0, 0, 0};
+    // one workspace, kept by the context until bh_tsne_set_p starts a descent (25 allocations and
+    // frees a call took 4.7 ms of a 20,000-point call)
+    size_t need = 0;
+    std::pair<void**, size_t> parts[32];
+    int np = 0;
+    auto part = [&](void** p, size_t bytes) {
+        parts[np++] = {p, need};
+        need += (bytes + 255) / 256 * 256;
+    };
+    part((void**)&dX, (size_t)n * dim * 4);
+    part((void**)&Xh, (size_t)n * dp * 2);
+    part((void**)&nh, (size_t)n * 4);
+    part((void**)&ah, (size_t)n * 4);
+    part((void**)&eb, (size_t)n * 4);
+    part((void**)&cand, (size_t)splits * n * cap * 8);
+    part((void**)&ccount, (size_t)splits * n * 4);
+    part((void**)&flags, 4 * 4);  // [0] rows over capacity, [1] sort error, [2] nnz, [3] max |x|
+    part((void**)&idx, nk * 4);
+    part((void**)&d2, nk * 8);
+    part((void**)&P, nk * 8);
+    part((void**)&dbeta, (size_t)n * 8);
+    part((void**)&keys_a, (size_t)m * 8);
+    part((void**)&keys_b, (size_t)m * 8);
+    part((void**)&vals_a, (size_t)m * 4);
+    part((void**)&vals_b, (size_t)m * 4);
+    part((void**)&head, (size_t)m * 4);
+    part((void**)&pos, (size_t)m * 4);
+    part((void**)&spart, (nsp + 1) * 4);
+    part((void**)&scratch, sort_scratch_words(m) * 4);
+    part((void**)&dcol, (size_t)m * 4);
+    part((void**)&dval, (size_t)m * 4);
+    part((void**)&drp, ((size_t)n + 1) * 4);
+    if (need > c->aff_bytes) {
+        aff_release(c);
+        hipError_t e = hipMalloc(&c->aff_buf, need);
+        if (e != hipSuccess) {
+            c->aff_buf = nullptr;
+            return hip_check(c, e, "hipMalloc (affinities)");
+        }
+        c->aff_bytes = need;
+    }
+    for (int q = 0; q < np; ++q) *parts[q].first = (char*)c->aff_buf + parts[q].second;
+    hipEvent_t ready = nullptr;  // neighbours and bandwidths final: their copies overlap the rest
+    bh_status st = hip_check(c, hipEventCreateWithFlags(&ready, hipEventDisableTiming), "event");
+    if (st != BH_OK) return st;
+    uint32_t* h_flags = reinterpret_cast<uint32_t*>(c->h_counters);  // pinned
+    float scale = 1.0f;
+    st = hip_check(c, hipMemcpyAsync(dX, X, (size_t)n * dim * 4, hipMemcpyHostToDevice, s), "X");
     if (st == BH_OK) {
-        st = hip_check(c, hipMemcpyAsync(dX, X, (size_t)n * dim * 4, hipMemcpyHostToDevice, s), "X");
+        // scale by a power of two so that the largest |x| lands in [2^13, 2^14): no FP16 overflow.
+        // The magnitude bits of a float order its |x|; infinities and NaN have all exponent bits set
+        launch_fill_u32(s, flags, 4, 0u);
+        launch_aff_maxbits(s, dX, (uint64_t)n * dim, flags + 3);
+        st = hip_check(c, hipMemcpyAsync(h_flags, flags + 3, 4, hipMemcpyDeviceToHost, s), "max");
+    }
+    if (st == BH_OK) st = hip_check(c, hipStreamSynchronize(s), "max");
+    if (st == BH_OK && h_flags[0] >= 0x7F800000u)
+        st = fail(c, BH_ERR_ARG, "an input coordinate is not finite");
+    if (st == BH_OK) {
+        float maxf;
+        std::memcpy(&maxf, h_flags, 4);
+        int ex = 0;
+        if (maxf > 0.0f) (void)std::frexp((double)maxf, &ex);
+        scale = maxf > 0.0f ? std::ldexp(1.0f, 14 - ex) : 1.0f;
     }
     // Column ranges keep thresholds of their own, so a range's list can overflow where one list
     // over all columns would not: such a call is repeated with one range.
@@ -1317,6 +1342,8 @@ bh_status bh_tsne_affinities(bh_ctx* c, const float* X, uint32_t n, uint32_t dim
             launch_aff_candidates(s, Xh, nh, ah, eb, n, dim, k, splits, cand, ccount, flags);
             launch_aff_refine(s, dX, nh, ah, eb, n, dim, k, splits, cand, ccount, idx, d2, flags);
             launch_aff_bandwidth(s, d2, n, k, std::log(perplexity), 1e-5, 200, P, dbeta);
+            st = hip_check(c, hipMemcpyAsync(h_flags, flags, 4, hipMemcpyDeviceToHost, s), "flags");
+            if (st == BH_OK) st = hip_check(c, hipEventRecord(ready, s), "event");
             launch_sym_entries(s, idx, n, k, keys_a, vals_a);
             int key_bits = 1;
             while (key_bits < 64 && ((uint64_t)n * n - 1) >> key_bits) ++key_bits;
@@ -1328,31 +1355,34 @@ bh_status bh_tsne_affinities(bh_ctx* c, const float* X, uint32_t n, uint32_t dim
             launch_sym_heads(s, ks, m, head);
             launch_exclusive_scan(s, head, pos, m, spart, flags + 2);
             launch_sym_reduce(s, ks, vs, pos, m, n, (uint32_t)nk, P, dcol, dval, drp, flags + 2);
-            st = launch_status(c, "affinities launch");
+            if (st == BH_OK)
+                st = hip_check(c, hipMemcpyAsync(h_flags + 4, flags, 16, hipMemcpyDeviceToHost, s), "flags");
+            if (st == BH_OK) st = launch_status(c, "affinities launch");
         }
-        if (st == BH_OK)
-            st = hip_check(c, hipMemcpyAsync(h_flags, flags, sizeof(h_flags), hipMemcpyDeviceToHost, s), "flags");
-        if (st == BH_OK) st = hip_check(c, hipStreamSynchronize(s), "affinities");
+        if (st == BH_OK) st = hip_check(c, hipEventSynchronize(ready), "affinities");
         if (st != BH_OK || !h_flags[0] || splits == 1) break;
+        st = hip_check(c, hipStreamSynchronize(s), "affinities");
     }
     if (st == BH_OK && h_flags[0])
         st = fail(c, BH_ERR_CAPACITY,
                   "%u points have more than %u candidates within the FP16 error bound of their "
                   "k-th neighbour (many exact or near duplicates)", h_flags[0], aff_keep());
-    if (st == BH_OK && h_flags[1]) st = fail(c, BH_ERR_HIP, "the radix sort gave up waiting");
-    const uint32_t nz = h_flags[2];
+    // (s does not synchronise with the default stream these copies run on)
+    if (st == BH_OK && knn_idx) st = hip_check(c, hipMemcpy(knn_idx, idx, nk * 4, hipMemcpyDeviceToHost), "idx");
+    if (st == BH_OK && knn_d2) st = hip_check(c, hipMemcpy(knn_d2, d2, nk * 8, hipMemcpyDeviceToHost), "d2");
+    if (st == BH_OK && beta) st = hip_check(c, hipMemcpy(beta, dbeta, (size_t)n * 8, hipMemcpyDeviceToHost), "beta");
+    if (st == BH_OK) st = hip_check(c, hipStreamSynchronize(s), "affinities");
+    if (st == BH_OK && h_flags[5]) st = fail(c, BH_ERR_HIP, "the radix sort gave up waiting");
+    const uint32_t nz = h_flags[6];
     if (st == BH_OK && (nz == 0 || nz > m)) st = fail(c, BH_ERR_HIP, "bad nonzero count %u", nz);
     if (st == BH_OK) {
         *nnz = nz;
         st = hip_check(c, hipMemcpy(row_ptr, drp, ((size_t)n + 1) * 4, hipMemcpyDeviceToHost), "row_ptr");
         if (st == BH_OK) st = hip_check(c, hipMemcpy(col, dcol, (size_t)nz * 4, hipMemcpyDeviceToHost), "col");
         if (st == BH_OK) st = hip_check(c, hipMemcpy(val, dval, (size_t)nz * 4, hipMemcpyDeviceToHost), "val");
-        if (st == BH_OK && knn_idx) st = hip_check(c, hipMemcpy(knn_idx, idx, nk * 4, hipMemcpyDeviceToHost), "idx");
-        if (st == BH_OK && knn_d2) st = hip_check(c, hipMemcpy(knn_d2, d2, nk * 8, hipMemcpyDeviceToHost), "d2");
-        if (st == BH_OK && beta) st = hip_check(c, hipMemcpy(beta, dbeta, (size_t)n * 8, hipMemcpyDeviceToHost), "beta");
     }
     (void)hipStreamSynchronize(s);
-    for (void* p : tmp) (void)hipFree(p);
+    (void)hipEventDestroy(ready);
     return st;
 }
 

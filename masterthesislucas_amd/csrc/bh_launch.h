@@ -249,6 +249,8 @@ uint32_t aff_dim_padded(uint32_t dim);
 uint32_t aff_cap();
 uint32_t aff_keep();  // most candidates of a row after the merge (more: counted in overflow)
 uint32_t aff_splits(uint32_t n);  // column ranges (lists per row) of the candidate search
+// out (cleared) = the largest magnitude bits of n values
+void launch_aff_maxbits(hipStream_t s, const float* x, uint64_t n, uint32_t* out);
 void launch_aff_pack(hipStream_t s, const float* X, uint32_t n, uint32_t dim, float scale,
                      _Float16* Xh, float* nh, float* ah, float* eb);
 void launch_aff_candidates(hipStream_t s, const _Float16* Xh, const float* nh, const float* ah,
