@@ -131,7 +131,7 @@ bh_status bh_forces_device(bh_ctx* ctx, double theta, float* d_ax, float* d_ay, 
 bh_status bh_leapfrog(bh_ctx* ctx, int steps, float dt, double theta);
 /* bh_leapfrog with each step (kick-drift, build, traversal, kick) captured once in a HIP graph
  * and replayed: same kernels and results, without per-launch host overhead. The graphs are
- * re-captured when dt, theta or the traversal variant change. */
+ * re-captured when dt, theta or a traversal setting change. */
 bh_status bh_leapfrog_graph(bh_ctx* ctx, int steps, float dt, double theta);
 
 /* Conserved quantities of a gravity context in FP64 (no counterpart in the reference, whose
@@ -330,51 +330,31 @@ bh_status bh_profile_phases(bh_ctx* ctx, uint32_t mask);
 bh_status bh_profile_read(bh_ctx* ctx, double* ms, uint64_t* launches, int reset);
 bh_status bh_synchronize(bh_ctx* ctx);
 
-/* ---- autotuning: kernel variants of the traversal (no reference counterpart; the reference
- * GPU traversal has one fixed shape, nBodySolverGpuBH.cu:260-348) ----
- * variant v in [0, bh_traverse_variant_count()). For v < 12: v / 4 selects 1, 2 or 4 sink
- * particles per lane (a wave serves 64, 128 or 256 Morton-consecutive particles); (v % 4) / 2
- * selects monopoles computed only when a lane accepts (0) or always, masked (1); v % 2 selects
- * 1 or 4 sources per scalar fetch in the particle-particle loop. For 12 <= v < 18: (v - 12) / 2
- * selects 1, 2 or 4 sinks per lane, (v - 12) % 2 the monopole mode as above, and the
- * particle-particle sources of a cell are loaded by the lanes with one vector load (up to 64 at
- * a time) and broadcast. Variants 18 <= v < 36 take the shape of v - 18 with the lane masks
- * kept in scalar registers (acceptance mask = ballot of the distance test and the active mask;
- * fewer vector instructions per visit, faster for some shapes and workloads, slower for
- * others). Split walks (bh_set_traverse_split) use the vector-mask form of the shape. Results
- * are identical up to FP32 summation order. */
+/* ---- traversal settings (no reference counterpart; the reference GPU traversal has one fixed
+ * shape, nBodySolverGpuBH.cu:260-348) ----
+ * Variant ids in [0, bh_traverse_variant_count()) are accepted and kept. They named shapes of an
+ * earlier walk; one walk now serves all of them with the same results. */
 int bh_traverse_variant_count(void);
 bh_status bh_set_traverse_variant(bh_ctx* ctx, int variant);
-/* Split walk for small N (no reference counterpart): `split` waves (1..8) share each sink
- * group and take the same path through the tree; wave f adds the monopoles of every split-th
- * node visit and, in each particle-particle cell, the sources of the f-th of `split` equal
- * slices of the cell. Every interaction is evaluated by exactly one wave and the partial
- * results are summed in wave order. Multiplies the waves of a launch when the sinks alone
- * cannot fill the device and divides the long particle-particle loops of crowded leaves.
- * Results equal split 1 up to FP32 summation order; interaction counts are identical.
- * Batched contexts split each work entry the same way; bh_forces_learned always walks with
- * split 1. */
+/* Waves per group of 64 sinks: split 1 (default) chooses 1, 2 or 4 from the number of groups (one
+ * for batched contexts), 2 asks for two and 3..8 for four. The waves of a group take the same path
+ * through the tree and each adds its own parts of the sums, which are fixed: results and
+ * interaction counts are bit-identical for every setting. (bh_forces with the t-SNE kernel on one
+ * system of at most 131,072 points keeps its own summation order at split 1 and agrees with the
+ * other settings up to FP32 summation order.) */
 bh_status bh_set_traverse_split(bh_ctx* ctx, int split);
-/* Issue priority of the walk's waves (no reference counterpart; on by default): each wave
- * starts at priority 3 and steps down a level every ~1/3 of a wave's node visits (a step set
- * from theta), so that waves that have made less progress are issued first and the waves of a
- * SIMD finish together instead of in dispatch order. Applied to one-system walks (not split,
- * not learned) whose waves all fit on the device at once (at most 8 per SIMD); other launches
- * walk without it. Scheduling only: results and interaction counts are bit-identical either
- * way. */
-/* Batched contexts (no reference counterpart): rebuild the work table of the current variant
- * from the interaction counts of the last walk (split 1): entries in descending cost per lane
- * (a wave's interactions / its sinks x its sinks per lane), and the costliest entries (at least
- * 16 times the mean cost, at most 8192 of them) walked as 8 slices each (every slice takes the
- * path; slice f adds every 8th visit's monopoles and the f-th eighth of each particle-particle
- * cell's sources; the slices' partial results are added in slice order). Waves are otherwise
- * dispatched in system order, and on the 256-system workload the waves over the thousands of
- * occupants of one-child chains (up to 17 ms each) then start late: ordered, its walk takes
- * 13.4 ms instead of 21.8 (2 sinks per lane). Interaction counts are unchanged; forces change
- * only in the summation order of the sliced entries. Calling it again after a walk on the
- * ordered table gives the same table. bh_set_traverse_split(ctx, F > 1) restores the system
- * order. */
+/* Batched contexts (no reference counterpart): rebuild the work table from the interaction counts
+ * of the last walk (split 1): entries (a wave's 64 sinks) in descending cost per sink, and the
+ * costliest entries (at least 16 times the mean cost, at most 8192 of them) walked as 8 slices each
+ * (every slice takes the path and adds the accepted cells of every 8th step and every 8th block of
+ * particle-particle sources; the slices' partial results are added in slice order). Waves are
+ * otherwise dispatched in system order, and waves over the thousands of occupants of one-child
+ * chains then start late. Interaction counts are unchanged; forces change only in the summation
+ * order of the sliced entries. Calling it again after a walk on the ordered table gives the same
+ * table. bh_set_traverse_split(ctx, F > 1) restores the system order. */
 bh_status bh_batch_order_by_cost(bh_ctx* ctx);
+/* Issue priority of the walk's waves: a scheduling setting of an earlier walk, accepted and kept
+ * (on by default); results never depended on it and the walk no longer uses it. */
 bh_status bh_set_walk_priority(bh_ctx* ctx, int on);
 bh_status bh_get_walk_priority(bh_ctx* ctx, int* on);
 

@@ -1,14 +1,10 @@
-"""Autotuner for the Barnes-Hut traversal kernel.
+"""Timing of the traversal's settings on a caller's context.
 
-The traversal has a few compile-time shapes (see bh_set_traverse_variant in include/bh.h):
-whether monopoles are computed only when a lane accepts or always (masked), and how many
-source particles each scalar fetch brings into the particle-particle loop. For small N the walk
-can also be split over several waves per sink group (bh_set_traverse_split), which multiplies the
-waves of a launch at the price of re-reading the path to each wave's tree range. Which is fastest
-depends on the particle distribution, N and theta, so the tuner times every variant on the
-caller's own context (already holding the workload) with the library's HIP-event phase timers
-and keeps the fastest. Choices are remembered per (kernel, tree mode, log2 N, theta) in a JSON
-table next to this file so later runs can skip the search.
+One walk serves every variant id (bh_set_traverse_variant in include/bh.h), and the library
+chooses the waves per sink group (bh_set_traverse_split) from the launch size, so a program need
+not tune. These calls time the settings on the caller's own context (already holding the
+workload) with the library's HIP-event phase timers, select the fastest, and can remember it per
+(kernel, tree mode, log2 N, theta) in a JSON table next to this file.
 """
 from __future__ import annotations
 
@@ -52,10 +48,8 @@ def tune(ctx, theta, repeats=3, save=False, path=TABLE):
     """Time all variants on ctx's current tree (ctx must have been built), select the fastest,
     and return (best_variant, {variant: ms}).
 
-    The variants are timed with the walk's progress-ordered issue priority on
-    (bh_set_walk_priority); the winner is timed once more without it, under the key
-    "<variant>:no-priority", and the context keeps whichever was faster. The priority pays when
-    all waves of a launch are resident at once and can cost a few percent when they are not."""
+    The winner is timed once more with the issue priority setting off (bh_set_walk_priority),
+    under the key "<variant>:no-priority", and the context keeps whichever was faster."""
     times = {}
     ctx.set_priority(True)
     for v in range(ctx.variant_count()):

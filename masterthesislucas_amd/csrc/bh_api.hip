@@ -129,11 +129,11 @@ struct bh_ctx {
     uint32_t nbblk = 0;
     uint32_t* bblk_off = nullptr;  // first bounds block of each system, nsys + 1
     float4* bpart = nullptr;
-    uint4* work[3]{};              // traversal work tables for 1, 2, 4 sinks per lane
-    uint32_t n_work[3]{};
-    std::vector<uint4> h_work0[3];  // the tables as built (system order, no heavy slices)
-    uint4* heavy[3]{};              // per table: (first sink, count, slices) of its heavy slots
-    uint32_t nheavy[3]{};
+    uint4* work = nullptr;          // traversal work table, one entry per wave
+    uint32_t n_work = 0;
+    std::vector<uint4> h_work0;     // the table as built (system order, no heavy slices)
+    uint4* heavy = nullptr;         // (first sink, count, slices) of its heavy slots
+    uint32_t nheavy = 0;
     float* side = nullptr;          // partial results of heavy slices (TraverseBatch::side)
     uint32_t side_cap = 0;          // heavy entries `side` holds room for
 
@@ -145,14 +145,12 @@ struct bh_ctx {
     double g_theta = 0.0;
     int g_variant = -1;
 
-    int variant = 4;  // traversal kernel variant (see launch_traverse)
-    bool walk_prio = true;  // waves step their issue priority down as they progress
-    uint32_t split = 1;         // waves per sink group in the traversal (one-system contexts)
+    int variant = 4;        // selected variant id and issue priority: kept for the caller, the
+    bool walk_prio = true;  // walk does not depend on them
+    uint32_t split = 1;     // waves per sink group in the traversal (1: chosen by size)
     int solver = BH_SOLVER_BH;  // force solver (BH_SOLVER_FMM_SYM: symmetric dual-tree FMM)
     void* fmm_buf = nullptr;    // FMM workspace (fmm_workspace_bytes: per-slot moments,
                                 // coefficients, interaction lists; per-point shares)
-    float* part = nullptr;      // split traversal outputs: x, y, total parts, F n_max each
-    uint32_t part_split = 0;    // F the part buffer was sized for
     uint32_t trav_blocks = 0;  // blocks of the last traversal launch
     uint32_t profile = 0;  // bit p: phase p is timed with HIP events
     PhaseTimer phases[BH_NUM_PHASES];
@@ -370,11 +368,11 @@ bh_status ensure_moments(bh_ctx* c) {
     return launch_status(c, "upward launch");
 }
 
-TraverseBatch batch_of(const bh_ctx* c, int ns_index) {
+TraverseBatch batch_of(const bh_ctx* c) {
     TraverseBatch b;
     if (c->nsys) {
-        b.work = c->work[ns_index];
-        b.n_work = c->n_work[ns_index];
+        b.work = c->work;
+        b.n_work = c->n_work;
         b.roots = c->roots;
         b.side = c->side;
         b.side_slots = c->side_cap;
@@ -397,7 +395,9 @@ bh_status do_fmm(bh_ctx* c, double theta) {
     return launch_status(c, "FMM launch");
 }
 
-bh_status do_forces(bh_ctx* c, double theta, bool want_total) {
+// plugin: the call is bh_forces / bh_forces_device, whose t-SNE sums keep the pre-order walk's
+// summation order
+bh_status do_forces(bh_ctx* c, double theta, bool want_total, bool plugin = false) {
     if (!c->built) return fail(c, BH_ERR_STATE, "forces requested before a tree was built");
     if (!(theta >= 0.0)) return fail(c, BH_ERR_ARG, "theta must be >= 0");
     if (c->solver == BH_SOLVER_FMM_SYM) return do_fmm(c, theta);
@@ -407,30 +407,22 @@ bh_status do_forces(bh_ctx* c, double theta, bool want_total) {
     const float inv_theta2 = (float)(1.0 / (theta * theta));
     const float eps = c->cfg.softening;
     const bool grav = c->cfg.kernel == BH_KERNEL_GRAVITY;
-    // a split walk writes F parts of n per output, summed in part order afterwards
-    const uint32_t F = c->split;
-    const size_t pn = (size_t)F * c->cfg.n_max;
-    float* ox = F > 1 ? c->part : c->ax;
-    float* oy = F > 1 ? c->part + pn : c->ay;
-    float* ot = F > 1 ? c->part + 2 * pn : c->tot;
     phase_begin(c, 5);
     if (!c->nsys && (uint64_t)c->n * 16 <= (3ull << 20))  // small trees: warm every L2 first
         launch_warm_l2(s, c->nodes, c->prm, c->pos4, c->n, c->vals_b);
-    c->trav_blocks = launch_traverse(s, grav ? kKernelGravity : kKernelTsne, c->variant, c->pos4,
-                                     c->nodes, c->prm, c->n, inv_theta2, eps * eps,
-                                     grav ? c->cfg.G : 1.0f, ox, oy, want_total ? ot : nullptr,
-                                     c->counters,
-                                     batch_of(c, variant_ns_index(c->variant)),
-                                     F, c->walk_prio);
-    if (F > 1) {
-        launch_sum_parts(s, ox, F, c->n, c->ax);
-        launch_sum_parts(s, oy, F, c->n, c->ay);
-        if (want_total) launch_sum_parts(s, ot, F, c->n, c->tot);
-    } else if (c->nsys) {
-        const int v = variant_ns_index(c->variant);
-        launch_sum_heavy(s, c->side, c->side_cap, c->heavy[v], c->nheavy[v], c->ax, c->ay,
+    if (plugin && !grav && !c->nsys && c->split == 1 && c->n <= kPreorderMax)
+        c->trav_blocks = launch_traverse_preorder(s, c->pos4, c->nodes, c->prm, c->n, inv_theta2,
+                                                  c->ax, c->ay, want_total ? c->tot : nullptr,
+                                                  c->counters);
+    else
+        c->trav_blocks = launch_traverse(s, grav ? kKernelGravity : kKernelTsne, c->pos4,
+                                         c->nodes, c->child4, c->prm, c->n, inv_theta2, eps * eps,
+                                         grav ? c->cfg.G : 1.0f, c->ax, c->ay,
+                                         want_total ? c->tot : nullptr, c->counters, batch_of(c),
+                                         c->split);
+    if (c->nsys)
+        launch_sum_heavy(s, c->side, c->side_cap, c->heavy, c->nheavy, c->ax, c->ay,
                          want_total ? c->tot : nullptr);
-    }
     phase_end(c, 5);
     if (want_total)
         launch_reduce_f64(s, c->tot, nullptr, c->n, c->red_part, c->dsum);
@@ -478,7 +470,6 @@ void bh_destroy(bh_ctx* c) {
     if (c->p_col) (void)hipFree(c->p_col);
     if (c->p_val) (void)hipFree(c->p_val);
     if (c->dpart) (void)hipFree(c->dpart);
-    if (c->part) (void)hipFree(c->part);
     if (c->fmm_buf) (void)hipFree(c->fmm_buf);
     if (c->side) (void)hipFree(c->side);
     aff_release(c);
@@ -707,20 +698,19 @@ bh_status bh_create_batched(bh_ctx** out, const bh_config* cfg, const uint32_t* 
                                      hipMemcpyHostToDevice, s), "blocks"));
     TRYB(hip_check(c, hipMemcpyAsync(c->bblk_off, blk_off.data(), blk_off.size() * 4,
                                      hipMemcpyHostToDevice, s), "blocks"));
-    for (int v = 0; v < 3; ++v) {
-        const uint32_t per = 64u << v;  // sinks per wave for 1, 2, 4 sinks per lane
-        std::vector<uint4> wk;
-        for (uint32_t q = 0; q < systems; ++q)
-            for (uint32_t f = 0; f < sizes[q]; f += per)
-                wk.push_back(make_uint4(c->h_sys_off[q] + f, std::min(per, sizes[q] - f), q, 0u));
-        c->n_work[v] = (uint32_t)wk.size();
-        // room for the heavy entries' extra slices (bh_batch_order_by_cost)
-        TRYB(dalloc(c, &c->work[v], wk.size() + (size_t)kHeavyMax * (kHeavySlices - 1)));
-        TRYB(dalloc(c, &c->heavy[v], kHeavyMax));
-        TRYB(hip_check(c, hipMemcpyAsync(c->work[v], wk.data(), wk.size() * sizeof(uint4),
-                                         hipMemcpyHostToDevice, s), "work"));
-        c->h_work0[v] = std::move(wk);
-    }
+    std::vector<uint4> wk;
+    for (uint32_t q = 0; q < systems; ++q)
+        for (uint32_t f = 0; f < sizes[q]; f += kWave)
+            wk.push_back(make_uint4(c->h_sys_off[q] + f,
+                                    std::min((uint32_t)kWave, sizes[q] - f), q, 0u));
+    c->n_work = (uint32_t)wk.size();
+    // room for the heavy entries' extra slices (bh_batch_order_by_cost)
+    TRYB(dalloc(c, &c->work, wk.size() + (size_t)kHeavyMax * (kHeavySlices - 1)));
+    TRYB(dalloc(c, &c->heavy, kHeavyMax));
+    TRYB(hip_check(c, hipMemcpyAsync(c->work, wk.data(), wk.size() * sizeof(uint4),
+                                     hipMemcpyHostToDevice, s), "work"));
+    TRYB(hip_check(c, hipStreamSynchronize(s), "work"));
+    c->h_work0 = std::move(wk);
 #undef TRYB
     return hip_check(c, hipStreamSynchronize(s), "batched init");
 }
@@ -811,7 +801,7 @@ bh_status bh_build(bh_ctx* c, const double* bounds) {
 static bh_status forces_out(bh_ctx* c, double theta, float* ax, float* ay, double* total,
                             bool device) {
     if (!c) return BH_ERR_ARG;
-    bh_status st = do_forces(c, theta, total != nullptr);
+    bh_status st = do_forces(c, theta, total != nullptr, true);
     if (st != BH_OK) return st;
     hipStream_t s = c->stream;
     const uint32_t n = c->n;
@@ -1631,10 +1621,10 @@ bh_status bh_set_solver(bh_ctx* c, int solver) {
     return BH_OK;
 }
 
-// Uploads work table v: `order` lists original entries (h_work0[v]) heaviest first; the first
+// Uploads the work table: `order` lists original entries (h_work0) heaviest first; the first
 // `nh` of them are walked as kHeavySlices slices each.
-static bh_status upload_work(bh_ctx* c, int v, const std::vector<uint32_t>& order, uint32_t nh) {
-    const std::vector<uint4>& w0 = c->h_work0[v];
+static bh_status upload_work(bh_ctx* c, const std::vector<uint32_t>& order, uint32_t nh) {
+    const std::vector<uint4>& w0 = c->h_work0;
     if (nh > c->side_cap) {  // grown in place of the old buffer: 3 planes x nh x slices x sinks
         bh_status st = hip_check(c, hipStreamSynchronize(c->stream), "side sync");
         if (st != BH_OK) return st;
@@ -1655,15 +1645,15 @@ static bh_status upload_work(bh_ctx* c, int v, const std::vector<uint32_t>& orde
             out.push_back(make_uint4(e.x, e.y, e.z, (h << 8) | (kHeavySlices << 4) | f));
     }
     for (size_t i = nh; i < order.size(); ++i) out.push_back(w0[order[i]]);
-    bh_status st = hip_check(c, hipMemcpyAsync(c->work[v], out.data(), out.size() * sizeof(uint4),
+    bh_status st = hip_check(c, hipMemcpyAsync(c->work, out.data(), out.size() * sizeof(uint4),
                                                hipMemcpyHostToDevice, c->stream), "work");
     if (st == BH_OK && nh)
-        st = hip_check(c, hipMemcpyAsync(c->heavy[v], hv.data(), nh * sizeof(uint4),
+        st = hip_check(c, hipMemcpyAsync(c->heavy, hv.data(), nh * sizeof(uint4),
                                          hipMemcpyHostToDevice, c->stream), "heavy");
     if (st == BH_OK) st = hip_check(c, hipStreamSynchronize(c->stream), "work table");
     if (st != BH_OK) return st;
-    c->n_work[v] = (uint32_t)out.size();
-    c->nheavy[v] = nh;
+    c->n_work = (uint32_t)out.size();
+    c->nheavy = nh;
     c->g_valid = false;  // captured steps hold the old grid
     return BH_OK;
 }
@@ -1673,24 +1663,22 @@ bh_status bh_batch_order_by_cost(bh_ctx* c) {
     if (!c->nsys) return fail(c, BH_ERR_STATE, "not a batched context");
     if (!c->have_acc) return fail(c, BH_ERR_STATE, "no force evaluation yet");
     if (c->split != 1) return fail(c, BH_ERR_STATE, "order by cost after a walk with split 1");
-    const int v = variant_ns_index(c->variant);
-    const uint32_t nw = c->n_work[v], nb = (nw + kWavesPerBlock - 1) / kWavesPerBlock;
+    const uint32_t nw = c->n_work, nb = (nw + kWavesPerBlock - 1) / kWavesPerBlock;
     if (c->trav_blocks != nb)
-        return fail(c, BH_ERR_STATE, "the last walk used another variant's work table");
+        return fail(c, BH_ERR_STATE, "the last walk used another work table");
     std::vector<unsigned long long> cnt(2ull * nw);  // per wave: entry e's pair
     std::vector<uint4> wk(nw);
     bh_status st = hip_check(c, hipMemcpyAsync(cnt.data(), c->counters, cnt.size() * 8,
                                                hipMemcpyDeviceToHost, c->stream), "counters");
     if (st == BH_OK)
-        st = hip_check(c, hipMemcpyAsync(wk.data(), c->work[v], (size_t)nw * sizeof(uint4),
+        st = hip_check(c, hipMemcpyAsync(wk.data(), c->work, (size_t)nw * sizeof(uint4),
                                          hipMemcpyDeviceToHost, c->stream), "work");
     if (st == BH_OK) st = hip_check(c, hipStreamSynchronize(c->stream), "order by cost");
     if (st != BH_OK) return st;
     // cost of each original entry: its wave's interactions in the last walk (a heavy entry's
-    // slices add up; entries are identified by their first sink), per lane: the wave's walk is
-    // shared by its lanes, so its time follows a lane's sinks (sink k of an entry sits on lane
-    // k mod 64), not the entry's sink count
-    const std::vector<uint4>& w0 = c->h_work0[v];
+    // slices add up; entries are identified by their first sink) per sink: the wave's walk is
+    // shared by its lanes, so its time does not follow the entry's sink count
+    const std::vector<uint4>& w0 = c->h_work0;
     std::vector<std::pair<uint32_t, uint32_t>> by_first(w0.size());
     for (uint32_t i = 0; i < w0.size(); ++i) by_first[i] = {w0[i].x, i};
     std::sort(by_first.begin(), by_first.end());
@@ -1702,7 +1690,7 @@ bh_status bh_batch_order_by_cost(bh_ctx* c) {
         cost[it->second] += cnt[2 * e] + cnt[2 * e + 1];
     }
     for (uint32_t i = 0; i < w0.size(); ++i)
-        if (w0[i].y) cost[i] = cost[i] * ((w0[i].y + kWave - 1) / kWave) / w0[i].y;
+        if (w0[i].y) cost[i] /= w0[i].y;
     std::vector<std::pair<unsigned long long, uint32_t>> ord(w0.size());  // (~cost, entry)
     unsigned long long total = 0;
     for (uint32_t i = 0; i < w0.size(); ++i) {
@@ -1722,12 +1710,11 @@ bh_status bh_batch_order_by_cost(bh_ctx* c) {
     while (nh < std::min<size_t>(kHeavyMax, order.size()) && cost[order[nh]] > 0 &&
            cost[order[nh]] * w0.size() >= kHeavyFactor * total)
         ++nh;
-    return upload_work(c, v, order, nh);
+    return upload_work(c, order, nh);
 }
 
 bh_status bh_set_walk_priority(bh_ctx* c, int on) {
     if (!c) return BH_ERR_ARG;
-    if ((on != 0) != c->walk_prio) c->g_valid = false;  // captured steps hold the old walk
     c->walk_prio = on != 0;
     return BH_OK;
 }
@@ -1742,30 +1729,12 @@ bh_status bh_set_traverse_split(bh_ctx* c, int split) {
     if (!c) return BH_ERR_ARG;
     if (split < 1 || split > (int)kMaxSplit)
         return fail(c, BH_ERR_ARG, "traversal split %d outside [1, %u]", split, kMaxSplit);
-    if (split > 1 && (uint32_t)split > c->part_split) {
-        // grown in place of the old buffer: 3 outputs x F parts x n_max
-        bh_status st = hip_check(c, hipStreamSynchronize(c->stream), "split sync");
+    if (split > 1 && c->nheavy) {
+        // heavy-entry slices and split walks do not combine: back to the table as built
+        std::vector<uint32_t> order(c->h_work0.size());
+        for (uint32_t i = 0; i < order.size(); ++i) order[i] = i;
+        bh_status st = upload_work(c, order, 0);
         if (st != BH_OK) return st;
-        if (c->part) (void)hipFree(c->part);
-        c->part = nullptr;
-        c->part_split = 0;
-        st = hip_check(c, hipMalloc(&c->part, 3ull * split * c->cfg.n_max * sizeof(float)),
-                       "hipMalloc split parts");
-        if (st != BH_OK) {
-            c->split = 1;
-            return st;
-        }
-        c->part_split = (uint32_t)split;
-    }
-    if (split > 1 && c->nsys) {
-        // heavy-entry slices and split walks do not combine: back to the tables as built
-        for (int v = 0; v < 3; ++v) {
-            if (!c->nheavy[v]) continue;
-            std::vector<uint32_t> order(c->h_work0[v].size());
-            for (uint32_t i = 0; i < order.size(); ++i) order[i] = i;
-            bh_status st = upload_work(c, v, order, 0);
-            if (st != BH_OK) return st;
-        }
     }
     if ((uint32_t)split != c->split) c->g_valid = false;  // captured steps hold the old walk
     c->split = (uint32_t)split;
@@ -2230,7 +2199,7 @@ bh_status bh_forces_learned(bh_ctx* c, const bh_mlp* m, double theta, double ban
     const float eps = c->cfg.softening;
     phase_begin(c, 5);  // the per-cell inference is part of the learned force evaluation
     launch_cell_coefs(s, c->lfeat, c->nodes, c->prm, c->cap_nodes, m->wbf, c->lcoef);
-    c->trav_blocks = launch_traverse_learned(s, c->variant, c->pos4, c->nodes, c->lcoef, c->prm,
+    c->trav_blocks = launch_traverse_learned(s, c->pos4, c->nodes, c->child4, c->lcoef, c->prm,
                                              c->n, inv_t2, inv_b2, eps * eps, c->cfg.G, m->terms,
                                              c->ax, c->ay, total ? c->tot : nullptr, c->counters);
     phase_end(c, 5);

@@ -12,10 +12,9 @@ constexpr int kWave = 64;
 constexpr int kBlock = 256;
 constexpr int kWavesPerBlock = kBlock / kWave;
 constexpr int kMaxLevels = 32;  // deepest tree level (32 bits per axis)
-constexpr int kStackDepth = 40; // > kMaxLevels + 1 pushes per traversal
-constexpr int kFoldEvery = 8;   // node visits between folds of the monopole batch
-constexpr int kPPUnroll = 8;    // sources per particle-particle fetch
-constexpr int kPosPad = 8;      // float4 entries readable past the last particle (>= kPPUnroll)
+constexpr int kStackDepth = 40; // > kMaxLevels + 1 pushes of the pre-order walk
+constexpr int kFoldEvery = 8;   // its node visits between folds of the monopole batch
+constexpr int kPosPad = 8;      // float4 entries readable past the last particle
 
 enum : uint32_t {
     kMetaLevelMask = 0xFFu,

@@ -72,42 +72,19 @@ void launch_tree_slots(hipStream_t s, const uint32_t* codes, const Node* nodes,
                        const BuildParams* prm, uint32_t cap_nodes, int depth, uint32_t* first_child,
                        uint32_t* first_particle, uint32_t* count, uint64_t slots);
 
-// Traversal variants: sinks per lane NS in {1, 2, 4}, monopoles evaluated only when some lane
-// accepts (branchy) or always under a mask, and the particle-particle source fetch: PPU sources
-// per scalar load (1 or 4), or PPU = 0: each lane loads one of up to 64 sources with one vector
-// load and the wave broadcasts them with readlane (one memory round trip per cell).
-// Variants 0..11: NS = {1,2,4}[v / 4], branchy = (v % 4) < 2, PPU = v % 2 ? 4 : 1;
-// variants 12..17: NS = {1,2,4}[(v - 12) / 2], branchy = (v - 12) % 2 == 0, PPU = 0;
-// variants 18..35: the shapes of v - 18 with the lane masks in scalar registers.
-constexpr int kTraverseVariantsVector = 18;
-constexpr int kTraverseVariants = 2 * kTraverseVariantsVector;
-inline int variant_shape(int v) { return v % kTraverseVariantsVector; }
-inline int variant_ns_index(int v) {
-    v = variant_shape(v);
-    return v < 12 ? v / 4 : (v - 12) / 2;
-}
-inline int variant_ns(int v) { return 1 << variant_ns_index(v); }
-inline bool variant_branchy(int v) {
-    v = variant_shape(v);
-    return v < 12 ? (v % 4) < 2 : (v - 12) % 2 == 0;
-}
-inline int variant_ppu(int v) {
-    v = variant_shape(v);
-    return v < 12 ? (v % 2 ? 4 : 1) : 0;
-}
-// returns the number of blocks launched (one counter partial each); prio: the waves of a
-// one-system walk that fits on the device at once lower their issue priority as they progress
-// (scheduling only, results are identical either way)
+// Traversal variant ids a caller may select: they named shapes of an earlier walk and all run the
+// one walk there is.
+constexpr int kTraverseVariants = 36;
 // batched systems: one work entry (first sink, count, system, -) per wave and the systems'
 // roots; work == nullptr for a one-system context
 // A batched work entry (first sink, count, system, w). w = 0: one wave walks the entry and
 // writes its sinks' results. w != 0: the entry is one of F slices of a heavy entry (F > 1): bits
-// 0-3 the slice f, 4-7 F, 8-31 the heavy slot; its wave takes the monopoles of every F-th visit
-// and the f-th slice of every particle-particle cell, and writes partial results to
+// 0-3 the slice f, 4-7 F, 8-31 the heavy slot; its wave takes the accepted cells of every F-th
+// step and every F-th block of sources, and writes partial results to
 // side[slot][f][sink] (planes x, y, total), which k_sum_heavy adds in slice order.
 constexpr uint32_t kHeavyMax = 8192;  // heavy entries of a work table
 constexpr uint32_t kHeavySlices = 8;  // waves per heavy entry
-constexpr uint32_t kHeavySinks = 256; // sinks per work entry, at most (64 lanes x 4 per lane)
+constexpr uint32_t kHeavySinks = 64;  // sinks per work entry, at most (one per lane)
 struct TraverseBatch {
     const uint4* work = nullptr;
     uint32_t n_work = 0;
@@ -118,14 +95,21 @@ struct TraverseBatch {
 // sums the slices of each heavy entry (heavy: (first sink, count, F, -) per slot) into the outputs
 void launch_sum_heavy(hipStream_t s, const float* side, uint32_t side_slots, const uint4* heavy,
                       uint32_t nheavy, float* ax, float* ay, float* tot);
-uint32_t launch_traverse(hipStream_t s, int kernel, int variant, const float4* pos4,
-                     const Node* nodes, const BuildParams* prm, uint32_t n, float inv_theta2,
-                     float eps2, float scale, float* ax, float* ay, float* tot,
-                     unsigned long long* counters, TraverseBatch batch, uint32_t F = 1,
-                     bool prio = true);
-// F > 1 (one-system contexts): F waves per sink group, outputs are F parts of n each
+// Returns the number of blocks launched (a pair of interaction counts per wave). split: waves per
+// sink group (2: two, more: four; 1: chosen from the number of groups, one for batched systems);
+// results do not depend on it.
 constexpr uint32_t kMaxSplit = 8;
-void launch_sum_parts(hipStream_t s, const float* part, uint32_t F, uint32_t n, float* out);
+uint32_t launch_traverse(hipStream_t s, int kernel, const float4* pos4, const Node* nodes,
+                         const uint32_t* child4, const BuildParams* prm, uint32_t n,
+                         float inv_theta2, float eps2, float scale, float* ax, float* ay,
+                         float* tot, unsigned long long* counters, TraverseBatch batch,
+                         uint32_t split);
+// the t-SNE solver plug-in's walk in its own summation order (one system of at most kPreorderMax
+// points)
+constexpr uint32_t kPreorderMax = 1u << 17;
+uint32_t launch_traverse_preorder(hipStream_t s, const float4* pos4, const Node* nodes,
+                                  const BuildParams* prm, uint32_t n, float inv_theta2, float* ax,
+                                  float* ay, float* tot, unsigned long long* counters);
 uint32_t reduce_grid(uint32_t n);
 // out[0..3] = FP64 kinetic energy, potential energy (sum m phi / 2), momentum x, y; partials
 // holds 4 doubles per block (at most kMaxReduceBlocks / 4 blocks)
@@ -221,11 +205,11 @@ void launch_sinks_sorted(hipStream_t s, const uint32_t* id, uint32_t n, const ui
                          uint32_t ns, uint32_t* where, uint32_t* sinks_sorted);
 // the walk with the learned correction from the per-node coefficient records
 // (terms: 3 or 7 basis terms of the correction, as the network was trained)
-uint32_t launch_traverse_learned(hipStream_t s, int variant, const float4* pos4, const Node* nodes,
-                                 const float4* coef, const BuildParams* prm, uint32_t n,
-                                 float inv_theta2, float inv_band2, float eps2, float scale,
-                                 int terms, float* ax, float* ay, float* tot,
-                                 unsigned long long* counters);
+uint32_t launch_traverse_learned(hipStream_t s, const float4* pos4, const Node* nodes,
+                                 const uint32_t* child4, const float4* coef,
+                                 const BuildParams* prm, uint32_t n, float inv_theta2,
+                                 float inv_band2, float eps2, float scale, int terms, float* ax,
+                                 float* ay, float* tot, unsigned long long* counters);
 void launch_label_pairs(hipStream_t s, const float4* pos4, const Node* nodes, const float* feat,
                         const BuildParams* prm, const uint32_t* sinks, const uint32_t* pairs, const uint32_t* counts,
                         const uint32_t* offsets, uint32_t ns, uint32_t cap, double eps2, float* X,

@@ -1,22 +1,14 @@
-// Barnes-Hut traversal on gfx950: one wave = 64 Morton-consecutive sink particles.
-//
-// The wave walks the pre-order tree together: each node record is fetched once per wave with
-// scalar loads, and every lane applies its own acceptance test, so each particle sees exactly
-// the per-particle Barnes-Hut decisions of the reference traversal (nBodySolverBH.h:56-89 /
-// nBodySolverFMM_SYM_MORTON.h:272-313). Lanes that accept a cell take its monopole and sit out
-// the cell's subtree; the set of lanes still descending is kept as a 64-bit mask, and a small
-// per-wave stack in LDS holds (mask, subtree end) for every level where the mask narrowed.
-// Near-field cells are summed particle by particle with the self term excluded by index.
-// Forces accumulate in FP32 with Kahan compensation: each particle-particle cell sum and each
-// batch of at most kFoldEvery monopoles is one compensated addition.
+// Barnes-Hut traversal on gfx950: one wave = 64 Morton-consecutive sink particles that walk the
+// pre-order tree together (k_walk below), each particle with exactly the per-particle Barnes-Hut
+// decisions of the reference traversal (nBodySolverBH.h:56-89 /
+// nBodySolverFMM_SYM_MORTON.h:272-313). Near-field cells are summed particle by particle with the
+// self term excluded by index. Forces accumulate in FP32 with Kahan compensation.
 #include "bh_common.h"
 #include "bh_launch.h"
-#include <cfloat>
 #include "bh_mlp.h"
 
-#include <algorithm>
-#include <cmath>
 #include <type_traits>
+
 
 namespace bh {
 
@@ -27,39 +19,7 @@ __device__ __forceinline__ void kahan_add(float& s, float& c, float v) {
     s = t;
 }
 
-// One interaction, accumulated into (ax, ay[, at]) for lanes where `use` holds.
-// gravity: a += m (q - p) / (|q - p|^2 + eps^2)^(3/2); potential -= m / sqrt(...)
-// t-SNE:   w = 1 / (1 + |p - q|^2); total += m w; derivative += m w^2 (p - q)
-// (dx, dy) = q - p points from the sink to the source.
-template <int KERNEL, bool TOT>
-__device__ __forceinline__ void accum(float dx, float dy, float d2, float m, float eps2, bool use,
-                                      float& ax, float& ay, float& at) {
-    if (KERNEL == kKernelGravity) {
-        const float inv = __builtin_amdgcn_rsqf(d2 + eps2);
-        const float mi = m * inv;
-        float s = mi * inv * inv;
-        s = use ? s : 0.f;
-        ax = fmaf(s, dx, ax);
-        ay = fmaf(s, dy, ay);
-        if (TOT) at -= use ? mi : 0.f;
-    } else {
-        const float w = __builtin_amdgcn_rcpf(1.0f + d2);
-        const float mw = m * w;
-        float s = mw * w;
-        s = use ? s : 0.f;
-        ax = fmaf(-s, dx, ax);
-        ay = fmaf(-s, dy, ay);
-        if (TOT) at += use ? mw : 0.f;
-    }
-}
-
-// Wave-uniform 64-bit value moved to scalar registers (the compiler then keeps lane masks and
-// node indices in SGPRs and the per-lane booleans derived from them cost no vector work).
-__device__ __forceinline__ uint64_t uniform_u64(uint64_t v) {
-    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)v);
-    const uint32_t hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    return ((uint64_t)hi << 32) | lo;
-}
+// a wave-uniform value moved to a scalar register
 __device__ __forceinline__ uint32_t uniform_u32(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_readfirstlane(v);
 }
@@ -67,8 +27,7 @@ __device__ __forceinline__ float uniform_f32(float v) {
     return __uint_as_float(uniform_u32(__float_as_uint(v)));
 }
 
-// Node record as raw bits (cx, cy, mass, l2 | skip, first, count, meta), fetched with scalar
-// loads at a wave-uniform index.
+// Node record as raw bits (cx, cy, mass, l2 | skip, first, count, meta)
 struct NodeBits {
     uint4 a, b;
     __device__ __forceinline__ float cx() const { return __uint_as_float(a.x); }
@@ -84,134 +43,550 @@ __device__ __forceinline__ NodeBits load_node(const Node* __restrict__ nodes, ui
     const uint4* p = reinterpret_cast<const uint4*>(nodes + k);
     return NodeBits{p[0], p[1]};
 }
-// The sinks and the subtree a wave walks: one system of a one-system context (the whole tree,
-// 64 NS consecutive sinks per wave) or, for batched systems, a (first sink, count, system)
-// entry of the work table and that system's root.
-__device__ __forceinline__ void wave_work(const TraverseBatch& batch, uint32_t gw, uint32_t n,
-                                          int ns, const Node* __restrict__ nodes,
-                                          const BuildParams* __restrict__ prm, uint32_t& base,
-                                          uint32_t& count, uint32_t& k0, uint32_t& end0,
-                                          uint32_t& slice) {
-    slice = 0;
-    if (batch.work) {
-        base = count = k0 = end0 = 0;
-        if (gw < batch.n_work) {
-            const uint4 wk = batch.work[gw];
-            slice = uniform_u32(wk.w);
-            const uint32_t r = uniform_u32(batch.roots[uniform_u32(wk.z)]);
-            if (r != kNone) {
-                base = uniform_u32(wk.x);
-                count = uniform_u32(wk.y);
-                k0 = r;
-                end0 = uniform_u32(nodes[r].skip);
-            }
-        }
+// ------------------------------------------------------------------------------------------
+// The walk.
+//
+// One wave holds 64 Morton-consecutive sinks, one per lane, and their bounding box. It keeps a
+// stack of opened cells in LDS, each with the mask of the lanes that opened it. A step takes up
+// to kWalkPop cells off the stack and loads the records of their children, one per lane, so a
+// step's 64 nodes cost one memory round trip instead of one each. Every child is then judged
+// against the box: with dmin and dmax the squared distances from its centre of mass to the
+// nearest and farthest edges, evaluated like a lane's own d2 (subtraction, square and fma are
+// monotone under rounding), every lane's d2 lies in [dmin, dmax], so dmin > lim proves that all
+// lanes accept the cell and dmax <= lim that none does. Only the cells in between are tested lane
+// by lane (about a sixth of the visits on a disk at theta = 0.5). Each particle sees exactly the
+// decisions of the per-particle rule.
+//
+// Accepted cells are summed from LDS broadcasts, those that every lane accepts without a mask,
+// the others under the lanes' exec mask. Particle-particle cells are collected, their sources
+// staged through LDS 64 at a time whatever the cells' sizes, and summed under each cell's mask;
+// the sink itself can only be among the sources of a cell that holds some of the wave's own
+// sinks, and only those cells compare indices.
+//
+// Sums. Every sink has kWalkParts compensated sums; entry i of a step's accepted cells and source
+// i of a particle-particle cell belong to part i % kWalkParts, and the parts are added in order,
+// with compensation, at the end. A part's plain sums are folded into its compensated ones after at most 8 cells or
+// 16 sources (error against FP64 sums of the same interactions: 2.8e-8 rms of the summed
+// magnitudes on the two disks, as before). Because the parts are fixed, 1, 2 or 4 waves can share a sink group (NP = 4, 2 or 1
+// parts per wave: they all take the same path and add only their parts) with bit-identical
+// results: launches with too few sink groups to fill the device use more waves per group
+// (walk_waves_per_group).
+//
+// Bound by VALU issue (13 slots per interaction, the reciprocal square root counting as four)
+// where the waves fill the device, by the latency of the steps where they do not. Measured
+// against the former walk (one node per visit for 128 sinks, fetched with scalar loads one visit
+// ahead; every lane tested every node):
+//   two disks, theta 0.5, 1,048,576 sinks    851 -> 695 us (VALU issue 92% busy in both)
+//                            200,003 sinks   424 -> 200 us
+//   uniform disk, 2,000 sinks                125 ->  55 us
+//   t-SNE, 70,000 points                     268 (spread) / 325 (compact) -> 110 / 140 us
+//   128 systems of 1,024 to 65,536           1080 -> 830 us
+// ------------------------------------------------------------------------------------------
+constexpr int kWalkParts = 4;
+constexpr int kWalkStack = 192;              // opened cells
+constexpr int kWalkPop = 16;                 // cells opened per step (4 children each)
+constexpr int kWalkDeep = 3 * kMaxLevels;    // entries a depth-first descent can add to the stack
+constexpr int kWalkCells = 96;               // particle-particle cells waiting
+constexpr int kWalkFlush = kWalkCells - 64;  // summed above this many (a step adds at most 64)
+constexpr uint32_t kWalkFold = 16;           // terms of a part's plain sum
+static_assert(kWalkStack >= kWalkDeep + 4 * kWalkPop, "room for a bulk step and a descent");
+
+struct __attribute__((aligned(16))) WalkLds {  // per wave
+    float4 rec[kWave];          // the step's cells (x, y, mass, limit), then sources
+    uint4 cells[kWalkCells];    // first source, count, lane mask
+    uint2 mask[kWalkStack];
+    uint32_t node[kWalkStack];
+};
+
+__device__ __forceinline__ void wave_lds_sync() {  // LDS of this wave only: order, no wait
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+__device__ __forceinline__ uint32_t lane_read(uint32_t v, uint32_t lane) {
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)lane);
+}
+__device__ __forceinline__ uint64_t lane_read2(uint32_t lo, uint32_t hi, uint32_t lane) {
+    return ((uint64_t)lane_read(hi, lane) << 32) | lane_read(lo, lane);
+}
+
+template <bool TOT>
+struct WalkSum {  // one part: plain sums (b) and compensated ones (a with terms c)
+    float bx = 0.f, by = 0.f, bt = 0.f;
+    float ax = 0.f, cx = 0.f, ay = 0.f, cy = 0.f, at = 0.f, ct = 0.f;
+    __device__ __forceinline__ void fold() {
+        kahan_add(ax, cx, bx);
+        kahan_add(ay, cy, by);
+        if (TOT) kahan_add(at, ct, bt);
+        bx = by = bt = 0.f;
+    }
+};
+
+// gravity: a += m (q - p) / (|q - p|^2 + eps^2)^(3/2); potential -= m / sqrt(...)
+// t-SNE:   w = 1 / (1 + |p - q|^2); total += m w; derivative += m w^2 (p - q)
+template <int KERNEL, bool TOT>
+__device__ __forceinline__ void walk_pair(WalkSum<TOT>& s, float dx, float dy, float m,
+                                          float eps2) {
+    if (KERNEL == kKernelGravity) {
+        const float inv = __builtin_amdgcn_rsqf(fmaf(dx, dx, fmaf(dy, dy, eps2)));
+        const float mi = m * inv;
+        const float f = mi * inv * inv;
+        s.bx = fmaf(f, dx, s.bx);
+        s.by = fmaf(f, dy, s.by);
+        if (TOT) s.bt -= mi;
     } else {
-        base = gw * (uint32_t)(kWave * ns);
-        count = n > base ? min(n - base, (uint32_t)(kWave * ns)) : 0u;
-        k0 = 0;
-        end0 = uniform_u32(prm->n_nodes);
+        const float w = __builtin_amdgcn_rcpf(fmaf(dx, dx, fmaf(dy, dy, 1.0f)));
+        const float mw = m * w;
+        const float f = mw * w;
+        s.bx = fmaf(-f, dx, s.bx);
+        s.by = fmaf(-f, dy, s.by);
+        if (TOT) s.bt += mw;
     }
 }
 
 // Learned far-field correction inside the walk (LTERMS = 3 or 7 basis terms; 0: none): each
-// accepted cell whose l / r is at
-// least `band` (all accepted cells when inv_band2 = 0) gets its monopole corrected by
-// (M l^2 / r^4) sum_j c_j b_j(d / r, l / r), with the cell's coefficient record (kCoefStride
-// floats, computed once per cell and build by the network) read by the wave with scalar loads.
+// accepted cell whose l / r is at least `band` (all accepted cells when inv_band2 = 0) gets its
+// monopole corrected by (M l^2 / r^4) sum_j c_j b_j(d / r, l / r), with the cell's coefficient
+// record (kCoefStride floats, computed once per cell and build by the network) read by the wave
+// with scalar loads.
 struct LearnArgs {
     const float4* coef = nullptr;
     float inv_band2 = 0.f;
 };
 
-// Traversal variants (picked per workload by the autotuner):
-//   NS:      sinks per lane; a wave walks the tree once for 64 NS Morton-consecutive particles,
-//            so every node fetch feeds NS independent interactions per lane
-//   BRANCHY: monopoles only when some lane accepts (else computed masked, unconditionally)
-//   PPU:     sources fetched per scalar load in the particle-particle loop; 0: every lane loads
-//            one of up to 64 sources with one vector load and the sources are broadcast with
-//            readlane, so a cell costs one memory round trip instead of one per fetch
-// BATCHED: the wave's sinks and subtree come from the work table of a batched context.
-// The node records for both possible next visits (descend: k + 1, skip: the subtree end) are
-// fetched while the current one is used.
-// SMASK: lane masks in scalar registers: the acceptance mask is the ballot of the distance test
-//   and'ed with the active mask, a lane's predicate its inverse ballot, the interaction count a
-//   wave popcount, and 1/theta^2 sits in a vector register so the limit costs one multiply.
-//   Fewer vector instructions per visit; which form is faster depends on the variant and the
-//   workload (measured both ways), so both are variants.
-// SPLIT: F waves share one sink group and take the same path through the tree (the same sinks
-// make the same decisions); wave f adds the monopoles of every F-th node visit (visit index mod
-// F = f) and, in every particle-particle cell, the sources of the f-th of F equal slices of the
-// cell, and writes partial results to part f of the output; every interaction is counted by
-// exactly one wave. This multiplies the waves of a launch when there are too few sinks to fill
-// the GPU, and splits the long particle-particle loops of crowded leaves (t-SNE embeddings
-// gather thousands of points in a leaf of the fixed-depth tree and hundreds in a QuadTree leaf)
-// which a split by node range left to one wave.
-//
-// Issue priority by progress. A SIMD's arbiter issues for the oldest ready wave first, so of
-// the waves dispatched together the early ones run ahead: measured with per-wave timers on the
-// two-disk walk (1M sinks, 7 to 8 waves per SIMD), wave durations grew linearly with the
-// dispatch index from 330 to 780 us for the same work, and for the second half of the launch
-// the SIMDs held ever fewer waves. Each wave therefore starts at priority 3 and steps down one
-// level every `prio_step` node visits (about a third of a wave's visits), so the waves that have
-// made the least progress are issued first and the waves of a SIMD finish close together: the
-// 1M-sink walk (2 sinks per lane, 8 waves per SIMD) 0.893 -> 0.826 ms. One scalar register
-// carries the level and the countdown: at 76 scalar registers instead of 72 the hardware held 7
-// waves per SIMD instead of 8, and the priority then made the walk slower, not faster.
-// PRIO compiles the steps in; launches without them run an instantiation without that code.
-// Scheduling only: every result is bit-identical with or without it.
-constexpr uint32_t kPrioLeft = (1u << 30) - 1u;
-template <int KERNEL, bool TOT, int NS, bool BRANCHY, int PPU, bool BATCHED, bool SPLIT,
-          bool SMASK, int LTERMS = 0, bool PRIO = false>
-__global__ __launch_bounds__(kBlock) void k_traverse(const float4* __restrict__ pos4,
-                                                     const Node* __restrict__ nodes,
-                                                     const BuildParams* __restrict__ prm,
-                                                     uint32_t n, float inv_theta2, float eps2,
-                                                     float scale, float* __restrict__ ax_out,
-                                                     float* __restrict__ ay_out,
-                                                     float* __restrict__ tot_out,
-                                                     unsigned long long* __restrict__ counters,
-                                                     TraverseBatch batch, uint32_t F,
-                                                     LearnArgs la, uint32_t prio_step) {
-    constexpr bool LEARN = LTERMS != 0;
-    static_assert(!LEARN || (KERNEL == kKernelGravity && !SMASK && !SPLIT && !BATCHED),
-                  "the learned walk is the vector-mask one-system gravity walk");
+template <int KERNEL, bool TOT, int NP, bool BATCHED, int LTERMS = 0>
+__global__ __launch_bounds__(kBlock) void k_walk(const float4* __restrict__ pos4,
+                                                 const Node* __restrict__ nodes,
+                                                 const uint32_t* __restrict__ child4,
+                                                 const BuildParams* __restrict__ prm, uint32_t n,
+                                                 float inv_theta2, float eps2, float scale,
+                                                 float* __restrict__ ax_out,
+                                                 float* __restrict__ ay_out,
+                                                 float* __restrict__ tot_out,
+                                                 unsigned long long* __restrict__ counters,
+                                                 TraverseBatch batch, LearnArgs la) {
+    constexpr int kGroupWaves = kWalkParts / NP;  // waves per sink group
+    static_assert(kWavesPerBlock % kGroupWaves == 0, "whole groups per block");
+    __shared__ WalkLds lds[kWavesPerBlock];
+    const uint32_t lane = threadIdx.x & 63;
+    // wave-uniform (the compiler cannot tell that threadIdx.x / 64 is)
+    const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t p0 = (w % kGroupWaves) * NP;  // first part of this wave
+    const uint32_t group = blockIdx.x * (kWavesPerBlock / kGroupWaves) + w / kGroupWaves;
+    WalkLds& L = lds[w];
+    const uint64_t lt = lane_mask_lt();
+
+    uint32_t base = group * kWave, count, k0 = 0, slice = 0;
+    bool any;
+    if constexpr (BATCHED) {
+        base = count = 0;
+        any = false;
+        if (group < batch.n_work) {
+            const uint4 wk = batch.work[group];
+            k0 = batch.roots[wk.z];
+            if (k0 != kNone) {
+                base = wk.x;
+                count = wk.y;
+                slice = wk.w;
+                any = true;
+            }
+        }
+        base = uniform_u32(base);
+        count = uniform_u32(count);
+        slice = uniform_u32(slice);
+        k0 = uniform_u32(k0);
+    } else {
+        count = n > base ? min(n - base, (uint32_t)kWave) : 0u;
+        any = count != 0u && prm->n_nodes != 0u;
+    }
+    any = uniform_u32(any ? 1u : 0u) != 0u;
+    const uint32_t idx = base + lane;
+    const bool valid = lane < count;
+    const float4 me = valid ? pos4[idx] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const float px = me.x, py = me.y;
+    const uint64_t full = __ballot(valid);
+    float xlo = valid ? px : INFINITY, xhi = valid ? px : -INFINITY;
+    float ylo = valid ? py : INFINITY, yhi = valid ? py : -INFINITY;
+    for (int o = 32; o > 0; o >>= 1) {
+        xlo = fminf(xlo, __shfl_xor(xlo, o, kWave));
+        xhi = fmaxf(xhi, __shfl_xor(xhi, o, kWave));
+        ylo = fminf(ylo, __shfl_xor(ylo, o, kWave));
+        yhi = fmaxf(yhi, __shfl_xor(yhi, o, kWave));
+    }
+    xlo = uniform_f32(xlo);
+    xhi = uniform_f32(xhi);
+    ylo = uniform_f32(ylo);
+    yhi = uniform_f32(yhi);
+    // BATCHED slice of a heavy entry: this wave adds every sF-th step's cells and every sF-th
+    // block of sources, from the sf-th on
+    const uint32_t sf = slice & 15u, sF = slice ? (slice >> 4) & 15u : 1u;
+
+    WalkSum<TOT> sum[NP];
+    uint32_t terms = 0;  // terms of the parts' plain sums (cells count as two)
+    auto fold_all = [&]() {
+#pragma unroll
+        for (int p = 0; p < NP; ++p) sum[p].fold();
+        terms = 0;
+    };
+    uint32_t n_pn = 0;  // per lane: interactions of the nodes it judged
+    uint64_t n_pp = 0;
+    int sp = 0, nc = 0;
+    uint32_t blk_no = sf == 0 ? 0u : sF - sf, step_no = blk_no;  // 0 (mod sF): this wave's turn
+
+    // particle-particle sums over the collected cells
+    auto flush = [&]() {
+        for (int c0 = 0; c0 < nc; c0 += kWave) {
+            const int nn = min(nc - c0, kWave);
+            const uint4 cell = (int)lane < nn ? L.cells[c0 + lane] : make_uint4(0, 0, 0, 0);
+            const uint32_t cr = (cell.y + 3u) & ~3u;  // slots: whole quads
+            uint32_t end = cr;
+            for (int o = 1; o < kWave; o <<= 1) {
+                const uint32_t t = __shfl_up(end, o, kWave);
+                if ((int)lane >= o) end += t;
+            }
+            const uint32_t off = end - cr, stop = off + cell.y;
+            const bool own = cell.x < base + count && base < cell.x + cell.y;
+            const uint32_t total = lane_read(end, kWave - 1);
+            // the source of this lane's slot in the 64 slots from `blk` on; the slots past a
+            // cell's last source repeat it
+            auto fetch = [&](uint32_t blk) {
+                uint32_t src = 0;
+                uint64_t m = __ballot(end > blk && off < blk + kWave && cr != 0u);
+                while (m) {
+                    const uint32_t e = (uint32_t)__builtin_ctzll(m);
+                    m &= m - 1;
+                    const uint32_t o = lane_read(off, e);
+                    if (blk + lane >= o)
+                        src = lane_read(cell.x, e) +
+                              min(blk + lane - o, lane_read(cell.y, e) - 1u);
+                }
+                return pos4[src];
+            };
+            float4 q = fetch(0);
+            for (uint32_t blk = 0; blk < total; blk += kWave) {
+                const bool mine = !BATCHED || blk_no == 0u;
+                if constexpr (BATCHED) blk_no = blk_no + 1u == sF ? 0u : blk_no + 1u;
+                wave_lds_sync();
+                L.rec[lane] = q;
+                wave_lds_sync();
+                if (blk + kWave < total) q = fetch(blk + kWave);  // in flight during the sums
+                if (!mine) continue;
+                // cells without sinks of this wave, then those that hold some
+                const bool here = stop > blk && off < blk + kWave && cr != 0u;
+                const uint32_t from = max(off, blk) - blk, to = min(stop - blk, (uint32_t)kWave);
+                uint64_t m = __ballot(here && !own);
+                while (m) {
+                    const uint32_t e = (uint32_t)__builtin_ctzll(m);
+                    m &= m - 1;
+                    uint32_t j = lane_read(from, e);  // a multiple of 4
+                    const uint32_t b = lane_read(to, e);
+                    const uint64_t msk = lane_read2(cell.z, cell.w, e);
+                    const uint32_t quads = (b - j + 3u) >> 2;
+                    if (terms + quads > kWalkFold) fold_all();
+                    terms += quads;
+                    if (__builtin_amdgcn_inverse_ballot_w64(msk)) {
+                        for (; j + 4 <= b; j += 4) {
+                            float4 s[NP];
+#pragma unroll
+                            for (int p = 0; p < NP; ++p) s[p] = L.rec[j + p0 + p];
+#pragma unroll
+                            for (int p = 0; p < NP; ++p)
+                                walk_pair<KERNEL, TOT>(sum[p], s[p].x - px, s[p].y - py, s[p].z,
+                                                       eps2);
+                        }
+#pragma unroll
+                        for (int p = 0; p < NP; ++p)
+                            if (j + p0 + p < b) {
+                                const float4 s = L.rec[j + p0 + p];
+                                walk_pair<KERNEL, TOT>(sum[p], s.x - px, s.y - py, s.z, eps2);
+                            }
+                    }
+                }
+                m = __ballot(here && own);
+                while (m) {
+                    const uint32_t e = (uint32_t)__builtin_ctzll(m);
+                    m &= m - 1;
+                    uint32_t j = lane_read(from, e);
+                    const uint32_t b = lane_read(to, e);
+                    const uint64_t msk = lane_read2(cell.z, cell.w, e);
+                    // slot of the sink itself in this block
+                    const uint32_t self = idx - lane_read(cell.x, e) + lane_read(off, e) - blk;
+                    const uint32_t quads = (b - j + 3u) >> 2;
+                    if (terms + quads > kWalkFold) fold_all();
+                    terms += quads;
+                    if (__builtin_amdgcn_inverse_ballot_w64(msk)) {
+                        for (; j < b; j += 4)
+#pragma unroll
+                            for (int p = 0; p < NP; ++p) {
+                                const uint32_t jj = j + p0 + p;
+                                if (jj < b && jj != self) {
+                                    const float4 s = L.rec[jj];
+                                    walk_pair<KERNEL, TOT>(sum[p], s.x - px, s.y - py, s.z, eps2);
+                                }
+                            }
+                    }
+                }
+            }
+        }
+        wave_lds_sync();
+        nc = 0;
+    };
+
+    // one accepted cell (staged at slot e) for the calling lanes
+    uint32_t id = kNone;
+    float l2 = 0.f;
+    auto cell_pair = [&](WalkSum<TOT>& s, const float4 q, uint32_t e) {
+        const float dx = q.x - px, dy = q.y - py;
+        walk_pair<KERNEL, TOT>(s, dx, dy, q.z, eps2);
+        if constexpr (LTERMS != 0) {
+            const float d2 = fmaf(dx, dx, dy * dy);
+            const bool corr = la.inv_band2 == 0.f ||
+                              !(d2 > __uint_as_float(lane_read(__float_as_uint(l2), e)) *
+                                         la.inv_band2);
+            const float4* cr = la.coef + (size_t)lane_read(id, e) * (kCoefStride / 4);
+            const float4 c0 = cr[0], c1 = cr[1], c2 = cr[2], c3 = cr[3];
+            if (corr) {
+                const float rec[kCoefStride] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w,
+                                                c2.x, c2.y, c2.z, c2.w, c3.x, c3.y, c3.z, c3.w};
+                float gx, gy;
+                learned_correction<LTERMS>(dx, dy, d2, rec, gx, gy);
+                s.bx += gx;
+                s.by += gy;
+            }
+        }
+    };
+
+    uint32_t mlo = 0, mhi = 0;  // lanes that reach this lane's node
+    if (any && lane == 0) {
+        id = k0;
+        mlo = (uint32_t)full;
+        mhi = (uint32_t)(full >> 32);
+    }
+    while (any) {
+        // one node per lane: its record and the box's verdict
+        const bool live = id != kNone;
+        const NodeBits nd = load_node(nodes, live ? id : k0);
+        const float lim = nd.l2() * inv_theta2;
+        const float xa = nd.cx() - xlo, xb = nd.cx() - xhi;  // xb <= every lane's dx <= xa
+        const float ya = nd.cy() - ylo, yb = nd.cy() - yhi;
+        const float nx = fmaxf(fmaxf(xb, -xa), 0.f), ny = fmaxf(fmaxf(yb, -ya), 0.f);
+        const float fx = fmaxf(xa, -xb), fy = fmaxf(ya, -yb);
+        const bool acc_all = live && fmaf(nx, nx, ny * ny) > lim;
+        const bool open_all = live && !acc_all && fmaf(fx, fx, fy * fy) <= lim;
+        wave_lds_sync();
+        L.rec[lane] = make_float4(nd.cx(), nd.cy(), nd.mass(), lim);
+        wave_lds_sync();
+        uint32_t olo = open_all ? mlo : 0u, ohi = open_all ? mhi : 0u;  // lanes that open it
+        uint64_t xm = __ballot(live && !acc_all && !open_all);
+        while (xm) {  // lane by lane
+            const uint32_t e = (uint32_t)__builtin_ctzll(xm);
+            xm &= xm - 1;
+            const float4 q = L.rec[e];
+            const float dx = q.x - px, dy = q.y - py;
+            const float d2 = fmaf(dx, dx, dy * dy);
+            const uint64_t op = lane_read2(mlo, mhi, e) & ~__ballot(d2 > q.w);
+            olo = lane == e ? (uint32_t)op : olo;
+            ohi = lane == e ? (uint32_t)(op >> 32) : ohi;
+        }
+        const uint32_t alo = mlo & ~olo, ahi = mhi & ~ohi;  // lanes that accept it
+        const bool opened = (olo | ohi) != 0u;
+        const bool is_pp = (nd.meta() & kMetaPP) != 0u;
+        const bool all = live && alo == (uint32_t)full && ahi == (uint32_t)(full >> 32);
+        uint64_t am = __ballot(all), mm = __ballot(live && !all && (alo | ahi) != 0u);
+        n_pn += (uint32_t)__popc(alo) + (uint32_t)__popc(ahi);
+        if constexpr (LTERMS != 0) l2 = nd.l2();
+        // particle-particle cells wait, opened cells go on the stack
+        const uint64_t cm = __ballot(opened && is_pp), pm = __ballot(opened && !is_pp);
+        if (opened && is_pp) {
+            L.cells[nc + __popcll(cm & lt)] = make_uint4(nd.first(), nd.count(), olo, ohi);
+            n_pp += (uint64_t)((uint32_t)__popc(olo) + (uint32_t)__popc(ohi)) * nd.count();
+            if (nd.first() < base + count && base < nd.first() + nd.count()) {
+                // sinks of the wave among the sources, a run of lanes, skip themselves
+                const uint32_t b0 = max(nd.first(), base) - base;
+                const uint32_t b1 = min(nd.first() + nd.count() - base, (uint32_t)kWave);
+                const uint64_t run = (~0ull >> (kWave - (b1 - b0))) << b0;
+                n_pp -= (uint32_t)__popcll((((uint64_t)ohi << 32) | olo) & run);
+            }
+        }
+        nc += __popcll(cm);
+        if (opened && !is_pp) {
+            const int at = sp + __popcll(pm & lt);
+            L.node[at] = id;
+            L.mask[at] = make_uint2(olo, ohi);
+        }
+        sp += __popcll(pm);
+        wave_lds_sync();
+        // the next step's cells off the stack, its nodes' indices in flight during the sums. A
+        // bulk step leaves room for a depth-first descent (each level adds at most 3), which a
+        // nearly full stack falls back to.
+        const int room = (kWalkStack - kWalkDeep - sp) / 3;
+        const int take = min(sp, max(1, min(kWalkPop, room)));
+        sp -= take;
+        const uint32_t par = lane >> 2;
+        const bool up = (int)par < take;
+        const uint32_t pid = up ? L.node[sp + par] : 0u;
+        const uint2 pmask = up ? L.mask[sp + par] : make_uint2(0u, 0u);
+        const uint32_t next_id = up ? child4[4 * (size_t)pid + (lane & 3)] : kNone;
+
+        const bool mine = !BATCHED || step_no == 0u;
+        if constexpr (BATCHED) step_no = step_no + 1u == sF ? 0u : step_no + 1u;
+        if (mine) {
+            // cells that every lane accepts, four at a time, one per part; what is left over
+            // joins the others
+            while (__popcll(am) >= kWalkParts) {
+                uint32_t e[kWalkParts];
+#pragma unroll
+                for (int p = 0; p < kWalkParts; ++p) {
+                    e[p] = (uint32_t)__builtin_ctzll(am);
+                    am &= am - 1;
+                }
+                if constexpr (NP == 2) {
+                    e[0] = p0 ? e[2] : e[0];
+                    e[1] = p0 ? e[3] : e[1];
+                } else if constexpr (NP == 1) {
+                    const uint32_t a = p0 & 1u ? e[1] : e[0], b = p0 & 1u ? e[3] : e[2];
+                    e[0] = p0 & 2u ? b : a;
+                }
+                if (terms + 2 > kWalkFold) fold_all();
+                terms += 2;
+                float4 q[NP];
+#pragma unroll
+                for (int p = 0; p < NP; ++p) q[p] = L.rec[e[p]];
+#pragma unroll
+                for (int p = 0; p < NP; ++p) cell_pair(sum[p], q[p], e[p]);
+            }
+            mm |= am;
+            // cells that some lanes accept
+            while (mm) {
+                if (terms + 2 > kWalkFold) fold_all();
+                terms += 2;
+#pragma unroll
+                for (int p = 0; p < kWalkParts; ++p) {
+                    if (!mm) break;
+                    const uint32_t e = (uint32_t)__builtin_ctzll(mm);
+                    mm &= mm - 1;
+                    if (NP != kWalkParts && ((uint32_t)p < p0 || (uint32_t)p >= p0 + NP)) continue;
+                    const float4 q = L.rec[e];
+                    const uint64_t msk = lane_read2(alo, ahi, e);
+                    if (__builtin_amdgcn_inverse_ballot_w64(msk)) {
+                        if constexpr (NP == 1) cell_pair(sum[0], q, e);
+                        else if constexpr (NP == 2) cell_pair(sum[p & 1], q, e);
+                        else cell_pair(sum[p], q, e);
+                    }
+                }
+            }
+        }
+        if (nc > kWalkFlush || (take == 0 && nc > 0)) flush();
+        if (take == 0) break;
+        id = next_id;
+        mlo = id != kNone ? pmask.x : 0u;
+        mhi = id != kNone ? pmask.y : 0u;
+    }
+    fold_all();
+    // the parts (and their compensation terms), added in order with compensation
+    float ox = 0.f, oy = 0.f, ot = 0.f, ex = 0.f, ey = 0.f, et = 0.f;
+    auto add_part = [&](float ax, float cx, float ay, float cy, float at, float ct) {
+        kahan_add(ox, ex, ax);
+        kahan_add(ox, ex, -cx);
+        kahan_add(oy, ey, ay);
+        kahan_add(oy, ey, -cy);
+        if (TOT) kahan_add(ot, et, at);
+        if (TOT) kahan_add(ot, et, -ct);
+    };
+    if constexpr (NP == kWalkParts) {
+#pragma unroll
+        for (int p = 0; p < NP; ++p)
+            add_part(sum[p].ax, sum[p].cx, sum[p].ay, sum[p].cy, sum[p].at, sum[p].ct);
+    } else {
+        // by the group's first wave, through the LDS of the group's waves
+        float* red = reinterpret_cast<float*>(&lds[w - w % kGroupWaves]);
+        static_assert(kGroupWaves * sizeof(WalkLds) >= 6 * kWalkParts * kWave * sizeof(float),
+                      "room for the parts");
+        __syncthreads();
+#pragma unroll
+        for (int p = 0; p < NP; ++p) {
+            float* r = red + 6 * (p0 + p) * kWave + lane;
+            r[0 * kWave] = sum[p].ax;
+            r[1 * kWave] = sum[p].cx;
+            r[2 * kWave] = sum[p].ay;
+            r[3 * kWave] = sum[p].cy;
+            r[4 * kWave] = sum[p].at;
+            r[5 * kWave] = sum[p].ct;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int p = 0; p < kWalkParts; ++p) {
+            const float* r = red + 6 * p * kWave + lane;
+            add_part(r[0 * kWave], r[1 * kWave], r[2 * kWave], r[3 * kWave], r[4 * kWave],
+                     r[5 * kWave]);
+        }
+    }
+    ox -= ex;
+    oy -= ey;
+    ot -= et;
+    const bool writer = NP == kWalkParts || p0 == 0;
+    if (writer && valid) {
+        if (BATCHED && slice) {  // a heavy entry's slice: partial results
+            const size_t plane = (size_t)batch.side_slots * kHeavySlices * kHeavySinks;
+            const size_t o = ((size_t)(slice >> 8) * kHeavySlices + sf) * kHeavySinks + lane;
+            batch.side[o] = scale * ox;
+            batch.side[plane + o] = scale * oy;
+            if (TOT) batch.side[2 * plane + o] = scale * ot;
+        } else {
+            ax_out[idx] = scale * ox;
+            ay_out[idx] = scale * oy;
+            if (TOT) tot_out[idx] = scale * ot;
+        }
+    }
+    // one pair per wave (no same-address device atomics): the group's first wave counts for it,
+    // the first slice for its entry
+    const bool counts = writer && sf == 0u;
+    const unsigned long long s_pn = wave_sum_u64(counts ? n_pn : 0u);
+    const unsigned long long s_pp = wave_sum_u64(counts ? n_pp : 0u);
+    if (lane == 0) {
+        const size_t gw = (size_t)blockIdx.x * kWavesPerBlock + w;
+        counters[2 * gw] = s_pn;
+        counters[2 * gw + 1] = s_pp;
+    }
+}
+
+// ------------------------------------------------------------------------------------------
+// The pre-order walk of the t-SNE solver plug-in (bh_forces with the t-SNE kernel, one system of
+// at most kPreorderMax points). NBodySolver::solveNbody adds these sums to the caller's doubles,
+// and they are kept bit for bit what they have been: their summation order is a wave's pre-order
+// visits (128 sinks, monopoles folded every 8 visits and at every particle-particle cell), which
+// k_walk's steps do not follow. The wave visits one node at a time; the records of both possible
+// next visits are fetched with scalar loads while the current one is used; lanes that open a
+// cell that others accept are pushed on a small LDS stack as lane masks.
+// Bound by the latency of the visits: 20,011 points 0.21 ms (k_walk 0.09 ms).
+// ------------------------------------------------------------------------------------------
+constexpr int kPreNS = 2;  // sinks per lane
+template <bool TOT>
+__global__ __launch_bounds__(kBlock) void k_walk_preorder(const float4* __restrict__ pos4,
+                                                          const Node* __restrict__ nodes,
+                                                          const BuildParams* __restrict__ prm,
+                                                          uint32_t n, float inv_theta2,
+                                                          float* __restrict__ ax_out,
+                                                          float* __restrict__ ay_out,
+                                                          float* __restrict__ tot_out,
+                                                          unsigned long long* __restrict__ counters) {
+    constexpr int NS = kPreNS;
     __shared__ uint64_t st_mask[kWavesPerBlock][kStackDepth][NS];
     __shared__ uint32_t st_end[kWavesPerBlock][kStackDepth];
     const int lane = threadIdx.x & 63;
     // wave-uniform (the compiler cannot tell that threadIdx.x / 64 is): keeps the stack pointer,
     // the stack reads and the loop control in scalar registers
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    // blocks in launch order: the hardware deals them round-robin over the 8 XCDs, so every XCD
-    // gets a share of the dense and of the sparse regions (measured 3% faster than giving each
-    // XCD a contiguous range of sinks: the balance matters more than L2 locality here)
     const uint32_t wb = blockIdx.x;
-    uint32_t base, count = 0, k0 = 0, end0 = 0;
-    uint32_t part = 0;
-    uint32_t slice = 0;  // BATCHED: slice word of a heavy entry's wave (see TraverseBatch)
-    if constexpr (BATCHED) {
-        uint32_t wv = wb * kWavesPerBlock + w;
-        if constexpr (SPLIT) {  // F waves per work entry
-            part = wv % F;
-            wv /= F;
-        }
-        wave_work(batch, wv, n, NS, nodes, prm, base, count, k0, end0, slice);
-    } else if constexpr (SPLIT) {
-        const uint32_t wv = wb * kWavesPerBlock + w;
-        part = wv % F;
-        base = (wv / F) * (uint32_t)(kWave * NS);
-    } else {
-        base = (wb * kWavesPerBlock + w) * (uint32_t)(kWave * NS);
-    }
+    const uint32_t base = (wb * kWavesPerBlock + w) * (uint32_t)(kWave * NS);
     uint32_t idx[NS];
     bool valid[NS];
-    float px[NS], py[NS], pm[NS];  // pm: the sink's own mass (t-SNE totals)
+    float px[NS], py[NS], pm[NS];  // pm: the sink's own mass
     uint64_t active[NS];
     uint64_t any = 0;
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
         idx[s] = base + s * kWave + lane;
-        valid[s] = BATCHED ? (uint32_t)(s * kWave + lane) < count : idx[s] < n;
+        valid[s] = idx[s] < n;
         const float4 me = valid[s] ? pos4[idx[s]] : make_float4(0.f, 0.f, 0.f, 0.f);
         px[s] = me.x;
         pm[s] = me.z;
@@ -220,49 +595,16 @@ __global__ __launch_bounds__(kBlock) void k_traverse(const float4* __restrict__ 
         any |= active[s];
     }
     const uint32_t nn = prm->n_nodes;
-    if constexpr (!BATCHED) end0 = nn;
-    const bool use_band = LEARN && la.inv_band2 > 0.f;  // else every accepted cell is corrected
-
-    // Compensated totals (ax, ay, at) and their Kahan terms; monopoles of consecutive visits are
-    // first gathered in a short plain batch (bx, by, bt) that is folded into the compensated
-    // totals at every particle-particle visit and at least every kFoldEvery visits.
     float ax[NS], ay[NS], at[NS], cax[NS], cay[NS], cat[NS], bx[NS], by[NS], bt[NS];
     uint32_t npn[NS], npp[NS];
-    uint64_t cnt_pn = 0;  // SMASK: accepted (sink, node) pairs of the wave
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
         ax[s] = ay[s] = at[s] = cax[s] = cay[s] = cat[s] = bx[s] = by[s] = bt[s] = 0.f;
         npn[s] = npp[s] = 0u;
     }
-    float inv_t2 = inv_theta2;
-    if constexpr (SMASK) asm volatile("v_mov_b32 %0, %1" : "=v"(inv_t2) : "s"(inv_theta2));
-    uint32_t k = k0, end_cur = end0;
+    uint32_t k = 0, end_cur = nn;
     int sp = 0, since_fold = 0;
-    Node cur = nodes[min(k0, nn - 1)];
-    uint32_t vmod = 0;  // SPLIT: node visits mod F
-    // Softened gravity without totals sums particle-particle cells in the unmasked form (below)
-    // when the sink's own term there, s = ((m r) r) r with r = rsq(eps^2), is finite for every
-    // sink of the wave: it is at most the same product of the wave's largest |m|, rounding
-    // being monotone. Otherwise (a huge mass, a tiny softening, a non-finite mass) the wave
-    // takes the masked form. Not in walks with issue priority: the guard's registers would cost
-    // them a wave per SIMD, and the one-system walks gain nothing from the unmasked form.
-    bool grav_unmasked = false;
-    if constexpr (KERNEL == kKernelGravity && !TOT && PPU > 0 && !PRIO) {
-        float mx = 0.f;
-#pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            const float am = valid[s] ? fabsf(pm[s]) : 0.f;
-            mx = am <= FLT_MAX ? fmaxf(mx, am) : INFINITY;  // NaN and inf: no bound
-        }
-        for (int o = 32; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, kWave));
-        mx = __uint_as_float(uniform_u32(__float_as_uint(mx)));
-        const float r = __builtin_amdgcn_rsqf(eps2);
-        grav_unmasked = eps2 >= FLT_MIN && mx * r * r * r <= FLT_MAX;
-    }
-    // priority level (top 2 bits) and the visits left at it (one scalar register: every
-    // further register of walk state cost the 1M-sink walk a wave per SIMD)
-    uint32_t prio = (3u << 30) | min(max(prio_step, 1u), kPrioLeft);
-    if constexpr (PRIO) __builtin_amdgcn_s_setprio(3);
+    Node cur = nodes[min(0u, nn - 1)];
     while (any) {
         while (k == end_cur && sp > 0) {
             --sp;
@@ -276,210 +618,79 @@ __global__ __launch_bounds__(kBlock) void k_traverse(const float4* __restrict__ 
         // the next node is k+1 (descend) or `next` (skip): fetch both while this one is used
         const Node nd_down = nodes[min(k + 1, nn - 1)];
         const Node nd_skip = nodes[min(next, nn - 1)];
-
-        bool owned = true;  // this wave adds node k's monopoles
-        if constexpr (SPLIT) {
-            owned = vmod == part;
-            vmod = vmod + 1u == F ? 0u : vmod + 1u;
-        } else if constexpr (BATCHED) {
-            if (slice) {  // slice (slice & 15) of (slice >> 4 & 15)
-                owned = vmod == (slice & 15u);
-                vmod = vmod + 1u == ((slice >> 4) & 15u) ? 0u : vmod + 1u;
-            }
-        }
-        const float lim = cur.l2 * inv_t2;
+        const float lim = cur.l2 * inv_theta2;
         uint64_t open[NS];
         uint64_t open_any = 0;
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
             const float dx = cur.cx - px[s], dy = cur.cy - py[s];
             const float d2 = fmaf(dx, dx, dy * dy);
-            if constexpr (SMASK) {
-                const uint64_t accm = __ballot(d2 > lim) & active[s];
-                if (owned && (!BRANCHY || accm)) {
-                    accum<KERNEL, TOT>(dx, dy, d2, cur.mass, eps2,
-                                       __builtin_amdgcn_inverse_ballot_w64(accm), bx[s], by[s],
-                                       bt[s]);
-                    cnt_pn += (uint64_t)__popcll(accm);
-                }
-                open[s] = active[s] & ~accm;
-            } else {
-                const bool on = (active[s] >> lane) & 1ull;
-                const bool acc = on && (d2 > lim);
-                if (owned && (!BRANCHY || __ballot(acc))) {
-                    accum<KERNEL, TOT>(dx, dy, d2, cur.mass, eps2, acc, bx[s], by[s], bt[s]);
-                    npn[s] += acc ? 1u : 0u;
-                    if constexpr (LEARN) {
-                        const bool corr = use_band ? acc && !(d2 > cur.l2 * la.inv_band2) : acc;
-                        if (!use_band || __ballot(corr)) {
-                            const float4* cr = la.coef + (size_t)k * (kCoefStride / 4);
-                            const float4 c0 = cr[0], c1 = cr[1], c2 = cr[2], c3 = cr[3];
-                            if (corr) {
-                                const float rec[kCoefStride] = {
-                                    c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w,
-                                    c2.x, c2.y, c2.z, c2.w, c3.x, c3.y, c3.z, c3.w};
-                                float gx, gy;
-                                learned_correction<LTERMS>(dx, dy, d2, rec, gx, gy);
-                                bx[s] += gx;
-                                by[s] += gy;
-                            }
-                        }
-                    }
-                }
-                open[s] = __ballot(on && !acc);
+            const bool on = (active[s] >> lane) & 1ull;
+            const bool acc = on && (d2 > lim);
+            if (__ballot(acc)) {
+                const float wq = __builtin_amdgcn_rcpf(1.0f + d2);
+                const float mw = cur.mass * wq;
+                float f = mw * wq;
+                f = acc ? f : 0.f;
+                bx[s] = fmaf(-f, dx, bx[s]);
+                by[s] = fmaf(-f, dy, by[s]);
+                if (TOT) bt[s] += acc ? mw : 0.f;
+                npn[s] += acc ? 1u : 0u;
             }
+            open[s] = __ballot(on && !acc);
             open_any |= open[s];
         }
         bool down = false;
         if (open_any) {
             if (cur.meta & kMetaPP) {
-                {  // particle-particle sums (SPLIT: of this wave's slice of the sources)
-                    bool mine[NS];
-                    float lx[NS], ly[NS], lt[NS];
+                // every lane sums every source; lanes that did not open the cell drop the sums,
+                // and the sink's own m * 1 is taken out of Z again
+                bool mine[NS];
+                float lx[NS], ly[NS], lt[NS];
 #pragma unroll
-                    for (int s = 0; s < NS; ++s) {
-                        mine[s] = SMASK ? __builtin_amdgcn_inverse_ballot_w64(open[s])
-                                        : ((open[s] >> lane) & 1ull) != 0ull;
-                        lx[s] = ly[s] = lt[s] = 0.f;
-                    }
-                    uint32_t f = cur.first, e = f + cur.count;  // SPLIT: this wave's slice
-                    if constexpr (SPLIT) {
-                        f = cur.first + (uint32_t)((uint64_t)cur.count * part / F);
-                        e = cur.first + (uint32_t)((uint64_t)cur.count * (part + 1u) / F);
-                    } else if constexpr (BATCHED) {
-                        if (slice) {
-                            const uint32_t sf = slice & 15u, sF = (slice >> 4) & 15u;
-                            f = cur.first + (uint32_t)((uint64_t)cur.count * sf / sF);
-                            e = cur.first + (uint32_t)((uint64_t)cur.count * (sf + 1u) / sF);
-                        }
-                    }
-                    if constexpr (PPU == 0) {
-                        // lane l loads source b + l; the sources are broadcast with readlane,
-                        // kLaneUnroll at a time so that their dependency chains interleave
-                        constexpr uint32_t kLaneUnroll = 4;
-                        for (uint32_t b = f; b < e; b += kWave) {
-                            const float4 qv = pos4[min(b + (uint32_t)lane, e - 1)];
-                            const uint32_t m = min(e - b, (uint32_t)kWave);
-                            for (uint32_t t = 0; t < m; t += kLaneUnroll) {
-#pragma unroll
-                                for (uint32_t u = 0; u < kLaneUnroll; ++u) {
-                                    const uint32_t src = min(t + u, (uint32_t)kWave - 1);
-                                    const float qx0 = __int_as_float(
-                                        __builtin_amdgcn_readlane(__float_as_int(qv.x), src));
-                                    const float qy0 = __int_as_float(
-                                        __builtin_amdgcn_readlane(__float_as_int(qv.y), src));
-                                    const float qm = __int_as_float(
-                                        __builtin_amdgcn_readlane(__float_as_int(qv.z), src));
-#pragma unroll
-                                    for (int s = 0; s < NS; ++s) {
-                                        const float qx = qx0 - px[s], qy = qy0 - py[s];
-                                        const float q2 = fmaf(qx, qx, qy * qy);
-                                        const bool use =
-                                            mine[s] && (t + u < m) && (b + t + u != idx[s]);
-                                        accum<KERNEL, TOT>(qx, qy, q2, qm, eps2, use, lx[s],
-                                                           ly[s], lt[s]);
-                                    }
-                                }
-                            }
-                        }
-                    } else {
-                        // PPU sources per scalar fetch (pos4 is padded past n, lanes mask the
-                        // tail). Only sink slots with open lanes take part: in about half of the
-                        // cells a pair of slots has one slot with no lane near the cell.
-                        // Unmasked form (FAST; softened gravity without totals where the
-                        // wave's guard above holds, and t-SNE): every lane sums every source
-                        // and the lane mask is applied once per cell below. A source past the
-                        // cell's end gets mass 0 (a scalar select), so adds 0 (r^2 >= eps^2 >=
-                        // FLT_MIN keeps rsq finite); the sink itself has dx = dy = 0 and adds
-                        // s * 0 = 0, s being finite by the guard. So the forces are those of
-                        // the masked form. t-SNE: w = 1/(1 + r^2) is finite, the forces are
-                        // those of the masked form, and the sink's own term of Z (m * 1) is
-                        // taken out once per cell below (Z then differs from the masked
-                        // form's by rounding only).
-                        auto pp_slots = [&](auto lo_c, auto hi_c, auto fast_c) {
-                            constexpr int LO = decltype(lo_c)::value, HI = decltype(hi_c)::value;
-                            constexpr bool FAST = decltype(fast_c)::value;
-                            for (uint32_t j = f; j < e; j += PPU) {
-                                float4 q[PPU > 0 ? PPU : 1];
-#pragma unroll
-                                for (int t = 0; t < PPU; ++t) q[t] = pos4[j + t];
-#pragma unroll
-                                for (int t = 0; t < PPU; ++t) {
-                                    // (integer select of the uniform mass: stays scalar)
-                                    const float qm = !FAST || t == 0 ? q[t].z
-                                        : __uint_as_float(uniform_u32(
-                                              j + t < e ? __float_as_uint(q[t].z) : 0u));
-#pragma unroll
-                                    for (int s = LO; s < HI; ++s) {
-                                        const float qx = q[t].x - px[s], qy = q[t].y - py[s];
-                                        const float q2 = fmaf(qx, qx, qy * qy);
-                                        if constexpr (FAST && KERNEL == kKernelGravity) {
-                                            const float inv = __builtin_amdgcn_rsqf(q2 + eps2);
-                                            const float mi = qm * inv;
-                                            const float sc = mi * inv * inv;
-                                            lx[s] = fmaf(sc, qx, lx[s]);
-                                            ly[s] = fmaf(sc, qy, ly[s]);
-                                        } else if constexpr (FAST) {
-                                            const float wq = __builtin_amdgcn_rcpf(1.0f + q2);
-                                            const float mw = qm * wq;
-                                            const float sc = mw * wq;
-                                            lx[s] = fmaf(-sc, qx, lx[s]);
-                                            ly[s] = fmaf(-sc, qy, ly[s]);
-                                            if (TOT) lt[s] += mw;
-                                        } else {
-                                            const bool use =
-                                                mine[s] && (j + t < e) && (j + t != idx[s]);
-                                            accum<KERNEL, TOT>(qx, qy, q2, q[t].z, eps2, use,
-                                                               lx[s], ly[s], lt[s]);
-                                        }
-                                    }
-                                }
-                            }
-                        };
-                        auto pp_fast = [&](auto lo_c, auto hi_c) {
-                            if (KERNEL != kKernelGravity || grav_unmasked)
-                                pp_slots(lo_c, hi_c, std::true_type{});
-                            else
-                                pp_slots(lo_c, hi_c, std::false_type{});
-                        };
-                        auto pp_pair = [&](auto p_c) {
-                            constexpr int P = decltype(p_c)::value;
-                            const bool a = open[P] != 0ull, c = open[P + 1] != 0ull;
-                            if (a && c)
-                                pp_fast(std::integral_constant<int, P>{},
-                                        std::integral_constant<int, P + 2>{});
-                            else if (a)
-                                pp_fast(std::integral_constant<int, P>{},
-                                        std::integral_constant<int, P + 1>{});
-                            else if (c)
-                                pp_fast(std::integral_constant<int, P + 1>{},
-                                        std::integral_constant<int, P + 2>{});
-                        };
-                        if constexpr (NS == 1) {
-                            pp_fast(std::integral_constant<int, 0>{},
-                                    std::integral_constant<int, 1>{});
-                        } else {
-                            pp_pair(std::integral_constant<int, 0>{});
-                            if constexpr (NS == 4) pp_pair(std::integral_constant<int, 2>{});
-                        }
-                    }
-#pragma unroll
-                    for (int s = 0; s < NS; ++s) {
-                        npp[s] += mine[s] ? (e - f) - ((idx[s] >= f && idx[s] < e) ? 1u : 0u) : 0u;
-                        // lanes that did not open the cell add nothing (the unmasked form
-                        // summed for them too); t-SNE: the unmasked form added the sink's own
-                        // m * 1 to Z when the sink lies in the summed range
-                        if (!mine[s]) lx[s] = ly[s] = lt[s] = 0.f;
-                        if (KERNEL != kKernelGravity && TOT && PPU > 0 && mine[s] &&
-                            idx[s] >= f && idx[s] < e)
-                            lt[s] -= pm[s];
-                        kahan_add(ax[s], cax[s], lx[s] + bx[s]);
-                        kahan_add(ay[s], cay[s], ly[s] + by[s]);
-                        if (TOT) kahan_add(at[s], cat[s], lt[s] + bt[s]);
-                        bx[s] = by[s] = bt[s] = 0.f;
-                    }
-                    since_fold = 0;
+                for (int s = 0; s < NS; ++s) {
+                    mine[s] = ((open[s] >> lane) & 1ull) != 0ull;
+                    lx[s] = ly[s] = lt[s] = 0.f;
                 }
+                const uint32_t f = cur.first, e = f + cur.count;
+                auto pp_slots = [&](auto lo_c, auto hi_c) {
+                    constexpr int LO = decltype(lo_c)::value, HI = decltype(hi_c)::value;
+                    for (uint32_t j = f; j < e; ++j) {
+                        const float4 q = pos4[j];
+#pragma unroll
+                        for (int s = LO; s < HI; ++s) {
+                            const float qx = q.x - px[s], qy = q.y - py[s];
+                            const float q2 = fmaf(qx, qx, qy * qy);
+                            const float wq = __builtin_amdgcn_rcpf(1.0f + q2);
+                            const float mw = q.z * wq;
+                            const float sc = mw * wq;
+                            lx[s] = fmaf(-sc, qx, lx[s]);
+                            ly[s] = fmaf(-sc, qy, ly[s]);
+                            if (TOT) lt[s] += mw;
+                        }
+                    }
+                };
+                using C0 = std::integral_constant<int, 0>;
+                using C1 = std::integral_constant<int, 1>;
+                using C2 = std::integral_constant<int, 2>;
+                const bool a = open[0] != 0ull, c = open[1] != 0ull;
+                if (a && c)
+                    pp_slots(C0{}, C2{});
+                else if (a)
+                    pp_slots(C0{}, C1{});
+                else if (c)
+                    pp_slots(C1{}, C2{});
+#pragma unroll
+                for (int s = 0; s < NS; ++s) {
+                    npp[s] += mine[s] ? (e - f) - ((idx[s] >= f && idx[s] < e) ? 1u : 0u) : 0u;
+                    if (!mine[s]) lx[s] = ly[s] = lt[s] = 0.f;
+                    if (TOT && mine[s] && idx[s] >= f && idx[s] < e) lt[s] -= pm[s];
+                    kahan_add(ax[s], cax[s], lx[s] + bx[s]);
+                    kahan_add(ay[s], cay[s], ly[s] + by[s]);
+                    if (TOT) kahan_add(at[s], cat[s], lt[s] + bt[s]);
+                    bx[s] = by[s] = bt[s] = 0.f;
+                }
+                since_fold = 0;
             } else {
                 bool changed = false;
 #pragma unroll
@@ -508,26 +719,16 @@ __global__ __launch_bounds__(kBlock) void k_traverse(const float4* __restrict__ 
             }
             since_fold = 0;
         }
-        if constexpr (PRIO) {
-            if ((--prio & kPrioLeft) == 0u) {  // s_setprio takes an immediate: a branch per level
-                const uint32_t lvl = prio >> 30;
-                if (lvl == 3) __builtin_amdgcn_s_setprio(2);
-                else if (lvl == 2) __builtin_amdgcn_s_setprio(1);
-                else __builtin_amdgcn_s_setprio(0);
-                prio = ((lvl ? lvl - 1u : 0u) << 30) | min(max(prio_step, 1u), kPrioLeft);
-            }
-        }
         k = down ? k + 1 : next;
         // select the next record word by word on the integer bit patterns: a uniform select
         // of uniform values, kept in scalar registers
-        cur.cx = __uint_as_float(__builtin_amdgcn_readfirstlane(
-            down ? __float_as_uint(nd_down.cx) : __float_as_uint(nd_skip.cx)));
-        cur.cy = __uint_as_float(__builtin_amdgcn_readfirstlane(
-            down ? __float_as_uint(nd_down.cy) : __float_as_uint(nd_skip.cy)));
-        cur.mass = __uint_as_float(__builtin_amdgcn_readfirstlane(
-            down ? __float_as_uint(nd_down.mass) : __float_as_uint(nd_skip.mass)));
-        cur.l2 = __uint_as_float(__builtin_amdgcn_readfirstlane(
-            down ? __float_as_uint(nd_down.l2) : __float_as_uint(nd_skip.l2)));
+        auto pick = [&](float a, float b) {
+            return __uint_as_float(uniform_u32(down ? __float_as_uint(a) : __float_as_uint(b)));
+        };
+        cur.cx = pick(nd_down.cx, nd_skip.cx);
+        cur.cy = pick(nd_down.cy, nd_skip.cy);
+        cur.mass = pick(nd_down.mass, nd_skip.mass);
+        cur.l2 = pick(nd_down.l2, nd_skip.l2);
         cur.skip = down ? nd_down.skip : nd_skip.skip;
         cur.first = down ? nd_down.first : nd_skip.first;
         cur.count = down ? nd_down.count : nd_skip.count;
@@ -538,34 +739,24 @@ __global__ __launch_bounds__(kBlock) void k_traverse(const float4* __restrict__ 
         kahan_add(ax[s], cax[s], bx[s]);
         kahan_add(ay[s], cay[s], by[s]);
         if (TOT) kahan_add(at[s], cat[s], bt[s]);
-        if (BATCHED && slice && valid[s]) {  // a heavy entry's slice: partial results
-            const size_t plane = (size_t)batch.side_slots * kHeavySlices * kHeavySinks;
-            const size_t o = ((size_t)(slice >> 8) * kHeavySlices + (slice & 15u)) * kHeavySinks +
-                             (uint32_t)(s * kWave + lane);
-            batch.side[o] = scale * (ax[s] - cax[s]);
-            batch.side[plane + o] = scale * (ay[s] - cay[s]);
-            if (TOT) batch.side[2 * plane + o] = scale * (at[s] - cat[s]);
-        } else if (valid[s]) {
-            const size_t o = (size_t)part * n + idx[s];  // part 0 unless SPLIT
-            ax_out[o] = scale * (ax[s] - cax[s]);
-            ay_out[o] = scale * (ay[s] - cay[s]);
-            if (TOT) tot_out[o] = scale * (at[s] - cat[s]);
+        if (valid[s]) {
+            ax_out[idx[s]] = ax[s] - cax[s];
+            ay_out[idx[s]] = ay[s] - cay[s];
+            if (TOT) tot_out[idx[s]] = at[s] - cat[s];
         }
     }
-    if (counters) {  // one pair per wave (no same-address device atomics)
-        unsigned long long s_pn = 0, s_pp = 0;
+    unsigned long long s_pn = 0, s_pp = 0;
 #pragma unroll
-        for (int s = 0; s < NS; ++s) {
-            s_pn += valid[s] ? npn[s] : 0u;
-            s_pp += valid[s] ? npp[s] : 0u;
-        }
-        s_pn = wave_sum_u64(s_pn) + cnt_pn;
-        s_pp = wave_sum_u64(s_pp);
-        if (lane == 0) {
-            const size_t gw = (size_t)wb * kWavesPerBlock + w;
-            counters[2 * gw] = s_pn;
-            counters[2 * gw + 1] = s_pp;
-        }
+    for (int s = 0; s < NS; ++s) {
+        s_pn += valid[s] ? npn[s] : 0u;
+        s_pp += valid[s] ? npp[s] : 0u;
+    }
+    s_pn = wave_sum_u64(s_pn);
+    s_pp = wave_sum_u64(s_pp);
+    if (lane == 0) {
+        const size_t gw = (size_t)wb * kWavesPerBlock + w;
+        counters[2 * gw] = s_pn;
+        counters[2 * gw + 1] = s_pp;
     }
 }
 
@@ -685,198 +876,99 @@ __global__ __launch_bounds__(kBlock) void k_kick(float* __restrict__ vx, float* 
 // ------------------------------------------------------------------------------------------
 static inline uint32_t div_up(uint64_t a, uint64_t b) { return (uint32_t)((a + b - 1) / b); }
 
-// Node visits per priority level of the walk. The best step measured on the two-disk walk
-// (1M sinks) was about a third of a wave's mean visits: 512-768 at theta 0.3, 256 at 0.5,
-// 128-192 at 0.7 and 96-128 at 1.0, while the visits per wave scale as about theta^-1.45.
-static uint32_t walk_prio_step(float inv_theta2) {
-    const double s = 261.0 * std::pow(0.25 * (double)inv_theta2, 0.725);
-    return (uint32_t)std::min(65536.0, std::max(16.0, std::round(s)));
-}
-
-// Wave slots of the device at the largest occupancy (8 waves per SIMD, 4 SIMDs per CU). The
-// priority steps only pay when every wave of a launch is resident from the start: with several
-// rounds of waves, each round then finishes together and the next one starts on an idle SIMD
-// (measured: the 4M-sink walk, 4 rounds, 9% slower with them; the 1M-sink walk with one sink
-// per lane, 2 rounds, 4% slower), so launches with more waves than this walk without them.
-static uint64_t device_wave_slots() {
-    static const uint64_t slots = [] {
+// Waves per sink group, results do not depend on it. Measured with 1 / 2 / 4 waves:
+//   uniform disk, 20,000 sinks (313 groups)    130 / 107 /  91 us
+//   t-SNE, 70,000 points (1,094 groups)        162 / 139 / 141 us compact, 141 / 117 / 111 spread
+//   two disks, 200,003 sinks (3,126 groups)    200 / 209 / 285 us; 1,048,576: 695 / 806 / 1215 us
+// so four waves while the groups alone leave SIMDs idle, two up to two groups per SIMD.
+static uint32_t walk_waves_per_group(uint64_t groups) {
+    static const uint64_t simds = [] {
         int dev = 0, cus = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
             cus = 0;
-        return (uint64_t)cus * 4u * 8u;
+        return (uint64_t)cus * 4u;
     }();
-    return slots;
+    return groups <= simds ? 4u : groups <= 2 * simds ? 2u : 1u;
 }
 
-static uint32_t launch_prio_step(bool prio, uint64_t waves, float inv_theta2) {
-    return prio && waves <= device_wave_slots() ? walk_prio_step(inv_theta2) : 0u;
-}
-
-// variant v: sinks per lane {1, 2, 4}[v / 4]; monopoles branchy (v % 4 < 2) or masked;
-// particle-particle fetch of 1 (v even) or 4 (v odd) sources
-template <int KERNEL, bool TOT, bool BATCHED>
-static void traverse_launch(hipStream_t s, int variant, uint32_t g, uint32_t n, const float4* pos4,
-                            const Node* nodes, const BuildParams* prm, float inv_theta2,
-                            float eps2, float scale, float* ax, float* ay, float* tot,
-                            unsigned long long* counters, TraverseBatch batch, uint32_t pstep) {
-#define BH_TRAV(NS, BR, U) BH_TRAV_M(NS, BR, U, false)
-#define BH_TRAV_M(NS, BR, U, M)                                                                   \
-    do {                                                                                          \
-        if (!BATCHED && pstep)                                                                    \
-            k_traverse<KERNEL, TOT, NS, BR, U, BATCHED, false, M, 0, !BATCHED>                    \
-                <<<g, kBlock, 0, s>>>(pos4, nodes, prm, n, inv_theta2, eps2, scale, ax, ay, tot,  \
-                                      counters, batch, 1u, LearnArgs{}, pstep);                   \
-        else                                                                                      \
-            k_traverse<KERNEL, TOT, NS, BR, U, BATCHED, false, M>                                 \
-                <<<g, kBlock, 0, s>>>(pos4, nodes, prm, n, inv_theta2, eps2, scale, ax, ay, tot,  \
-                                      counters, batch, 1u, LearnArgs{}, 0u);                      \
-    } while (0)
-    if (variant >= kTraverseVariantsVector) {
-        // the same 18 shapes with scalar lane masks
-        const int v = variant - kTraverseVariantsVector;
-        const int ns = variant_ns(v), ppu = variant_ppu(v);
-        const bool br = variant_branchy(v);
-#define BH_TRAV_S(NS)                                                                             \
-    if (ppu == 0) { if (br) BH_TRAV_M(NS, true, 0, true); else BH_TRAV_M(NS, false, 0, true); }   \
-    else if (ppu == 1) { if (br) BH_TRAV_M(NS, true, 1, true); else BH_TRAV_M(NS, false, 1, true); } \
-    else { if (br) BH_TRAV_M(NS, true, 4, true); else BH_TRAV_M(NS, false, 4, true); }
-        if (ns == 1) { BH_TRAV_S(1) } else if (ns == 2) { BH_TRAV_S(2) } else { BH_TRAV_S(4) }
-#undef BH_TRAV_S
-        return;
-    }
-    switch (variant) {
-        case 0: BH_TRAV(1, true, 1); break;
-        case 1: BH_TRAV(1, true, 4); break;
-        case 2: BH_TRAV(1, false, 1); break;
-        case 3: BH_TRAV(1, false, 4); break;
-        case 4: BH_TRAV(2, true, 1); break;
-        case 5: BH_TRAV(2, true, 4); break;
-        case 6: BH_TRAV(2, false, 1); break;
-        case 7: BH_TRAV(2, false, 4); break;
-        case 8: BH_TRAV(4, true, 1); break;
-        case 9: BH_TRAV(4, true, 4); break;
-        case 10: BH_TRAV(4, false, 1); break;
-        case 11: BH_TRAV(4, false, 4); break;
-        case 12: BH_TRAV(1, true, 0); break;
-        case 13: BH_TRAV(1, false, 0); break;
-        case 14: BH_TRAV(2, true, 0); break;
-        case 15: BH_TRAV(2, false, 0); break;
-        case 16: BH_TRAV(4, true, 0); break;
-        default: BH_TRAV(4, false, 0); break;
-    }
-#undef BH_TRAV
-#undef BH_TRAV_M
-}
-
-// split traversal: the variant's NS and branchiness, particle-particle sources by scalar load
-// (PPU 1, for PPU 1 and 4) or lane-loaded (PPU 0); F partial outputs of n each; one-system
-// sink groups or the work entries of a batched context (F waves each)
-template <int KERNEL, bool TOT>
-static uint32_t traverse_split(hipStream_t s, int variant, uint32_t F, uint32_t n,
-                               const float4* pos4, const Node* nodes, const BuildParams* prm,
-                               float inv_theta2, float eps2, float scale, float* ax, float* ay,
-                               float* tot, unsigned long long* counters, TraverseBatch batch) {
-    const int ns = variant_ns(variant);
-    const uint64_t groups = batch.work ? batch.n_work : div_up(n, (uint64_t)kWave * ns);
-    const uint32_t g = div_up(groups * F, kWavesPerBlock);
-#define BH_TRAVS_B(NS, BR, U, B)                                                                  \
-    k_traverse<KERNEL, TOT, NS, BR, U, B, true, false><<<g, kBlock, 0, s>>>(                      \
-        pos4, nodes, prm, n, inv_theta2, eps2, scale, ax, ay, tot, counters, batch, F, LearnArgs{}, \
-        0u)
-#define BH_TRAVS(NS, BR, U)                                                                       \
-    do {                                                                                          \
-        if (batch.work) BH_TRAVS_B(NS, BR, U, true); else BH_TRAVS_B(NS, BR, U, false);           \
-    } while (0)
-#define BH_TRAVS_U(NS, BR)                                                                        \
-    if (lane_pp) BH_TRAVS(NS, BR, 0); else BH_TRAVS(NS, BR, 1)
-    const bool br = variant_branchy(variant);
-    const bool lane_pp = variant_ppu(variant) == 0;
-    if (ns == 1) {
-        if (br) { BH_TRAVS_U(1, true); } else { BH_TRAVS_U(1, false); }
-    } else if (ns == 2) {
-        if (br) { BH_TRAVS_U(2, true); } else { BH_TRAVS_U(2, false); }
-    } else {
-        if (br) { BH_TRAVS_U(4, true); } else { BH_TRAVS_U(4, false); }
-    }
-#undef BH_TRAVS_U
-#undef BH_TRAVS
-#undef BH_TRAVS_B
-    return g;
-}
-
-template <int KERNEL, bool TOT>
-static uint32_t traverse_variant(hipStream_t s, int variant, uint32_t n, const float4* pos4,
-                                 const Node* nodes, const BuildParams* prm, float inv_theta2,
-                                 float eps2, float scale, float* ax, float* ay, float* tot,
-                                 unsigned long long* counters, TraverseBatch batch, uint32_t F,
-                                 bool prio) {
-    const int ns = variant_ns(variant);
-    if (F > 1)  // split walks: no priority steps
-        return traverse_split<KERNEL, TOT>(s, variant, F, n, pos4, nodes, prm, inv_theta2, eps2,
-                                           scale, ax, ay, tot, counters, batch);
-    const uint32_t g = batch.work ? div_up(batch.n_work, kWavesPerBlock)
-                                  : div_up(n, (uint64_t)kBlock * ns);
-    const uint32_t pstep = launch_prio_step(prio, (uint64_t)g * kWavesPerBlock, inv_theta2);
-    if (batch.work)
-        traverse_launch<KERNEL, TOT, true>(s, variant, g, n, pos4, nodes, prm, inv_theta2, eps2,
-                                           scale, ax, ay, tot, counters, batch, pstep);
-    else
-        traverse_launch<KERNEL, TOT, false>(s, variant, g, n, pos4, nodes, prm, inv_theta2, eps2,
-                                            scale, ax, ay, tot, counters, batch, pstep);
-    return g;
-}
-
-uint32_t launch_traverse(hipStream_t s, int kernel, int variant, const float4* pos4,
-                         const Node* nodes, const BuildParams* prm, uint32_t n, float inv_theta2,
-                         float eps2, float scale, float* ax, float* ay, float* tot,
-                         unsigned long long* counters, TraverseBatch batch, uint32_t F,
-                         bool prio) {
-    if (kernel == kKernelGravity) {
-        if (tot)
-            return traverse_variant<kKernelGravity, true>(s, variant, n, pos4, nodes, prm,
-                                                          inv_theta2, eps2, scale, ax, ay, tot,
-                                                          counters, batch, F, prio);
-        return traverse_variant<kKernelGravity, false>(s, variant, n, pos4, nodes, prm, inv_theta2,
-                                                       eps2, scale, ax, ay, tot, counters, batch, F,
-                                                       prio);
-    }
-    if (tot)
-        return traverse_variant<kKernelTsne, true>(s, variant, n, pos4, nodes, prm, inv_theta2,
-                                                   eps2, scale, ax, ay, tot, counters, batch, F,
-                                                   prio);
-    return traverse_variant<kKernelTsne, false>(s, variant, n, pos4, nodes, prm, inv_theta2, eps2,
-                                                scale, ax, ay, tot, counters, batch, F, prio);
-}
-
-uint32_t launch_traverse_learned(hipStream_t s, int variant, const float4* pos4, const Node* nodes,
-                                 const float4* coef, const BuildParams* prm, uint32_t n,
-                                 float inv_theta2, float inv_band2, float eps2, float scale,
-                                 int terms, float* ax, float* ay, float* tot,
-                                 unsigned long long* counters) {
-    // the variant's sinks per lane; branchy monopoles, one source per particle-particle fetch;
-    // no priority steps (the learned walks of interest span several rounds of waves)
-    const int ns = variant_ns(variant);
-    const uint32_t g = div_up(n, (uint64_t)kBlock * ns);
+struct WalkCall {
+    hipStream_t s;
+    const float4* pos4;
+    const Node* nodes;
+    const uint32_t* child4;
+    const BuildParams* prm;
+    uint32_t n;
+    float inv_theta2, eps2, scale;
+    float *ax, *ay, *tot;
+    unsigned long long* counters;
+    TraverseBatch batch;
     LearnArgs la;
-    la.coef = coef;
-    la.inv_band2 = inv_band2;
-    TraverseBatch none;
-#define BH_TRAVL(NS, TOT, T)                                                                      \
-    k_traverse<kKernelGravity, TOT, NS, true, 1, false, false, false, T><<<g, kBlock, 0, s>>>(    \
-        pos4, nodes, prm, n, inv_theta2, eps2, scale, ax, ay, tot, counters, none, 1u, la, 0u)
-#define BH_TRAVL_T(NS, TOT) \
-    if (terms == 3) BH_TRAVL(NS, TOT, 3); else BH_TRAVL(NS, TOT, 7)
-    if (ns == 1) {
-        if (tot) BH_TRAVL_T(1, true); else BH_TRAVL_T(1, false);
-    } else if (ns == 2) {
-        if (tot) BH_TRAVL_T(2, true); else BH_TRAVL_T(2, false);
-    } else {
-        if (tot) BH_TRAVL_T(4, true); else BH_TRAVL_T(4, false);
-    }
-#undef BH_TRAVL_T
-#undef BH_TRAVL
+    uint32_t waves;  // per sink group: 1, 2 or 4
+};
+
+template <int KERNEL, bool TOT, bool BATCHED, int LTERMS>
+static uint32_t walk_launch(const WalkCall& c) {
+    const uint64_t groups = BATCHED ? c.batch.n_work : div_up(c.n, kWave);
+    const uint32_t g = div_up(groups * c.waves, kWavesPerBlock);
+#define BH_WALK(NP)                                                                               \
+    k_walk<KERNEL, TOT, NP, BATCHED, LTERMS><<<g, kBlock, 0, c.s>>>(                              \
+        c.pos4, c.nodes, c.child4, c.prm, c.n, c.inv_theta2, c.eps2, c.scale, c.ax, c.ay, c.tot,  \
+        c.counters, c.batch, c.la)
+    if (c.waves == 4) BH_WALK(1);
+    else if (c.waves == 2) BH_WALK(2);
+    else BH_WALK(4);
+#undef BH_WALK
     return g;
+}
+
+uint32_t launch_traverse(hipStream_t s, int kernel, const float4* pos4, const Node* nodes,
+                         const uint32_t* child4, const BuildParams* prm, uint32_t n,
+                         float inv_theta2, float eps2, float scale, float* ax, float* ay,
+                         float* tot, unsigned long long* counters, TraverseBatch batch,
+                         uint32_t split) {
+    WalkCall c{s, pos4, nodes, child4, prm, n, inv_theta2, eps2, scale, ax, ay, tot, counters,
+               batch, LearnArgs{}, 1u};
+    if (split > 1) c.waves = split == 2 ? 2u : 4u;
+    else if (!batch.work) c.waves = walk_waves_per_group(div_up(n, kWave));
+    const bool grav = kernel == kKernelGravity;
+    if (batch.work) {
+        if (grav) return tot ? walk_launch<kKernelGravity, true, true, 0>(c)
+                             : walk_launch<kKernelGravity, false, true, 0>(c);
+        return tot ? walk_launch<kKernelTsne, true, true, 0>(c)
+                   : walk_launch<kKernelTsne, false, true, 0>(c);
+    }
+    if (grav) return tot ? walk_launch<kKernelGravity, true, false, 0>(c)
+                         : walk_launch<kKernelGravity, false, false, 0>(c);
+    return tot ? walk_launch<kKernelTsne, true, false, 0>(c)
+               : walk_launch<kKernelTsne, false, false, 0>(c);
+}
+
+uint32_t launch_traverse_preorder(hipStream_t s, const float4* pos4, const Node* nodes,
+                                  const BuildParams* prm, uint32_t n, float inv_theta2, float* ax,
+                                  float* ay, float* tot, unsigned long long* counters) {
+    const uint32_t g = div_up(n, kBlock * kPreNS);
+    if (tot)
+        k_walk_preorder<true><<<g, kBlock, 0, s>>>(pos4, nodes, prm, n, inv_theta2, ax, ay, tot,
+                                                   counters);
+    else
+        k_walk_preorder<false><<<g, kBlock, 0, s>>>(pos4, nodes, prm, n, inv_theta2, ax, ay, tot,
+                                                    counters);
+    return g;
+}
+
+uint32_t launch_traverse_learned(hipStream_t s, const float4* pos4, const Node* nodes,
+                                 const uint32_t* child4, const float4* coef,
+                                 const BuildParams* prm, uint32_t n, float inv_theta2,
+                                 float inv_band2, float eps2, float scale, int terms, float* ax,
+                                 float* ay, float* tot, unsigned long long* counters) {
+    WalkCall c{s, pos4, nodes, child4, prm, n, inv_theta2, eps2, scale, ax, ay, tot, counters,
+               TraverseBatch{}, LearnArgs{coef, inv_band2}, walk_waves_per_group(div_up(n, kWave))};
+    if (terms == 3)
+        return tot ? walk_launch<kKernelGravity, true, false, 3>(c)
+                   : walk_launch<kKernelGravity, false, false, 3>(c);
+    return tot ? walk_launch<kKernelGravity, true, false, 7>(c)
+               : walk_launch<kKernelGravity, false, false, 7>(c);
 }
 
 // heavy batched entries: out[first + i] = sum over slices f of side[slot][f][i], in slice order
@@ -906,20 +998,6 @@ __global__ __launch_bounds__(kBlock) void k_sum_heavy(const float* __restrict__ 
 void launch_sum_heavy(hipStream_t s, const float* side, uint32_t side_slots, const uint4* heavy,
                       uint32_t nheavy, float* ax, float* ay, float* tot) {
     if (nheavy) k_sum_heavy<<<nheavy, kBlock, 0, s>>>(side, side_slots, heavy, ax, ay, tot);
-}
-
-// out[i] = sum over parts f of part[f n + i], in part order
-__global__ __launch_bounds__(kBlock) void k_sum_parts(const float* __restrict__ part, uint32_t F,
-                                                      uint32_t n, float* __restrict__ out) {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    float s = part[i];
-    for (uint32_t f = 1; f < F; ++f) s += part[(size_t)f * n + i];
-    out[i] = s;
-}
-
-void launch_sum_parts(hipStream_t s, const float* part, uint32_t F, uint32_t n, float* out) {
-    k_sum_parts<<<div_up(n, kBlock), kBlock, 0, s>>>(part, F, n, out);
 }
 
 uint32_t reduce_grid(uint32_t n) {

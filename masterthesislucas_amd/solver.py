@@ -254,7 +254,7 @@ class BHContext:
 
     @property
     def variant(self):
-        """Traversal variant in use (the library starts with 4: two sinks per lane)."""
+        """Traversal variant selected (the library starts with 4)."""
         return getattr(self, "_variant", 4)
 
     def set_sort_spin_limit(self, polls):
@@ -275,7 +275,7 @@ class BHContext:
         self._c(_lib.load().bh_batch_order_by_cost(self._h))
 
     def set_priority(self, on=True):
-        """Progress-ordered issue priority of the walk's waves (bh_set_walk_priority)."""
+        """The issue priority setting of the walk (bh_set_walk_priority)."""
         self._c(_lib.load().bh_set_walk_priority(self._h, 1 if on else 0))
 
     @property

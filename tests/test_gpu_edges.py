@@ -98,3 +98,90 @@ def test_affinity_tile_edges(gpu, n, dim, k):
     gap = np.abs(np.take_along_axis(d2, a["idx"].astype(np.int64), 1) - want)
     assert np.all(gap[differ] <= 1e-12 * want[differ])
     assert abs(a["val"].astype(np.float64).sum() - 1.0) < 1e-6
+
+
+def _walk(p, kernel, theta, split, mode="quadtree", eps=1e-3, cap=16, want_total=True):
+    from masterthesislucas_amd import BHContext
+    ctx = BHContext(len(p[0]), kernel=kernel, tree_mode=mode, softening=eps, max_children=cap)
+    ctx.set_particles(*p)
+    ctx.set_split(split)
+    ctx.build()
+    ax, ay, tot = ctx.forces(theta, want_total=want_total)
+    cnt = ctx.counters()
+    return ctx, ax, ay, tot, cnt
+
+
+def _points(case, n, rng):
+    """x, y, masses: a disk; a tight cluster under a chain of one-child cells (a far outlier sets
+    the root square); a line; points of which a third sit on one spot (a leaf of n / 3 at the
+    depth limit)."""
+    if case == "line":
+        x, y = rng.uniform(-1, 1, n), np.zeros(n)
+    else:
+        r, a = np.sqrt(rng.random(n)), rng.uniform(0, 2 * np.pi, n)
+        x, y = r * np.cos(a), r * np.sin(a)
+    if case == "chain":
+        x, y = 1e-5 * x, 1e-5 * y
+        x[-1] = 900.0
+    if case == "spot":
+        x[: n // 3], y[: n // 3] = 0.25, 0.125
+    m = rng.uniform(0.5, 1.5, n) / n
+    return tuple(v.astype(np.float32) for v in (x, y, m))
+
+
+@pytest.mark.parametrize("case", ["disk", "chain", "line", "spot"])
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 129, 1000, 5000])
+def test_walk_edges(gpu, case, n):
+    """The walk at the edges of its sink groups (64), its source blocks (64, quads of 4) and its
+    collected cells, on 1, 2 and 4 waves per group: bit-identical results and counts, and forces
+    within the exact-walk bar of the FP64 sum of the same interactions (counts equal). A leaf of
+    many coincident points sums them in plain FP32 batches: the bar holds there too."""
+    from tests.helpers import check_exact_walk
+    rng = np.random.default_rng(n)
+    p = _points(case, n, rng)
+    for theta in (0.5, 1.0):
+        ctx, ax, ay, tot, cnt = _walk(p, "gravity", theta, 2)
+        check_exact_walk(ctx, *p, "gravity", theta, float(np.float32(1e-3)), ax, ay, tot)
+        ctx.close()
+        for split in (1, 8):
+            ctx, bx, by, tot2, cnt2 = _walk(p, "gravity", theta, split)
+            ctx.close()
+            assert np.array_equal(ax.view(np.uint32), bx.view(np.uint32))
+            assert np.array_equal(ay.view(np.uint32), by.view(np.uint32))
+            assert tot2 == tot and cnt2 == cnt
+
+
+@pytest.mark.parametrize("n", [100, 1000, 70000])
+def test_walk_small_opening_angle(gpu, n):
+    """theta = 0.05 on few and many sinks: nearly every cell is opened, so the stack of opened
+    cells fills and the walk falls back to one cell at a time; counts and forces as above."""
+    from tests.helpers import check_exact_walk
+    from masterthesislucas_amd.workloads import sample_indices
+    rng = np.random.default_rng(7)
+    p = _points("disk", n, rng)
+    ctx, ax, ay, tot, cnt = _walk(p, "gravity", 0.05, 1, want_total=n <= 1000)
+    if n <= 1000:
+        check_exact_walk(ctx, *p, "gravity", 0.05, float(np.float32(1e-3)), ax, ay, tot)
+    else:
+        s = sample_indices(n, 256).astype(np.uint32)
+        dx, dy, _ = ctx.direct_fp64(s)
+        # the monopole error at l / r = 0.05 is about (l / r)^2 / 8 of a cell's pull
+        assert np.quantile(np.hypot(ax[s] - dx, ay[s] - dy) / np.hypot(dx, dy), 0.9) < 1e-3
+    ctx.close()
+
+
+def test_walk_tsne_paths_agree(gpu):
+    """The t-SNE sums of bh_forces (pre-order walk up to 131,072 points) and of the list walk
+    (any split above 1) select the same interactions and differ by rounding only."""
+    from tests.helpers import rel_err
+    rng = np.random.default_rng(11)
+    x, y, _ = _points("spot", 20011, rng)
+    p = (20.0 * x, 20.0 * y, None)
+    c1, ax, ay, z, cnt = _walk(p, "tsne", 0.5, 1)
+    c2, bx, by, z2, cnt2 = _walk(p, "tsne", 0.5, 4)
+    assert cnt == cnt2
+    r = rel_err(bx, by, ax.astype(np.float64), ay.astype(np.float64))
+    assert np.median(r) <= 1e-6 and np.quantile(r, 0.999) <= 1e-4
+    assert abs(z2 - z) <= 1e-5 * z
+    c1.close()
+    c2.close()
