@@ -285,7 +285,7 @@ bh_status bh_learned_export(bh_ctx* ctx, const bh_mlp* mlp, float* features, flo
  * cudaHelper.cuh:22-31) ----
  * Every call that builds a tree (bh_build, bh_leapfrog, bh_leapfrog_graph, bh_tsne_step,
  * bh_tsne_run, bh_tsne_kl) returns BH_ERR_ARG when a particle position is NaN or infinite (the
- * bounds pass flags it) and BH_ERR_HIP when the radix sort's look-back gave up waiting (the
+ * bounds pass flags it) and BH_ERR_HIP when the sort's look-back gave up waiting (the
  * order would not be valid); the tree is then marked unbuilt. Set the look-back bound (polls of
  * a tile waiting on an earlier tile; default 2^22, a wait that always ends on a working device)
  * to a small value only to exercise that error path. */

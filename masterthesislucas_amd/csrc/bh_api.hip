@@ -62,7 +62,7 @@ struct bh_ctx {
     float *out_a = nullptr, *out_b = nullptr, *out_c = nullptr, *out_d = nullptr;
     void *keys_a = nullptr, *keys_b = nullptr;
     uint32_t *vals_a = nullptr, *vals_b = nullptr;
-    uint32_t* sort_scratch = nullptr;  // radix sort counts, look-back words, totals, tickets
+    uint32_t* sort_scratch = nullptr;  // sort counts, look-back words, totals, tickets
     uint32_t* scan_part = nullptr;
     uint8_t *leaf_lvl = nullptr, *lcp1 = nullptr;
     uint32_t *cnt = nullptr, *noff = nullptr;
@@ -251,7 +251,7 @@ bh_status status_check(bh_ctx* c) {
         c->built = false;
         c->have_acc = false;
         return fail(c, BH_ERR_HIP,
-                    "radix sort: a look-back wait exceeded %u polls; the sort order is not valid",
+                    "sort: a look-back wait exceeded %u polls; the sort order is not valid",
                     c->sort_spin);
     }
     return BH_OK;
@@ -318,7 +318,7 @@ bh_status do_build(bh_ctx* c, const double* bounds) {
     phase_begin(c, 1);
     bool in_b = false;
     const int key_bits = c->nsys ? 2 * c->qbits + 2 * c->R : 2 * c->B;
-    launch_radix_sort(s, c->keys_a, c->vals_a, c->keys_b, c->vals_b, n, key_bits, c->wide,
+    launch_sort(s, c->keys_a, c->vals_a, c->keys_b, c->vals_b, n, key_bits, c->wide,
                       c->sort_scratch, c->dstatus, c->sort_spin, &in_b);
     phase_end(c, 1);
     c->keys_in_b = in_b;
@@ -1338,7 +1338,7 @@ bh_status bh_tsne_affinities(bh_ctx* c, const float* X, uint32_t n, uint32_t dim
             int key_bits = 1;
             while (key_bits < 64 && ((uint64_t)n * n - 1) >> key_bits) ++key_bits;
             bool in_b = false;
-            launch_radix_sort(s, keys_a, vals_a, keys_b, vals_b, m, key_bits, true, scratch,
+            launch_sort(s, keys_a, vals_a, keys_b, vals_b, m, key_bits, true, scratch,
                               flags + 1, kSortSpinLimit, &in_b);
             const uint64_t* ks = in_b ? keys_b : keys_a;
             const uint32_t* vs = in_b ? vals_b : vals_a;
@@ -1362,7 +1362,7 @@ bh_status bh_tsne_affinities(bh_ctx* c, const float* X, uint32_t n, uint32_t dim
     if (st == BH_OK && knn_d2) st = hip_check(c, hipMemcpy(knn_d2, d2, nk * 8, hipMemcpyDeviceToHost), "d2");
     if (st == BH_OK && beta) st = hip_check(c, hipMemcpy(beta, dbeta, (size_t)n * 8, hipMemcpyDeviceToHost), "beta");
     if (st == BH_OK) st = hip_check(c, hipStreamSynchronize(s), "affinities");
-    if (st == BH_OK && h_flags[5]) st = fail(c, BH_ERR_HIP, "the radix sort gave up waiting");
+    if (st == BH_OK && h_flags[5]) st = fail(c, BH_ERR_HIP, "the sort gave up waiting");
     const uint32_t nz = h_flags[6];
     if (st == BH_OK && (nz == 0 || nz > m)) st = fail(c, BH_ERR_HIP, "bad nonzero count %u", nz);
     if (st == BH_OK) {

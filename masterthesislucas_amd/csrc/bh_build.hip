@@ -338,7 +338,8 @@ __global__ __launch_bounds__(kBlock) void k_scan_down(const uint32_t* __restrict
 }
 
 // ------------------------------------------------------------------------------------------
-// LSD radix sort, 8-bit digits, one launch per pass after one counting launch ("one-sweep").
+// LSD radix sort, 8-bit digits, one launch per pass after one counting launch ("one-sweep"),
+// for more than kBucketSortMax keys.
 //   k_radix_counts: one block per 4096-key tile; the tile's digit counts for every pass (the
 //     multiset of digits of a pass does not depend on the order) and the clearing of the tile's
 //     look-back words of every pass.
@@ -352,18 +353,61 @@ __global__ __launch_bounds__(kBlock) void k_scan_down(const uint32_t* __restrict
 // only waits on tiles whose tickets were taken before its own (their blocks are running), so
 // every wait ends.
 // ------------------------------------------------------------------------------------------
-// Tiles of 4096 keys for large sorts, 2048 for sorts of at most kSortSmallMax keys (more
-// blocks share a small sort: 70k keys 20% faster, while 1M keys are 14% slower with them).
-// kSortItems* is the tile in keys per thread of a 256-thread block (the counting kernel); the
-// pass kernel ranks a tile with 4 keys per lane (1024 threads, or 512 for small tiles), which
-// measured faster than 8 or 16 keys per lane on fewer waves.
+// Tiles of 4096 keys for large sorts, 2048 for sorts of at most kSortSmallMax keys (more blocks
+// share a small sort). kSortItems* is the tile in keys per thread of a 256-thread block; the
+// kernels take a tile with 4 keys per lane, which measured faster in the radix pass than 8 or 16
+// keys per lane on fewer waves.
 constexpr int kSortItemsLarge = 16, kSortItemsSmall = 8;
 constexpr uint32_t kSortSmallMax = 1u << 18;  // sorts up to this size use the small tiles
 __host__ __device__ constexpr int sort_tile(int items) { return kBlock * items; }
 constexpr int kSortMaxPasses = 8;
 constexpr uint32_t kLbCount = 1u << 30, kLbPrefix = 2u << 30, kLbMask = kLbCount - 1;
 constexpr int kLbWindow = 8;  // look-back loads in flight per digit
+// the sample-based sorts below
+constexpr uint32_t kRankSortMax = 8192, kBucketSortMax = 1u << 21;
+static_assert(kSortMaxPasses * 256 >= 2048, "bucket look-back words fit the radix sort's");
+constexpr int kBucketMax = 2048, kBucketSamples = 8 * kBucketMax, kBucketItems = 4, kBucketItemsMax = 8;
 static_assert(kBlock == 256, "one thread per digit");
+
+// The sum of a digit's counts over the tiles before `tile` (> 0), whose words of the digit stand
+// `stride` apart from `status` on: kLbWindow tiles per round with independent loads, nearest
+// first; stops at the first inclusive prefix (tile 0 always publishes one), waits at a tile not
+// ready.
+__device__ __forceinline__ uint32_t look_back(const uint32_t* __restrict__ status, uint32_t stride,
+                                              uint32_t tile, uint32_t* __restrict__ err,
+                                              uint32_t spin_limit) {
+    int j = (int)tile - 1;
+    uint32_t excl = 0, spins = 0;
+    bool done = false;
+    while (!done) {
+        uint32_t v[kLbWindow];
+#pragma unroll
+        for (int k = 0; k < kLbWindow; ++k)
+            v[k] = j - k >= 0 ? __hip_atomic_load(status + (size_t)(j - k) * stride,
+                                                  __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
+                              : kLbPrefix;
+        int used = 0;
+#pragma unroll
+        for (int k = 0; k < kLbWindow; ++k) {
+            if (done || used < k) continue;  // stopped earlier in this round
+            if ((v[k] & ~kLbMask) == 0u) continue;  // not ready: poll again from here
+            excl += v[k] & kLbMask;
+            done = (v[k] & kLbPrefix) != 0u;
+            used = k + 1;
+        }
+        j -= used;
+        if (!done && used < kLbWindow) {
+            // never expected: record it and stop waiting. The tile's prefix is then short of the
+            // true one, so this and every later tile still place their keys inside [0, n)
+            if (++spins > spin_limit) {
+                __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
+    }
+    return excl;
+}
 
 template <typename K, int THREADS, int ITEMS>
 __global__ __launch_bounds__(THREADS) void k_radix_counts(const K* __restrict__ keys, uint32_t n,
@@ -501,39 +545,7 @@ __global__ __launch_bounds__(THREADS) void k_radix_pass(const K* __restrict__ ke
             excl = block_exclusive_scan_t<THREADS>(dig ? totals[d] : 0u, &tot);
         } else if (dig) {
             __hip_atomic_store(mine, kLbCount | cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            // look back kLbWindow tiles per round with independent loads, nearest first; stop at
-            // the first inclusive prefix (tile 0 always publishes one), wait at a tile not ready
-            int j = (int)tile - 1;
-            uint32_t spins = 0;
-            bool done = false;
-            while (!done) {
-                uint32_t v[kLbWindow];
-#pragma unroll
-                for (int k = 0; k < kLbWindow; ++k)
-                    v[k] = j - k >= 0 ? __hip_atomic_load(status + (size_t)(j - k) * 256 + d,
-                                                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                                      : kLbPrefix;
-                int used = 0;
-#pragma unroll
-                for (int k = 0; k < kLbWindow; ++k) {
-                    if (done || used < k) continue;  // stopped earlier in this round
-                    if ((v[k] & ~kLbMask) == 0u) continue;  // not ready: poll again from here
-                    excl += v[k] & kLbMask;
-                    done = (v[k] & kLbPrefix) != 0u;
-                    used = k + 1;
-                }
-                j -= used;
-                if (!done && used < kLbWindow) {
-                    // never expected: record it and stop waiting. The tile's prefix is then
-                    // short of the true one, so this and every later tile still place their
-                    // keys inside [0, n)
-                    if (++spins > spin_limit) {
-                        __hip_atomic_store(err, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        break;
-                    }
-                    __builtin_amdgcn_s_sleep(1);
-                }
-            }
+            excl = look_back(status + d, 256, tile, err, spin_limit);
         }
         if (dig) {
             __hip_atomic_store(mine, kLbPrefix | (excl + cnt), __ATOMIC_RELAXED,
@@ -559,6 +571,433 @@ __global__ __launch_bounds__(THREADS) void k_radix_pass(const K* __restrict__ ke
         keys_out[g] = k;
         vals_out[g] = s_vals[p];
     }
+}
+
+// ------------------------------------------------------------------------------------------
+// Sorts of up to kBucketSortMax keys. vals holds 0 .. n-1 on entry, so an order by (key, value)
+// is the stable order, and every pair is distinct.
+//   k_rank_sort: each key's rank is counted against all others, 64 keys per block. The other key
+//     is a scalar operand, so a comparison is two vector instructions. One launch; used for whole
+//     sorts of at most kRankSortMax keys and for the sample of the larger ones.
+//   k_bucket_prepare: a sample of the keys, one from each of equal strata of the input, and the
+//     clearing of the look-back words.
+//   k_rank_sort on the sample: every bucket's share of it ends at a splitter (key, position).
+//   k_bucket_count: each key's bucket by binary search among the splitters in LDS, kept as a
+//     16-bit id (equal keys spread over buckets by position); per-tile bucket counts with
+//     decoupled look-back over the tiles, as in k_radix_pass.
+//   k_bucket_scatter: keys and values to their bucket, staged in LDS so that a tile's keys of one
+//     bucket are written as a run. No waits: the look-back words now hold every tile's prefix.
+//   k_bucket_sort: one block per bucket merge-sorts its pairs in LDS. A bucket that outgrew LDS (a
+//     sample that missed the distribution) is sorted in pieces that its block merges through
+//     memory: slow, and right.
+// Three passes over the keys and five launches instead of the radix sort's nine and ten (64-bit
+// keys), whose waits for earlier tiles are paid once. Measured, radix sort -> this: 2k keys 52 ->
+// 8 us (and nine launches fewer), 70k 85 -> 55 beside another kernel, 1M 173 -> 99, 1.5M (batch)
+// 217 -> 143; at 4M keys 382 -> 357 (buckets of 2048), within the spread of the passes, so
+// larger sorts keep the radix sort: it needs no sample to hold.
+// In k_bucket_sort ranking runs of 64 by lane broadcasts before the merges (1M: 57 us instead of
+// 46) and merging four runs at a time by binary searches (90 us) were slower.
+// ------------------------------------------------------------------------------------------
+constexpr int kRankWaves = 16;
+
+template <typename K>
+__device__ __forceinline__ bool pair_less(K ka, uint32_t va, K kb, uint32_t vb) {
+    return ka < kb || (ka == kb && va < vb);
+}
+
+__device__ __forceinline__ uint32_t lane_value(uint32_t x, int j) {
+    return (uint32_t)__builtin_amdgcn_readlane((int)x, j);
+}
+__device__ __forceinline__ uint64_t lane_value(uint64_t x, int j) {
+    return ((uint64_t)lane_value((uint32_t)(x >> 32), j) << 32) | lane_value((uint32_t)x, j);
+}
+
+// how many of the wave's pairs (qk, qv) stand before (k, v)
+template <typename K>
+__device__ __forceinline__ uint32_t lanes_before(K qk, uint32_t qv, K k, uint32_t v) {
+    uint32_t c = 0;
+#pragma unroll 8
+    for (int j = 0; j < kWave; ++j)
+        c += pair_less(lane_value(qk, j), lane_value(qv, j), k, v) ? 1u : 0u;
+    return c;
+}
+
+
+template <typename K, bool SPLIT>
+__global__ __launch_bounds__(kRankWaves * kWave) void k_rank_sort(const K* __restrict__ keys,
+                                                                  const uint32_t* __restrict__ vals,
+                                                                  uint32_t n,
+                                                                  uint32_t per,
+                                                                  K* __restrict__ keys_out,
+                                                                  uint32_t* __restrict__ vals_out) {
+    __shared__ uint32_t s_rank[kWave];
+    const uint32_t lane = threadIdx.x & 63, b = blockIdx.x, i = b * kWave + lane;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const K k = i < n ? keys[i] : (K)0;
+    if (threadIdx.x < kWave) s_rank[lane] = 0u;
+    __syncthreads();
+    // keys equal to this one count when they stand before it
+    const uint32_t chunks = (n + kWave - 1) / kWave;
+    uint32_t rank = 0;
+    for (uint32_t c = w; c < chunks; c += kRankWaves) {
+        const K* __restrict__ q = keys + c * kWave;
+        if (c == b || c + 1 == chunks) {
+            const uint32_t e = c * kWave + lane;
+            rank += lanes_before(e < n ? keys[e] : ~(K)0, e, k, i);
+        } else if (c < b) {
+#pragma unroll 16
+            for (int j = 0; j < kWave; ++j) rank += q[j] <= k ? 1u : 0u;
+        } else {
+#pragma unroll 16
+            for (int j = 0; j < kWave; ++j) rank += q[j] < k ? 1u : 0u;
+        }
+    }
+    atomicAdd(&s_rank[lane], rank);
+    __syncthreads();
+    if (threadIdx.x >= kWave || i >= n) return;
+    rank = s_rank[lane];
+    if (SPLIT) {
+        if (rank == 0 || (rank & (per - 1))) return;
+        rank = rank / per - 1;
+    }
+    keys_out[rank] = k;
+    vals_out[rank] = vals[i];
+}
+
+template <typename K>
+__global__ __launch_bounds__(kBlock) void k_bucket_prepare(const K* __restrict__ keys, uint32_t n,
+                                                           uint32_t samples, K* __restrict__ skey,
+                                                           uint32_t* __restrict__ spos,
+                                                           uint32_t* __restrict__ status,
+                                                           uint32_t words,
+                                                           uint32_t* __restrict__ ticket) {
+    const uint32_t j = blockIdx.x * kBlock + threadIdx.x;
+    if (j == 0) *ticket = 0u;
+    for (uint32_t i = j; i < words; i += gridDim.x * kBlock) status[i] = 0u;
+    if (j >= samples) return;
+    // a scrambled place in the stratum, so that a period in the input is not met in step
+    const uint32_t p0 = (uint32_t)((uint64_t)n * j / samples);
+    const uint32_t p1 = (uint32_t)((uint64_t)n * (j + 1) / samples);  // > p0: n >= samples
+    uint32_t h = j * 0x9E3779B1u;
+    h ^= h >> 15;
+    h *= 0x85EBCA77u;
+    const uint32_t p = p0 + (uint32_t)(((uint64_t)h * (p1 - p0)) >> 32);
+    skey[j] = keys[p];
+    spos[j] = p;
+}
+
+template <typename K, int THREADS>
+__global__ __launch_bounds__(THREADS) void k_bucket_count(const K* __restrict__ keys, uint32_t n,
+                                                          uint32_t buckets,
+                                                          const K* __restrict__ split_key,
+                                                          const uint32_t* __restrict__ split_pos,
+                                                          uint16_t* __restrict__ id,
+                                                          uint32_t* __restrict__ status,
+                                                          uint32_t* __restrict__ ticket,
+                                                          uint32_t* __restrict__ err,
+                                                          uint32_t spin_limit) {
+    constexpr int kItems = kBucketItems;
+    if (__hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0u) return;
+    __shared__ K sk[kBucketMax];
+    __shared__ uint32_t sp[kBucketMax];
+    __shared__ uint32_t hist[kBucketMax];
+    __shared__ uint32_t s_tile;
+    if (threadIdx.x == 0) s_tile = atomicAdd(ticket, 1u);
+    for (uint32_t d = threadIdx.x; d < buckets; d += THREADS) {
+        hist[d] = 0u;
+        if (d + 1 < buckets) {
+            sk[d] = split_key[d];
+            sp[d] = split_pos[d];
+        }
+    }
+    __syncthreads();
+    const uint32_t tile = s_tile, base = tile * (THREADS * kItems);
+    const int lane = threadIdx.x & 63;
+    const uint64_t le = lane_mask_lt() | (1ull << lane);
+    K k[kItems];
+    uint32_t lo[kItems], len = buckets - 1;
+#pragma unroll
+    for (int r = 0; r < kItems; ++r) {
+        const uint32_t i = base + r * THREADS + threadIdx.x;
+        k[r] = i < n ? keys[i] : (K)0;
+        lo[r] = 0;
+    }
+    // splitters below (key, position), for the thread's keys side by side
+    while (len) {
+        const uint32_t half = (len + 1) >> 1;
+#pragma unroll
+        for (int r = 0; r < kItems; ++r) {
+            const uint32_t i = base + r * THREADS + threadIdx.x;
+            const uint32_t mid = lo[r] + half - 1;
+            const K s = sk[mid];
+            bool below = s < k[r];
+            if (s == k[r]) below = sp[mid] < i;
+            lo[r] = below ? mid + 1 : lo[r];
+        }
+        len -= half;
+    }
+    // runs of equal buckets among neighbouring lanes count with one add (nearly sorted keys)
+#pragma unroll
+    for (int r = 0; r < kItems; ++r) {
+        const uint32_t i = base + r * THREADS + threadIdx.x;
+        const bool valid = i < n;
+        const uint32_t prev = __shfl_up(lo[r], 1, kWave);
+        const bool head = valid && (lane == 0 || lo[r] != prev);
+        const uint64_t after = (__ballot(head) | __ballot(!valid)) & ~le;
+        const uint32_t end = after ? (uint32_t)__builtin_ctzll(after) : 64u;
+        if (head) atomicAdd(&hist[lo[r]], end - (uint32_t)lane);
+        if (valid) id[i] = (uint16_t)lo[r];
+    }
+    __syncthreads();
+    uint32_t* mine = status + (size_t)tile * buckets;
+    for (uint32_t d = threadIdx.x; d < buckets; d += THREADS)
+        __hip_atomic_store(mine + d, (tile ? kLbCount : kLbPrefix) | hist[d], __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    if (tile == 0) return;
+    for (uint32_t d = threadIdx.x; d < buckets; d += THREADS) {
+        const uint32_t excl = look_back(status + d, buckets, tile, err, spin_limit);
+        __hip_atomic_store(mine + d, kLbPrefix | (excl + hist[d]), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    }
+}
+
+// start[d] = sum of count(0 .. d-1)
+template <int THREADS, typename F>
+__device__ __forceinline__ void bucket_starts(uint32_t buckets, uint32_t* start, F count) {
+    constexpr int kPer = kBucketMax / THREADS;
+    uint32_t c[kPer], s = 0, tot;
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        const uint32_t d = threadIdx.x * kPer + q;
+        c[q] = d < buckets ? count(d) : 0u;
+        s += c[q];
+    }
+    uint32_t run = block_exclusive_scan_t<THREADS>(s, &tot);
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        const uint32_t d = threadIdx.x * kPer + q;
+        if (d < buckets) start[d] = run;
+        run += c[q];
+    }
+}
+
+template <typename K, int THREADS>
+__global__ __launch_bounds__(THREADS) void k_bucket_scatter(const K* __restrict__ keys,
+                                                            const uint32_t* __restrict__ vals,
+                                                            uint32_t n, uint32_t buckets,
+                                                            const uint16_t* __restrict__ id,
+                                                            const uint32_t* __restrict__ status,
+                                                            const uint32_t* __restrict__ err,
+                                                            K* __restrict__ keys_out,
+                                                            uint32_t* __restrict__ vals_out,
+                                                            uint32_t* __restrict__ starts) {
+    constexpr int kItems = kBucketItems, kTile = THREADS * kItems;
+    if (*err != 0u) return;  // the counts are not whole: nothing is placed
+    __shared__ K s_key[kTile];
+    __shared__ uint32_t s_val[kTile];
+    __shared__ uint16_t s_id[kTile];
+    __shared__ uint32_t hist[kBucketMax], first[kBucketMax], place[kBucketMax];
+    const uint32_t tile = blockIdx.x, base = tile * kTile;
+    const int lane = threadIdx.x & 63;
+    K k[kItems];
+    uint32_t v[kItems], d[kItems], rank[kItems];
+#pragma unroll
+    for (int r = 0; r < kItems; ++r) {
+        const uint32_t i = base + r * THREADS + threadIdx.x;
+        k[r] = i < n ? keys[i] : (K)0;
+        v[r] = i < n ? vals[i] : 0u;
+        d[r] = i < n ? id[i] : 0u;
+    }
+    for (uint32_t q = threadIdx.x; q < buckets; q += THREADS) hist[q] = 0u;
+    const uint32_t* last = status + (size_t)(gridDim.x - 1) * buckets;
+    bucket_starts<THREADS>(buckets, place, [&](uint32_t q) { return last[q] & kLbMask; });
+    __syncthreads();
+    const uint64_t le = lane_mask_lt() | (1ull << lane);
+#pragma unroll
+    for (int r = 0; r < kItems; ++r) {
+        const bool valid = base + r * THREADS + threadIdx.x < n;
+        const uint32_t prev = __shfl_up(d[r], 1, kWave);
+        const bool head = valid && (lane == 0 || d[r] != prev);
+        const uint64_t heads = __ballot(head);
+        const uint64_t after = (heads | __ballot(!valid)) & ~le;
+        const uint32_t end = after ? (uint32_t)__builtin_ctzll(after) : 64u;
+        const uint64_t upto = heads & le;
+        const int mine = upto ? 63 - (int)__builtin_clzll(upto) : 0;  // the head of my run
+        uint32_t at = 0;
+        if (head) at = atomicAdd(&hist[d[r]], end - (uint32_t)lane);
+        rank[r] = __shfl(at, mine, kWave) + (uint32_t)(lane - mine);
+    }
+    __syncthreads();
+    if (tile == 0)
+        for (uint32_t q = threadIdx.x; q < buckets; q += THREADS) starts[q] = place[q];
+    else
+        for (uint32_t q = threadIdx.x; q < buckets; q += THREADS)
+            place[q] += status[(size_t)(tile - 1) * buckets + q] & kLbMask;
+    bucket_starts<THREADS>(buckets, first, [&](uint32_t q) { return hist[q]; });
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < kItems; ++r) {
+        if (base + r * THREADS + threadIdx.x >= n) continue;
+        const uint32_t p = first[d[r]] + rank[r];
+        s_key[p] = k[r];
+        s_val[p] = v[r];
+        s_id[p] = (uint16_t)d[r];
+    }
+    __syncthreads();
+    const uint32_t cnt = min((uint32_t)kTile, n - base);
+    for (uint32_t p = threadIdx.x; p < cnt; p += THREADS) {
+        const uint32_t q = s_id[p], g = place[q] + (p - first[q]);
+        keys_out[g] = s_key[p];
+        vals_out[g] = s_val[p];
+    }
+}
+
+// Merge sort of the n <= THREADS * ITEMS pairs in sk / sv, in place. The slots from n up to
+// THREADS * ITEMS are filled with pairs above every other (no value is 2^32 - 1).
+template <typename K, int THREADS, int ITEMS>
+__device__ __forceinline__ void block_merge_sort(K* sk, uint32_t* sv, uint32_t n) {
+    const uint32_t at = threadIdx.x * ITEMS;
+    K k[ITEMS];
+    uint32_t v[ITEMS];
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        k[i] = at + i < n ? sk[at + i] : ~(K)0;
+        v[i] = at + i < n ? sv[at + i] : 0xFFFFFFFFu;
+    }
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r)  // odd-even transposition within the thread
+#pragma unroll
+        for (int i = r & 1; i + 1 < ITEMS; i += 2) {
+            const bool sw = pair_less(k[i + 1], v[i + 1], k[i], v[i]);
+            const K ka = sw ? k[i + 1] : k[i], kb = sw ? k[i] : k[i + 1];
+            const uint32_t va = sw ? v[i + 1] : v[i], vb = sw ? v[i] : v[i + 1];
+            k[i] = ka;
+            k[i + 1] = kb;
+            v[i] = va;
+            v[i + 1] = vb;
+        }
+    for (uint32_t w = ITEMS; w < n; w <<= 1) {
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            sk[at + i] = k[i];
+            sv[at + i] = v[i];
+        }
+        __syncthreads();
+        const uint32_t a0 = at & ~(2 * w - 1), b0 = a0 + w, diag = at - a0;
+        if (b0 >= n) continue;  // the second run is filling alone
+        // runs [a0, b0) and [b0, b0 + w): the outputs from `diag` on take the first from a0 + lo
+        uint32_t lo = diag > w ? diag - w : 0u, hi = min(diag, w);
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi) >> 1, o = b0 + diag - 1 - mid;
+            const K ka = sk[a0 + mid], kb = sk[o];
+            bool less = ka < kb;
+            if (ka == kb) less = sv[a0 + mid] < sv[o];
+            lo = less ? mid + 1 : lo;
+            hi = less ? hi : mid;
+        }
+        uint32_t ia = a0 + lo, ib = b0 + diag - lo;
+        const uint32_t b1 = b0 + w;
+        K ka = sk[min(ia, b0 - 1)], kb = sk[min(ib, b1 - 1)];
+        uint32_t va = sv[min(ia, b0 - 1)], vb = sv[min(ib, b1 - 1)];
+#pragma unroll
+        for (int i = 0; i < ITEMS; ++i) {
+            const bool a = ib >= b1 || (ia < b0 && pair_less(ka, va, kb, vb));
+            k[i] = a ? ka : kb;
+            v[i] = a ? va : vb;
+            ia += a ? 1u : 0u;
+            ib += a ? 0u : 1u;
+            if (i + 1 < ITEMS) {
+                const uint32_t next = a ? min(ia, b0 - 1) : min(ib, b1 - 1);
+                const K kn = sk[next];
+                const uint32_t vn = sv[next];
+                ka = a ? kn : ka;
+                va = a ? vn : va;
+                kb = a ? kb : kn;
+                vb = a ? vb : vn;
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < ITEMS; ++i) {
+        sk[at + i] = k[i];
+        sv[at + i] = v[i];
+    }
+    __syncthreads();
+}
+
+// merge of the sorted runs [a0, b0) and [b0, b1) from one place to another, by the whole block
+template <typename K, int THREADS>
+__device__ void block_merge_runs(const K* sk, const uint32_t* sv, K* dk, uint32_t* dv, uint32_t a0,
+                                 uint32_t b0, uint32_t b1) {
+    const uint32_t na = b0 - a0, nb = b1 - b0, per = (na + nb + THREADS - 1) / THREADS;
+    const uint32_t d0 = min(threadIdx.x * per, na + nb), d1 = min(d0 + per, na + nb);
+    uint32_t lo = d0 > nb ? d0 - nb : 0u, hi = min(d0, na);
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1, o = b0 + d0 - 1 - mid;
+        if (pair_less(sk[a0 + mid], sv[a0 + mid], sk[o], sv[o]))
+            lo = mid + 1;
+        else
+            hi = mid;
+    }
+    uint32_t ia = a0 + lo, ib = b0 + d0 - lo;
+    for (uint32_t d = d0; d < d1; ++d) {
+        const bool a = ib >= b1 || (ia < b0 && pair_less(sk[ia], sv[ia], sk[ib], sv[ib]));
+        const uint32_t s = a ? ia++ : ib++;
+        dk[a0 + d] = sk[s];
+        dv[a0 + d] = sv[s];
+    }
+}
+
+template <typename K, int THREADS>
+__global__ __launch_bounds__(THREADS) void k_bucket_sort(K* keys, uint32_t* vals, uint32_t n,
+                                                         uint32_t buckets,
+                                                         const uint32_t* __restrict__ starts,
+                                                         const uint32_t* __restrict__ err,
+                                                         K* keys_out, uint32_t* vals_out) {
+    constexpr uint32_t kCap = THREADS * kBucketItemsMax;
+    if (*err != 0u) return;
+    __shared__ K sk[kCap];
+    __shared__ uint32_t sv[kCap];
+    const uint32_t b = blockIdx.x, start = starts[b];
+    const uint32_t cnt = (b + 1 < buckets ? starts[b + 1] : n) - start;
+    for (uint32_t c0 = 0; c0 < cnt; c0 += kCap) {  // one piece unless the bucket outgrew LDS
+        const uint32_t m = min(cnt - c0, kCap), g = start + c0;
+        for (uint32_t i = threadIdx.x; i < m; i += THREADS) {
+            sk[i] = keys[g + i];
+            sv[i] = vals[g + i];
+        }
+        __syncthreads();
+        if (m <= THREADS) block_merge_sort<K, THREADS, 1>(sk, sv, m);
+        else if (m <= 2 * THREADS) block_merge_sort<K, THREADS, 2>(sk, sv, m);
+        else if (m <= 4 * THREADS) block_merge_sort<K, THREADS, 4>(sk, sv, m);
+        else block_merge_sort<K, THREADS, kBucketItemsMax>(sk, sv, m);
+        for (uint32_t i = threadIdx.x; i < m; i += THREADS) {
+            keys_out[g + i] = sk[i];
+            vals_out[g + i] = sv[i];
+        }
+        __syncthreads();
+    }
+    if (cnt <= kCap) return;
+    K *from_k = keys_out, *to_k = keys;
+    uint32_t *from_v = vals_out, *to_v = vals;
+    for (uint32_t w = kCap; w < cnt; w *= 2) {
+        __threadfence_block();
+        __syncthreads();
+        for (uint32_t a0 = 0; a0 < cnt; a0 += 2 * w)
+            block_merge_runs<K, THREADS>(from_k, from_v, to_k, to_v, start + a0,
+                                         start + min(a0 + w, cnt), start + min(a0 + 2 * w, cnt));
+        K* tk = from_k; from_k = to_k; to_k = tk;
+        uint32_t* tv = from_v; from_v = to_v; to_v = tv;
+    }
+    __threadfence_block();
+    __syncthreads();
+    if (from_k != keys_out)
+        for (uint32_t i = threadIdx.x; i < cnt; i += THREADS) {
+            keys_out[start + i] = from_k[start + i];
+            vals_out[start + i] = from_v[start + i];
+        }
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1333,30 +1772,97 @@ static int sort_items(uint32_t n) { return n <= kSortSmallMax ? kSortItemsSmall 
 
 uint32_t sort_blocks(uint32_t n) { return div_up(n, sort_tile(sort_items(n))); }
 
-// counts [8][256][tiles] + look-back words [8][tiles][256] + totals [8][256] + tickets and an
-// error word, for the largest tile count of any n' <= n
+// radix sort: counts [8][256][tiles] + look-back words [8][tiles][256] + totals [8][256] + tickets;
+// bucket sort: ids (2 bytes per key) + look-back words [tiles][buckets] + ticket + sample and
+// splitter keys and positions, bucket starts. The largest tile count of any n' <= n.
 uint64_t sort_scratch_words(uint32_t n) {
     const uint32_t tiles = max(sort_blocks(n), div_up(min(n, kSortSmallMax), sort_tile(kSortItemsSmall)));
-    return 2ull * kSortMaxPasses * 256 * tiles + kSortMaxPasses * 256 + 16;
+    return 2ull * kSortMaxPasses * 256 * tiles + kSortMaxPasses * 256 + 16 +
+           3ull * kBucketSamples + 4ull * kBucketMax;
 }
 
-void launch_radix_sort(hipStream_t s, void* keys_a, uint32_t* vals_a, void* keys_b,
-                       uint32_t* vals_b, uint32_t n, int key_bits, bool wide, uint32_t* scratch,
-                       uint32_t* err, uint32_t spin_limit, bool* result_in_b) {
+// Mean bucket of a sort, a quarter of what its sorting block holds in LDS: the smaller one leaves
+// more buckets to share a small sort (20k keys: 40 blocks), the larger keeps the splitters of a
+// large one few (and the runs that a tile writes long).
+static uint32_t bucket_mean(uint32_t n) { return n <= (1u << 19) ? 512 : 1024; }
+static_assert(kBucketSortMax <= 1024u * kBucketMax && (1u << 19) <= 512u * kBucketMax, "buckets");
+
+// Samples per bucket, a power of two: 4096 keys together, within 8 .. 64 a bucket. Few samples leave
+// uneven buckets, and the largest one is the sort's last wave (20k keys: 17 us of k_bucket_sort
+// with 8, 12 with 64); ranking 8192 instead of 4096 costs 4 us more.
+static uint32_t bucket_sample(uint32_t buckets) {
+    uint32_t per = 8;
+    while (per < 64 && buckets * per * 2 <= 4096) per *= 2;
+    return per;
+}
+
+template <typename K>
+static void bucket_sort(hipStream_t s, K* keys_a, uint32_t* vals_a, K* keys_b, uint32_t* vals_b,
+                        uint32_t n, uint32_t* scratch, uint32_t* err, uint32_t spin_limit) {
+    const uint32_t nt = sort_blocks(n), mean = bucket_mean(n), buckets = div_up(n, mean);
+    const uint32_t per = bucket_sample(buckets);
+    const uint32_t samples = buckets * per;
+    uint16_t* id = (uint16_t*)scratch;
+    uint32_t* status = scratch + (size_t)kSortMaxPasses * 256 * nt;
+    uint32_t* ticket = status + (size_t)kSortMaxPasses * 256 * nt;
+    K* sample_key = (K*)(ticket + 16);
+    K* split_key = sample_key + kBucketSamples;
+    uint32_t* sample_pos = (uint32_t*)(split_key + kBucketMax);
+    uint32_t* split_pos = sample_pos + kBucketSamples;
+    uint32_t* starts = split_pos + kBucketMax;
+    k_bucket_prepare<K><<<div_up(samples, kBlock), kBlock, 0, s>>>(
+        keys_a, n, samples, sample_key, sample_pos, status, nt * buckets, ticket);
+    k_rank_sort<K, true><<<div_up(samples, kWave), kRankWaves * kWave, 0, s>>>(
+        sample_key, sample_pos, samples, per, split_key, split_pos);
+#define BH_SPREAD(T)                                                                              \
+    k_bucket_count<K, T><<<nt, T, 0, s>>>(keys_a, n, buckets, split_key, split_pos, id, status,   \
+                                          ticket, err, spin_limit);                               \
+    k_bucket_scatter<K, T><<<nt, T, 0, s>>>(keys_a, vals_a, n, buckets, id, status, err, keys_b,  \
+                                            vals_b, starts)
+    if (sort_items(n) == kSortItemsSmall) { BH_SPREAD(512); } else { BH_SPREAD(1024); }
+#undef BH_SPREAD
+    static_assert(kBucketItems * 512 == sort_tile(kSortItemsSmall) &&
+                  kBucketItems * 1024 == sort_tile(kSortItemsLarge), "tiles match");
+#define BH_SORT(T)                                                                                \
+    k_bucket_sort<K, T><<<buckets, T, 0, s>>>(keys_b, vals_b, n, buckets, starts, err, keys_a, \
+                                                 vals_a)
+    if (mean == 512) BH_SORT(256); else BH_SORT(512);
+#undef BH_SORT
+}
+
+void launch_sort(hipStream_t s, void* keys_a, uint32_t* vals_a, void* keys_b, uint32_t* vals_b,
+                 uint32_t n, int key_bits, bool wide, uint32_t* scratch, uint32_t* err,
+                 uint32_t spin_limit, bool* result_in_b) {
+    if (n <= kRankSortMax) {
+        const dim3 g(div_up(n, kWave)), t(kRankWaves * kWave);
+        if (wide)
+            k_rank_sort<uint64_t, false><<<g, t, 0, s>>>((const uint64_t*)keys_a, vals_a, n, 1,
+                                                         (uint64_t*)keys_b, vals_b);
+        else
+            k_rank_sort<uint32_t, false><<<g, t, 0, s>>>((const uint32_t*)keys_a, vals_a, n, 1,
+                                                         (uint32_t*)keys_b, vals_b);
+        *result_in_b = true;
+        return;
+    }
+    if (n <= kBucketSortMax) {
+        if (wide)
+            bucket_sort<uint64_t>(s, (uint64_t*)keys_a, vals_a, (uint64_t*)keys_b, vals_b, n,
+                                  scratch, err, spin_limit);
+        else
+            bucket_sort<uint32_t>(s, (uint32_t*)keys_a, vals_a, (uint32_t*)keys_b, vals_b, n,
+                                  scratch, err, spin_limit);
+        *result_in_b = false;
+        return;
+    }
     const uint32_t nt = sort_blocks(n);
     const int passes = (key_bits + 7) / 8;
     uint32_t* counts = scratch;
     uint32_t* status = counts + (size_t)kSortMaxPasses * 256 * nt;
     uint32_t* totals = status + (size_t)kSortMaxPasses * 256 * nt;
     uint32_t* tickets = totals + kSortMaxPasses * 256;
-    const bool small = sort_items(n) == kSortItemsSmall;
 #define BH_COUNTS(K, T, I)                                                                        \
     k_radix_counts<K, T, I><<<nt, T, 0, s>>>((const K*)keys_a, n, passes, nt, counts, status)
-    if (wide) {
-        if (small) BH_COUNTS(uint64_t, 512, 4); else BH_COUNTS(uint64_t, 1024, 4);
-    } else {
-        if (small) BH_COUNTS(uint32_t, 512, 4); else BH_COUNTS(uint32_t, 1024, 4);
-    }
+    if (wide) BH_COUNTS(uint64_t, 1024, 4); else BH_COUNTS(uint32_t, 1024, 4);
 #undef BH_COUNTS
     k_radix_totals<<<div_up(passes * 256, kWavesPerBlock), kBlock, 0, s>>>(counts, nt, passes,
                                                                             totals, tickets);
@@ -1370,13 +1876,9 @@ void launch_radix_sort(hipStream_t s, void* keys_a, uint32_t* vals_a, void* keys
 #define BH_PASS(K, T, I)                                                                          \
     k_radix_pass<K, T, I><<<nt, T, 0, s>>>((const K*)kin, vin, (K*)kout, vout, n, 8 * p, tp, st,  \
                                            tickets + p, err, spin_limit)
-        static_assert(kSortItemsLarge * kBlock == 1024 * 4 && kSortItemsSmall * kBlock == 512 * 4,
+        static_assert(kSortItemsLarge * kBlock == 1024 * 4 && kBucketSortMax >= kSortSmallMax,
                       "pass tiles match the counting tiles");
-        if (wide) {
-            if (small) BH_PASS(uint64_t, 512, 4); else BH_PASS(uint64_t, 1024, 4);
-        } else {
-            if (small) BH_PASS(uint32_t, 512, 4); else BH_PASS(uint32_t, 1024, 4);
-        }
+        if (wide) BH_PASS(uint64_t, 1024, 4); else BH_PASS(uint32_t, 1024, 4);
 #undef BH_PASS
         void* tk = kin; kin = kout; kout = tk;
         uint32_t* tv = vin; vin = vout; vout = tv;

@@ -17,7 +17,7 @@ constexpr int kKernelTsne = 1;
 
 uint32_t bounds_grid(uint32_t n);
 // Build status words (device, cleared by the host before a build sequence, read after it):
-// [0] the radix sort's look-back gave up waiting, [1] a position was not finite.
+// [0] the sort's look-back gave up waiting, [1] a position was not finite.
 constexpr int kStatusWords = 4;
 constexpr uint32_t kSortSpinLimit = 1u << 22;  // look-back polls before giving up
 void launch_bounds(hipStream_t s, const float* xs, const float* ys, uint32_t n, float4* partials,
@@ -31,12 +31,13 @@ uint32_t scan_partials_size(uint64_t n);
 void launch_exclusive_scan(hipStream_t s, const uint32_t* in, uint32_t* out, uint32_t n,
                            uint32_t* partials, uint32_t* total);
 uint32_t sort_blocks(uint32_t n);
-uint64_t sort_scratch_words(uint32_t n);  // uint32 words of scratch launch_radix_sort needs
+uint64_t sort_scratch_words(uint32_t n);  // uint32 words of scratch launch_sort needs
+// Stable sort of the n keys; vals_a holds 0 .. n-1 on entry.
 // err: status word set when a look-back wait exceeds spin_limit polls (the order is then not
 // valid; later passes do nothing and launch_gather falls back to the input order)
-void launch_radix_sort(hipStream_t s, void* keys_a, uint32_t* vals_a, void* keys_b,
-                       uint32_t* vals_b, uint32_t n, int key_bits, bool wide, uint32_t* scratch,
-                       uint32_t* err, uint32_t spin_limit, bool* result_in_b);
+void launch_sort(hipStream_t s, void* keys_a, uint32_t* vals_a, void* keys_b, uint32_t* vals_b,
+                 uint32_t n, int key_bits, bool wide, uint32_t* scratch, uint32_t* err,
+                 uint32_t spin_limit, bool* result_in_b);
 // codes: the sorted codes, zeroed (with the identity order) when *sort_err is set
 void launch_gather(hipStream_t s, const uint32_t* perm, uint32_t n, const float* x, const float* y,
                    const float* m, const float* vx, const float* vy, const uint32_t* id, float* xo,

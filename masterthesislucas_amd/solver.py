@@ -258,7 +258,7 @@ class BHContext:
         return getattr(self, "_variant", 4)
 
     def set_sort_spin_limit(self, polls):
-        """Look-back polls before the radix sort gives up (default 2^22); a small value only
+        """Look-back polls before the sort gives up (default 2^22); a small value only
         exercises the error path (bh_set_sort_spin_limit)."""
         self._c(_lib.load().bh_set_sort_spin_limit(self._h, int(polls)))
 

@@ -3,7 +3,7 @@ or one launch's blocks, each against the FP64 oracle or plain numpy."""
 import numpy as np
 import pytest
 
-from masterthesislucas_amd import tsne
+from masterthesislucas_amd import BHContext, tsne
 from masterthesislucas_amd.learned import N_OUT, FarFieldMLP, flatten, unflatten
 from oracle import oracle as O
 
@@ -185,3 +185,54 @@ def test_walk_tsne_paths_agree(gpu):
     assert abs(z2 - z) <= 1e-5 * z
     c1.close()
     c2.close()
+
+
+def _check_sort(x, y, mode):
+    n = len(x)
+    xd, yd = x.astype(np.float64), y.astype(np.float64)
+    minx, miny, maxx, maxy = xd.min(), yd.min(), xd.max(), yd.max()
+    if mode == "quadtree":
+        ref = O.morton64(xd, yd, minx, miny, O.quadtree_side(minx, miny, maxx, maxy), 32)
+    else:
+        ref = O.morton32(xd, yd, minx, miny, max(maxx + (-minx), maxy + (-miny))).astype(np.uint64)
+    p = np.argsort(ref, kind="stable")
+    ctx = BHContext(n, kernel="gravity", tree_mode=mode, softening=0.01)
+    ctx.set_particles(x, y)
+    ctx.build()
+    codes, perm = ctx.morton()
+    assert np.array_equal(perm, p)
+    assert np.array_equal(codes, ref[p])
+    ctx.close()
+
+
+@pytest.mark.parametrize("mode", ["quadtree", "morton_fixed"])
+@pytest.mark.parametrize("n", [2, 63, 64, 65, 1025, 8192, 8193, 10_241, 262_144, 524_288, 524_289,
+                               1_048_577, 2_097_152, 2_097_153])
+def test_sort_edges(gpu, mode, n):
+    """Both sides of every size at which the sort changes its kernels or bucket size, one point
+    in eight on one of three spots: codes and order bit-exact against a stable sort."""
+    rng = np.random.default_rng(n)
+    x, y = rng.normal(0, 1, (2, n)).astype(np.float32)
+    dup = rng.random(n) < 1 / 8
+    x[dup] = y[dup] = np.float32(0.25) * rng.integers(0, 3, dup.sum())
+    _check_sort(x, y, mode)
+
+
+@pytest.mark.parametrize("mode", ["quadtree", "morton_fixed"])
+@pytest.mark.parametrize("low", ["spread", "equal"])
+@pytest.mark.parametrize("n,mean", [(20_000, 512), (600_000, 1024)])
+def test_sort_sample_misses_the_distribution(gpu, mode, low, n, mean):
+    """Every key that the sort samples lies above every other key, so all the others fall into
+    the first bucket, many times what one block sorts in LDS: still bit-exact."""
+    b = -(-n // mean)
+    s = b * next(q for q in (64, 32, 16, 8) if q == 8 or b * q <= 4096)
+    j = np.arange(s, dtype=np.uint64)
+    p0, p1 = n * j // s, n * (j + 1) // s
+    h = (j * 0x9E3779B1) & 0xFFFFFFFF
+    h ^= h >> 15
+    h = (h * 0x85EBCA77) & 0xFFFFFFFF
+    pick = p0 + ((h * (p1 - p0)) >> 32)
+    rng = np.random.default_rng(n)
+    t = rng.uniform(0, 0.5, n).astype(np.float32) if low == "spread" else np.zeros(n, np.float32)
+    t[pick] = rng.uniform(0.75, 1.0, s).astype(np.float32)
+    _check_sort(t, t.copy(), mode)
