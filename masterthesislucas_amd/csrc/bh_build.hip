@@ -1328,47 +1328,56 @@ __device__ __forceinline__ Moments combine(const Moments* ch, const bool* has, b
     return r;
 }
 
-__global__ __launch_bounds__(kUpThreads) void k_up_chunk(const float4* __restrict__ pos4,
+// A block's time is a chain of latencies: node records, then leaf points, then one LDS round per
+// level. The child slots are therefore loaded with the records, the level loop covers the chunk's
+// own levels only, and small trees take small chunks (rule at launch_upward): 25 -> 12 us at 70k
+// points beside another kernel, 27 -> 13 us at 200k, 28 -> 26 us at 1M (60 MB of records).
+template <int CHUNK, int THREADS, bool M2>
+__global__ __launch_bounds__(THREADS) void k_up_chunk(const float4* __restrict__ pos4,
                                                      Node* __restrict__ nodes,
                                                      const uint4* __restrict__ child4,
                                                      float4* __restrict__ m2,
                                                      const BuildParams* __restrict__ prm,
                                                      uint32_t* __restrict__ deferred,
                                                      uint32_t cap_nodes, int big_done) {
-    __shared__ float s_m[kUpChunk], s_x[kUpChunk], s_y[kUpChunk];
-    __shared__ float s_xx[kUpChunk], s_xy[kUpChunk], s_yy[kUpChunk];
-    __shared__ uint32_t s_maxl;
+    __shared__ float s_m[CHUNK], s_x[CHUNK], s_y[CHUNK];
+    __shared__ float s_xx[M2 ? CHUNK : 1], s_xy[M2 ? CHUNK : 1], s_yy[M2 ? CHUNK : 1];
+    __shared__ uint32_t s_maxl, s_minl;
     __shared__ uint32_t s_ndef;
-    constexpr int kPer = kUpChunk / kUpThreads;
+    constexpr int kPer = CHUNK / THREADS;
     const uint32_t total = min(prm->n_nodes, cap_nodes);
-    const uint32_t c0 = blockIdx.x * kUpChunk;
+    const uint32_t c0 = blockIdx.x * CHUNK;
     uint32_t* my_def = deferred + (size_t)blockIdx.x * kDeferStride;
     if (c0 >= total) {
         if (threadIdx.x == 0) my_def[0] = 0;
         return;
     }
-    const uint32_t c1 = min(c0 + kUpChunk, total);
-    const bool with_m2 = m2 != nullptr;
+    const uint32_t c1 = min(c0 + CHUNK, total);
     if (threadIdx.x == 0) {
         s_maxl = 0;
+        s_minl = 255;
         s_ndef = 0;
     }
     __syncthreads();
     Node nd[kPer];
-    uint32_t lmax = 0;
+    uint4 kids[kPer];
+    uint32_t lmax = 0, lmin = 255;
 #pragma unroll
     for (int r = 0; r < kPer; ++r) {
-        const uint32_t k = c0 + threadIdx.x + r * kUpThreads;
+        const uint32_t k = c0 + threadIdx.x + r * THREADS;
         if (k < c1) {
             nd[r] = nodes[k];
+            kids[r] = child4[k];
             lmax = max(lmax, nd[r].meta & kMetaLevelMask);
+            lmin = min(lmin, nd[r].meta & kMetaLevelMask);
         }
     }
     atomicMax(&s_maxl, lmax);
+    atomicMin(&s_minl, lmin);
     // leaves first, all at once: their particle loads overlap instead of waiting level by level
 #pragma unroll
     for (int r = 0; r < kPer; ++r) {
-        const uint32_t k = c0 + threadIdx.x + r * kUpThreads;
+        const uint32_t k = c0 + threadIdx.x + r * THREADS;
         if (k >= c1 || !(nd[r].meta & kMetaLeaf)) continue;
         const uint32_t s = k - c0;
         // leaves of more than kBigLeaf points hold their moments already when k_big_leaf_moments
@@ -1376,47 +1385,47 @@ __global__ __launch_bounds__(kUpThreads) void k_up_chunk(const float4* __restric
         // adaptive tree, rare) this thread sums them
         const Moments mo = (big_done && nd[r].count > kBigLeaf)
                                ? Moments{nd[r].mass, nd[r].cx, nd[r].cy, 0.f, 0.f, 0.f}
-                               : leaf_moments(pos4, nd[r].first, nd[r].count, with_m2);
+                               : leaf_moments(pos4, nd[r].first, nd[r].count, M2);
         s_m[s] = mo.m; s_x[s] = mo.x; s_y[s] = mo.y;
-        s_xx[s] = mo.xx; s_xy[s] = mo.xy; s_yy[s] = mo.yy;
+        if (M2) { s_xx[s] = mo.xx; s_xy[s] = mo.xy; s_yy[s] = mo.yy; }
     }
     __syncthreads();
-    for (int L = (int)s_maxl; L >= 0; --L) {
+    for (int L = (int)s_maxl; L >= (int)s_minl; --L) {
 #pragma unroll
         for (int r = 0; r < kPer; ++r) {
-            const uint32_t k = c0 + threadIdx.x + r * kUpThreads;
+            const uint32_t k = c0 + threadIdx.x + r * THREADS;
             if (k >= c1 || (int)(nd[r].meta & kMetaLevelMask) != L) continue;
             const uint32_t s = k - c0;
             if (nd[r].meta & kMetaLeaf) {
                 continue;
             } else if (nd[r].skip <= c1) {
-                const uint4 cs = child4[k];
-                const uint32_t ci[4] = {cs.x, cs.y, cs.z, cs.w};
+                const uint32_t ci[4] = {kids[r].x, kids[r].y, kids[r].z, kids[r].w};
                 Moments ch[4];
                 bool has[4];
 #pragma unroll
                 for (int t = 0; t < 4; ++t) {
                     has[t] = ci[t] != kNone;
                     const uint32_t q = has[t] ? ci[t] - c0 : s;
-                    ch[t] = Moments{s_m[q], s_x[q], s_y[q], s_xx[q], s_xy[q], s_yy[q]};
+                    ch[t] = Moments{s_m[q], s_x[q], s_y[q], M2 ? s_xx[q] : 0.f,
+                                    M2 ? s_xy[q] : 0.f, M2 ? s_yy[q] : 0.f};
                 }
-                const Moments mo = combine(ch, has, with_m2);
+                const Moments mo = combine(ch, has, M2);
                 s_m[s] = mo.m; s_x[s] = mo.x; s_y[s] = mo.y;
-                s_xx[s] = mo.xx; s_xy[s] = mo.xy; s_yy[s] = mo.yy;
+                if (M2) { s_xx[s] = mo.xx; s_xy[s] = mo.xy; s_yy[s] = mo.yy; }
             }
         }
         __syncthreads();
     }
 #pragma unroll
     for (int r = 0; r < kPer; ++r) {
-        const uint32_t k = c0 + threadIdx.x + r * kUpThreads;
+        const uint32_t k = c0 + threadIdx.x + r * THREADS;
         if (k >= c1) continue;
         const uint32_t s = k - c0;
         if ((nd[r].meta & kMetaLeaf) || nd[r].skip <= c1) {
             nodes[k].cx = s_x[s];
             nodes[k].cy = s_y[s];
             nodes[k].mass = s_m[s];
-            if (with_m2) m2[k] = make_float4(s_xx[s], s_xy[s], s_yy[s], 0.f);
+            if (M2) m2[k] = make_float4(s_xx[s], s_xy[s], s_yy[s], 0.f);
         } else {
             // ancestors of the chunk end (at most one per level)
             const uint32_t slot = atomicAdd(&s_ndef, 1u);
@@ -1457,23 +1466,24 @@ static_assert(kTopMax < 65536, "entry indices are 16-bit");
 
 __device__ __forceinline__ uint32_t top_hash(uint32_t k) { return (k * 0x9E3779B1u) >> 20; }
 
+template <bool M2>
 __global__ __launch_bounds__(kUpThreads) void k_up_top(Node* __restrict__ nodes,
                                                        const uint4* __restrict__ child4,
                                                        float4* __restrict__ m2,
                                                        const BuildParams* __restrict__ prm,
                                                        const uint32_t* __restrict__ deferred,
                                                        uint32_t* __restrict__ bylevel,
-                                                       uint32_t nchunks, uint32_t cap_nodes) {
+                                                       uint32_t nchunks, uint32_t chunk,
+                                                       uint32_t cap_nodes) {
     __shared__ uint32_t s_k[kTopMax];
     __shared__ uint8_t s_l[kTopMax];
     __shared__ uint32_t s_hk[kTopHash];  // node index + 1, 0 = empty
     __shared__ uint16_t s_hv[kTopHash];  // its entry
-    __shared__ float s_mo[6][kTopMax];   // moments of settled entries
+    __shared__ float s_mo[M2 ? 6 : 3][kTopMax];   // moments of settled entries
     __shared__ uint32_t s_count, s_maxl;
     const uint32_t tid = threadIdx.x;
     const uint32_t total = min(prm->n_nodes, cap_nodes);
-    const uint32_t nch = min(nchunks, (total + kUpChunk - 1) / kUpChunk);
-    const bool with_m2 = m2 != nullptr;
+    const uint32_t nch = min(nchunks, (total + chunk - 1) / chunk);
     if (tid == 0) {
         s_count = 0;
         s_maxl = 0;
@@ -1487,9 +1497,14 @@ __global__ __launch_bounds__(kUpThreads) void k_up_top(Node* __restrict__ nodes,
         uint32_t tot;
         const uint32_t off = block_exclusive_scan_t<kUpThreads>(c, &tot);
         const uint32_t base = s_count;
-        for (uint32_t j = 0; j < c; ++j) {
-            const uint32_t at = base + off + j;
-            if (at < kTopMax) s_k[at] = deferred[(size_t)b * kDeferStride + 1 + j];
+        const uint32_t* lst = deferred + (size_t)b * kDeferStride + 1;
+        for (uint32_t j0 = 0; j0 < c; j0 += 8) {  // eight loads in flight
+            uint32_t q[8];
+#pragma unroll
+            for (uint32_t u = 0; u < 8; ++u) q[u] = lst[min(j0 + u, c - 1)];
+#pragma unroll
+            for (uint32_t u = 0; u < 8; ++u)
+                if (j0 + u < c && base + off + j0 + u < kTopMax) s_k[base + off + j0 + u] = q[u];
         }
         __syncthreads();
         if (tid == 0) s_count = base + tot;
@@ -1541,13 +1556,13 @@ __global__ __launch_bounds__(kUpThreads) void k_up_top(Node* __restrict__ nodes,
 #pragma unroll
                 for (int t2 = 0; t2 < 4; ++t2) {
                     has[t2] = ci[t2] != kNone;
-                    ch[t2] = load_moments(nodes, m2, has[t2] ? ci[t2] : k, with_m2);
+                    ch[t2] = load_moments(nodes, m2, has[t2] ? ci[t2] : k, M2);
                 }
-                const Moments mo = combine(ch, has, with_m2);
+                const Moments mo = combine(ch, has, M2);
                 __hip_atomic_store(&nodes[k].cx, mo.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 __hip_atomic_store(&nodes[k].cy, mo.y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                 __hip_atomic_store(&nodes[k].mass, mo.m, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                if (with_m2) {
+                if (M2) {
                     __hip_atomic_store(&m2[k].x, mo.xx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                     __hip_atomic_store(&m2[k].y, mo.xy, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
                     __hip_atomic_store(&m2[k].z, mo.yy, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
@@ -1559,13 +1574,20 @@ __global__ __launch_bounds__(kUpThreads) void k_up_top(Node* __restrict__ nodes,
     }
     // on chip: levels and the hash of this thread's entries
     uint32_t lmax = 0;
-    uint32_t kk[kTopPer];
+    uint32_t kk[kTopPer], lev[kTopPer];
+    uint4 kids[kTopPer];
 #pragma unroll
     for (int r = 0; r < kTopPer; ++r) {
         const uint32_t e = tid + r * kUpThreads;
         kk[r] = e < D ? s_k[e] : 0u;
+        lev[r] = e < D ? nodes[kk[r]].meta & kMetaLevelMask : 0u;
+        kids[r] = e < D ? child4[kk[r]] : make_uint4(kNone, kNone, kNone, kNone);
+    }
+#pragma unroll
+    for (int r = 0; r < kTopPer; ++r) {
+        const uint32_t e = tid + r * kUpThreads;
         if (e >= D) continue;
-        const uint32_t l = nodes[kk[r]].meta & kMetaLevelMask;
+        const uint32_t l = lev[r];
         s_l[e] = (uint8_t)l;
         lmax = max(lmax, l);
         uint32_t h = top_hash(kk[r]) & (kTopHash - 1);
@@ -1580,9 +1602,7 @@ __global__ __launch_bounds__(kUpThreads) void k_up_top(Node* __restrict__ nodes,
     bool has[kTopPer][4];
 #pragma unroll
     for (int r = 0; r < kTopPer; ++r) {
-        const uint32_t e = tid + r * kUpThreads;
-        const uint4 cs = e < D ? child4[kk[r]] : make_uint4(kNone, kNone, kNone, kNone);
-        const uint32_t ci[4] = {cs.x, cs.y, cs.z, cs.w};
+        const uint32_t ci[4] = {kids[r].x, kids[r].y, kids[r].z, kids[r].w};
 #pragma unroll
         for (int t2 = 0; t2 < 4; ++t2) {
             has[r][t2] = ci[t2] != kNone;
@@ -1599,7 +1619,7 @@ __global__ __launch_bounds__(kUpThreads) void k_up_top(Node* __restrict__ nodes,
                 ch[r][t2].m = q.mass;
                 ch[r][t2].x = q.cx;
                 ch[r][t2].y = q.cy;
-                if (with_m2) {
+                if (M2) {
                     const float4 q2 = m2[ci[t2]];
                     ch[r][t2].xx = q2.x;
                     ch[r][t2].xy = q2.y;
@@ -1617,16 +1637,16 @@ __global__ __launch_bounds__(kUpThreads) void k_up_top(Node* __restrict__ nodes,
             for (int t2 = 0; t2 < 4; ++t2) {
                 const int q = ce[r][t2];
                 if (q < 0) continue;
-                ch[r][t2] = Moments{s_mo[0][q], s_mo[1][q], s_mo[2][q],
-                                    s_mo[3][q], s_mo[4][q], s_mo[5][q]};
+                ch[r][t2] = Moments{s_mo[0][q], s_mo[1][q], s_mo[2][q], M2 ? s_mo[M2 ? 3 : 0][q] : 0.f,
+                                    M2 ? s_mo[M2 ? 4 : 0][q] : 0.f, M2 ? s_mo[M2 ? 5 : 0][q] : 0.f};
             }
-            const Moments mo = combine(ch[r], has[r], with_m2);
+            const Moments mo = combine(ch[r], has[r], M2);
             s_mo[0][e] = mo.m; s_mo[1][e] = mo.x; s_mo[2][e] = mo.y;
-            s_mo[3][e] = mo.xx; s_mo[4][e] = mo.xy; s_mo[5][e] = mo.yy;
+            if (M2) { s_mo[M2 ? 3 : 0][e] = mo.xx; s_mo[M2 ? 4 : 0][e] = mo.xy; s_mo[M2 ? 5 : 0][e] = mo.yy; }
             nodes[kk[r]].cx = mo.x;
             nodes[kk[r]].cy = mo.y;
             nodes[kk[r]].mass = mo.m;
-            if (with_m2) m2[kk[r]] = make_float4(mo.xx, mo.xy, mo.yy, 0.f);
+            if (M2) m2[kk[r]] = make_float4(mo.xx, mo.xy, mo.yy, 0.f);
         }
         __syncthreads();
     }
@@ -1939,20 +1959,35 @@ void launch_batch_roots(hipStream_t s, const uint32_t* sys_off, uint32_t nsys,
     k_batch_roots<<<div_up(nsys, kBlock), kBlock, 0, s>>>(sys_off, nsys, noff, prm, roots);
 }
 
-uint32_t up_chunks(uint32_t cap_nodes) { return div_up(cap_nodes, kUpChunk); }
+uint32_t up_chunks(uint32_t cap_nodes) { return div_up(cap_nodes, kUpChunkSmall); }
 
+// Chunks of 512 nodes up to kUpSmallMax points: with 2048, 70k points are 20 blocks. Larger trees take
+// 2048, so that the nodes left to k_up_top (up to one per level and chunk) fit its LDS at 1M.
 void launch_upward(hipStream_t s, const float4* pos4, Node* nodes, const uint32_t* child4,
                    float4* m2, const BuildParams* prm, uint32_t* deferred, uint32_t* bylevel,
-                   uint32_t cap_nodes, bool big_leaves) {
-    const uint32_t nch = up_chunks(cap_nodes);
+                   uint32_t cap_nodes, uint32_t n, bool big_leaves) {
+    const bool small = n <= kUpSmallMax;
+    const uint32_t chunk = small ? kUpChunkSmall : kUpChunk;
+    const uint32_t nch = div_up(cap_nodes, chunk);
     const bool big_done = big_leaves && !m2;
     if (big_done)
         k_big_leaf_moments<<<div_up(cap_nodes, kWavesPerBlock), kBlock, 0, s>>>(pos4, nodes, prm,
                                                                                 cap_nodes);
-    k_up_chunk<<<nch, kUpThreads, 0, s>>>(pos4, nodes, (const uint4*)child4, m2, prm, deferred,
-                                      cap_nodes, big_done ? 1 : 0);
-    k_up_top<<<1, kUpThreads, 0, s>>>(nodes, (const uint4*)child4, m2, prm, deferred, bylevel,
-                                      nch, cap_nodes);
+#define BH_UP(M2)                                                                                 \
+    if (small)                                                                                    \
+        k_up_chunk<kUpChunkSmall, kUpChunkSmall, M2><<<nch, kUpChunkSmall, 0, s>>>(               \
+            pos4, nodes, (const uint4*)child4, m2, prm, deferred, cap_nodes, big_done ? 1 : 0);   \
+    else                                                                                          \
+        k_up_chunk<kUpChunk, kUpThreads, M2><<<nch, kUpThreads, 0, s>>>(                          \
+            pos4, nodes, (const uint4*)child4, m2, prm, deferred, cap_nodes, big_done ? 1 : 0);   \
+    k_up_top<M2><<<1, kUpThreads, 0, s>>>(nodes, (const uint4*)child4, m2, prm, deferred,         \
+                                          bylevel, nch, chunk, cap_nodes)
+    if (m2) {
+        BH_UP(true);
+    } else {
+        BH_UP(false);
+    }
+#undef BH_UP
 }
 
 void launch_tree_stats(hipStream_t s, const Node* nodes, const BuildParams* prm,

@@ -25,6 +25,8 @@ enum : uint32_t {
 
 constexpr uint32_t kNone = 0xFFFFFFFFu;
 constexpr int kUpChunk = 2048;                 // nodes per block in the upward pass
+constexpr int kUpChunkSmall = 512;             // the same for trees of at most kUpSmallMax points
+constexpr uint32_t kUpSmallMax = 1u << 18;
 constexpr int kUpThreads = 1024;               // threads per block in the upward pass
 constexpr int kDeferStride = kMaxLevels + 2;   // count + at most one deferred node per level
 constexpr int kTopMax = 2560;                  // deferred nodes the top pass keeps in LDS

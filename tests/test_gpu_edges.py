@@ -236,3 +236,33 @@ def test_sort_sample_misses_the_distribution(gpu, mode, low, n, mean):
     t = rng.uniform(0, 0.5, n).astype(np.float32) if low == "spread" else np.zeros(n, np.float32)
     t[pick] = rng.uniform(0.75, 1.0, s).astype(np.float32)
     _check_sort(t, t.copy(), mode)
+
+
+@pytest.mark.parametrize("mode", ["quadtree", "morton_fixed"])
+@pytest.mark.parametrize("n", [1, 40, 700, 3000, 262_144, 262_145])
+def test_node_moments_edges(gpu, mode, n):
+    """Mass and centre of every node against FP64 prefix sums over the sorted particles, for trees
+    of one chunk, of several, and on both sides of the size at which the chunks grow. A node's sum
+    is at most 8 terms of a leaf batch after another and then 4 children per level: a relative
+    error of about 100 x 2^-24 at most, 1e-5 with the centre's offsets measured in cell sides."""
+    rng = np.random.default_rng(n + 1)
+    x, y = rng.normal(0, 1, (2, n)).astype(np.float32)
+    if n > 100:
+        x[: n // 50] = y[: n // 50] = 0.5  # a crowded spot: a deep chain of cells, a large leaf
+    m = rng.uniform(0.5, 1.5, n).astype(np.float32)
+    ctx = BHContext(n, kernel="gravity", tree_mode=mode, softening=0.01)
+    ctx.set_particles(x, y, m)
+    ctx.build()
+    _, perm = ctx.morton()
+    t = ctx.tree()
+    ctx.close()
+    ms = m[perm].astype(np.float64)
+    s0, sx, sy = (np.concatenate([[0.0], np.cumsum(v)])
+                  for v in (ms, ms * x[perm].astype(np.float64), ms * y[perm].astype(np.float64)))
+    f, e = t["first"].astype(np.int64), t["first"].astype(np.int64) + t["count"].astype(np.int64)
+    assert f[0] == 0 and e[0] == n and t["skip"][0] == len(f)
+    mass = s0[e] - s0[f]
+    assert np.max(np.abs(t["mass"] - mass) / mass) < 1e-5
+    extent = max(np.ptp(x), np.ptp(y), 1e-3)
+    assert np.max(np.abs(t["cx"] - (sx[e] - sx[f]) / mass)) < 1e-5 * extent
+    assert np.max(np.abs(t["cy"] - (sy[e] - sy[f]) / mass)) < 1e-5 * extent
