@@ -63,7 +63,7 @@ struct bh_ctx {
     void *keys_a = nullptr, *keys_b = nullptr;
     uint32_t *vals_a = nullptr, *vals_b = nullptr;
     uint32_t* sort_scratch = nullptr;  // sort counts, look-back words, totals, tickets
-    uint32_t* scan_part = nullptr;
+    uint32_t* tree_sums = nullptr;
     uint8_t *leaf_lvl = nullptr, *lcp1 = nullptr;
     uint32_t *cnt = nullptr, *noff = nullptr;
     Node* nodes = nullptr;
@@ -336,7 +336,7 @@ bh_status do_build(bh_ctx* c, const double* bounds) {
     if (!quadtree) c->depth = fixed;
     phase_begin(c, 3);
     launch_tree(s, codes, c->wide, n, c->B, c->cfg.max_children, fixed, quadtree ? 1 : 0,
-                c->leaf_lvl, c->lcp1, c->cnt, c->noff, c->scan_part, c->prm, c->nodes, c->parent,
+                c->leaf_lvl, c->lcp1, c->cnt, c->noff, c->tree_sums, c->prm, c->nodes, c->parent,
                 c->child4, c->cap_nodes, c->R, c->nsys ? c->sys_prm : nullptr, c->dstatus);
     if (c->nsys) launch_batch_roots(s, c->sys_off, c->nsys, c->noff, c->prm, c->roots);
     phase_end(c, 3);
@@ -576,7 +576,7 @@ static bh_status create_impl(bh_ctx** out, const bh_config* cfg, uint32_t extra_
     TRY(dalloc(c, &c->vals_a, N));
     TRY(dalloc(c, &c->vals_b, N));
     TRY(dalloc(c, &c->sort_scratch, sort_scratch_words(N)));
-    TRY(dalloc(c, &c->scan_part, scan_partials_size(N) + 256));
+    TRY(dalloc(c, &c->tree_sums, tree_tiles(N)));
     TRY(dalloc(c, &c->leaf_lvl, N));
     TRY(dalloc(c, &c->lcp1, N));
     TRY(dalloc(c, &c->cnt, N));

@@ -1044,27 +1044,32 @@ __global__ __launch_bounds__(kBlock) void k_gather(const uint32_t* __restrict__ 
 // ------------------------------------------------------------------------------------------
 // tree: leaf level per particle, node count per particle
 // ------------------------------------------------------------------------------------------
+// The node count of each tile of kTreeTile particles goes to sums: k_tree_emit_heads takes the
+// counts of the tiles before its own from there, so the device-wide scan needs no launch of its
+// own (three launches of 2 to 4 us each before).
+constexpr int kTreeTile = 1024;
 template <typename K>
-__global__ __launch_bounds__(kBlock) void k_tree_levels(const K* __restrict__ codes, uint32_t n,
+__global__ __launch_bounds__(kTreeTile) void k_tree_levels(const K* __restrict__ codes, uint32_t n,
                                                         int B, int R, int cap, int fixed_depth,
                                                         uint8_t* __restrict__ leaf_lvl,
                                                         uint8_t* __restrict__ lcp1,
                                                         uint32_t* __restrict__ cnt,
+                                                        uint32_t* __restrict__ sums,
                                                         const uint32_t* __restrict__ status) {
-    __shared__ K s_code[kBlock + 2 * kMaxLeafCap];
-    __shared__ int8_t s_w[kBlock + kMaxLeafCap];
-    const int64_t b0 = (int64_t)blockIdx.x * kBlock;
+    __shared__ K s_code[kTreeTile + 2 * kMaxLeafCap];
+    __shared__ int8_t s_w[kTreeTile + kMaxLeafCap];
+    const int64_t b0 = (int64_t)blockIdx.x * kTreeTile;
     const int adaptive = fixed_depth < 0;
     if (adaptive) {
-        const int span = kBlock + 2 * cap;
-        for (int t = threadIdx.x; t < span; t += kBlock) {
+        const int span = kTreeTile + 2 * cap;
+        for (int t = threadIdx.x; t < span; t += kTreeTile) {
             const int64_t j = b0 - cap + t;
             s_code[t] = (j >= 0 && j < (int64_t)n) ? codes[j] : (K)0;
         }
         __syncthreads();
         // w(j) = common level of particles j and j+cap: the window [j, j+cap] shares a cell of
         // that level, so a cell holding i splits while some window through i shares it
-        for (int t = threadIdx.x; t < kBlock + cap; t += kBlock) {
+        for (int t = threadIdx.x; t < kTreeTile + cap; t += kTreeTile) {
             const int64_t j = b0 - cap + t;
             int8_t wv = -1;
             if (j >= 0 && j + cap < (int64_t)n) wv = (int8_t)lcp_level(s_code[t], s_code[t + cap], B);
@@ -1073,79 +1078,90 @@ __global__ __launch_bounds__(kBlock) void k_tree_levels(const K* __restrict__ co
         __syncthreads();
     }
     const int64_t i = b0 + threadIdx.x;
-    if (i >= (int64_t)n) return;
-    int leaf;
-    if (adaptive) {
-        int m = -1;
-        for (int t = 0; t <= cap; ++t) m = max(m, (int)s_w[threadIdx.x + t]);
-        leaf = max(min(m + 1, B), R);  // more than `cap` in the finest cell: stop at depth B
-    } else {
-        leaf = fixed_depth;
+    uint32_t c = 0;
+    if (i < (int64_t)n) {
+        int leaf;
+        if (adaptive) {
+            int m = -1;
+            for (int t = 0; t <= cap; ++t) m = max(m, (int)s_w[threadIdx.x + t]);
+            leaf = max(min(m + 1, B), R);  // more than `cap` in the finest cell: stop at depth B
+        } else {
+            leaf = fixed_depth;
+        }
+        // levels below R only separate batched systems: every system's tree starts at level R
+        const int lp = max((i == 0) ? -1 : lcp_level(codes[i - 1], codes[i], B), R - 1);
+        leaf_lvl[i] = (uint8_t)leaf;
+        lcp1[i] = (uint8_t)(lp + 1);
+        // a build whose sort gave up or whose input is not finite gets an empty tree: every walk
+        // over it ends at once (the call reports the error)
+        const bool failed = (status[0] | status[1]) != 0u;
+        c = (!failed && leaf > lp) ? (uint32_t)(leaf - lp) : 0u;
+        cnt[i] = c;
     }
-    // levels below R only separate batched systems: every system's tree starts at level R
-    const int lp = max((i == 0) ? -1 : lcp_level(codes[i - 1], codes[i], B), R - 1);
-    leaf_lvl[i] = (uint8_t)leaf;
-    lcp1[i] = (uint8_t)(lp + 1);
-    // a build whose sort gave up or whose input is not finite gets an empty tree: every walk
-    // over it ends at once (the call reports the error)
-    const bool failed = (status[0] | status[1]) != 0u;
-    cnt[i] = (!failed && leaf > lp) ? (uint32_t)(leaf - lp) : 0u;
+    uint32_t tot;
+    block_exclusive_scan_t<kTreeTile>(c, &tot);
+    if (threadIdx.x == 0) sums[blockIdx.x] = tot;
 }
 
-// first j >= lo with codes[j] > hi_key (codes ascending), galloping then binary search
-template <typename K>
-__device__ __forceinline__ uint32_t upper_from(const K* __restrict__ codes, uint32_t n, K hi_key,
-                                               uint32_t lo) {
-    uint32_t step = 1, hi = lo;
-    while (hi < n && codes[hi] <= hi_key) {
-        lo = hi + 1;
-        hi = lo + step;
-        step <<= 1;
-    }
-    if (hi > n) hi = n;
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (codes[mid] <= hi_key)
-            lo = mid + 1;
-        else
-            hi = mid;
-    }
-    return lo;
-}
+// k_tree_emit_nodes is bound by its loads: scattered ones (one line per lane) and, past the L2
+// (another XCD wrote the data), chains of them. A node's two searches in the sorted codes run side
+// by side, start with kProbes codes at distances 1, 2, 4 .. (most cells are small), narrow what is
+// still open in LDS (every block holds one code in `stride`, s_key[t] = codes[t * stride]) and end
+// with an 8-ary search; only lanes that need a search load for it. A gallop and a binary search
+// in memory took up to 2 log2(n) loads one after another for the topmost cells: 16 -> 10 us at 70k
+// points, 17 -> 9.5 at 200k, 25 -> 17 at 1M. Blocks of 256: with 1024 threads the scattered loads
+// of a small tree meet on few CUs (17 us at 70k), and 6 probes load more than they save.
+constexpr int kTreeKeys = 1024, kTreeThreads = 256, kProbes = 4;
 
-// first j <= hi with codes[j] >= lo_key (codes ascending), galloping backwards
+// a search for the first j in [a, b) with codes[j] > key, else b
 template <typename K>
-__device__ __forceinline__ uint32_t lower_back(const K* __restrict__ codes, K lo_key, uint32_t hi) {
-    uint32_t step = 1, lo = hi;
-    while (lo > 0 && codes[lo - 1] >= lo_key) {
-        hi = lo - 1;
-        lo = (hi > step) ? hi - step : 0;
-        step <<= 1;
-    }
-    // answer in [lo, hi]: first index with codes[j] >= lo_key
-    while (lo < hi) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (codes[mid] >= lo_key)
-            hi = mid;
+struct CodeSearch {
+    K key;
+    uint32_t a, b;
+    __device__ __forceinline__ void see(uint32_t j, K c) {  // codes[j] = c; any order of probes
+        if (c > key)
+            b = min(b, j);
         else
-            lo = mid + 1;
+            a = max(a, j + 1);
     }
-    return lo;
-}
+    __device__ __forceinline__ void table(const K* s_key, uint32_t keys, uint32_t stride) {
+        uint32_t u = 0, v = keys;  // first sample above key
+        while (u < v) {
+            const uint32_t mid = (u + v) >> 1;
+            if (s_key[mid] <= key)
+                u = mid + 1;
+            else
+                v = mid;
+        }
+        if (u) a = max(a, (u - 1) * stride);
+        if (u < keys) b = min(b, u * stride);
+    }
+    __device__ __forceinline__ uint32_t probe(uint32_t t) const {  // t in 0 .. 6, a < b
+        const uint32_t len = b - a;
+        return a + (len >> 3) * (t + 1) + (((len & 7) * (t + 1)) >> 3);
+    }
+};
 
 // nodes of particle i: k = noff[i] + t at level lcp1[i] + t, t < cnt[i]
-__global__ __launch_bounds__(kBlock) void k_tree_emit_heads(uint32_t n,
-                                                            const uint8_t* __restrict__ lcp1,
-                                                            const uint32_t* __restrict__ cnt,
-                                                            const uint32_t* __restrict__ noff,
-                                                            Node* __restrict__ nodes,
-                                                            uint4* __restrict__ child4,
-                                                            uint32_t cap_nodes) {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+__global__ __launch_bounds__(kTreeTile) void k_tree_emit_heads(uint32_t n,
+                                                               const uint8_t* __restrict__ lcp1,
+                                                               const uint32_t* __restrict__ cnt,
+                                                               const uint32_t* __restrict__ sums,
+                                                               uint32_t* __restrict__ noff,
+                                                               BuildParams* __restrict__ prm,
+                                                               Node* __restrict__ nodes,
+                                                               uint4* __restrict__ child4,
+                                                               uint32_t cap_nodes) {
+    const uint32_t i = blockIdx.x * kTreeTile + threadIdx.x;
+    const uint32_t c = i < n ? cnt[i] : 0u;
+    const uint32_t l0 = i < n ? lcp1[i] : 0u;
+    uint32_t before = 0, all, tot;
+    for (uint32_t b = threadIdx.x; b < blockIdx.x; b += kTreeTile) before += sums[b];
+    block_exclusive_scan_t<kTreeTile>(before, &all);
+    const uint32_t base = all + block_exclusive_scan_t<kTreeTile>(c, &tot);
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) prm->n_nodes = all + tot;
     if (i >= n) return;
-    const uint32_t c = cnt[i];
-    const uint32_t base = noff[i];
-    const uint32_t l0 = lcp1[i];
+    noff[i] = base;
     for (uint32_t t = 0; t < c; ++t) {
         const uint32_t k = base + t;
         if (k >= cap_nodes) break;  // cannot happen for the capacity the context allocates
@@ -1157,7 +1173,7 @@ __global__ __launch_bounds__(kBlock) void k_tree_emit_heads(uint32_t n,
 
 // one thread per node: subtree extent, flags, side, parent and the parent's child slot
 template <typename K>
-__global__ __launch_bounds__(kBlock) void k_tree_emit_nodes(const K* __restrict__ codes,
+__global__ __launch_bounds__(kTreeThreads) void k_tree_emit_nodes(const K* __restrict__ codes,
                                                             uint32_t n, int B, int R,
                                                             const uint8_t* __restrict__ lcp1,
                                                             const uint32_t* __restrict__ noff,
@@ -1168,48 +1184,90 @@ __global__ __launch_bounds__(kBlock) void k_tree_emit_nodes(const K* __restrict_
                                                             uint32_t* __restrict__ parent,
                                                             uint32_t* __restrict__ child4,
                                                             uint32_t cap_nodes) {
-    const uint32_t k = blockIdx.x * kBlock + threadIdx.x;
+    __shared__ K s_key[kTreeKeys];
+    const uint32_t k = blockIdx.x * kTreeThreads + threadIdx.x;
+    const Node n0 = nodes[min(k, cap_nodes - 1)];  // not yet written past the last node
     const uint32_t total = prm->n_nodes;
+    if (blockIdx.x * kTreeThreads >= min(total, cap_nodes)) return;
+    const uint32_t stride = (n + kTreeKeys - 1) / kTreeKeys, keys = (n + stride - 1) / stride;
+    for (uint32_t t = threadIdx.x; t < keys; t += kTreeThreads) s_key[t] = codes[t * stride];
+    __syncthreads();
     if (k >= total || k >= cap_nodes) return;
-    const uint32_t i = nodes[k].first;
-    uint32_t meta = nodes[k].meta;
+    const uint32_t i = n0.first;
+    uint32_t meta = n0.meta;
     const int l = (int)(meta & kMetaLevelMask);
     const K ci = codes[i];
-    uint32_t e;
-    if (l == 0) {  // the single root of a one-system tree (R = 0)
-        e = n;
-    } else {
-        const int sh = 2 * (B - l);
-        const K hk = ci | (K)(((K)1 << sh) - 1);
-        e = upper_from(codes, n, hk, i + 1);
+    // end of the cell: first code above its last one (the single root of a one-system tree, level
+    // 0, ends at n); first particle of the parent's cell, for the head of a run of nodes
+    const bool up = l > 0, back = l > max(R, 1) && (meta & kMetaHead);
+    CodeSearch<K> e{(K)0, n, n}, ip{(K)0, 0, 0};
+    if (up) e = CodeSearch<K>{ci | (K)(((K)1 << (2 * (B - l))) - 1), i + 1, n};
+    if (back) {
+        const K lk = ci & ~(K)(((K)1 << (2 * (B - l + 1))) - 1);
+        if (lk) ip = CodeSearch<K>{lk - 1, 0, i};
     }
+    {
+        K q[kProbes], r[kProbes];
+        if (up) {
+#pragma unroll
+            for (uint32_t t = 0; t < kProbes; ++t) q[t] = codes[min(i + (1u << t), n - 1)];
+        }
+        if (back) {
+#pragma unroll
+            for (uint32_t t = 0; t < kProbes; ++t) r[t] = codes[i >= (1u << t) ? i - (1u << t) : 0u];
+        }
+#pragma unroll
+        for (uint32_t t = 0; t < kProbes; ++t) {
+            if (up && i + (1u << t) < n) e.see(i + (1u << t), q[t]);
+            if (ip.b && i >= (1u << t)) ip.see(i - (1u << t), r[t]);
+        }
+    }
+    if (e.b - e.a > (1u << kProbes)) e.table(s_key, keys, stride);
+    if (ip.b - ip.a > (1u << kProbes)) ip.table(s_key, keys, stride);
+    for (;;) {
+        const bool se = e.a < e.b, si = ip.a < ip.b;
+        if (!se && !si) break;
+        uint32_t je[7], ji[7];
+        K q[7], r[7];
+#pragma unroll
+        for (uint32_t t = 0; t < 7; ++t) {
+            je[t] = e.probe(t);
+            ji[t] = ip.probe(t);
+        }
+        if (se) {
+#pragma unroll
+            for (uint32_t t = 0; t < 7; ++t) q[t] = codes[je[t]];
+        }
+        if (si) {
+#pragma unroll
+            for (uint32_t t = 0; t < 7; ++t) r[t] = codes[ji[t]];
+        }
+#pragma unroll
+        for (uint32_t t = 0; t < 7; ++t) {
+            if (se) e.see(je[t], q[t]);
+            if (si) ip.see(ji[t], r[t]);
+        }
+    }
+    const uint32_t end = e.a;
+    const K last = codes[end - 1];
+    const uint32_t skip = end < n ? noff[end] : total;
+    const uint32_t pk = back ? noff[ip.a] + (uint32_t)(l - 1 - (int)lcp1[ip.a]) : 0u;
     if (meta & kMetaLeaf) {
         meta |= kMetaPP;
     } else if (single_child_pp) {
         const int shc = 2 * (B - l - 1);
-        if (((uint32_t)(ci >> shc) & 3u) == ((uint32_t)(codes[e - 1] >> shc) & 3u)) meta |= kMetaPP;
+        if (((uint32_t)(ci >> shc) & 3u) == ((uint32_t)(last >> shc) & 3u)) meta |= kMetaPP;
     }
     const BuildParams* sp = R ? sys_prm + (uint32_t)(ci >> (2 * (B - R))) : prm;
     const float sl = ldexpf(sp->side, -(l - R));
     Node* nd = nodes + k;
     nd->l2 = sl * sl;
-    nd->skip = (e < n) ? noff[e] : total;
-    nd->count = e - i;
+    nd->skip = skip;
+    nd->count = end - i;
     nd->meta = meta;
     uint32_t par = kNone;
     if (l > R) {
-        if (!(meta & kMetaHead)) {
-            par = k - 1;
-        } else {
-            const int pl = l - 1;
-            uint32_t ip = 0;
-            if (pl > 0) {
-                const int psh = 2 * (B - pl);
-                const K lk = ci & ~(K)(((K)1 << psh) - 1);
-                ip = lower_back(codes, lk, i);
-            }
-            par = noff[ip] + (uint32_t)(pl - (int)lcp1[ip]);
-        }
+        par = !(meta & kMetaHead) ? k - 1 : pk;
         child4[4ull * par + ((uint32_t)(ci >> (2 * (B - l))) & 3u)] = k;
     }
     parent[k] = par;
@@ -1914,29 +1972,27 @@ void launch_gather(hipStream_t s, const uint32_t* perm, uint32_t n, const float*
                                                   vyo, ido, pos4, sort_err, codes, wide ? 1 : 0);
 }
 
+uint32_t tree_tiles(uint32_t n) { return div_up(n, kTreeTile); }
+
 void launch_tree(hipStream_t s, const void* codes, bool wide, uint32_t n, int B, int cap,
                  int fixed_depth, int single_child_pp, uint8_t* leaf_lvl, uint8_t* lcp1,
-                 uint32_t* cnt, uint32_t* noff, uint32_t* scan_partials, BuildParams* prm,
+                 uint32_t* cnt, uint32_t* noff, uint32_t* sums, BuildParams* prm,
                  Node* nodes, uint32_t* parent, uint32_t* child4, uint32_t cap_nodes, int R,
                  const BuildParams* sys_prm, const uint32_t* status) {
-    const uint32_t g = div_up(n, kBlock);
-    if (wide)
-        k_tree_levels<uint64_t><<<g, kBlock, 0, s>>>((const uint64_t*)codes, n, B, R, cap,
-                                                     fixed_depth, leaf_lvl, lcp1, cnt, status);
-    else
-        k_tree_levels<uint32_t><<<g, kBlock, 0, s>>>((const uint32_t*)codes, n, B, R, cap,
-                                                     fixed_depth, leaf_lvl, lcp1, cnt, status);
-    launch_exclusive_scan(s, cnt, noff, n, scan_partials, &prm->n_nodes);
-    k_tree_emit_heads<<<g, kBlock, 0, s>>>(n, lcp1, cnt, noff, nodes, (uint4*)child4, cap_nodes);
-    const uint32_t gn = div_up(cap_nodes, kBlock);
-    if (wide)
-        k_tree_emit_nodes<uint64_t><<<gn, kBlock, 0, s>>>((const uint64_t*)codes, n, B, R, lcp1,
-                                                          noff, prm, sys_prm, single_child_pp,
-                                                          nodes, parent, child4, cap_nodes);
-    else
-        k_tree_emit_nodes<uint32_t><<<gn, kBlock, 0, s>>>((const uint32_t*)codes, n, B, R, lcp1,
-                                                          noff, prm, sys_prm, single_child_pp,
-                                                          nodes, parent, child4, cap_nodes);
+    const uint32_t g = div_up(n, kTreeTile), gn = div_up(cap_nodes, kTreeThreads);
+#define BH_LEVELS(K)                                                                              \
+    k_tree_levels<K><<<g, kTreeTile, 0, s>>>((const K*)codes, n, B, R, cap, fixed_depth,          \
+                                             leaf_lvl, lcp1, cnt, sums, status)
+#define BH_NODES(K)                                                                               \
+    k_tree_emit_nodes<K><<<gn, kTreeThreads, 0, s>>>((const K*)codes, n, B, R, lcp1, noff, prm,      \
+                                                  sys_prm, single_child_pp, nodes, parent,        \
+                                                  child4, cap_nodes)
+    if (wide) BH_LEVELS(uint64_t); else BH_LEVELS(uint32_t);
+    k_tree_emit_heads<<<g, kTreeTile, 0, s>>>(n, lcp1, cnt, sums, noff, prm, nodes,
+                                              (uint4*)child4, cap_nodes);
+    if (wide) BH_NODES(uint64_t); else BH_NODES(uint32_t);
+#undef BH_LEVELS
+#undef BH_NODES
 }
 
 void launch_bounds_batched(hipStream_t s, const float* xs, const float* ys, const uint2* blk,

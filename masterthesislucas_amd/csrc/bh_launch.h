@@ -44,9 +44,10 @@ void launch_gather(hipStream_t s, const uint32_t* perm, uint32_t n, const float*
                    float* yo, float* mo, float* vxo, float* vyo, uint32_t* ido, float4* pos4,
                    const uint32_t* sort_err, void* codes, bool wide);
 // R: level of the tree roots (0; batched systems: the system id occupies the levels above R)
+uint32_t tree_tiles(uint32_t n);  // words of launch_tree's sums
 void launch_tree(hipStream_t s, const void* codes, bool wide, uint32_t n, int B, int cap,
                  int fixed_depth, int single_child_pp, uint8_t* leaf_lvl, uint8_t* lcp1,
-                 uint32_t* cnt, uint32_t* noff, uint32_t* scan_partials, BuildParams* prm,
+                 uint32_t* cnt, uint32_t* noff, uint32_t* sums, BuildParams* prm,
                  Node* nodes, uint32_t* parent, uint32_t* child4, uint32_t cap_nodes, int R,
                  const BuildParams* sys_prm, const uint32_t* status);
 void launch_bounds_batched(hipStream_t s, const float* xs, const float* ys, const uint2* blk,

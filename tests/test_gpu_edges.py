@@ -6,6 +6,7 @@ import pytest
 from masterthesislucas_amd import BHContext, tsne
 from masterthesislucas_amd.learned import N_OUT, FarFieldMLP, flatten, unflatten
 from oracle import oracle as O
+from tests.helpers import oracle_tree
 
 pytestmark = pytest.mark.gpu
 
@@ -266,3 +267,26 @@ def test_node_moments_edges(gpu, mode, n):
     extent = max(np.ptp(x), np.ptp(y), 1e-3)
     assert np.max(np.abs(t["cx"] - (sx[e] - sx[f]) / mass)) < 1e-5 * extent
     assert np.max(np.abs(t["cy"] - (sy[e] - sy[f]) / mass)) < 1e-5 * extent
+
+
+@pytest.mark.parametrize("mode", ["quadtree", "morton_fixed"])
+@pytest.mark.parametrize("n", [1, 17, 1023, 1024, 1025, 2049, 33_000])
+def test_tree_emission_edges(gpu, mode, n):
+    """Node numbering over tiles of 1024 particles, cells found near a particle, through the block's
+    table of codes and by the wide search: every record equals the oracle's. A crowded spot gives
+    long chains of single cells and leaves past the table's stride."""
+    rng = np.random.default_rng(n + 2)
+    x, y = rng.normal(0, 1, (2, n)).astype(np.float32)
+    if n > 1000:
+        x[: n // 3] = (0.5 + 1e-3 * rng.normal(0, 1, n // 3)).astype(np.float32)
+        y[: n // 3] = (0.5 + 1e-3 * rng.normal(0, 1, n // 3)).astype(np.float32)
+        x[: n // 20] = y[: n // 20] = np.float32(0.5)
+    ctx = BHContext(n, kernel="gravity", tree_mode=mode, softening=0.01)
+    ctx.set_particles(x, y)
+    ctx.build()
+    g = ctx.tree()
+    ctx.close()
+    t = oracle_tree(x, y, mode=mode)
+    for k in ("level", "first", "count", "skip"):
+        assert np.array_equal(g[k].astype(np.int64), t["tree"][k].astype(np.int64)), k
+    assert np.array_equal((g["flags"] >> 1) & 1, t["pp"])
