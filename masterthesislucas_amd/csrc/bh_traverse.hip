@@ -65,12 +65,17 @@ __device__ __forceinline__ NodeBits load_node(const Node* __restrict__ nodes, ui
 //
 // Sums. Every sink has kWalkParts compensated sums; entry i of a step's accepted cells and source
 // i of a particle-particle cell belong to part i % kWalkParts, and the parts are added in order,
-// with compensation, at the end. A part's plain sums are folded into its compensated ones after at most 8 cells or
-// 16 sources (error against FP64 sums of the same interactions: 2.8e-8 rms of the summed
+// with compensation, at the end. A part's plain sums are folded into its compensated ones after at
+// most 8 cells or 16 sources (error against FP64 sums of the same interactions: 2.8e-8 rms of the summed
 // magnitudes on the two disks, as before). Because the parts are fixed, 1, 2 or 4 waves can share a sink group (NP = 4, 2 or 1
 // parts per wave: they all take the same path and add only their parts) with bit-identical
 // results: launches with too few sink groups to fill the device use more waves per group
-// (walk_waves_per_group).
+// (walk_waves_per_group). A particle-particle cell of more than kWalkGiant points, gravity (a cell
+// with one child is one, and can hold a whole cluster), is one plain sum over its sources in
+// order, added to part 0: the rounding of so long a plain sum can exceed the rest of a sink's
+// error by far (half of 1M points in one cell: 0.6%), so its order is part of the result and
+// stays what it has always been. Telling such cells apart costs 0.5% of a walk without them; a
+// walk over one with 524,288 points 331 -> 258 ms.
 //
 // Bound by VALU issue (13 slots per interaction, the reciprocal square root counting as four)
 // where the waves fill the device, by the latency of the steps where they do not. Measured
@@ -89,6 +94,7 @@ constexpr int kWalkDeep = 3 * kMaxLevels;    // entries a depth-first descent ca
 constexpr int kWalkCells = 96;               // particle-particle cells waiting
 constexpr int kWalkFlush = kWalkCells - 64;  // summed above this many (a step adds at most 64)
 constexpr uint32_t kWalkFold = 16;           // terms of a part's plain sum
+constexpr uint32_t kWalkGiant = 4096;        // points of a cell that is summed by itself
 static_assert(kWalkStack >= kWalkDeep + 4 * kWalkPop, "room for a bulk step and a descent");
 
 struct __attribute__((aligned(16))) WalkLds {  // per wave
@@ -237,94 +243,134 @@ __global__ __launch_bounds__(kBlock) void k_walk(const float4* __restrict__ pos4
         for (int c0 = 0; c0 < nc; c0 += kWave) {
             const int nn = min(nc - c0, kWave);
             const uint4 cell = (int)lane < nn ? L.cells[c0 + lane] : make_uint4(0, 0, 0, 0);
-            const uint32_t cr = (cell.y + 3u) & ~3u;  // slots: whole quads
-            uint32_t end = cr;
-            for (int o = 1; o < kWave; o <<= 1) {
-                const uint32_t t = __shfl_up(end, o, kWave);
-                if ((int)lane >= o) end += t;
-            }
-            const uint32_t off = end - cr, stop = off + cell.y;
-            const bool own = cell.x < base + count && base < cell.x + cell.y;
-            const uint32_t total = lane_read(end, kWave - 1);
-            // the source of this lane's slot in the 64 slots from `blk` on; the slots past a
-            // cell's last source repeat it
-            auto fetch = [&](uint32_t blk) {
-                uint32_t src = 0;
-                uint64_t m = __ballot(end > blk && off < blk + kWave && cr != 0u);
-                while (m) {
-                    const uint32_t e = (uint32_t)__builtin_ctzll(m);
-                    m &= m - 1;
-                    const uint32_t o = lane_read(off, e);
-                    if (blk + lane >= o)
-                        src = lane_read(cell.x, e) +
-                              min(blk + lane - o, lane_read(cell.y, e) - 1u);
+            // the ordinary cells, then the giant ones each by itself
+            uint64_t giants = __ballot(KERNEL == kKernelGravity && cell.y > kWalkGiant);
+            uint32_t giant = kNone;
+            bool now = KERNEL != kKernelGravity || cell.y <= kWalkGiant;
+            for (;;) {
+                const uint32_t cr = now ? (cell.y + 3u) & ~3u : 0u;  // slots: whole quads
+                uint32_t end = cr;
+                for (int o = 1; o < kWave; o <<= 1) {
+                    const uint32_t t = __shfl_up(end, o, kWave);
+                    if ((int)lane >= o) end += t;
                 }
-                return pos4[src];
-            };
-            float4 q = fetch(0);
-            for (uint32_t blk = 0; blk < total; blk += kWave) {
-                const bool mine = !BATCHED || blk_no == 0u;
-                if constexpr (BATCHED) blk_no = blk_no + 1u == sF ? 0u : blk_no + 1u;
-                wave_lds_sync();
-                L.rec[lane] = q;
-                wave_lds_sync();
-                if (blk + kWave < total) q = fetch(blk + kWave);  // in flight during the sums
-                if (!mine) continue;
-                // cells without sinks of this wave, then those that hold some
-                const bool here = stop > blk && off < blk + kWave && cr != 0u;
-                const uint32_t from = max(off, blk) - blk, to = min(stop - blk, (uint32_t)kWave);
-                uint64_t m = __ballot(here && !own);
-                while (m) {
-                    const uint32_t e = (uint32_t)__builtin_ctzll(m);
-                    m &= m - 1;
-                    uint32_t j = lane_read(from, e);  // a multiple of 4
-                    const uint32_t b = lane_read(to, e);
-                    const uint64_t msk = lane_read2(cell.z, cell.w, e);
-                    const uint32_t quads = (b - j + 3u) >> 2;
-                    if (terms + quads > kWalkFold) fold_all();
-                    terms += quads;
-                    if (__builtin_amdgcn_inverse_ballot_w64(msk)) {
-                        for (; j + 4 <= b; j += 4) {
-                            float4 s[NP];
+                const uint32_t off = end - cr, stop = off + cell.y;
+                const bool own = cell.x < base + count && base < cell.x + cell.y;
+                const uint32_t total = lane_read(end, kWave - 1);
+                // the source of this lane's slot in the 64 slots from `blk` on; the slots past a
+                // cell's last source repeat it
+                auto fetch = [&](uint32_t blk) {
+                    uint32_t src = 0;
+                    uint64_t m = __ballot(end > blk && off < blk + kWave && cr != 0u);
+                    while (m) {
+                        const uint32_t e = (uint32_t)__builtin_ctzll(m);
+                        m &= m - 1;
+                        const uint32_t o = lane_read(off, e);
+                        if (blk + lane >= o)
+                            src = lane_read(cell.x, e) +
+                                  min(blk + lane - o, lane_read(cell.y, e) - 1u);
+                    }
+                    return pos4[src];
+                };
+                float4 q = fetch(0);
+                for (uint32_t blk = 0; blk < total; blk += kWave) {
+                    const bool mine = !BATCHED || blk_no == 0u;
+                    if constexpr (BATCHED) blk_no = blk_no + 1u == sF ? 0u : blk_no + 1u;
+                    wave_lds_sync();
+                    L.rec[lane] = q;
+                    wave_lds_sync();
+                    if (blk + kWave < total) q = fetch(blk + kWave);  // in flight during the sums
+                    if (!mine) continue;
+                    if (giant != kNone) {  // one cell in order, in one plain sum
+                        if (p0 != 0) continue;
+                        const uint32_t b = min(lane_read(cell.y, giant) - blk, (uint32_t)kWave);
+                        const int s0 = (int)(base - lane_read(cell.x, giant) - blk);  // first sink
+                        const uint64_t msk = lane_read2(cell.z, cell.w, giant);
+                        if (!__builtin_amdgcn_inverse_ballot_w64(msk)) continue;
+                        if (s0 >= (int)b || s0 + (int)count <= 0) {
+                            uint32_t j = 0;
+                            for (; j + 4 <= b; j += 4) {
+                                float4 s[4];
 #pragma unroll
-                            for (int p = 0; p < NP; ++p) s[p] = L.rec[j + p0 + p];
+                                for (int t = 0; t < 4; ++t) s[t] = L.rec[j + t];
+#pragma unroll
+                                for (int t = 0; t < 4; ++t)
+                                    walk_pair<KERNEL, TOT>(sum[0], s[t].x - px, s[t].y - py, s[t].z,
+                                                           eps2);
+                            }
+                            for (; j < b; ++j)
+                                walk_pair<KERNEL, TOT>(sum[0], L.rec[j].x - px, L.rec[j].y - py,
+                                                       L.rec[j].z, eps2);
+                        } else {
+                            for (uint32_t j = 0; j < b; ++j)
+                                if ((int)j != s0 + (int)lane)
+                                    walk_pair<KERNEL, TOT>(sum[0], L.rec[j].x - px, L.rec[j].y - py,
+                                                           L.rec[j].z, eps2);
+                        }
+                        continue;
+                    }
+                    // cells without sinks of this wave, then those that hold some
+                    const bool here = stop > blk && off < blk + kWave && cr != 0u;
+                    const uint32_t from = max(off, blk) - blk, to = min(stop - blk, (uint32_t)kWave);
+                    uint64_t m = __ballot(here && !own);
+                    while (m) {
+                        const uint32_t e = (uint32_t)__builtin_ctzll(m);
+                        m &= m - 1;
+                        uint32_t j = lane_read(from, e);  // a multiple of 4
+                        const uint32_t b = lane_read(to, e);
+                        const uint64_t msk = lane_read2(cell.z, cell.w, e);
+                        const uint32_t quads = (b - j + 3u) >> 2;
+                        if (terms + quads > kWalkFold) fold_all();
+                        terms += quads;
+                        if (__builtin_amdgcn_inverse_ballot_w64(msk)) {
+                            for (; j + 4 <= b; j += 4) {
+                                float4 s[NP];
+#pragma unroll
+                                for (int p = 0; p < NP; ++p) s[p] = L.rec[j + p0 + p];
+#pragma unroll
+                                for (int p = 0; p < NP; ++p)
+                                    walk_pair<KERNEL, TOT>(sum[p], s[p].x - px, s[p].y - py, s[p].z,
+                                                           eps2);
+                            }
 #pragma unroll
                             for (int p = 0; p < NP; ++p)
-                                walk_pair<KERNEL, TOT>(sum[p], s[p].x - px, s[p].y - py, s[p].z,
-                                                       eps2);
-                        }
-#pragma unroll
-                        for (int p = 0; p < NP; ++p)
-                            if (j + p0 + p < b) {
-                                const float4 s = L.rec[j + p0 + p];
-                                walk_pair<KERNEL, TOT>(sum[p], s.x - px, s.y - py, s.z, eps2);
-                            }
-                    }
-                }
-                m = __ballot(here && own);
-                while (m) {
-                    const uint32_t e = (uint32_t)__builtin_ctzll(m);
-                    m &= m - 1;
-                    uint32_t j = lane_read(from, e);
-                    const uint32_t b = lane_read(to, e);
-                    const uint64_t msk = lane_read2(cell.z, cell.w, e);
-                    // slot of the sink itself in this block
-                    const uint32_t self = idx - lane_read(cell.x, e) + lane_read(off, e) - blk;
-                    const uint32_t quads = (b - j + 3u) >> 2;
-                    if (terms + quads > kWalkFold) fold_all();
-                    terms += quads;
-                    if (__builtin_amdgcn_inverse_ballot_w64(msk)) {
-                        for (; j < b; j += 4)
-#pragma unroll
-                            for (int p = 0; p < NP; ++p) {
-                                const uint32_t jj = j + p0 + p;
-                                if (jj < b && jj != self) {
-                                    const float4 s = L.rec[jj];
+                                if (j + p0 + p < b) {
+                                    const float4 s = L.rec[j + p0 + p];
                                     walk_pair<KERNEL, TOT>(sum[p], s.x - px, s.y - py, s.z, eps2);
                                 }
-                            }
+                        }
+                    }
+                    m = __ballot(here && own);
+                    while (m) {
+                        const uint32_t e = (uint32_t)__builtin_ctzll(m);
+                        m &= m - 1;
+                        uint32_t j = lane_read(from, e);
+                        const uint32_t b = lane_read(to, e);
+                        const uint64_t msk = lane_read2(cell.z, cell.w, e);
+                        // slot of the sink itself in this block
+                        const uint32_t self = idx - lane_read(cell.x, e) + lane_read(off, e) - blk;
+                        const uint32_t quads = (b - j + 3u) >> 2;
+                        if (terms + quads > kWalkFold) fold_all();
+                        terms += quads;
+                        if (__builtin_amdgcn_inverse_ballot_w64(msk)) {
+                            for (; j < b; j += 4)
+#pragma unroll
+                                for (int p = 0; p < NP; ++p) {
+                                    const uint32_t jj = j + p0 + p;
+                                    if (jj < b && jj != self) {
+                                        const float4 s = L.rec[jj];
+                                        walk_pair<KERNEL, TOT>(sum[p], s.x - px, s.y - py, s.z, eps2);
+                                    }
+                                }
+                        }
                     }
                 }
+                if (giant != kNone) fold_all();
+                if (!giants) break;
+                giant = (uint32_t)__builtin_ctzll(giants);
+                giants &= giants - 1;
+                now = lane == giant;
+                fold_all();
             }
         }
         wave_lds_sync();

@@ -290,3 +290,48 @@ def test_tree_emission_edges(gpu, mode, n):
     for k in ("level", "first", "count", "skip"):
         assert np.array_equal(g[k].astype(np.int64), t["tree"][k].astype(np.int64)), k
     assert np.array_equal((g["flags"] >> 1) & 1, t["pp"])
+
+
+@pytest.mark.parametrize("n", [20_000, 100_000, 140_000])
+def test_giant_cell_sums_in_order(gpu, n):
+    """A cell with one child is a particle-particle cell; one that holds a whole cluster is summed
+    in particle order in plain FP32 (1, 2 and 4 parts per wave). One source outweighs the others
+    by 2^26, so a plain sum loses most of them and any other order would differ by about 1e-4;
+    against the same sum in numpy to 2e-6 (terms to a few 2^-24)."""
+    rng = np.random.default_rng(n)
+    x, y = (0.30 + 0.02 * rng.random((2, n))).astype(np.float32)
+    m = np.full(n, 2.0 ** -26, np.float32)
+    x[0], y[0], m[0] = 0.30, 0.30, 1.0  # first in Morton order
+    x[1], y[1] = 1.0, 1.0
+    x[2], y[2] = 0.0, 0.0
+    y[2], x[2] = 0.99, 0.0  # keeps the box at [0, 1]
+    y[3], x[3] = 0.0, 0.99
+    eps = float(np.float32(1e-3))
+    ctx = BHContext(n, kernel="gravity", softening=eps)
+    ctx.set_particles(x, y, m)
+    ctx.build()
+    fx, fy = ctx.forces(0.5)[:2]
+    _, perm = ctx.morton()
+    t = ctx.tree()
+    ctx.close()
+    giant = np.nonzero(((t["flags"] >> 1) & 1).astype(bool) & (t["count"] > 4096))[0][0]
+    lo, hi = int(t["first"][giant]), int(t["first"][giant] + t["count"][giant])
+    assert hi - lo > n - 8
+    src = perm[lo:hi]
+    sinks = src[rng.integers(1, hi - lo, 64)]
+    f64, f32 = np.float64, np.float32
+    px, py = x[sinks], y[sinks]
+    gx, gy = np.zeros(64, f32), np.zeros(64, f32)
+    eps2 = f32(eps) * f32(eps)
+    for j in src:
+        dx, dy = x[j] - px, y[j] - py
+        d2 = (dx.astype(f64) ** 2 + (dy * dy).astype(f64)).astype(f32) + eps2
+        inv = (1.0 / np.sqrt(d2.astype(f64))).astype(f32)
+        g = m[j] * inv * inv * inv
+        on = sinks != j
+        gx = np.where(on, (gx.astype(f64) + g.astype(f64) * dx).astype(f32), gx)
+        gy = np.where(on, (gy.astype(f64) + g.astype(f64) * dy).astype(f32), gy)
+    # the few points outside the cell are far and light: below 1e-6 of the sums
+    scale = np.hypot(gx, gy)
+    assert np.max(np.abs(fx[sinks] - gx) / scale) < 2e-6
+    assert np.max(np.abs(fy[sinks] - gy) / scale) < 2e-6
