@@ -58,6 +58,8 @@ struct bh_ctx {
     float *x[2]{}, *y[2]{}, *m[2]{}, *vx[2]{}, *vy[2]{};
     uint32_t* id[2]{};
     float4* pos4 = nullptr;
+    float4* packed = nullptr;  // (x, y, mass, index) in input order, made and used by a build
+    bool v_zero = true;        // the velocities are all zero (no caller gave any, no kick yet)
     float *ax = nullptr, *ay = nullptr, *tot = nullptr;
     float *out_a = nullptr, *out_b = nullptr, *out_c = nullptr, *out_d = nullptr;
     void *keys_a = nullptr, *keys_b = nullptr;
@@ -296,21 +298,18 @@ bh_status do_build(bh_ctx* c, const double* bounds) {
     if (c->nsys) {
         launch_bounds_batched(s, c->x[cur], c->y[cur], c->bblk, c->nbblk, c->bblk_off, c->sys_off,
                               c->nsys, c->bpart, c->sys_prm, c->prm, c->dstatus);
-        launch_morton_batched(s, c->x[cur], c->y[cur], n, c->sys_off, c->nsys, c->sys_prm,
-                              c->qbits, (uint64_t*)c->keys_a, c->vals_a);
+        launch_morton_batched(s, c->x[cur], c->y[cur], c->m[cur], c->id[cur], n, c->sys_off, c->nsys,
+                              c->sys_prm, c->qbits, (uint64_t*)c->keys_a, c->vals_a, c->packed);
     } else {
         if (c->cfg.tree_mode == BH_TREE_GPU_REF) {
             // the reference GPU step takes the bounds of the points themselves
-            launch_bounds(s, c->x[cur], c->y[cur], n, c->bounds_part, c->prm, kTreeGpuRef, nullptr,
-                          c->dstatus);
-            launch_morton_gpuref(s, c->x[cur], c->y[cur], n, c->prm, fixed, (uint32_t*)c->keys_a,
-                                 c->vals_a);
+            launch_morton_gpuref(s, c->x[cur], c->y[cur], c->m[cur], c->id[cur], n, c->bounds_part,
+                                 c->prm, fixed, c->dstatus, (uint32_t*)c->keys_a, c->vals_a,
+                                 c->packed);
         } else {
-            launch_bounds(s, c->x[cur], c->y[cur], n, c->bounds_part, c->prm,
+            launch_morton(s, c->x[cur], c->y[cur], c->m[cur], c->id[cur], n, c->bounds_part, c->prm,
                           quadtree ? kTreeQuadTree : kTreeMortonFixed, quadtree ? nullptr : bounds,
-                          c->dstatus);
-            launch_morton(s, c->x[cur], c->y[cur], n, c->prm, c->B, c->keys_a, c->vals_a,
-                          c->wide);
+                          c->dstatus, c->B, c->keys_a, c->vals_a, c->wide, c->packed);
         }
     }
     phase_end(c, 0);
@@ -318,8 +317,8 @@ bh_status do_build(bh_ctx* c, const double* bounds) {
     phase_begin(c, 1);
     bool in_b = false;
     const int key_bits = c->nsys ? 2 * c->qbits + 2 * c->R : 2 * c->B;
-    launch_sort(s, c->keys_a, c->vals_a, c->keys_b, c->vals_b, n, key_bits, c->wide,
-                      c->sort_scratch, c->dstatus, c->sort_spin, &in_b);
+    launch_sort(s, c->keys_a, c->vals_a, c->keys_b, c->vals_b, n, key_bits, c->wide, c->sort_scratch,
+                c->dstatus, c->sort_spin, &in_b);
     phase_end(c, 1);
     c->keys_in_b = in_b;
     void* codes = in_b ? c->keys_b : c->keys_a;
@@ -327,9 +326,9 @@ bh_status do_build(bh_ctx* c, const double* bounds) {
 
     phase_begin(c, 2);
     const int nxt = 1 - cur;
-    launch_gather(s, perm, n, c->x[cur], c->y[cur], c->m[cur], c->vx[cur], c->vy[cur], c->id[cur],
-                  c->x[nxt], c->y[nxt], c->m[nxt], c->vx[nxt], c->vy[nxt], c->id[nxt], c->pos4,
-                  c->dstatus, codes, c->wide);
+    const float *vx = c->v_zero ? nullptr : c->vx[cur], *vy = c->v_zero ? nullptr : c->vy[cur];
+    launch_gather(s, perm, n, c->packed, vx, vy, c->x[nxt], c->y[nxt], c->m[nxt], c->vx[nxt],
+                  c->vy[nxt], c->id[nxt], c->pos4, c->dstatus, codes, c->wide);
     phase_end(c, 2);
     c->cur = nxt;
 
@@ -556,6 +555,7 @@ static bh_status create_impl(bh_ctx** out, const bh_config* cfg, uint32_t extra_
         TRY(dalloc(c, &c->id[k], N));
     }
     TRY(dalloc(c, &c->pos4, (size_t)N + kPosPad));
+    TRY(dalloc(c, &c->packed, N));
     TRY(dalloc(c, &c->ax, N));
     TRY(dalloc(c, &c->ay, N));
     TRY(dalloc(c, &c->tot, N));
@@ -745,20 +745,15 @@ static bh_status set_particles(bh_ctx* c, uint32_t n, const float* x, const floa
     bh_status st = hip_check(c, hipMemcpyAsync(c->x[0], x, b, kind, s), "upload x");
     if (st == BH_OK) st = hip_check(c, hipMemcpyAsync(c->y[0], y, b, kind, s), "upload y");
     if (st != BH_OK) return st;
-    if (m)
-        st = hip_check(c, hipMemcpyAsync(c->m[0], m, b, kind, s), "upload m");
-    else
-        launch_fill_f32(s, c->m[0], n, 1.0f);
-    if (st != BH_OK) return st;
-    if (vx) {
+    if (m) st = hip_check(c, hipMemcpyAsync(c->m[0], m, b, kind, s), "upload m");
+    if (st == BH_OK && vx) {
         st = hip_check(c, hipMemcpyAsync(c->vx[0], vx, b, kind, s), "upload vx");
         if (st == BH_OK) st = hip_check(c, hipMemcpyAsync(c->vy[0], vy, b, kind, s), "upload vy");
-        if (st != BH_OK) return st;
-    } else {
-        launch_fill_f32(s, c->vx[0], n, 0.0f);
-        launch_fill_f32(s, c->vy[0], n, 0.0f);
     }
-    launch_iota(s, c->id[0], n);
+    if (st != BH_OK) return st;
+    c->v_zero = vx == nullptr;
+    launch_init_state(s, n, c->id[0], m ? nullptr : c->m[0], vx ? nullptr : c->vx[0],
+                      vx ? nullptr : c->vy[0]);
     return hip_check(c, hipStreamSynchronize(s), "upload");
 }
 
@@ -842,6 +837,7 @@ bh_status bh_leapfrog(bh_ctx* c, int steps, float dt, double theta) {
     if (c->n == 0) return fail(c, BH_ERR_STATE, "no particles");
     bh_status st = status_begin(c);
     if (st != BH_OK) return st;
+    c->v_zero = false;  // the kicks, also those of replayed graphs
     if (!c->have_acc) {
         st = do_build(c, nullptr);
         if (st == BH_OK) st = do_forces(c, theta, false);
@@ -896,6 +892,7 @@ bh_status bh_leapfrog_graph(bh_ctx* c, int steps, float dt, double theta) {
     if (c->n == 0) return fail(c, BH_ERR_STATE, "no particles");
     bh_status st = status_begin(c);
     if (st != BH_OK) return st;
+    c->v_zero = false;  // the kicks, also those of replayed graphs
     if (!c->have_acc) {
         st = do_build(c, nullptr);
         if (st == BH_OK) st = do_forces(c, theta, false);

@@ -65,31 +65,42 @@ __global__ __launch_bounds__(kBlock) void k_bounds_partial(const float* __restri
 __device__ void fill_params(BuildParams* prm, float4 r, uint64_t mnx64, uint64_t mny64,
                             uint64_t mxx64, uint64_t mxy64, uint32_t tree_mode, uint32_t n);
 
-__global__ __launch_bounds__(kBlock) void k_bounds_final(const float4* __restrict__ partials,
-                                                         uint32_t nb, uint32_t n,
-                                                         BuildParams* __restrict__ prm,
-                                                         uint32_t tree_mode, int use_caller,
-                                                         double cminx, double cminy,
-                                                         double cmaxx, double cmaxy,
-                                                         uint32_t* __restrict__ status) {
+// the caller's bounds, or none
+struct CallerBounds {
+    int use;
+    double minx, miny, maxx, maxy;
+};
+
+// every thread of the block takes part; thread 0 fills *out (LDS or memory)
+__device__ __forceinline__ void bounds_final(const float4* __restrict__ partials, uint32_t nb,
+                                             uint32_t n, uint32_t tree_mode, CallerBounds cb,
+                                             BuildParams* out, uint32_t* status) {
     float4 r = make_float4(INFINITY, INFINITY, -INFINITY, -INFINITY);
     for (uint32_t b = threadIdx.x; b < nb; b += kBlock) r = minmax4(r, partials[b]);
     r = block_minmax4(r);
     if (threadIdx.x != 0) return;
-    flag_nonfinite(r, status);
+    if (status) flag_nonfinite(r, status);
     uint64_t mnx64, mny64, mxx64, mxy64;
-    if (use_caller) {
-        mnx64 = bh_sfp_f64_bits(cminx);
-        mny64 = bh_sfp_f64_bits(cminy);
-        mxx64 = bh_sfp_f64_bits(cmaxx);
-        mxy64 = bh_sfp_f64_bits(cmaxy);
+    if (cb.use) {
+        mnx64 = bh_sfp_f64_bits(cb.minx);
+        mny64 = bh_sfp_f64_bits(cb.miny);
+        mxx64 = bh_sfp_f64_bits(cb.maxx);
+        mxy64 = bh_sfp_f64_bits(cb.maxy);
     } else {
         mnx64 = bh_sfp_from_f32(r.x);
         mny64 = bh_sfp_from_f32(r.y);
         mxx64 = bh_sfp_from_f32(r.z);
         mxy64 = bh_sfp_from_f32(r.w);
     }
-    fill_params(prm, r, mnx64, mny64, mxx64, mxy64, tree_mode, n);
+    fill_params(out, r, mnx64, mny64, mxx64, mxy64, tree_mode, n);
+}
+
+__global__ __launch_bounds__(kBlock) void k_bounds_final(const float4* __restrict__ partials,
+                                                         uint32_t nb, uint32_t n,
+                                                         BuildParams* __restrict__ prm,
+                                                         uint32_t tree_mode, CallerBounds cb,
+                                                         uint32_t* __restrict__ status) {
+    bounds_final(partials, nb, n, tree_mode, cb, prm, status);
 }
 
 // batched systems: bounds per system from per-block partials over each system's blocks
@@ -157,26 +168,63 @@ __device__ void fill_params(BuildParams* prm, float4 r, uint64_t mnx64, uint64_t
 // ------------------------------------------------------------------------------------------
 // Morton codes: bit-exact with the reference's FP64 rule via integer emulation
 // ------------------------------------------------------------------------------------------
-template <typename K>
+// One particle's state as the gather after the sort reads it: x, y, mass and index in one record,
+// a single line of random access where four arrays are four (1M particles in random order, with
+// velocities known to be zero: 80 -> 22 us; 4M 467 -> 102; for 2 and 17 us more here).
+__device__ __forceinline__ void pack_state(float4* __restrict__ pk, uint32_t i, float x, float y,
+                                           const float* __restrict__ m,
+                                           const uint32_t* __restrict__ id) {
+    pk[i] = make_float4(x, y, m[i], __uint_as_float(id[i]));
+}
+
+// Every block derives the root square from the partial bounds itself (block 0 records it): a
+// launch of its own for that cost 5 us of every build (70k points: 14 -> 10 us with the codes).
+template <typename K, int ITEMS>
 __global__ __launch_bounds__(kBlock) void k_morton(const float* __restrict__ xs,
-                                                   const float* __restrict__ ys, uint32_t n,
-                                                   const BuildParams* __restrict__ prm, int B,
+                                                   const float* __restrict__ ys,
+                                                   const float* __restrict__ ms,
+                                                   const uint32_t* __restrict__ ids, uint32_t n,
+                                                   const float4* __restrict__ partials,
+                                                   uint32_t nb, uint32_t tree_mode,
+                                                   CallerBounds cb, BuildParams* __restrict__ prm,
+                                                   uint32_t* __restrict__ status, int B,
                                                    K* __restrict__ keys,
-                                                   uint32_t* __restrict__ vals) {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    const bh_sfp_quant Q = prm->quant;
-    const uint64_t dx = bh_sfp_add(bh_sfp_from_f32(xs[i]), prm->neg_minx64);
-    const uint64_t dy = bh_sfp_add(bh_sfp_from_f32(ys[i]), prm->neg_miny64);
-    const uint64_t qx = bh_sfp_quantize(dx, Q, B);
-    const uint64_t qy = bh_sfp_quantize(dy, Q, B);
-    K code;
-    if (sizeof(K) == 4)
-        code = (K)((bh_spread16((uint32_t)qy) << 1) | bh_spread16((uint32_t)qx));
-    else
-        code = (K)((bh_spread32(qy) << 1) | bh_spread32(qx));
-    keys[i] = code;
-    vals[i] = i;
+                                                   uint32_t* __restrict__ vals,
+                                                   float4* __restrict__ pk) {
+    __shared__ BuildParams s_prm;
+    const uint32_t base = blockIdx.x * (kBlock * ITEMS) + threadIdx.x;
+    float x[ITEMS], y[ITEMS];
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const uint32_t i = min(base + r * kBlock, n - 1);
+        x[r] = xs[i];
+        y[r] = ys[i];
+    }
+    bounds_final(partials, nb, n, tree_mode, cb, &s_prm, blockIdx.x == 0 ? status : nullptr);
+    if (threadIdx.x == 0) s_prm.n_nodes = 0;
+    __syncthreads();
+    static_assert(sizeof(BuildParams) % 4 == 0 && sizeof(BuildParams) / 4 <= kBlock, "one word each");
+    if (blockIdx.x == 0 && threadIdx.x < sizeof(BuildParams) / 4)
+        reinterpret_cast<uint32_t*>(prm)[threadIdx.x] =
+            reinterpret_cast<const uint32_t*>(&s_prm)[threadIdx.x];
+    const bh_sfp_quant Q = s_prm.quant;
+#pragma unroll
+    for (int r = 0; r < ITEMS; ++r) {
+        const uint32_t i = base + r * kBlock;
+        if (i >= n) return;
+        const uint64_t dx = bh_sfp_add(bh_sfp_from_f32(x[r]), s_prm.neg_minx64);
+        const uint64_t dy = bh_sfp_add(bh_sfp_from_f32(y[r]), s_prm.neg_miny64);
+        const uint64_t qx = bh_sfp_quantize(dx, Q, B);
+        const uint64_t qy = bh_sfp_quantize(dy, Q, B);
+        K code;
+        if (sizeof(K) == 4)
+            code = (K)((bh_spread16((uint32_t)qy) << 1) | bh_spread16((uint32_t)qx));
+        else
+            code = (K)((bh_spread32(qy) << 1) | bh_spread32(qx));
+        keys[i] = code;
+        vals[i] = i;
+        pack_state(pk, i, x[r], y[r], ms, ids);
+    }
 }
 
 // The tree of the reference's GPU step (NBodySolverGpuBH: createRoot, createChildren,
@@ -189,10 +237,13 @@ __global__ __launch_bounds__(kBlock) void k_morton(const float* __restrict__ xs,
 // top 2 depth bits of the 32-bit key.
 __global__ __launch_bounds__(kBlock) void k_morton_gpuref(const float* __restrict__ xs,
                                                           const float* __restrict__ ys,
+                                                          const float* __restrict__ ms,
+                                                          const uint32_t* __restrict__ ids,
                                                           uint32_t n,
                                                           const BuildParams* __restrict__ prm,
                                                           int depth, uint32_t* __restrict__ keys,
-                                                          uint32_t* __restrict__ vals) {
+                                                          uint32_t* __restrict__ vals,
+                                                          float4* __restrict__ pk) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
     const float mnx = prm->minx, mny = prm->miny, mxx = prm->maxx, mxy = prm->maxy;
@@ -210,16 +261,20 @@ __global__ __launch_bounds__(kBlock) void k_morton_gpuref(const float* __restric
     }
     keys[i] = depth > 0 ? code << (32 - 2 * depth) : 0u;
     vals[i] = i;
+    pack_state(pk, i, x, y, ms, ids);
 }
 
 // batched systems: key = system << 2B | code, with each system's own root square
 __global__ __launch_bounds__(kBlock) void k_morton_seg(const float* __restrict__ xs,
-                                                       const float* __restrict__ ys, uint32_t n,
+                                                       const float* __restrict__ ys,
+                                                       const float* __restrict__ ms,
+                                                       const uint32_t* __restrict__ ids, uint32_t n,
                                                        const uint32_t* __restrict__ sys_off,
                                                        uint32_t nsys,
                                                        const BuildParams* __restrict__ sys_prm,
                                                        int B, uint64_t* __restrict__ keys,
-                                                       uint32_t* __restrict__ vals) {
+                                                       uint32_t* __restrict__ vals,
+                                                       float4* __restrict__ pk) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i >= n) return;
     uint32_t lo = 0, hi = nsys;  // largest s with sys_off[s] <= i
@@ -229,12 +284,14 @@ __global__ __launch_bounds__(kBlock) void k_morton_seg(const float* __restrict__
     }
     const BuildParams* prm = sys_prm + lo;
     const bh_sfp_quant Q = prm->quant;
-    const uint64_t dx = bh_sfp_add(bh_sfp_from_f32(xs[i]), prm->neg_minx64);
-    const uint64_t dy = bh_sfp_add(bh_sfp_from_f32(ys[i]), prm->neg_miny64);
+    const float x = xs[i], y = ys[i];
+    const uint64_t dx = bh_sfp_add(bh_sfp_from_f32(x), prm->neg_minx64);
+    const uint64_t dy = bh_sfp_add(bh_sfp_from_f32(y), prm->neg_miny64);
     const uint64_t qx = bh_sfp_quantize(dx, Q, B);
     const uint64_t qy = bh_sfp_quantize(dy, Q, B);
     keys[i] = ((uint64_t)lo << (2 * B)) | (bh_spread32(qy) << 1) | bh_spread32(qx);
     vals[i] = i;
+    pack_state(pk, i, x, y, ms, ids);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1003,13 +1060,11 @@ __global__ __launch_bounds__(THREADS) void k_bucket_sort(K* keys, uint32_t* vals
 // ------------------------------------------------------------------------------------------
 // gather the particle state into sorted order
 // ------------------------------------------------------------------------------------------
+// vx, vy: null when the velocities are known to be zero (zeros are then written, not gathered)
 __global__ __launch_bounds__(kBlock) void k_gather(const uint32_t* __restrict__ perm, uint32_t n,
-                                                   const float* __restrict__ x,
-                                                   const float* __restrict__ y,
-                                                   const float* __restrict__ m,
+                                                   const float4* __restrict__ pk,
                                                    const float* __restrict__ vx,
                                                    const float* __restrict__ vy,
-                                                   const uint32_t* __restrict__ id,
                                                    float* __restrict__ xo, float* __restrict__ yo,
                                                    float* __restrict__ mo, float* __restrict__ vxo,
                                                    float* __restrict__ vyo,
@@ -1029,16 +1084,15 @@ __global__ __launch_bounds__(kBlock) void k_gather(const uint32_t* __restrict__ 
         else
             static_cast<uint32_t*>(codes)[i] = 0u;
     }
-    const float px = x[j], py = y[j], pm = m[j];
-    xo[i] = px;
-    yo[i] = py;
-    mo[i] = pm;
-    if (vx) {
-        vxo[i] = vx[j];
-        vyo[i] = vy[j];
-    }
-    ido[i] = id[j];
-    pos4[i] = make_float4(px, py, pm, 0.0f);
+    const float4 q = pk[j];
+    const float u = vx ? vx[j] : 0.0f, v = vy ? vy[j] : 0.0f;
+    xo[i] = q.x;
+    yo[i] = q.y;
+    mo[i] = q.z;
+    vxo[i] = u;
+    vyo[i] = v;
+    ido[i] = __float_as_uint(q.w);
+    pos4[i] = make_float4(q.x, q.y, q.z, 0.0f);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1776,9 +1830,19 @@ __global__ __launch_bounds__(kBlock) void k_clear_slots(uint32_t* __restrict__ a
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_iota(uint32_t* __restrict__ p, uint32_t n) {
+// what a caller did not give: index order, unit masses (m not null), zero velocities (vx not null)
+__global__ __launch_bounds__(kBlock) void k_init_state(uint32_t n, uint32_t* __restrict__ id,
+                                                       float* __restrict__ m,
+                                                       float* __restrict__ vx,
+                                                       float* __restrict__ vy) {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i < n) p[i] = i;
+    if (i >= n) return;
+    id[i] = i;
+    if (m) m[i] = 1.0f;
+    if (vx) {
+        vx[i] = 0.0f;
+        vy[i] = 0.0f;
+    }
 }
 
 __global__ __launch_bounds__(kBlock) void k_tree_slots(const uint32_t* __restrict__ codes,
@@ -1812,28 +1876,41 @@ uint32_t bounds_grid(uint32_t n) {
     return g;
 }
 
-void launch_bounds(hipStream_t s, const float* xs, const float* ys, uint32_t n, float4* partials,
-                   BuildParams* prm, uint32_t tree_mode, const double* caller, uint32_t* status) {
+static CallerBounds caller_bounds(const double* b) {
+    if (!b) return CallerBounds{0, 0.0, 0.0, 0.0, 0.0};
+    return CallerBounds{1, b[0], b[1], b[2], b[3]};
+}
+
+void launch_morton_gpuref(hipStream_t s, const float* xs, const float* ys, const float* ms,
+                          const uint32_t* ids, uint32_t n, float4* partials, BuildParams* prm,
+                          int depth, uint32_t* status, uint32_t* keys, uint32_t* vals, float4* pk) {
     const uint32_t g = bounds_grid(n);
     k_bounds_partial<<<g, kBlock, 0, s>>>(xs, ys, n, partials);
-    k_bounds_final<<<1, kBlock, 0, s>>>(partials, g, n, prm, tree_mode, caller ? 1 : 0,
-                                        caller ? caller[0] : 0.0, caller ? caller[1] : 0.0,
-                                        caller ? caller[2] : 0.0, caller ? caller[3] : 0.0,
+    k_bounds_final<<<1, kBlock, 0, s>>>(partials, g, n, prm, kTreeGpuRef, caller_bounds(nullptr),
                                         status);
+    k_morton_gpuref<<<div_up(n, kBlock), kBlock, 0, s>>>(xs, ys, ms, ids, n, prm, depth, keys,
+                                                         vals, pk);
 }
 
-void launch_morton_gpuref(hipStream_t s, const float* xs, const float* ys, uint32_t n,
-                          const BuildParams* prm, int depth, uint32_t* keys, uint32_t* vals) {
-    k_morton_gpuref<<<div_up(n, kBlock), kBlock, 0, s>>>(xs, ys, n, prm, depth, keys, vals);
-}
+// 4 particles per thread above kMortonWide: fewer blocks to repeat the bounds' last step
+constexpr uint32_t kMortonWide = 1u << 18;
 
-void launch_morton(hipStream_t s, const float* xs, const float* ys, uint32_t n,
-                   const BuildParams* prm, int B, void* keys, uint32_t* vals, bool wide) {
-    const uint32_t g = div_up(n, kBlock);
-    if (wide)
-        k_morton<uint64_t><<<g, kBlock, 0, s>>>(xs, ys, n, prm, B, (uint64_t*)keys, vals);
-    else
-        k_morton<uint32_t><<<g, kBlock, 0, s>>>(xs, ys, n, prm, B, (uint32_t*)keys, vals);
+void launch_morton(hipStream_t s, const float* xs, const float* ys, const float* ms,
+                   const uint32_t* ids, uint32_t n, float4* partials, BuildParams* prm,
+                   uint32_t tree_mode, const double* caller, uint32_t* status, int B, void* keys,
+                   uint32_t* vals, bool wide, float4* pk) {
+    const uint32_t nb = bounds_grid(n);
+    k_bounds_partial<<<nb, kBlock, 0, s>>>(xs, ys, n, partials);
+    const CallerBounds cb = caller_bounds(caller);
+#define BH_MORTON(K, I)                                                                           \
+    k_morton<K, I><<<div_up(n, kBlock * I), kBlock, 0, s>>>(                                      \
+        xs, ys, ms, ids, n, partials, nb, tree_mode, cb, prm, status, B, (K*)keys, vals, pk)
+    if (n <= kMortonWide) {
+        if (wide) BH_MORTON(uint64_t, 1); else BH_MORTON(uint32_t, 1);
+    } else {
+        if (wide) BH_MORTON(uint64_t, 4); else BH_MORTON(uint32_t, 4);
+    }
+#undef BH_MORTON
 }
 
 uint32_t scan_partials_size(uint64_t n) { return div_up(n, kScanTile) + 1; }
@@ -1964,12 +2041,12 @@ void launch_sort(hipStream_t s, void* keys_a, uint32_t* vals_a, void* keys_b, ui
     *result_in_b = (passes & 1) != 0;
 }
 
-void launch_gather(hipStream_t s, const uint32_t* perm, uint32_t n, const float* x, const float* y,
-                   const float* m, const float* vx, const float* vy, const uint32_t* id, float* xo,
-                   float* yo, float* mo, float* vxo, float* vyo, uint32_t* ido, float4* pos4,
-                   const uint32_t* sort_err, void* codes, bool wide) {
-    k_gather<<<div_up(n, kBlock), kBlock, 0, s>>>(perm, n, x, y, m, vx, vy, id, xo, yo, mo, vxo,
-                                                  vyo, ido, pos4, sort_err, codes, wide ? 1 : 0);
+void launch_gather(hipStream_t s, const uint32_t* perm, uint32_t n, const float4* pk,
+                   const float* vx, const float* vy, float* xo, float* yo, float* mo, float* vxo,
+                   float* vyo, uint32_t* ido, float4* pos4, const uint32_t* sort_err, void* codes,
+                   bool wide) {
+    k_gather<<<div_up(n, kBlock), kBlock, 0, s>>>(perm, n, pk, vx, vy, xo, yo, mo, vxo, vyo, ido,
+                                                  pos4, sort_err, codes, wide ? 1 : 0);
 }
 
 uint32_t tree_tiles(uint32_t n) { return div_up(n, kTreeTile); }
@@ -2003,11 +2080,12 @@ void launch_bounds_batched(hipStream_t s, const float* xs, const float* ys, cons
     k_bounds_seg_final<<<nsys, kBlock, 0, s>>>(partials, blk_off, sys_off, sys_prm, prm, status);
 }
 
-void launch_morton_batched(hipStream_t s, const float* xs, const float* ys, uint32_t n,
-                           const uint32_t* sys_off, uint32_t nsys, const BuildParams* sys_prm,
-                           int B, uint64_t* keys, uint32_t* vals) {
-    k_morton_seg<<<div_up(n, kBlock), kBlock, 0, s>>>(xs, ys, n, sys_off, nsys, sys_prm, B, keys,
-                                                     vals);
+void launch_morton_batched(hipStream_t s, const float* xs, const float* ys, const float* ms,
+                           const uint32_t* ids, uint32_t n, const uint32_t* sys_off, uint32_t nsys,
+                           const BuildParams* sys_prm, int B, uint64_t* keys, uint32_t* vals,
+                           float4* pk) {
+    k_morton_seg<<<div_up(n, kBlock), kBlock, 0, s>>>(xs, ys, ms, ids, n, sys_off, nsys, sys_prm, B,
+                                                      keys, vals, pk);
 }
 
 void launch_batch_roots(hipStream_t s, const uint32_t* sys_off, uint32_t nsys,
@@ -2065,8 +2143,8 @@ void launch_fill_f32(hipStream_t s, float* p, uint64_t n, float v) {
     launch_fill_u32(s, (uint32_t*)p, n, c.u);
 }
 
-void launch_iota(hipStream_t s, uint32_t* p, uint32_t n) {
-    if (n) k_iota<<<div_up(n, kBlock), kBlock, 0, s>>>(p, n);
+void launch_init_state(hipStream_t s, uint32_t n, uint32_t* id, float* m, float* vx, float* vy) {
+    if (n) k_init_state<<<div_up(n, kBlock), kBlock, 0, s>>>(n, id, m, vx, vy);
 }
 
 void launch_tree_slots(hipStream_t s, const uint32_t* codes, const Node* nodes,

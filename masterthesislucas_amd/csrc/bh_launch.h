@@ -20,13 +20,16 @@ uint32_t bounds_grid(uint32_t n);
 // [0] the sort's look-back gave up waiting, [1] a position was not finite.
 constexpr int kStatusWords = 4;
 constexpr uint32_t kSortSpinLimit = 1u << 22;  // look-back polls before giving up
-void launch_bounds(hipStream_t s, const float* xs, const float* ys, uint32_t n, float4* partials,
-                   BuildParams* prm, uint32_t tree_mode, const double* caller, uint32_t* status);
-// keys of the reference GPU step's tree (32-bit, path in the top 2 depth bits)
-void launch_morton_gpuref(hipStream_t s, const float* xs, const float* ys, uint32_t n,
-                          const BuildParams* prm, int depth, uint32_t* keys, uint32_t* vals);
-void launch_morton(hipStream_t s, const float* xs, const float* ys, uint32_t n,
-                   const BuildParams* prm, int B, void* keys, uint32_t* vals, bool wide);
+// Bounds, root square and Morton keys of the positions, the identity in vals, and every particle's
+// state packed for launch_gather (x, y, mass, index). ms, ids: masses and indices.
+// gpuref: keys of the reference GPU step's tree (32-bit, path in the top 2 depth bits)
+void launch_morton_gpuref(hipStream_t s, const float* xs, const float* ys, const float* ms,
+                          const uint32_t* ids, uint32_t n, float4* partials, BuildParams* prm,
+                          int depth, uint32_t* status, uint32_t* keys, uint32_t* vals, float4* pk);
+void launch_morton(hipStream_t s, const float* xs, const float* ys, const float* ms,
+                   const uint32_t* ids, uint32_t n, float4* partials, BuildParams* prm,
+                   uint32_t tree_mode, const double* caller, uint32_t* status, int B, void* keys,
+                   uint32_t* vals, bool wide, float4* pk);
 uint32_t scan_partials_size(uint64_t n);
 void launch_exclusive_scan(hipStream_t s, const uint32_t* in, uint32_t* out, uint32_t n,
                            uint32_t* partials, uint32_t* total);
@@ -38,11 +41,12 @@ uint64_t sort_scratch_words(uint32_t n);  // uint32 words of scratch launch_sort
 void launch_sort(hipStream_t s, void* keys_a, uint32_t* vals_a, void* keys_b, uint32_t* vals_b,
                  uint32_t n, int key_bits, bool wide, uint32_t* scratch, uint32_t* err,
                  uint32_t spin_limit, bool* result_in_b);
-// codes: the sorted codes, zeroed (with the identity order) when *sort_err is set
-void launch_gather(hipStream_t s, const uint32_t* perm, uint32_t n, const float* x, const float* y,
-                   const float* m, const float* vx, const float* vy, const uint32_t* id, float* xo,
-                   float* yo, float* mo, float* vxo, float* vyo, uint32_t* ido, float4* pos4,
-                   const uint32_t* sort_err, void* codes, bool wide);
+// codes: the sorted codes, zeroed (with the identity order) when *sort_err is set; vx, vy: null when
+// the velocities are known to be zero
+void launch_gather(hipStream_t s, const uint32_t* perm, uint32_t n, const float4* pk,
+                   const float* vx, const float* vy, float* xo, float* yo, float* mo, float* vxo,
+                   float* vyo, uint32_t* ido, float4* pos4, const uint32_t* sort_err, void* codes,
+                   bool wide);
 // R: level of the tree roots (0; batched systems: the system id occupies the levels above R)
 uint32_t tree_tiles(uint32_t n);  // words of launch_tree's sums
 void launch_tree(hipStream_t s, const void* codes, bool wide, uint32_t n, int B, int cap,
@@ -54,9 +58,10 @@ void launch_bounds_batched(hipStream_t s, const float* xs, const float* ys, cons
                            uint32_t nblk, const uint32_t* blk_off, const uint32_t* sys_off,
                            uint32_t nsys, float4* partials, BuildParams* sys_prm,
                            BuildParams* prm, uint32_t* status);
-void launch_morton_batched(hipStream_t s, const float* xs, const float* ys, uint32_t n,
-                           const uint32_t* sys_off, uint32_t nsys, const BuildParams* sys_prm,
-                           int B, uint64_t* keys, uint32_t* vals);
+void launch_morton_batched(hipStream_t s, const float* xs, const float* ys, const float* ms,
+                           const uint32_t* ids, uint32_t n, const uint32_t* sys_off, uint32_t nsys,
+                           const BuildParams* sys_prm, int B, uint64_t* keys, uint32_t* vals,
+                           float4* pk);
 void launch_batch_roots(hipStream_t s, const uint32_t* sys_off, uint32_t nsys,
                         const uint32_t* noff, const BuildParams* prm, uint32_t* roots);
 uint32_t up_chunks(uint32_t cap_nodes);  // at most
@@ -69,7 +74,8 @@ void launch_tree_stats(hipStream_t s, const Node* nodes, const BuildParams* prm,
                        uint32_t blocks);
 void launch_fill_u32(hipStream_t s, uint32_t* p, uint64_t n, uint32_t v);
 void launch_fill_f32(hipStream_t s, float* p, uint64_t n, float v);
-void launch_iota(hipStream_t s, uint32_t* p, uint32_t n);
+// id = 0 .. n-1; unit masses and zero velocities where the arrays are not null
+void launch_init_state(hipStream_t s, uint32_t n, uint32_t* id, float* m, float* vx, float* vy);
 void launch_tree_slots(hipStream_t s, const uint32_t* codes, const Node* nodes,
                        const BuildParams* prm, uint32_t cap_nodes, int depth, uint32_t* first_child,
                        uint32_t* first_particle, uint32_t* count, uint64_t slots);
