@@ -279,7 +279,8 @@ int effective_depth(const bh_ctx* c) {
 
 void launch_node_moments(bh_ctx* c);
 
-bh_status do_build(bh_ctx* c, const double* bounds) {
+// have_partials: partial bounds of the positions that stand in bounds_part already (0: none)
+bh_status do_build(bh_ctx* c, const double* bounds, uint32_t have_partials = 0) {
     const uint32_t n = c->n;
     if (n == 0) return fail(c, BH_ERR_STATE, "no particles");
     hipStream_t s = c->stream;
@@ -309,7 +310,7 @@ bh_status do_build(bh_ctx* c, const double* bounds) {
         } else {
             launch_morton(s, c->x[cur], c->y[cur], c->m[cur], c->id[cur], n, c->bounds_part, c->prm,
                           quadtree ? kTreeQuadTree : kTreeMortonFixed, quadtree ? nullptr : bounds,
-                          c->dstatus, c->B, c->keys_a, c->vals_a, c->wide, c->packed);
+                          c->dstatus, c->B, c->keys_a, c->vals_a, c->wide, c->packed, have_partials);
         }
     }
     phase_end(c, 0);
@@ -395,8 +396,10 @@ bh_status do_fmm(bh_ctx* c, double theta) {
 }
 
 // plugin: the call is bh_forces / bh_forces_device, whose t-SNE sums keep the pre-order walk's
-// summation order
-bh_status do_forces(bh_ctx* c, double theta, bool want_total, bool plugin = false) {
+// summation order. sum_later: with want_total, the per-point terms in tot are left to the caller to
+// add up (the FMM solver has no terms, its total is in dsum)
+bh_status do_forces(bh_ctx* c, double theta, bool want_total, bool plugin = false,
+                    bool sum_later = false) {
     if (!c->built) return fail(c, BH_ERR_STATE, "forces requested before a tree was built");
     if (!(theta >= 0.0)) return fail(c, BH_ERR_ARG, "theta must be >= 0");
     if (c->solver == BH_SOLVER_FMM_SYM) return do_fmm(c, theta);
@@ -423,8 +426,7 @@ bh_status do_forces(bh_ctx* c, double theta, bool want_total, bool plugin = fals
         launch_sum_heavy(s, c->side, c->side_cap, c->heavy, c->nheavy, c->ax, c->ay,
                          want_total ? c->tot : nullptr);
     phase_end(c, 5);
-    if (want_total)
-        launch_reduce_f64(s, c->tot, nullptr, c->n, c->red_part, c->dsum);
+    if (want_total && !sum_later) launch_reduce_f64(s, c->tot, nullptr, c->n, c->red_part, c->dsum);
     c->have_acc = true;
     return launch_status(c, "traverse launch");
 }
@@ -1124,10 +1126,12 @@ bh_status bh_tsne_set_embedding(bh_ctx* c, const float* yx, const float* yy) {
     if (!c->p_n) return fail(c, BH_ERR_STATE, "set the P matrix first");
     const size_t b = (size_t)c->p_n * 4;
     bh_status st = BH_OK;
-    for (int k = 0; k < 3 && st == BH_OK; ++k) {
-        st = hip_check(c, hipMemcpy(c->ty_x[k], yx, b, hipMemcpyHostToDevice), "embedding");
-        if (st == BH_OK) st = hip_check(c, hipMemcpy(c->ty_y[k], yy, b, hipMemcpyHostToDevice), "embedding");
-    }
+    st = hip_check(c, hipMemcpy(c->ty_x[0], yx, b, hipMemcpyHostToDevice), "embedding");
+    if (st == BH_OK) st = hip_check(c, hipMemcpy(c->ty_y[0], yy, b, hipMemcpyHostToDevice), "embedding");
+    if (st != BH_OK) return st;
+    for (int k = 1; k < 3; ++k)
+        launch_copy2(c->stream, c->p_n, c->ty_x[0], c->ty_y[0], c->ty_x[k], c->ty_y[k]);
+    st = launch_status(c, "embedding");
     if (st != BH_OK) return st;
     c->ty_cur = 0;
     c->ty_set = true;
@@ -1160,34 +1164,51 @@ static bh_status tsne_stage_build(bh_ctx* c) {
     return do_build(c, nullptr);
 }
 
-// The attraction needs only the staged embedding: it runs on att_stream from the stage on, while
-// the tree is built and walked on the context's stream; the update waits for both.
-static bh_status tsne_iteration(bh_ctx* c, const bh_tsne_params* p, int32_t t, bool keep_deriv) {
+// The attraction needs only the staged embedding: it runs on att_stream beside the walk, whose
+// waves leave issue slots and memory idle, and the update waits for both. (Started beside the
+// build, it kept the sort's large blocks waiting for room: 70k points, early phase, 339 us an
+// iteration instead of 315.) staged: the iteration before left this one's particles and
+// bounds; stage_next: leave the next one's (both within one call only).
+static bh_status tsne_iteration(bh_ctx* c, const bh_tsne_params* p, int32_t t, bool keep_deriv,
+                                bool staged, bool stage_next) {
     hipStream_t s = c->stream;
     const uint32_t n = c->p_n;
     const float exag = (float)(t < p->exag_switch ? p->exag_early : p->exag_late);
     const float mu = (float)(t < p->momentum_switch ? p->momentum_early : p->momentum_late);
-    tsne_stage(c);
-    bh_status st = hip_check(c, hipEventRecord(c->ev_staged, s), "event");
+    if (staged)
+        c->cur = 0;
+    else
+        tsne_stage(c);
+    bh_status st = do_build(c, nullptr, staged ? tsne_update_blocks(n) : 0);
+    if (st != BH_OK) return st;
+    st = hip_check(c, hipEventRecord(c->ev_staged, s), "event");
     if (st == BH_OK) st = hip_check(c, hipStreamWaitEvent(c->att_stream, c->ev_staged, 0), "wait");
     if (st != BH_OK) return st;
     launch_tsne_attract(c->att_stream, c->p_row, c->p_col, c->p_val, n, c->ty_xy, exag, c->att_x,
                         c->att_y);
     st = hip_check(c, hipEventRecord(c->ev_att, c->att_stream), "event");
     if (st != BH_OK) return st;
-    st = do_build(c, nullptr);
+    // repulsion and Z: per-point terms (tree walk) or their sum in dsum (FMM)
+    const bool terms = c->solver != BH_SOLVER_FMM_SYM;
+    st = do_forces(c, tsne_theta(p, t), true, false, true);
     if (st != BH_OK) return st;
-    st = do_forces(c, tsne_theta(p, t), true);  // repulsion + per-point Z terms, Z -> dsum
-    if (st != BH_OK) return st;
-    launch_unsort2(s, c->id[c->cur], n, c->ax, c->ay, c->rep_x, c->rep_y);
+    uint32_t nz = 1;
+    if (terms)
+        nz = launch_unsort2_sum(s, c->id[c->cur], n, c->ax, c->ay, c->tot, c->rep_x, c->rep_y,
+                                c->red_part);
+    else
+        launch_unsort2(s, c->id[c->cur], n, c->ax, c->ay, c->rep_x, c->rep_y);
     st = hip_check(c, hipStreamWaitEvent(s, c->ev_att, 0), "wait");
     if (st != BH_OK) return st;
     const int cur = c->ty_cur, prev = (cur + 2) % 3, next = (cur + 1) % 3;
-    launch_tsne_combine(s, n, c->ty_x[cur], c->ty_y[cur], c->ty_x[prev], c->ty_y[prev], c->rep_x,
-                        c->rep_y, c->att_x, c->att_y, c->dsum,
-                        p->repulsion_scale > 0.0 ? p->repulsion_scale : 4.0,
-                        (float)p->learning_rate, mu, c->ty_x[next], c->ty_y[next],
-                        keep_deriv ? c->tder_x : nullptr, keep_deriv ? c->tder_y : nullptr);
+    launch_tsne_update(s, n, c->ty_x[cur], c->ty_y[cur], c->ty_x[prev], c->ty_y[prev], c->rep_x,
+                       c->rep_y, c->att_x, c->att_y, terms ? c->red_part : c->dsum, nz,
+                       terms ? c->dsum : nullptr,
+                       p->repulsion_scale > 0.0 ? p->repulsion_scale : 4.0,
+                       (float)p->learning_rate, mu, c->ty_x[next], c->ty_y[next],
+                       keep_deriv ? c->tder_x : nullptr, keep_deriv ? c->tder_y : nullptr,
+                       stage_next ? c->x[0] : nullptr, stage_next ? c->y[0] : nullptr, c->ty_xy,
+                       c->bounds_part);
     // rotate: next becomes current, current becomes previous
     c->ty_cur = next;
     return launch_status(c, "t-SNE step");
@@ -1198,7 +1219,7 @@ bh_status bh_tsne_step(bh_ctx* c, const bh_tsne_params* p, int32_t iteration, fl
     if (!c || !p || iteration < 0) return BH_ERR_ARG;
     if (!c->ty_set) return fail(c, BH_ERR_STATE, "set P and the embedding first");
     bh_status st = status_begin(c);
-    if (st == BH_OK) st = tsne_iteration(c, p, iteration, dx || dy);
+    if (st == BH_OK) st = tsne_iteration(c, p, iteration, dx || dy, false, false);
     if (st != BH_OK) return st;
     hipStream_t s = c->stream;
     const size_t b = (size_t)c->p_n * 4;
@@ -1217,7 +1238,7 @@ bh_status bh_tsne_run(bh_ctx* c, const bh_tsne_params* p, int32_t first, int32_t
     bh_status st = status_begin(c);
     if (st != BH_OK) return st;
     for (int32_t t = first; t < first + count; ++t) {
-        st = tsne_iteration(c, p, t, false);
+        st = tsne_iteration(c, p, t, false, t > first, t + 1 < first + count);
         if (st != BH_OK) return st;
     }
     return finish_build_call(c, "t-SNE run");

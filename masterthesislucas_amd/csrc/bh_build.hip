@@ -18,34 +18,6 @@ namespace bh {
 // ------------------------------------------------------------------------------------------
 // bounds: FP32 min/max per block, then one block derives the root square and the quantiser
 // ------------------------------------------------------------------------------------------
-__device__ __forceinline__ float4 minmax4(float4 a, float4 b) {
-    return make_float4(fminf(a.x, b.x), fminf(a.y, b.y), fmaxf(a.z, b.z), fmaxf(a.w, b.w));
-}
-
-__device__ __forceinline__ float4 block_minmax4(float4 r) {
-    __shared__ float4 red[kWavesPerBlock];
-    for (int o = 32; o > 0; o >>= 1) {
-        r.x = fminf(r.x, __shfl_xor(r.x, o, kWave));
-        r.y = fminf(r.y, __shfl_xor(r.y, o, kWave));
-        r.z = fmaxf(r.z, __shfl_xor(r.z, o, kWave));
-        r.w = fmaxf(r.w, __shfl_xor(r.w, o, kWave));
-    }
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    if (lane == 0) red[w] = r;
-    __syncthreads();
-    r = red[0];
-    for (int k = 1; k < kWavesPerBlock; ++k) r = minmax4(r, red[k]);
-    __syncthreads();
-    return r;
-}
-
-// One position as a bounds item. fminf/fmaxf drop NaN, so a NaN coordinate enters as -inf:
-// the bounds are then finite exactly when every position is (an infinity stays infinite).
-__device__ __forceinline__ float4 bounds_item(float x, float y) {
-    const float xl = x == x ? x : -INFINITY, yl = y == y ? y : -INFINITY;
-    return make_float4(xl, yl, x, y);
-}
-
 // status word 1: the build saw a non-finite position (read by the host after the build)
 __device__ __forceinline__ void flag_nonfinite(float4 r, uint32_t* status) {
     if (!(isfinite(r.x) && isfinite(r.y) && isfinite(r.z) && isfinite(r.w))) status[1] = 1u;
@@ -1898,9 +1870,9 @@ constexpr uint32_t kMortonWide = 1u << 18;
 void launch_morton(hipStream_t s, const float* xs, const float* ys, const float* ms,
                    const uint32_t* ids, uint32_t n, float4* partials, BuildParams* prm,
                    uint32_t tree_mode, const double* caller, uint32_t* status, int B, void* keys,
-                   uint32_t* vals, bool wide, float4* pk) {
-    const uint32_t nb = bounds_grid(n);
-    k_bounds_partial<<<nb, kBlock, 0, s>>>(xs, ys, n, partials);
+                   uint32_t* vals, bool wide, float4* pk, uint32_t have_partials) {
+    const uint32_t nb = have_partials ? have_partials : bounds_grid(n);
+    if (!have_partials) k_bounds_partial<<<nb, kBlock, 0, s>>>(xs, ys, n, partials);
     const CallerBounds cb = caller_bounds(caller);
 #define BH_MORTON(K, I)                                                                           \
     k_morton<K, I><<<div_up(n, kBlock * I), kBlock, 0, s>>>(                                      \

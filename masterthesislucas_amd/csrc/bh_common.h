@@ -99,4 +99,46 @@ __device__ __forceinline__ double wave_sum_d(double v) {
     return v;
 }
 
+// bounds of positions: (min x, min y, max x, max y)
+__device__ __forceinline__ float4 minmax4(float4 a, float4 b) {
+    return make_float4(fminf(a.x, b.x), fminf(a.y, b.y), fmaxf(a.z, b.z), fmaxf(a.w, b.w));
+}
+
+__device__ __forceinline__ float4 block_minmax4(float4 r) {
+    __shared__ float4 red[kWavesPerBlock];
+    for (int o = 32; o > 0; o >>= 1) {
+        r.x = fminf(r.x, __shfl_xor(r.x, o, kWave));
+        r.y = fminf(r.y, __shfl_xor(r.y, o, kWave));
+        r.z = fmaxf(r.z, __shfl_xor(r.z, o, kWave));
+        r.w = fmaxf(r.w, __shfl_xor(r.w, o, kWave));
+    }
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if (lane == 0) red[w] = r;
+    __syncthreads();
+    r = red[0];
+    for (int k = 1; k < kWavesPerBlock; ++k) r = minmax4(r, red[k]);
+    __syncthreads();
+    return r;
+}
+
+// One position as a bounds item. fminf/fmaxf drop NaN, so a NaN coordinate enters as -inf:
+// the bounds are then finite exactly when every position is (an infinity stays infinite).
+__device__ __forceinline__ float4 bounds_item(float x, float y) {
+    const float xl = x == x ? x : -INFINITY, yl = y == y ? y : -INFINITY;
+    return make_float4(xl, yl, x, y);
+}
+
+// sum over a block of kBlock threads, in every thread
+__device__ __forceinline__ double block_sum_d(double s) {
+    __shared__ double red[kWavesPerBlock];
+    s = wave_sum_d(s);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    if (lane == 0) red[wv] = s;
+    __syncthreads();
+    double b = 0.0;
+    for (int k = 0; k < kWavesPerBlock; ++k) b += red[k];
+    __syncthreads();
+    return b;
+}
+
 }  // namespace bh

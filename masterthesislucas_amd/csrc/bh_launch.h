@@ -22,6 +22,7 @@ constexpr int kStatusWords = 4;
 constexpr uint32_t kSortSpinLimit = 1u << 22;  // look-back polls before giving up
 // Bounds, root square and Morton keys of the positions, the identity in vals, and every particle's
 // state packed for launch_gather (x, y, mass, index). ms, ids: masses and indices.
+// have_partials: partial bounds that stand in `partials` already (0: made here).
 // gpuref: keys of the reference GPU step's tree (32-bit, path in the top 2 depth bits)
 void launch_morton_gpuref(hipStream_t s, const float* xs, const float* ys, const float* ms,
                           const uint32_t* ids, uint32_t n, float4* partials, BuildParams* prm,
@@ -29,7 +30,7 @@ void launch_morton_gpuref(hipStream_t s, const float* xs, const float* ys, const
 void launch_morton(hipStream_t s, const float* xs, const float* ys, const float* ms,
                    const uint32_t* ids, uint32_t n, float4* partials, BuildParams* prm,
                    uint32_t tree_mode, const double* caller, uint32_t* status, int B, void* keys,
-                   uint32_t* vals, bool wide, float4* pk);
+                   uint32_t* vals, bool wide, float4* pk, uint32_t have_partials = 0);
 uint32_t scan_partials_size(uint64_t n);
 void launch_exclusive_scan(hipStream_t s, const uint32_t* in, uint32_t* out, uint32_t n,
                            uint32_t* partials, uint32_t* total);
@@ -141,6 +142,10 @@ void launch_warm_l2(hipStream_t s, const Node* nodes, const BuildParams* prm, co
                     uint32_t n, uint32_t* sink);
 void launch_unsort2(hipStream_t s, const uint32_t* id, uint32_t n, const float* a, const float* b,
                     float* ao, float* bo);
+// returns the number of partial sums of w (at most kMaxReduceBlocks)
+uint32_t launch_unsort2_sum(hipStream_t s, const uint32_t* id, uint32_t n, const float* a,
+                            const float* b, const float* w, float* ao, float* bo,
+                            double* partials);
 void launch_kick_drift(hipStream_t s, float* x, float* y, float* vx, float* vy, const float* ax,
                        const float* ay, uint32_t n, float hdt, float dt);
 void launch_kick(hipStream_t s, float* vx, float* vy, const float* ax, const float* ay, uint32_t n,
@@ -171,14 +176,18 @@ void launch_direct_f64_static(hipStream_t s, int kernel, const float4* pos4, con
 // stage also writes the interleaved copy xy that the update's neighbour gathers read
 void launch_tsne_stage(hipStream_t s, const float* yx, const float* yy, uint32_t n, float* x,
                        float* y, float* m, uint32_t* id, float2* xy);
+void launch_copy2(hipStream_t s, uint32_t n, const float* a, const float* b, float* ao, float* bo);
 void launch_tsne_attract(hipStream_t s, const uint32_t* row_ptr, const uint32_t* col,
                          const float* val, uint32_t n, const float2* xy, float exag, float* att_x,
                          float* att_y);
-void launch_tsne_combine(hipStream_t s, uint32_t n, const float* yx, const float* yy,
-                         const float* pyx, const float* pyy, const float* rep_x,
-                         const float* rep_y, const float* att_x, const float* att_y,
-                         const double* z, double rep_scale, float lr, float mu, float* nyx,
-                         float* nyy, float* dx, float* dy);
+// Z = sum of nz partial sums (written to z_out when not null); sx, sy, xy, bounds (null: not wanted):
+// the next iteration's particles and their partial bounds (tsne_update_blocks of them)
+uint32_t tsne_update_blocks(uint32_t n);
+void launch_tsne_update(hipStream_t s, uint32_t n, const float* yx, const float* yy,
+                        const float* pyx, const float* pyy, const float* rep_x, const float* rep_y,
+                        const float* att_x, const float* att_y, const double* zpart, uint32_t nz,
+                        double* z_out, double rep_scale, float lr, float mu, float* nyx, float* nyy,
+                        float* dx, float* dy, float* sx, float* sy, float2* xy, float4* bounds);
 uint32_t tsne_kl_blocks(uint32_t n);
 void launch_tsne_kl(hipStream_t s, const uint32_t* row_ptr, const uint32_t* col, const float* val,
                     uint32_t n, const float* yx, const float* yy, const double* z,

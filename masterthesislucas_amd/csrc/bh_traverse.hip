@@ -810,18 +810,6 @@ __global__ __launch_bounds__(kBlock) void k_walk_preorder(const float4* __restri
 // FP64 reduction of per-particle totals (t-SNE Z, potential energy): fixed partition into
 // block partials, then one block sums them in order, so the result is deterministic.
 // ------------------------------------------------------------------------------------------
-__device__ __forceinline__ double block_sum_d(double s) {
-    __shared__ double red[kWavesPerBlock];
-    s = wave_sum_d(s);
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    if (lane == 0) red[wv] = s;
-    __syncthreads();
-    double b = 0.0;
-    for (int k = 0; k < kWavesPerBlock; ++k) b += red[k];
-    __syncthreads();
-    return b;
-}
-
 __global__ __launch_bounds__(kBlock) void k_reduce_f64_partial(const float* __restrict__ v,
                                                                uint32_t n,
                                                                const float* __restrict__ w,
@@ -890,6 +878,25 @@ __global__ __launch_bounds__(kBlock) void k_unsort2(const uint32_t* __restrict__
     const uint32_t j = id[i];
     ao[j] = a[i];
     if (b) bo[j] = b[i];
+}
+
+// unsorts a and b and sums w per block (partials in FP64)
+__global__ __launch_bounds__(kBlock) void k_unsort2_sum(const uint32_t* __restrict__ id, uint32_t n,
+                                                        const float* __restrict__ a,
+                                                        const float* __restrict__ b,
+                                                        const float* __restrict__ w,
+                                                        float* __restrict__ ao,
+                                                        float* __restrict__ bo,
+                                                        double* __restrict__ partials) {
+    double s = 0.0;
+    for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
+        const uint32_t j = id[i];
+        ao[j] = a[i];
+        bo[j] = b[i];
+        s += (double)w[i];
+    }
+    s = block_sum_d(s);
+    if (threadIdx.x == 0) partials[blockIdx.x] = s;
 }
 
 // kick-drift of kick-drift-kick leapfrog: v += a dt/2; x += v dt
@@ -1115,6 +1122,14 @@ uint32_t traverse_blocks(uint32_t n) { return div_up(n, kBlock); }
 void launch_unsort2(hipStream_t s, const uint32_t* id, uint32_t n, const float* a, const float* b,
                     float* ao, float* bo) {
     k_unsort2<<<div_up(n, kBlock), kBlock, 0, s>>>(id, n, a, b, ao, bo);
+}
+
+uint32_t launch_unsort2_sum(hipStream_t s, const uint32_t* id, uint32_t n, const float* a,
+                            const float* b, const float* w, float* ao, float* bo,
+                            double* partials) {
+    const uint32_t g = min(div_up(n, kBlock), kMaxReduceBlocks);
+    k_unsort2_sum<<<g, kBlock, 0, s>>>(id, n, a, b, w, ao, bo, partials);
+    return g;
 }
 
 void launch_kick_drift(hipStream_t s, float* x, float* y, float* vx, float* vy, const float* ax,

@@ -11,6 +11,15 @@
 
 namespace bh {
 
+__global__ __launch_bounds__(kBlock) void k_copy2(uint32_t n, const float* __restrict__ a,
+                                                  const float* __restrict__ b,
+                                                  float* __restrict__ ao, float* __restrict__ bo) {
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= n) return;
+    ao[i] = a[i];
+    bo[i] = b[i];
+}
+
 // embedding -> solver particles (unit masses, identity ids)
 __global__ __launch_bounds__(kBlock) void k_tsne_stage(const float* __restrict__ yx,
                                                        const float* __restrict__ yy, uint32_t n,
@@ -63,34 +72,47 @@ __global__ __launch_bounds__(kBlock) void k_tsne_attract(const uint32_t* __restr
 // derivative d_i = (s/Z) rep_i + attraction with s = 4 (updateRepulsive scaling,
 // tsne.h:291-294; 1 in the reference's GPU step, nBodySolverGpuBH.cu:424), then
 // y' = y + lr d + mu (y - y_prev) (updatePoints, tsne.h:179-206); one thread per point
-__global__ __launch_bounds__(kBlock) void k_tsne_combine(uint32_t n, const float* __restrict__ yx,
-                                                         const float* __restrict__ yy,
-                                                         const float* __restrict__ pyx,
-                                                         const float* __restrict__ pyy,
-                                                         const float* __restrict__ rep_x,
-                                                         const float* __restrict__ rep_y,
-                                                         const float* __restrict__ att_x,
-                                                         const float* __restrict__ att_y,
-                                                         const double* __restrict__ z,
-                                                         double rep_scale, float lr, float mu,
-                                                         float* __restrict__ nyx,
-                                                         float* __restrict__ nyy,
-                                                         float* __restrict__ dx_out,
-                                                         float* __restrict__ dy_out) {
-    const uint32_t r = blockIdx.x * kBlock + threadIdx.x;
-    if (r >= n) return;
-    const float scale = (float)(rep_scale / *z);
-    const float dx = fmaf(scale, rep_x[r], att_x[r]);
-    const float dy = fmaf(scale, rep_y[r], att_y[r]);
-    if (dx_out) {
-        dx_out[r] = dx;
-        dy_out[r] = dy;
-    }
-    if (nyx) {
+// The update, and the next iteration's start where one follows (sx not null): its particles (the
+// masses and indices stay those of the first stage), the interleaved copy and the partial bounds.
+// Z comes as nz partial sums, which every block adds in the same order. Unsorting with Z's partial
+// sums and this kernel stand for six launches of about 5 us each (partial sums, their sum, unsort,
+// update, stage, bounds), a tenth of an iteration at 70k points.
+__global__ __launch_bounds__(kBlock) void k_tsne_update(
+    uint32_t n, const float* __restrict__ yx, const float* __restrict__ yy,
+    const float* __restrict__ pyx, const float* __restrict__ pyy, const float* __restrict__ rep_x,
+    const float* __restrict__ rep_y, const float* __restrict__ att_x,
+    const float* __restrict__ att_y, const double* zpart, uint32_t nz, double* z_out,
+    double rep_scale, float lr, float mu, float* __restrict__ nyx, float* __restrict__ nyy,
+    float* __restrict__ dx_out, float* __restrict__ dy_out, float* __restrict__ sx,
+    float* __restrict__ sy, float2* __restrict__ xy, float4* __restrict__ bounds) {
+    double z = 0.0;
+    for (uint32_t b = threadIdx.x; b < nz; b += kBlock) z += zpart[b];
+    z = block_sum_d(z);
+    if (blockIdx.x == 0 && threadIdx.x == 0 && z_out) *z_out = z;
+    const float scale = (float)(rep_scale / z);
+    float4 box = make_float4(INFINITY, INFINITY, -INFINITY, -INFINITY);
+    for (uint32_t r = blockIdx.x * kBlock + threadIdx.x; r < n; r += gridDim.x * kBlock) {
+        const float dx = fmaf(scale, rep_x[r], att_x[r]);
+        const float dy = fmaf(scale, rep_y[r], att_y[r]);
+        if (dx_out) {
+            dx_out[r] = dx;
+            dy_out[r] = dy;
+        }
         const float xi = yx[r], yi = yy[r];
-        nyx[r] = fmaf(lr, dx, xi) + mu * (xi - pyx[r]);
-        nyy[r] = fmaf(lr, dy, yi) + mu * (yi - pyy[r]);
+        const float x = fmaf(lr, dx, xi) + mu * (xi - pyx[r]);
+        const float y = fmaf(lr, dy, yi) + mu * (yi - pyy[r]);
+        nyx[r] = x;
+        nyy[r] = y;
+        if (sx) {
+            sx[r] = x;
+            sy[r] = y;
+            xy[r] = make_float2(x, y);
+            box = minmax4(box, bounds_item(x, y));
+        }
     }
+    if (!sx) return;
+    box = block_minmax4(box);
+    if (threadIdx.x == 0) bounds[blockIdx.x] = box;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -228,6 +250,10 @@ void launch_tsne_stage(hipStream_t s, const float* yx, const float* yy, uint32_t
     k_tsne_stage<<<div_up(n, kBlock), kBlock, 0, s>>>(yx, yy, n, x, y, m, id, xy);
 }
 
+void launch_copy2(hipStream_t s, uint32_t n, const float* a, const float* b, float* ao, float* bo) {
+    if (n) k_copy2<<<div_up(n, kBlock), kBlock, 0, s>>>(n, a, b, ao, bo);
+}
+
 void launch_tsne_attract(hipStream_t s, const uint32_t* row_ptr, const uint32_t* col,
                          const float* val, uint32_t n, const float2* xy, float exag, float* att_x,
                          float* att_y) {
@@ -235,14 +261,16 @@ void launch_tsne_attract(hipStream_t s, const uint32_t* row_ptr, const uint32_t*
                                                                 att_x, att_y);
 }
 
-void launch_tsne_combine(hipStream_t s, uint32_t n, const float* yx, const float* yy,
-                         const float* pyx, const float* pyy, const float* rep_x,
-                         const float* rep_y, const float* att_x, const float* att_y,
-                         const double* z, double rep_scale, float lr, float mu, float* nyx,
-                         float* nyy, float* dx, float* dy) {
-    k_tsne_combine<<<div_up(n, kBlock), kBlock, 0, s>>>(n, yx, yy, pyx, pyy, rep_x, rep_y, att_x,
-                                                        att_y, z, rep_scale, lr, mu, nyx, nyy, dx,
-                                                        dy);
+uint32_t tsne_update_blocks(uint32_t n) { return min(div_up(n, kBlock), kMaxBoundsBlocks); }
+
+void launch_tsne_update(hipStream_t s, uint32_t n, const float* yx, const float* yy,
+                        const float* pyx, const float* pyy, const float* rep_x, const float* rep_y,
+                        const float* att_x, const float* att_y, const double* zpart, uint32_t nz,
+                        double* z_out, double rep_scale, float lr, float mu, float* nyx, float* nyy,
+                        float* dx, float* dy, float* sx, float* sy, float2* xy, float4* bounds) {
+    k_tsne_update<<<tsne_update_blocks(n), kBlock, 0, s>>>(
+        n, yx, yy, pyx, pyy, rep_x, rep_y, att_x, att_y, zpart, nz, z_out, rep_scale, lr, mu, nyx,
+        nyy, dx, dy, sx, sy, xy, bounds);
 }
 
 uint32_t tsne_kl_blocks(uint32_t n) {

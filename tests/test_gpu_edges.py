@@ -370,3 +370,31 @@ def test_velocities_through_builds(gpu, n):
     if n > 1:
         assert np.abs(gu - dt * ax).max() < 0.05 * top and np.any(gu)
     ctx.close()
+
+
+@pytest.mark.parametrize("solver", ["bh", "fmm_sym"])
+@pytest.mark.parametrize("n", [40, 256, 257, 5000, 262_400])
+def test_tsne_run_equals_single_steps(gpu, solver, n):
+    """Iterations in one call start from what the update before left (particles, bounds), single
+    steps stage the embedding anew: the same embedding to the bit, through the change of the
+    exaggeration, past one block and past the blocks that sum Z and take the bounds."""
+    rng = np.random.default_rng(n)
+    y = rng.normal(0, 1e-2, (n, 2)).astype(np.float32)
+    cols = ((np.arange(n)[:, None] + np.array([1, 7, n - 7, n - 1])) % n).astype(np.uint32)
+    cols.sort(axis=1)
+    rp = (4 * np.arange(n + 1)).astype(np.uint32)
+    val = np.full(4 * n, 1.0 / (4 * n), np.float32)
+    out = []
+    for single in (False, True):
+        t = tsne.TSNE(rp, cols.ravel(), val, (y[:, 0].copy(), y[:, 1].copy()), solver=solver)
+        t.iteration_counter = 247
+        if single:
+            zs = [t.timeStep() for _ in range(6)]
+            assert all(np.isfinite(z) and z > 0 for z in zs)
+        else:
+            t.run(2)
+            t.run(4)
+        out.append(t.embeddedPoints)
+        t.close()
+    assert np.all(np.isfinite(out[0])) and np.any(out[0] != y)
+    assert np.array_equal(out[0], out[1])
