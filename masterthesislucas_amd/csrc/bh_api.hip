@@ -410,8 +410,6 @@ bh_status do_forces(bh_ctx* c, double theta, bool want_total, bool plugin = fals
     const float eps = c->cfg.softening;
     const bool grav = c->cfg.kernel == BH_KERNEL_GRAVITY;
     phase_begin(c, 5);
-    if (!c->nsys && (uint64_t)c->n * 16 <= (3ull << 20))  // small trees: warm every L2 first
-        launch_warm_l2(s, c->nodes, c->prm, c->pos4, c->n, c->vals_b);
     if (plugin && !grav && !c->nsys && c->split == 1 && c->n <= kPreorderMax)
         c->trav_blocks = launch_traverse_preorder(s, c->pos4, c->nodes, c->prm, c->n, inv_theta2,
                                                   c->ax, c->ay, want_total ? c->tot : nullptr,

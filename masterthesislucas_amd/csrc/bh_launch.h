@@ -137,9 +137,6 @@ void launch_fmm(hipStream_t s, const float4* pos4, const uint32_t* codes, const 
                 const uint32_t* count, int depth, uint64_t slot_stride, uint32_t n, uint64_t n_max,
                 const BuildParams* prm, double theta, void* workspace, float* ax, float* ay,
                 double* total);
-// streams the node records and sorted positions into every XCD's L2 when they fit (else no-op)
-void launch_warm_l2(hipStream_t s, const Node* nodes, const BuildParams* prm, const float4* pos4,
-                    uint32_t n, uint32_t* sink);
 void launch_unsort2(hipStream_t s, const uint32_t* id, uint32_t n, const float* a, const float* b,
                     float* ao, float* bo);
 // returns the number of partial sums of w (at most kMaxReduceBlocks)
