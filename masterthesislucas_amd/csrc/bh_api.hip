@@ -59,6 +59,8 @@ struct bh_ctx {
     uint32_t* id[2]{};
     float4* pos4 = nullptr;
     float4* packed = nullptr;  // (x, y, mass, index) in input order, made and used by a build
+    const double* zpart = nullptr;  // the last force call's partial sums of the total (sum_later)
+    uint32_t nzpart = 0;
     bool v_zero = true;        // the velocities are all zero (no caller gave any, no kick yet)
     float *ax = nullptr, *ay = nullptr, *tot = nullptr;
     float *out_a = nullptr, *out_b = nullptr, *out_c = nullptr, *out_d = nullptr;
@@ -380,15 +382,16 @@ TraverseBatch batch_of(const bh_ctx* c) {
     return b;
 }
 
-bh_status do_fmm(bh_ctx* c, double theta) {
+bh_status do_fmm(bh_ctx* c, double theta, bool sum_later) {
     if (!(theta > 0.0)) return fail(c, BH_ERR_ARG, "the FMM solver needs theta > 0");
     hipStream_t s = c->stream;
     phase_begin(c, 5);
     const uint32_t* keys = (const uint32_t*)(c->keys_in_b ? c->keys_b : c->keys_a);
     launch_tree_slots(s, keys, c->nodes, c->prm, c->cap_nodes, c->depth, c->slot_a, c->slot_b,
                       c->slot_c, fmm_slots(c->depth));
-    launch_fmm(s, c->pos4, keys, c->slot_b, c->slot_c, c->depth, c->slot_cap, c->n, c->cfg.n_max,
-               c->prm, theta, c->fmm_buf, c->ax, c->ay, c->dsum);
+    c->zpart = launch_fmm(s, c->pos4, keys, c->slot_b, c->slot_c, c->depth, c->slot_cap, c->n,
+                          c->cfg.n_max, c->prm, theta, c->fmm_buf, c->ax, c->ay,
+                          sum_later ? nullptr : c->dsum, &c->nzpart);
     phase_end(c, 5);
     c->trav_blocks = 0;  // interaction counters are those of the tree walk only
     c->have_acc = true;
@@ -396,13 +399,13 @@ bh_status do_fmm(bh_ctx* c, double theta) {
 }
 
 // plugin: the call is bh_forces / bh_forces_device, whose t-SNE sums keep the pre-order walk's
-// summation order. sum_later: with want_total, the per-point terms in tot are left to the caller to
-// add up (the FMM solver has no terms, its total is in dsum)
+// summation order. sum_later: with want_total, the per-point terms in tot (FMM solver: the nzpart
+// partial sums at zpart) are left to the caller to add up
 bh_status do_forces(bh_ctx* c, double theta, bool want_total, bool plugin = false,
                     bool sum_later = false) {
     if (!c->built) return fail(c, BH_ERR_STATE, "forces requested before a tree was built");
     if (!(theta >= 0.0)) return fail(c, BH_ERR_ARG, "theta must be >= 0");
-    if (c->solver == BH_SOLVER_FMM_SYM) return do_fmm(c, theta);
+    if (c->solver == BH_SOLVER_FMM_SYM) return do_fmm(c, theta, sum_later);
     bh_status mst = ensure_moments(c);
     if (mst != BH_OK) return mst;
     hipStream_t s = c->stream;
@@ -1186,22 +1189,21 @@ static bh_status tsne_iteration(bh_ctx* c, const bh_tsne_params* p, int32_t t, b
                         c->att_y);
     st = hip_check(c, hipEventRecord(c->ev_att, c->att_stream), "event");
     if (st != BH_OK) return st;
-    // repulsion and Z: per-point terms (tree walk) or their sum in dsum (FMM)
-    const bool terms = c->solver != BH_SOLVER_FMM_SYM;
+    // repulsion, and Z as partial sums
     st = do_forces(c, tsne_theta(p, t), true, false, true);
     if (st != BH_OK) return st;
-    uint32_t nz = 1;
-    if (terms)
-        nz = launch_unsort2_sum(s, c->id[c->cur], n, c->ax, c->ay, c->tot, c->rep_x, c->rep_y,
-                                c->red_part);
-    else
+    if (c->solver == BH_SOLVER_FMM_SYM) {
         launch_unsort2(s, c->id[c->cur], n, c->ax, c->ay, c->rep_x, c->rep_y);
+    } else {
+        c->nzpart = launch_unsort2_sum(s, c->id[c->cur], n, c->ax, c->ay, c->tot, c->rep_x,
+                                       c->rep_y, c->red_part);
+        c->zpart = c->red_part;
+    }
     st = hip_check(c, hipStreamWaitEvent(s, c->ev_att, 0), "wait");
     if (st != BH_OK) return st;
     const int cur = c->ty_cur, prev = (cur + 2) % 3, next = (cur + 1) % 3;
     launch_tsne_update(s, n, c->ty_x[cur], c->ty_y[cur], c->ty_x[prev], c->ty_y[prev], c->rep_x,
-                       c->rep_y, c->att_x, c->att_y, terms ? c->red_part : c->dsum, nz,
-                       terms ? c->dsum : nullptr,
+                       c->rep_y, c->att_x, c->att_y, c->zpart, c->nzpart, c->dsum,
                        p->repulsion_scale > 0.0 ? p->repulsion_scale : 4.0,
                        (float)p->learning_rate, mu, c->ty_x[next], c->ty_y[next],
                        keep_deriv ? c->tder_x : nullptr, keep_deriv ? c->tder_y : nullptr,

@@ -371,6 +371,27 @@ __device__ __forceinline__ void fmm_nn_gather(double rx, double ry, double ma, F
     t += (ma * M.m0[y]) / rS;
 }
 
+__device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, kWave);
+    return v;
+}
+
+// The last leaf lo with unit_off[lo] <= u: 64 entries per step, one per lane (3 dependent loads
+// for 65,536 leaves instead of 16).
+__device__ __forceinline__ uint32_t fmm_unit_leaf(const uint32_t* __restrict__ unit_off, uint32_t L,
+                                                  uint32_t u) {
+    const uint32_t lane = threadIdx.x & 63;
+    uint32_t lo = 0, len = L;
+    while (len > 1) {
+        const uint32_t step = (len + kWave - 1) / kWave, at = lane * step;
+        const uint32_t v = at < len ? unit_off[lo + at] : 0xFFFFFFFFu;
+        const uint32_t k = (uint32_t)__popcll(__ballot(at < len && v <= u)) - 1u;
+        lo += k * step;
+        len = min(step, len - k * step);
+    }
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)lo);
+}
+
 // One level of the list construction, one wave per node X of level l: candidates (children of
 // the parent's partners) over the lanes; accepted ones add their expansion to X (node-node
 // kernel, gathered: X is the sink), the others are appended to N(X) in candidate order. Leaf
@@ -440,8 +461,10 @@ __global__ __launch_bounds__(kBlock) void k_fmm_level(const uint32_t* __restrict
             }
             n_out += (uint32_t)__popcll(kb);
         }
-        meet = (uint32_t)wave_sum_u64(meet);
-        lower = (uint32_t)wave_sum_u64(lower);
+        if (l == depth) {  // at most n together: a partner appears once
+            meet = wave_sum_u32(meet);
+            lower = wave_sum_u32(lower);
+        }
     } else {
         // the parent's list overflowed: walk from the root (uniform), lanes take turns with the
         // accepted pairs
@@ -533,7 +556,7 @@ __device__ __forceinline__ void fmm_partners_meta(const uint32_t* __restrict__ f
 
 // exclusive scans of the per-leaf unit counts of the three unit classes (light, heavy,
 // expansion: units + c * unit_stride, unit_stride a multiple of 4) in place; entry L of each =
-// its total (one block). Each thread sums a contiguous run of entries (a multiple of 16, read
+// its total (one block per class: one block for all three took 15 us for 65,536 leaves, now 6). Each thread sums a contiguous run of entries (a multiple of 16, read
 // as uint4, four loads in flight), the run totals are scanned over the block, and the runs are
 // rewritten with their offsets.
 constexpr int kFmmScanArrays = 3;
@@ -547,69 +570,57 @@ __device__ __forceinline__ uint4 fmm_load4(const uint32_t* __restrict__ u, uint3
 __global__ __launch_bounds__(kFmmScanThreads) void k_fmm_scan(uint32_t* __restrict__ units,
                                                               uint32_t unit_stride, uint32_t L) {
     constexpr int kW = kFmmScanThreads / kWave;
-    __shared__ uint32_t wsum[kFmmScanArrays][kW];
+    __shared__ uint32_t wsum[kW];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const uint32_t per = ((L + kFmmScanThreads - 1) / kFmmScanThreads + 15) & ~15u;
     const uint32_t b = threadIdx.x * per;
     const uint32_t e = b + per;  // entries >= L read as 0 and are not written
-    uint32_t own[kFmmScanArrays], x[kFmmScanArrays];
-#pragma unroll
-    for (int a = 0; a < kFmmScanArrays; ++a) {
-        const uint32_t* u = units + a * unit_stride;
-        uint32_t s = 0;
-        for (uint32_t i = b; i < e && i < L; i += 16) {
-            const uint4 v0 = fmm_load4(u, i, L), v1 = fmm_load4(u, i + 4, L),
-                        v2 = fmm_load4(u, i + 8, L), v3 = fmm_load4(u, i + 12, L);
-            s += (v0.x + v0.y + v0.z + v0.w) + (v1.x + v1.y + v1.z + v1.w) +
-                 (v2.x + v2.y + v2.z + v2.w) + (v3.x + v3.y + v3.z + v3.w);
-        }
-        own[a] = s;
+    uint32_t* u = units + blockIdx.x * unit_stride;
+    uint32_t own = 0;
+    for (uint32_t i = b; i < e && i < L; i += 16) {
+        const uint4 v0 = fmm_load4(u, i, L), v1 = fmm_load4(u, i + 4, L),
+                    v2 = fmm_load4(u, i + 8, L), v3 = fmm_load4(u, i + 12, L);
+        own += (v0.x + v0.y + v0.z + v0.w) + (v1.x + v1.y + v1.z + v1.w) +
+               (v2.x + v2.y + v2.z + v2.w) + (v3.x + v3.y + v3.z + v3.w);
     }
+    uint32_t x = own;
 #pragma unroll
-    for (int a = 0; a < kFmmScanArrays; ++a) {
-        x[a] = own[a];
-#pragma unroll
-        for (int d = 1; d < kWave; d <<= 1) {
-            const uint32_t y = __shfl_up(x[a], d, kWave);
-            if (lane >= d) x[a] += y;
-        }
-        if (lane == kWave - 1) wsum[a][w] = x[a];
+    for (int d = 1; d < kWave; d <<= 1) {
+        const uint32_t y = __shfl_up(x, d, kWave);
+        if (lane >= d) x += y;
     }
+    if (lane == kWave - 1) wsum[w] = x;
     __syncthreads();
+    uint32_t off = 0, all = 0;
+    for (int j = 0; j < kW; ++j) {
+        const uint32_t s = wsum[j];
+        off += j < w ? s : 0u;
+        all += s;
+    }
+    uint32_t run = off + x - own;
+    for (uint32_t i = b; i < e && i < L; i += 16) {
+        uint4 v[4] = {fmm_load4(u, i, L), fmm_load4(u, i + 4, L), fmm_load4(u, i + 8, L),
+                      fmm_load4(u, i + 12, L)};
 #pragma unroll
-    for (int a = 0; a < kFmmScanArrays; ++a) {
-        uint32_t off = 0, all = 0;
-        for (int j = 0; j < kW; ++j) {
-            const uint32_t s = wsum[a][j];
-            off += j < w ? s : 0u;
-            all += s;
-        }
-        uint32_t* u = units + a * unit_stride;
-        uint32_t run = off + x[a] - own[a];
-        for (uint32_t i = b; i < e && i < L; i += 16) {
-            uint4 v[4] = {fmm_load4(u, i, L), fmm_load4(u, i + 4, L), fmm_load4(u, i + 8, L),
-                          fmm_load4(u, i + 12, L)};
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                const uint4 c = v[k];
-                uint4 o;
-                o.x = run;
-                o.y = o.x + c.x;
-                o.z = o.y + c.y;
-                o.w = o.z + c.z;
-                run = o.w + c.w;
-                const uint32_t j = i + 4 * k;
-                if (j + 3 < L) {
-                    *reinterpret_cast<uint4*>(u + j) = o;
-                } else {
-                    if (j < L) u[j] = o.x;
-                    if (j + 1 < L) u[j + 1] = o.y;
-                    if (j + 2 < L) u[j + 2] = o.z;
-                }
+        for (int k = 0; k < 4; ++k) {
+            const uint4 c = v[k];
+            uint4 o;
+            o.x = run;
+            o.y = o.x + c.x;
+            o.z = o.y + c.y;
+            o.w = o.z + c.z;
+            run = o.w + c.w;
+            const uint32_t j = i + 4 * k;
+            if (j + 3 < L) {
+                *reinterpret_cast<uint4*>(u + j) = o;
+            } else {
+                if (j < L) u[j] = o.x;
+                if (j + 1 < L) u[j + 1] = o.y;
+                if (j + 2 < L) u[j + 2] = o.z;
             }
         }
-        if (threadIdx.x == 0) u[L] = all;
     }
+    if (threadIdx.x == 0) u[L] = all;
 }
 
 // 1 / d for d >= 1: hardware reciprocal estimate (relative error below 1e-7) refined by one
@@ -619,11 +630,57 @@ __device__ __forceinline__ double fmm_inv(double d) {
     return __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
 }
 
+// Points of many partners dealt to the lanes as one flat sequence. Lane k holds partner k: the
+// slots [off, off + m) of the sequence are its points a, a + F, a + 2 F ... The point in slot
+// blk + lane (any point past the sequence's end), and the lane of its partner.
+struct FmmFlat {
+    uint32_t off, m, a, F;
+    __device__ __forceinline__ uint32_t total() const {
+        return (uint32_t)__builtin_amdgcn_readlane((int)(off + m), kWave - 1);
+    }
+    __device__ __forceinline__ uint32_t at(uint32_t blk, uint32_t& who) const {
+        const uint32_t lane = threadIdx.x & 63;
+        uint64_t on = __ballot(m != 0u && off + m > blk && off < blk + kWave);
+        uint32_t src = 0;
+        who = 0;
+        while (on) {
+            const uint32_t e = (uint32_t)__builtin_ctzll(on);
+            on &= on - 1;
+            const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)off, (int)e);
+            const uint32_t last = (uint32_t)__builtin_amdgcn_readlane((int)m, (int)e) - 1u;
+            if (blk + lane >= o) {
+                src = (uint32_t)__builtin_amdgcn_readlane((int)a, (int)e) +
+                      F * min(blk + lane - o, last);
+                who = e;
+            }
+        }
+        return src;
+    }
+};
+__device__ __forceinline__ FmmFlat fmm_flat(uint32_t m, uint32_t a, uint32_t F) {
+    const int lane = threadIdx.x & 63;
+    uint32_t end = m;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+        const uint32_t y = __shfl_up(end, d, kWave);
+        if (lane >= d) end += y;
+    }
+    return FmmFlat{end - m, m, a, F};
+}
+__device__ __forceinline__ void fmm_wave_sync() {  // LDS of this wave: order only
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 // Point-to-node expansions into leaf X (the reference's point-node kernel applied to X as the
 // second leaf of a pair): for every leaf partner Y of lower slot, each point q of Y farther than
 // l_X/theta from X's centre adds its C1 = -R D1 and C2, C3 (x M0_X) to X. Work units (X, e of
 // E_X) take the points e, e + E_X, ... of those partners over the lanes; each writes its 14
-// coefficients, reduced over the wave, to epart (14 per unit), summed into X by k_fmm_exp_add.
+// coefficients, reduced over the wave, to epart (14 per unit), summed into X on the way down.
+// Partners hold few points each (about 7 on a 70k embedding), so the points of 64 partners are
+// dealt to the lanes as one sequence, and the ones far enough are collected in LDS until there
+// is one per lane for the expansion's hundred FP64 operations: 45 -> 26 us at
+// 70,000 points, where a partner's points alone left most lanes idle.
 __global__ __launch_bounds__(kBlock) void k_fmm_exp(const double2* __restrict__ pd,
                                                     const uint32_t* __restrict__ first,
                                                     const uint32_t* __restrict__ count, int depth,
@@ -642,34 +699,65 @@ __global__ __launch_bounds__(kBlock) void k_fmm_exp(const double2* __restrict__ 
     if (!(side > 0.0)) side = 1.0;
     const double thr = ldexp(side, -depth) / theta;
     const uint32_t base = fmm_level_index(depth);
+    __shared__ double2 stage_all[kWavesPerBlock][2 * kWave];
+    double2* stage = stage_all[threadIdx.x >> 6];
     for (uint32_t u = __builtin_amdgcn_readfirstlane(blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6));
          u < total; u += waves) {
-        uint32_t lo = 0, hi = L;  // unit_off[lo] <= u < unit_off[hi]
-        while (hi - lo > 1) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (unit_off[mid] <= u) lo = mid;
-            else hi = mid;
-        }
-        const uint32_t ix = lo, X = base + ix;
+        const uint32_t ix = fmm_unit_leaf(unit_off, L, u), X = base + ix;
         const uint32_t E = unit_off[ix + 1] - unit_off[ix], e = u - unit_off[ix];
         const double cxX = M.cx[X], cyX = M.cy[X], m0X = M.m0[X];
         FmmCoef cX = {};
-        const uint32_t start = e + E * (uint32_t)lane, step = E * (uint32_t)kWave;
-        fmm_partners_meta(first, count, M, side, theta, depth, X, ix, lists, nlist,
-                          [&](uint32_t Y, uint32_t fY, uint32_t end, double, double) {
-            if (Y >= X) return;
-            for (uint32_t q = fY + start; q < end; q += step) {
-                const double2 qq = pd[q];
-                const double rx = qq.x - cxX, ry = qq.y - cyX;
-                if (rx * rx + ry * ry > thr * thr) {
-                    double rS, D1, D2, D3;
-                    fmm_derivs(rx, ry, rS, D1, D2, D3);
-                    cX.c1[0] += -rx * D1;
-                    cX.c1[1] += -ry * D1;
-                    fmm_add_c2c3(-rx, -ry, D1, D2, D3, m0X, cX);
+        auto expand = [&](double rx, double ry) {  // (rx, ry): point relative to X's centre
+            double rS, D1, D2, D3;
+            fmm_derivs(rx, ry, rS, D1, D2, D3);
+            cX.c1[0] += -rx * D1;
+            cX.c1[1] += -ry * D1;
+            fmm_add_c2c3(-rx, -ry, D1, D2, D3, m0X, cX);
+        };
+        const uint32_t np = nlist[X];
+        if (np != kFmmOverflow) {
+            const uint32_t* in = lists + (size_t)X * kFmmListCap;
+            uint32_t nst = 0;  // points collected
+            for (uint32_t b0 = 0; b0 < np; b0 += kWave) {
+                const uint32_t j = b0 + (uint32_t)lane;
+                const uint32_t Y = j < np ? in[j] : X;
+                const uint32_t nY = Y < X ? count[Y] : 0u;
+                const FmmFlat fl = fmm_flat(nY > e ? (nY - 1 - e) / E + 1 : 0u, first[Y] + e, E);
+                const uint32_t all = fl.total();
+                uint32_t who;
+                double2 next = all ? pd[fl.at(0, who)] : make_double2(0.0, 0.0);
+                for (uint32_t blk = 0; blk < all; blk += kWave) {
+                    const double2 qq = next;
+                    if (blk + kWave < all) next = pd[fl.at(blk + kWave, who)];
+                    const double rx = qq.x - cxX, ry = qq.y - cyX;
+                    const bool keep = blk + (uint32_t)lane < all && rx * rx + ry * ry > thr * thr;
+                    const uint64_t kb = __ballot(keep);
+                    if (keep) stage[nst + __popcll(kb & lane_mask_lt())] = make_double2(rx, ry);
+                    nst += (uint32_t)__popcll(kb);
+                    fmm_wave_sync();
+                    if (nst >= (uint32_t)kWave) {
+                        const double2 r = stage[lane], over = stage[kWave + lane];
+                        expand(r.x, r.y);
+                        nst -= kWave;
+                        fmm_wave_sync();
+                        if ((uint32_t)lane < nst) stage[lane] = over;
+                        fmm_wave_sync();
+                    }
                 }
             }
-        });
+            if ((uint32_t)lane < nst) expand(stage[lane].x, stage[lane].y);
+            fmm_wave_sync();
+        } else {
+            const uint32_t start = e + E * (uint32_t)lane, step = E * (uint32_t)kWave;
+            fmm_walk(count, M, side, theta, depth, ix,
+                     [&](int k, uint32_t y, bool acc, double, double) {
+                if (k != depth || acc || y >= X) return;
+                for (uint32_t q = first[y] + start; q < first[y] + count[y]; q += step) {
+                    const double rx = pd[q].x - cxX, ry = pd[q].y - cyX;
+                    if (rx * rx + ry * ry > thr * thr) expand(rx, ry);
+                }
+            });
+        }
         double v[14];
 #pragma unroll
         for (int k = 0; k < 2; ++k) v[k] = wave_sum_d(cX.c1[k]);
@@ -686,17 +774,10 @@ __global__ __launch_bounds__(kBlock) void k_fmm_exp(const double2* __restrict__ 
     }
 }
 
-// adds each leaf's expansion-unit partials (in unit order) to its coefficients; thread per leaf
-__global__ __launch_bounds__(kBlock) void k_fmm_exp_add(const uint32_t* __restrict__ unit_off,
-                                                        int depth, uint32_t S,
-                                                        const double* __restrict__ epart,
-                                                        double* __restrict__ C) {
-    const uint32_t ix = blockIdx.x * kBlock + threadIdx.x;
-    if (ix >= (1u << (2 * depth))) return;
+// adds leaf ix's expansion-unit partials (in unit order) to its coefficients
+__device__ __forceinline__ void fmm_exp_add(const uint32_t* __restrict__ unit_off, uint32_t ix,
+                                            const double* __restrict__ epart, FmmCoef& c) {
     const uint32_t b = unit_off[ix], e = unit_off[ix + 1];
-    if (b == e) return;
-    const uint32_t X = fmm_level_index(depth) + ix;
-    FmmCoef c = fmm_load(C, S, X);
     for (uint32_t u = b; u < e; ++u) {
         const double* p = epart + (size_t)u * 14;
 #pragma unroll
@@ -706,7 +787,6 @@ __global__ __launch_bounds__(kBlock) void k_fmm_exp_add(const uint32_t* __restri
 #pragma unroll
         for (int k = 0; k < 8; ++k) c.c3[k] += p[6 + k];
     }
-    fmm_store(C, S, X, c);
 }
 
 // point-point term of source q on the lane's sink (p.x, p.y)
@@ -837,11 +917,19 @@ __device__ __forceinline__ void fmm_pp_unit(const double2* __restrict__ pd,
     mine_out = mine;
 }
 
-// The same unit with its sources staged in LDS first (units of at most 64 partners whose
-// shares hold at most kFmmStage points): lane k copies the share of partner k into its segment
-// of the wave's stage buffer, dropping the points of a lower-slot partner that X's box accepts,
-// so every load of the unit is in flight at once; the sums then read the sources from LDS.
+// The same unit with its sources staged in LDS first (units of at most 64 partners whose shares
+// hold at most kFmmStage points), all loads of the unit in flight at once: the points of the
+// partners are dealt to the lanes as one sequence. Partners of lower slot (without the points that
+// X's box accepts) and X itself make one run of sources that every sink sums, no matter whose
+// they are. A partner of higher slot is tested by every sink first, so those keep their segments,
+// and the lane groups take different partners. 93 -> 57 us
+// at 70,000 points (theta 0.5), where a loop over the partners spent as many instructions on
+// stepping from one to the next as on its few points.
 // Returns false (nothing done) when the unit does not qualify.
+struct FmmPartner {
+    double cx, cy;
+    uint32_t first, end, Y, pad;
+};
 template <bool GROUPED>
 __device__ __forceinline__ bool fmm_pp_unit_staged(const double2* __restrict__ pd,
                                                    const uint32_t* __restrict__ first,
@@ -851,6 +939,7 @@ __device__ __forceinline__ bool fmm_pp_unit_staged(const double2* __restrict__ p
                                                    const uint32_t* __restrict__ nlist, uint32_t X,
                                                    uint32_t F, uint32_t c0, uint32_t f,
                                                    double2* __restrict__ stage,
+                                                   FmmPartner* __restrict__ upper,
                                                    uint64_t part_stride, double* __restrict__ part,
                                                    double& t_out, bool& mine_out) {
     const int lane = threadIdx.x & 63;
@@ -863,36 +952,32 @@ __device__ __forceinline__ bool fmm_pp_unit_staged(const double2* __restrict__ p
     const uint32_t Y = has ? lists[(size_t)X * kFmmListCap + lane] : X;
     const uint32_t fY = first[Y], nY = has ? count[Y] : 0u;
     const uint32_t m = nY > f ? (nY - 1 - f) / F + 1 : 0u;  // points of share f
-    uint32_t off = m;  // exclusive prefix over the lanes
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        const uint32_t y = __shfl_up(off, d, kWave);
-        if (lane >= d) off += y;
+    const bool up = has && Y > X;
+    const FmmFlat hi = fmm_flat(up ? m : 0u, fY + f, F), lo = fmm_flat(up ? 0u : m, fY + f, F);
+    const uint32_t nhi = hi.total(), nlo = lo.total();
+    if (nhi + nlo > kFmmStage) return false;
+    const uint64_t ub = __ballot(up);
+    const uint32_t nup = (uint32_t)__popcll(ub);
+    if (up)
+        upper[__popcll(ub & lane_mask_lt())] =
+            FmmPartner{M.cx[Y], M.cy[Y], hi.off, hi.off + m, Y, 0u};
+    uint32_t who;
+    for (uint32_t blk = 0; blk < nhi; blk += kWave) {
+        const double2 q = pd[hi.at(blk, who)];
+        if (blk + (uint32_t)lane < nhi) stage[blk + lane] = q;
     }
-    const uint32_t all = (uint32_t)__builtin_amdgcn_readlane((int)off, kWave - 1);
-    if (all > kFmmStage) return false;
-    off -= m;
-    const bool second = Y < X;
-    uint32_t kept = 0;
-    for (uint32_t i = 0; i < m; i += 4) {
-        double2 v[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] = pd[fY + f + F * (i + u < m ? i + u : i)];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            if (i + u >= m) break;
-            if (second) {
-                const double bx = v[u].x - cxX, by = v[u].y - cyX;
-                if (bx * bx + by * by > thr * thr) continue;
-            }
-            stage[off + kept] = v[u];
-            ++kept;
-        }
+    uint32_t end = nhi;
+    for (uint32_t blk = 0; blk < nlo; blk += kWave) {
+        const double2 q = pd[lo.at(blk, who)];
+        const bool own = (uint32_t)__shfl((int)Y, (int)who, kWave) == X;
+        const double bx = q.x - cxX, by = q.y - cyX;
+        const bool keep =
+            blk + (uint32_t)lane < nlo && (own || !(bx * bx + by * by > thr * thr));
+        const uint64_t kb = __ballot(keep);
+        if (keep) stage[end + __popcll(kb & lane_mask_lt())] = q;
+        end += (uint32_t)__popcll(kb);
     }
-    const double cxl = M.cx[Y], cyl = M.cy[Y];
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    fmm_wave_sync();
 
     const uint32_t Wc = GROUPED ? (nX > 16u ? 32u : (nX > 8u ? 16u : 8u)) : (uint32_t)kWave;
     const uint32_t G = GROUPED ? (uint32_t)kWave / Wc : 1u;
@@ -904,38 +989,36 @@ __device__ __forceinline__ bool fmm_pp_unit_staged(const double2* __restrict__ p
     const double2 pp = pd[p];
     const double px = pp.x, py = pp.y;
     double ax = 0.0, ay = 0.0, t = 0.0;
-    for (uint32_t k = 0; k < np; ++k) {
-        const uint32_t Yk = (uint32_t)__builtin_amdgcn_readlane((int)Y, (int)k);
-        const uint32_t sb = (uint32_t)__builtin_amdgcn_readlane((int)off, (int)k);
-        const uint32_t se = sb + (uint32_t)__builtin_amdgcn_readlane((int)kept, (int)k);
-        bool run = true;
-        if (X < Yk) {
-            const double rx = px - fmm_readlane_d(cxl, k), ry = py - fmm_readlane_d(cyl, k);
-            if (rx * rx + ry * ry > thr * thr) {
-                run = false;
-                if (f == 0 && g == 0) {
-                    double rS, D1, D2, D3;
-                    fmm_derivs(rx, ry, rS, D1, D2, D3);
-                    double vx, vy;
-                    fmm_c1(rx, ry, D1, D2, D3, M.m0[Yk], M.xx[Yk], M.xy[Yk], M.yy[Yk], vx, vy);
-                    ax += vx;
-                    ay += vy;
-                    t += 2.0 * M.m0[Yk] / rS;
-                }
-            }
-        }
-        if (!run) continue;
-        uint32_t j = sb + g;
-        for (; j + 3 * G < se; j += 4 * G) {
-            const double2 a = stage[j], b = stage[j + G], c = stage[j + 2 * G], d = stage[j + 3 * G];
+    auto sum = [&](uint32_t j, uint32_t e, uint32_t st) {
+        for (; j + 3 * st < e; j += 4 * st) {
+            const double2 a = stage[j], b = stage[j + st], c = stage[j + 2 * st],
+                          d = stage[j + 3 * st];
             fmm_pp1(a, px, py, ax, ay, t, true);
             fmm_pp1(b, px, py, ax, ay, t, true);
             fmm_pp1(c, px, py, ax, ay, t, true);
             fmm_pp1(d, px, py, ax, ay, t, true);
         }
-        for (; j < se; j += G) fmm_pp1(stage[j], px, py, ax, ay, t, true);
-        // the leaf's own share holds the sink itself once (w = 1, no force): take it out
-        if (Yk == X && o % F == f && (o / F) % G == g) t -= 1.0;
+        for (; j < e; j += st) fmm_pp1(stage[j], px, py, ax, ay, t, true);
+    };
+    sum(nhi + g, end, G);
+    // the run holds the sink itself once (w = 1, no force): take it out
+    if (g == 0 && o % F == f) t -= 1.0;
+    for (uint32_t k = g; k < nup; k += G) {
+        const FmmPartner q = upper[k];
+        const double rx = px - q.cx, ry = py - q.cy;
+        if (rx * rx + ry * ry > thr * thr) {
+            if (f == 0) {
+                double rS, D1, D2, D3;
+                fmm_derivs(rx, ry, rS, D1, D2, D3);
+                double vx, vy;
+                fmm_c1(rx, ry, D1, D2, D3, M.m0[q.Y], M.xx[q.Y], M.xy[q.Y], M.yy[q.Y], vx, vy);
+                ax += vx;
+                ay += vy;
+                t += 2.0 * M.m0[q.Y] / rS;
+            }
+        } else {
+            sum(q.first, q.end, 1);
+        }
     }
     if (GROUPED) {
         for (uint32_t w = Wc; w < (uint32_t)kWave; w <<= 1) {
@@ -949,9 +1032,7 @@ __device__ __forceinline__ bool fmm_pp_unit_staged(const double2* __restrict__ p
     }
     t_out = t;
     mine_out = mine;
-    // the next unit's staging must not overwrite sources still being read
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
+    fmm_wave_sync();  // the next unit's staging must not overwrite sources still being read
     return true;
 }
 
@@ -962,7 +1043,7 @@ __device__ __forceinline__ bool fmm_pp_unit_staged(const double2* __restrict__ p
 //  - X < Y (X first): a sink far enough from Y's centre takes Y's expansion (C1 of the
 //    point-node kernel, share 0 only), the others sum over Y's points;
 //  - Y < X (X second): Y's points not accepted against X's box act point by point on the sinks
-//    (the accepted ones went into X's expansion in k_fmm_exp).
+//    (the accepted ones go into X's expansion in k_fmm_exp).
 // Unit f takes partner points f, f + F, ... (split further over lane groups for small leaves);
 // the F shares are summed per point afterwards.
 template <bool LIGHT>
@@ -988,15 +1069,10 @@ __global__ __launch_bounds__(kBlock) void k_fmm_pp(const double2* __restrict__ p
     const double thr = ldexp(side, -depth) / theta;
     const uint32_t base = fmm_level_index(depth);
     __shared__ double2 stage_all[kWavesPerBlock][LIGHT ? kFmmStage : kWave];
+    __shared__ FmmPartner upper_all[LIGHT ? kWavesPerBlock : 1][kWave];
     for (uint32_t u = __builtin_amdgcn_readfirstlane(blockIdx.x * kWavesPerBlock + (threadIdx.x >> 6));
          u < total; u += waves) {
-        uint32_t lo = 0, hi = L;  // unit_off[lo] <= u < unit_off[hi]
-        while (hi - lo > 1) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (unit_off[mid] <= u) lo = mid;
-            else hi = mid;
-        }
-        const uint32_t ix = lo, X = base + ix;
+        const uint32_t ix = fmm_unit_leaf(unit_off, L, u), X = base + ix;
         const uint32_t F = split[ix], local = u - unit_off[ix];
         const uint32_t c0 = (local / F) * kWave, f = local % F;
         double t;
@@ -1005,10 +1081,12 @@ __global__ __launch_bounds__(kBlock) void k_fmm_pp(const double2* __restrict__ p
         bool done = false;
         double2* stage = stage_all[threadIdx.x >> 6];
         if (LIGHT) {
-            done = grouped ? fmm_pp_unit_staged<true>(pd, first, count, M, thr, lists, nlist, X, F,
-                                                      c0, f, stage, part_stride, part, t, mine)
-                           : fmm_pp_unit_staged<false>(pd, first, count, M, thr, lists, nlist, X, F,
-                                                       c0, f, stage, part_stride, part, t, mine);
+            FmmPartner* upper = upper_all[LIGHT ? threadIdx.x >> 6 : 0];
+            done = grouped
+                       ? fmm_pp_unit_staged<true>(pd, first, count, M, thr, lists, nlist, X, F, c0,
+                                                  f, stage, upper, part_stride, part, t, mine)
+                       : fmm_pp_unit_staged<false>(pd, first, count, M, thr, lists, nlist, X, F, c0,
+                                                   f, stage, upper, part_stride, part, t, mine);
         }
         if (!done) {
             if (grouped)
@@ -1025,23 +1103,15 @@ __global__ __launch_bounds__(kBlock) void k_fmm_pp(const double2* __restrict__ p
 
 // applyForces (:482-536), one level: C2, C3 of a node divided by its M0, then the parent's
 // (final) expansion translated to the node's centre of mass added. Level 0: the division only.
-__device__ __forceinline__ void fmm_down_node(const uint32_t* __restrict__ count, int l,
-                                              uint32_t i, uint32_t S, double* __restrict__ mom,
-                                              double* __restrict__ C) {
-    const uint32_t s = fmm_level_index(l) + i;
-    if (count[s] == 0u) return;
-    FmmMoments M = fmm_moments(mom, S);
-    FmmCoef c = fmm_load(C, S, s);
-    const double inv = 1.0 / M.m0[s];
+__device__ __forceinline__ void fmm_down_step(FmmCoef& c, double inv, bool has_par,
+                                              const FmmCoef& pc, double dx, double dy) {
 #pragma unroll
     for (int k = 0; k < 4; ++k) c.c2[k] *= inv;
 #pragma unroll
     for (int k = 0; k < 8; ++k) c.c3[k] *= inv;
-    if (l > 0) {
-        const uint32_t par = fmm_level_index(l - 1) + (i >> 2);
-        const FmmCoef pc = fmm_load(C, S, par);
+    if (has_par) {
         double vx, vy, t2[4];
-        fmm_translate(pc, M.cx[s] - M.cx[par], M.cy[s] - M.cy[par], vx, vy, t2);
+        fmm_translate(pc, dx, dy, vx, vy, t2);
         c.c1[0] += vx;
         c.c1[1] += vy;
 #pragma unroll
@@ -1049,22 +1119,90 @@ __device__ __forceinline__ void fmm_down_node(const uint32_t* __restrict__ count
 #pragma unroll
         for (int k = 0; k < 8; ++k) c.c3[k] += pc.c3[k];
     }
+}
+
+// unit_off, epart: the expansion units of the leaves (null above the leaf level)
+__global__ __launch_bounds__(kBlock) void k_fmm_down(const uint32_t* __restrict__ count, int l,
+                                                     uint32_t S, double* __restrict__ mom,
+                                                     double* __restrict__ C,
+                                                     const uint32_t* __restrict__ unit_off,
+                                                     const double* __restrict__ epart) {
+    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
+    if (i >= (1u << (2 * l))) return;
+    const uint32_t s = fmm_level_index(l) + i;
+    if (count[s] == 0u) return;
+    FmmMoments M = fmm_moments(mom, S);
+    FmmCoef c = fmm_load(C, S, s);
+    const uint32_t par = fmm_level_index(l - 1) + (i >> 2);  // l > 0
+    const FmmCoef pc = fmm_load(C, S, par);
+    const double dx = M.cx[s] - M.cx[par], dy = M.cy[s] - M.cy[par], inv = 1.0 / M.m0[s];
+    if (epart) fmm_exp_add(unit_off, i, epart, c);
+    fmm_down_step(c, inv, true, pc, dx, dy);
     fmm_store(C, S, s, c);
 }
 
-__global__ __launch_bounds__(kBlock) void k_fmm_down(const uint32_t* __restrict__ count, int l,
-                                                     uint32_t S, double* __restrict__ mom,
-                                                     double* __restrict__ C) {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i < (1u << (2 * l))) fmm_down_node(count, l, i, S, mom, C);
-}
-
+// The levels with at most kFmmTopNodes nodes, one block: a level's coefficients are loaded while the
+// one above is worked on, and parents are read from LDS (11 us with a trip to memory per level,
+// now 10).
 __global__ __launch_bounds__(kFmmTopNodes) void k_fmm_down_top(const uint32_t* __restrict__ count,
-                                                               int top, uint32_t S,
+                                                               int top, int depth, uint32_t S,
                                                                double* __restrict__ mom,
-                                                               double* __restrict__ C) {
+                                                               double* __restrict__ C,
+                                                               const uint32_t* __restrict__ unit_off,
+                                                               const double* __restrict__ epart) {
+    __shared__ double sp[16][kFmmTopNodes / 4];  // the level above: coefficients, centre
+    const uint32_t i = threadIdx.x;
+    FmmMoments M = fmm_moments(mom, S);
+    struct Own {
+        FmmCoef c;
+        double m0, cx, cy;
+        bool on;
+    };
+    auto load = [&](int l) {
+        Own o{};
+        o.on = i < (1u << (2 * l)) && count[fmm_level_index(l) + i] != 0u;
+        if (o.on) {
+            const uint32_t s = fmm_level_index(l) + i;
+            o.c = fmm_load(C, S, s);
+            o.m0 = M.m0[s];
+            o.cx = M.cx[s];
+            o.cy = M.cy[s];
+        }
+        return o;
+    };
+    Own next = load(0);
     for (int l = 0; l <= top; ++l) {
-        if (threadIdx.x < (1u << (2 * l))) fmm_down_node(count, l, threadIdx.x, S, mom, C);
+        Own o = next;
+        if (l < top) next = load(l + 1);
+        if (o.on) {
+            FmmCoef pc{};
+            double dx = 0.0, dy = 0.0;
+            if (l > 0) {
+                const uint32_t q = i >> 2;
+#pragma unroll
+                for (int k = 0; k < 2; ++k) pc.c1[k] = sp[k][q];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) pc.c2[k] = sp[2 + k][q];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) pc.c3[k] = sp[6 + k][q];
+                dx = o.cx - sp[14][q];
+                dy = o.cy - sp[15][q];
+            }
+            if (l == depth) fmm_exp_add(unit_off, i, epart, o.c);
+            fmm_down_step(o.c, 1.0 / o.m0, l > 0, pc, dx, dy);
+            fmm_store(C, S, fmm_level_index(l) + i, o.c);
+        }
+        __syncthreads();
+        if (o.on && l < top) {  // at most kFmmTopNodes / 4 of them
+#pragma unroll
+            for (int k = 0; k < 2; ++k) sp[k][i] = o.c.c1[k];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) sp[2 + k][i] = o.c.c2[k];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) sp[6 + k][i] = o.c.c3[k];
+            sp[14][i] = o.cx;
+            sp[15][i] = o.cy;
+        }
         __syncthreads();
     }
 }
@@ -1142,12 +1280,11 @@ constexpr uint32_t kFmmSumBlocks = 64;
 
 // workspace layout (each part 256-byte aligned): moments 6 x S, coefficients 14 x S, node
 // totals S, unit totals 2 x max_units (light, heavy), point-point shares 2 x kFmmMaxSplit x n_max,
-// FP64 positions n_max, Z partials, unit offsets 3 x (S + 1 rounded up to 4) (light, heavy,
-// expansion), splits S, list lengths S, lists kFmmListCap x S (uint32). The expansion partials (14 per expansion
-// unit, at most 14 (leaves + n/4) doubles) live in the point-point shares' space, which is
-// written only after they are summed.
+// expansion partials (14 per expansion unit, at most leaves + n/4 units), FP64 positions n_max, Z
+// partials, unit offsets 3 x (S + 1 rounded up to 4) (light, heavy, expansion), splits S, list
+// lengths S, lists kFmmListCap x S (uint32).
 struct FmmLayout {
-    uint64_t mom, coef, tot_nn, tot_unit, part, pd, partials, units, split, nlist, lists, bytes,
+    uint64_t mom, coef, tot_nn, tot_unit, part, epart, pd, partials, units, split, nlist, lists, bytes,
         max_units, unit_stride;
 };
 
@@ -1162,6 +1299,7 @@ FmmLayout fmm_layout(uint64_t S, uint64_t n_max) {
     L.tot_nn = o;    o += up(S * sizeof(double));
     L.tot_unit = o;  o += up(2 * L.max_units * sizeof(double));
     L.part = o;      o += up(2ull * kFmmMaxSplit * n_max * sizeof(double));
+    L.epart = o;     o += up(14 * (leaves + n_max / 4) * sizeof(double));
     L.pd = o;        o += up(n_max * sizeof(double2));
     L.partials = o;  o += up(kFmmSumBlocks * sizeof(double));
     L.unit_stride = (S + 1 + 3) & ~(uint64_t)3;
@@ -1178,10 +1316,11 @@ uint64_t fmm_workspace_bytes(uint64_t slot_stride, uint64_t n_max) {
     return fmm_layout(slot_stride, n_max).bytes;
 }
 
-void launch_fmm(hipStream_t s, const float4* pos4, const uint32_t* codes, const uint32_t* first,
-                const uint32_t* count, int depth, uint64_t slot_stride, uint32_t n, uint64_t n_max,
-                const BuildParams* prm, double theta, void* workspace, float* ax, float* ay,
-                double* total) {
+const double* launch_fmm(hipStream_t s, const float4* pos4, const uint32_t* codes,
+                         const uint32_t* first, const uint32_t* count, int depth,
+                         uint64_t slot_stride, uint32_t n, uint64_t n_max, const BuildParams* prm,
+                         double theta, void* workspace, float* ax, float* ay, double* total,
+                         uint32_t* nz) {
     const uint32_t S = (uint32_t)slot_stride;
     const FmmLayout Lw = fmm_layout(slot_stride, n_max);
     char* w = (char*)workspace;
@@ -1190,6 +1329,7 @@ void launch_fmm(hipStream_t s, const float4* pos4, const uint32_t* codes, const 
     double* tot_nn = (double*)(w + Lw.tot_nn);
     double* tot_unit = (double*)(w + Lw.tot_unit);
     double* part = (double*)(w + Lw.part);
+    double* epart = (double*)(w + Lw.epart);
     double* partials = (double*)(w + Lw.partials);
     uint32_t* units = (uint32_t*)(w + Lw.units);
     uint32_t* split = (uint32_t*)(w + Lw.split);
@@ -1207,16 +1347,14 @@ void launch_fmm(hipStream_t s, const float4* pos4, const uint32_t* codes, const 
     for (int l = 0; l <= depth; ++l)
         k_fmm_level<<<fmm_div_up(1u << (2 * l), kWavesPerBlock), kBlock, 0, s>>>(
             count, l, depth, S, prm, theta, mom, coef, tot_nn, lists, nlist, units, US, split);
-    k_fmm_scan<<<1, kFmmScanThreads, 0, s>>>(units, US, leaves);
+    k_fmm_scan<<<kFmmScanArrays, kFmmScanThreads, 0, s>>>(units, US, leaves);
     {
         const uint64_t ebound = (uint64_t)(leaves < n ? leaves : n) + n / 4;
         uint32_t eblocks = fmm_div_up(ebound, kWavesPerBlock);
         if (eblocks > kFmmUnitBlocks) eblocks = kFmmUnitBlocks;
         if (eblocks < 1) eblocks = 1;
         k_fmm_exp<<<eblocks, kBlock, 0, s>>>(pd, first, count, depth, S, prm, theta, mom, lists,
-                                             nlist, units + 2 * US, part);
-        k_fmm_exp_add<<<fmm_div_up(leaves, kBlock), kBlock, 0, s>>>(units + 2 * US, depth, S,
-                                                                    part, coef);
+                                             nlist, units + 2 * US, epart);
     }
     // the unit count stays on the device: a fixed grid of waves strides over the units
     const uint64_t unit_bound = (uint64_t)kFmmMaxSplit * ((n + kWave - 1) / kWave +
@@ -1230,16 +1368,19 @@ void launch_fmm(hipStream_t s, const float4* pos4, const uint32_t* codes, const 
                                               nlist, units + US, split, n_max, part,
                                               tot_unit + Lw.max_units);
     const int dtop = depth < kFmmTopLevel ? depth : kFmmTopLevel;
-    k_fmm_down_top<<<1, kFmmTopNodes, 0, s>>>(count, dtop, S, mom, coef);
+    k_fmm_down_top<<<1, kFmmTopNodes, 0, s>>>(count, dtop, depth, S, mom, coef, units + 2 * US, epart);
     for (int l = dtop + 1; l <= depth; ++l)
-        k_fmm_down<<<fmm_div_up(1u << (2 * l), kBlock), kBlock, 0, s>>>(count, l, S, mom, coef);
+        k_fmm_down<<<fmm_div_up(1u << (2 * l), kBlock), kBlock, 0, s>>>(
+            count, l, S, mom, coef, units + 2 * US, l == depth ? epart : nullptr);
     k_fmm_l2p<<<fmm_div_up(n, kBlock), kBlock, 0, s>>>(pos4, codes, n, depth, S, mom, coef, split,
                                                        n_max, part, ax, ay);
     const uint32_t used = (uint32_t)fmm_slots(depth);
     k_fmm_sum_partial<<<kFmmSumBlocks, kBlock, 0, s>>>(tot_nn, used, tot_unit, units + leaves,
                                                        tot_unit + Lw.max_units,
                                                        units + US + leaves, partials);
-    k_fmm_sum_final<<<1, 64, 0, s>>>(partials, kFmmSumBlocks, total);
+    if (total) k_fmm_sum_final<<<1, 64, 0, s>>>(partials, kFmmSumBlocks, total);
+    *nz = kFmmSumBlocks;
+    return partials;
 }
 
 }  // namespace bh

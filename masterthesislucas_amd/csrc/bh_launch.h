@@ -133,10 +133,12 @@ uint32_t traverse_blocks(uint32_t n);
 // FP32) and *total (Z).
 uint64_t fmm_slots(int depth);
 uint64_t fmm_workspace_bytes(uint64_t slot_stride, uint64_t n_max);
-void launch_fmm(hipStream_t s, const float4* pos4, const uint32_t* codes, const uint32_t* first,
-                const uint32_t* count, int depth, uint64_t slot_stride, uint32_t n, uint64_t n_max,
-                const BuildParams* prm, double theta, void* workspace, float* ax, float* ay,
-                double* total);
+// returns the partial sums of the total, *nz of them in the workspace; total: their sum, or null
+const double* launch_fmm(hipStream_t s, const float4* pos4, const uint32_t* codes,
+                         const uint32_t* first, const uint32_t* count, int depth,
+                         uint64_t slot_stride, uint32_t n, uint64_t n_max, const BuildParams* prm,
+                         double theta, void* workspace, float* ax, float* ay, double* total,
+                         uint32_t* nz);
 void launch_unsort2(hipStream_t s, const uint32_t* id, uint32_t n, const float* a, const float* b,
                     float* ao, float* bo);
 // returns the number of partial sums of w (at most kMaxReduceBlocks)

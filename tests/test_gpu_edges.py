@@ -6,7 +6,7 @@ import pytest
 from masterthesislucas_amd import BHContext, tsne
 from masterthesislucas_amd.learned import N_OUT, FarFieldMLP, flatten, unflatten
 from oracle import oracle as O
-from tests.helpers import oracle_tree
+from tests.helpers import oracle_tree, rel_err
 
 pytestmark = pytest.mark.gpu
 
@@ -398,3 +398,35 @@ def test_tsne_run_equals_single_steps(gpu, solver, n):
         t.close()
     assert np.all(np.isfinite(out[0])) and np.any(out[0] != y)
     assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("theta", [0.35, 0.8])
+@pytest.mark.parametrize("n", [64, 300, 4096, 16_384, 16_400, 66_000])
+def test_fmm_edges(gpu, n, theta):
+    """Leaf units at the edges of their lane groups (leaves of about 8, 16, 32 and many points side
+    by side), units of more points than are staged at once, and trees whose leaf level is and is
+    not among the levels of one block. FP64 on both sides, the order of the sums apart: FP32
+    rounding of the result (median 1e-6, p99 1e-5), Z to 1e-10."""
+    rng = np.random.default_rng(n)
+    # four quadrants of densities 1 : 2 : 4 : 9, and a crowded spot
+    q = np.searchsorted(np.cumsum([1, 2, 4, 9]) / 16, rng.random(n))
+    x = (rng.random(n) + (q & 1)).astype(np.float32)
+    y = (rng.random(n) + (q >> 1)).astype(np.float32)
+    c = n // 40
+    x[:c] = (0.3 + 1e-3 * rng.random(c)).astype(np.float32)
+    y[:c] = (0.3 + 1e-3 * rng.random(c)).astype(np.float32)
+    ctx = BHContext(n, kernel="tsne", tree_mode="morton_fixed")
+    ctx.set_solver("fmm_sym")
+    ctx.set_particles(x, y)
+    ctx.build()
+    ax, ay, z = ctx.forces(theta)
+    ctx.close()
+    t = oracle_tree(x, y, None, mode="morton_fixed")
+    minx, miny, maxx, maxy = t["bounds"]
+    tree = O.fixed_tree(t["xs"], t["ys"], t["depth"], minx, miny, maxx, maxy)
+    sx, sy, bz = O.fmm_sym(t["xs"], t["ys"], tree, t["depth"], theta)
+    bx, by = np.empty(n), np.empty(n)
+    bx[t["perm"]], by[t["perm"]] = sx, sy
+    r = rel_err(ax, ay, bx, by)
+    assert np.median(r) <= 1e-6 and np.quantile(r, 0.99) <= 1e-5, (np.median(r), r.max())
+    assert abs(z - bz) <= 1e-10 * abs(bz)
