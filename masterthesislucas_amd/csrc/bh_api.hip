@@ -330,16 +330,18 @@ bh_status do_build(bh_ctx* c, const double* bounds, uint32_t have_partials = 0) 
     phase_begin(c, 2);
     const int nxt = 1 - cur;
     const float *vx = c->v_zero ? nullptr : c->vx[cur], *vy = c->v_zero ? nullptr : c->vy[cur];
-    launch_gather(s, perm, n, c->packed, vx, vy, c->x[nxt], c->y[nxt], c->m[nxt], c->vx[nxt],
-                  c->vy[nxt], c->id[nxt], c->pos4, c->dstatus, codes, c->wide);
+    launch_gather_levels(s, perm, c->packed, vx, vy, c->x[nxt], c->y[nxt], c->m[nxt], c->vx[nxt],
+                         c->vy[nxt], c->id[nxt], c->pos4, codes, c->wide, n, c->B,
+                         c->cfg.max_children, fixed, c->leaf_lvl, c->lcp1, c->cnt, c->tree_sums,
+                         c->R, c->dstatus);
     phase_end(c, 2);
     c->cur = nxt;
 
     if (!quadtree) c->depth = fixed;
     phase_begin(c, 3);
-    launch_tree(s, codes, c->wide, n, c->B, c->cfg.max_children, fixed, quadtree ? 1 : 0,
-                c->leaf_lvl, c->lcp1, c->cnt, c->noff, c->tree_sums, c->prm, c->nodes, c->parent,
-                c->child4, c->cap_nodes, c->R, c->nsys ? c->sys_prm : nullptr, c->dstatus);
+    launch_tree(s, codes, c->wide, n, c->B, quadtree ? 1 : 0, c->lcp1, c->cnt, c->noff, c->tree_sums,
+                c->prm, c->nodes, c->parent, c->child4, c->cap_nodes, c->R,
+                c->nsys ? c->sys_prm : nullptr);
     if (c->nsys) launch_batch_roots(s, c->sys_off, c->nsys, c->noff, c->prm, c->roots);
     phase_end(c, 3);
 
@@ -851,11 +853,13 @@ bh_status bh_leapfrog(bh_ctx* c, int steps, float dt, double theta) {
         const int cur = c->cur;
         phase_begin(c, 6);
         launch_kick_drift(c->stream, c->x[cur], c->y[cur], c->vx[cur], c->vy[cur], c->ax, c->ay,
-                          c->n, hdt, dt);
+                          c->n, hdt, dt, k > 0, c->bounds_part);
         phase_end(c, 6);
-        st = do_build(c, nullptr);
+        st = do_build(c, nullptr, update_blocks(c->n));
         if (st == BH_OK) st = do_forces(c, theta, false);
         if (st != BH_OK) return st;
+    }
+    if (steps > 0) {
         const int nc = c->cur;
         phase_begin(c, 6);
         launch_kick(c->stream, c->vx[nc], c->vy[nc], c->ax, c->ay, c->n, hdt);
@@ -871,8 +875,8 @@ static bh_status leapfrog_step(bh_ctx* c, float dt, double theta) {
     const float hdt = 0.5f * dt;
     const int cur = c->cur;
     launch_kick_drift(c->stream, c->x[cur], c->y[cur], c->vx[cur], c->vy[cur], c->ax, c->ay, c->n,
-                      hdt, dt);
-    bh_status st = do_build(c, nullptr);
+                      hdt, dt, false, c->bounds_part);
+    bh_status st = do_build(c, nullptr, update_blocks(c->n));
     if (st == BH_OK) st = do_forces(c, theta, false);
     if (st != BH_OK) return st;
     const int nc = c->cur;
@@ -1180,7 +1184,7 @@ static bh_status tsne_iteration(bh_ctx* c, const bh_tsne_params* p, int32_t t, b
         c->cur = 0;
     else
         tsne_stage(c);
-    bh_status st = do_build(c, nullptr, staged ? tsne_update_blocks(n) : 0);
+    bh_status st = do_build(c, nullptr, staged ? update_blocks(n) : 0);
     if (st != BH_OK) return st;
     st = hip_check(c, hipEventRecord(c->ev_staged, s), "event");
     if (st == BH_OK) st = hip_check(c, hipStreamWaitEvent(c->att_stream, c->ev_staged, 0), "wait");

@@ -43,12 +43,17 @@ struct CallerBounds {
     double minx, miny, maxx, maxy;
 };
 
-// every thread of the block takes part; thread 0 fills *out (LDS or memory)
+// every thread of the block takes part; thread 0 fills *out (LDS or memory). Without partials (nb =
+// 0) the block takes the bounds of all positions itself.
 __device__ __forceinline__ void bounds_final(const float4* __restrict__ partials, uint32_t nb,
-                                             uint32_t n, uint32_t tree_mode, CallerBounds cb,
-                                             BuildParams* out, uint32_t* status) {
+                                             const float* __restrict__ xs,
+                                             const float* __restrict__ ys, uint32_t n,
+                                             uint32_t tree_mode, CallerBounds cb, BuildParams* out,
+                                             uint32_t* status) {
     float4 r = make_float4(INFINITY, INFINITY, -INFINITY, -INFINITY);
     for (uint32_t b = threadIdx.x; b < nb; b += kBlock) r = minmax4(r, partials[b]);
+    if (nb == 0)
+        for (uint32_t i = threadIdx.x; i < n; i += kBlock) r = minmax4(r, bounds_item(xs[i], ys[i]));
     r = block_minmax4(r);
     if (threadIdx.x != 0) return;
     if (status) flag_nonfinite(r, status);
@@ -72,7 +77,7 @@ __global__ __launch_bounds__(kBlock) void k_bounds_final(const float4* __restric
                                                          BuildParams* __restrict__ prm,
                                                          uint32_t tree_mode, CallerBounds cb,
                                                          uint32_t* __restrict__ status) {
-    bounds_final(partials, nb, n, tree_mode, cb, prm, status);
+    bounds_final(partials, nb, nullptr, nullptr, n, tree_mode, cb, prm, status);
 }
 
 // batched systems: bounds per system from per-block partials over each system's blocks
@@ -172,7 +177,8 @@ __global__ __launch_bounds__(kBlock) void k_morton(const float* __restrict__ xs,
         x[r] = xs[i];
         y[r] = ys[i];
     }
-    bounds_final(partials, nb, n, tree_mode, cb, &s_prm, blockIdx.x == 0 ? status : nullptr);
+    bounds_final(partials, nb, xs, ys, n, tree_mode, cb, &s_prm,
+                 blockIdx.x == 0 ? status : nullptr);
     if (threadIdx.x == 0) s_prm.n_nodes = 0;
     __syncthreads();
     static_assert(sizeof(BuildParams) % 4 == 0 && sizeof(BuildParams) / 4 <= kBlock, "one word each");
@@ -1030,52 +1036,27 @@ __global__ __launch_bounds__(THREADS) void k_bucket_sort(K* keys, uint32_t* vals
 }
 
 // ------------------------------------------------------------------------------------------
-// gather the particle state into sorted order
-// ------------------------------------------------------------------------------------------
-// vx, vy: null when the velocities are known to be zero (zeros are then written, not gathered)
-__global__ __launch_bounds__(kBlock) void k_gather(const uint32_t* __restrict__ perm, uint32_t n,
-                                                   const float4* __restrict__ pk,
-                                                   const float* __restrict__ vx,
-                                                   const float* __restrict__ vy,
-                                                   float* __restrict__ xo, float* __restrict__ yo,
-                                                   float* __restrict__ mo, float* __restrict__ vxo,
-                                                   float* __restrict__ vyo,
-                                                   uint32_t* __restrict__ ido,
-                                                   float4* __restrict__ pos4,
-                                                   const uint32_t* __restrict__ sort_err,
-                                                   void* __restrict__ codes, int wide) {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    // a sort that gave up leaves no valid permutation: keep the input order and make every code
-    // 0 (sorted), so the tree build sees a well-formed input; the build reports the error
-    const bool failed = sort_err[0] != 0u;
-    const uint32_t j = failed ? i : min(perm[i], n - 1);
-    if (failed) {
-        if (wide)
-            static_cast<uint64_t*>(codes)[i] = 0ull;
-        else
-            static_cast<uint32_t*>(codes)[i] = 0u;
-    }
-    const float4 q = pk[j];
-    const float u = vx ? vx[j] : 0.0f, v = vy ? vy[j] : 0.0f;
-    xo[i] = q.x;
-    yo[i] = q.y;
-    mo[i] = q.z;
-    vxo[i] = u;
-    vyo[i] = v;
-    ido[i] = __float_as_uint(q.w);
-    pos4[i] = make_float4(q.x, q.y, q.z, 0.0f);
-}
-
-// ------------------------------------------------------------------------------------------
-// tree: leaf level per particle, node count per particle
+// the particle state gathered into sorted order; tree: leaf level and node count per particle
 // ------------------------------------------------------------------------------------------
 // The node count of each tile of kTreeTile particles goes to sums: k_tree_emit_heads takes the
 // counts of the tiles before its own from there, so the device-wide scan needs no launch of its
-// own (three launches of 2 to 4 us each before).
+// own (three launches of 2 to 4 us each before). The gather has no launch of its own either: its
+// random reads are in flight while the block works on its codes.
+// vx, vy: null when the velocities are known to be zero (zeros are then written, not gathered).
 constexpr int kTreeTile = 1024;
 template <typename K>
-__global__ __launch_bounds__(kTreeTile) void k_tree_levels(const K* __restrict__ codes, uint32_t n,
+__global__ __launch_bounds__(kTreeTile) void k_gather_levels(const uint32_t* __restrict__ perm,
+                                                        const float4* __restrict__ pk,
+                                                        const float* __restrict__ vx,
+                                                        const float* __restrict__ vy,
+                                                        float* __restrict__ xo,
+                                                        float* __restrict__ yo,
+                                                        float* __restrict__ mo,
+                                                        float* __restrict__ vxo,
+                                                        float* __restrict__ vyo,
+                                                        uint32_t* __restrict__ ido,
+                                                        float4* __restrict__ pos4,
+                                                        K* codes, uint32_t n,
                                                         int B, int R, int cap, int fixed_depth,
                                                         uint8_t* __restrict__ leaf_lvl,
                                                         uint8_t* __restrict__ lcp1,
@@ -1085,6 +1066,19 @@ __global__ __launch_bounds__(kTreeTile) void k_tree_levels(const K* __restrict__
     __shared__ K s_code[kTreeTile + 2 * kMaxLeafCap];
     __shared__ int8_t s_w[kTreeTile + kMaxLeafCap];
     const int64_t b0 = (int64_t)blockIdx.x * kTreeTile;
+    const int64_t i = b0 + threadIdx.x;
+    // a build whose sort gave up or whose input is not finite gets an empty tree: every walk over
+    // it ends at once (the call reports the error). A sort that gave up leaves no valid
+    // permutation either: the input order is kept, with every code 0 (sorted).
+    const bool no_sort = status[0] != 0u, failed = no_sort || status[1] != 0u;
+    float4 q = make_float4(0.f, 0.f, 0.f, 0.f);
+    float qu = 0.0f, qv = 0.0f;
+    if (i < (int64_t)n) {
+        const uint32_t j = no_sort ? (uint32_t)i : min(perm[i], n - 1);
+        q = pk[j];
+        if (vx) qu = vx[j];
+        if (vy) qv = vy[j];
+    }
     const int adaptive = fixed_depth < 0;
     if (adaptive) {
         const int span = kTreeTile + 2 * cap;
@@ -1103,9 +1097,15 @@ __global__ __launch_bounds__(kTreeTile) void k_tree_levels(const K* __restrict__
         }
         __syncthreads();
     }
-    const int64_t i = b0 + threadIdx.x;
     uint32_t c = 0;
     if (i < (int64_t)n) {
+        xo[i] = q.x;
+        yo[i] = q.y;
+        mo[i] = q.z;
+        vxo[i] = qu;
+        vyo[i] = qv;
+        ido[i] = __float_as_uint(q.w);
+        pos4[i] = make_float4(q.x, q.y, q.z, 0.0f);
         int leaf;
         if (adaptive) {
             int m = -1;
@@ -1118,11 +1118,9 @@ __global__ __launch_bounds__(kTreeTile) void k_tree_levels(const K* __restrict__
         const int lp = max((i == 0) ? -1 : lcp_level(codes[i - 1], codes[i], B), R - 1);
         leaf_lvl[i] = (uint8_t)leaf;
         lcp1[i] = (uint8_t)(lp + 1);
-        // a build whose sort gave up or whose input is not finite gets an empty tree: every walk
-        // over it ends at once (the call reports the error)
-        const bool failed = (status[0] | status[1]) != 0u;
         c = (!failed && leaf > lp) ? (uint32_t)(leaf - lp) : 0u;
         cnt[i] = c;
+        if (no_sort) codes[i] = 0;
     }
     uint32_t tot;
     block_exclusive_scan_t<kTreeTile>(c, &tot);
@@ -1866,13 +1864,15 @@ void launch_morton_gpuref(hipStream_t s, const float* xs, const float* ys, const
 
 // 4 particles per thread above kMortonWide: fewer blocks to repeat the bounds' last step
 constexpr uint32_t kMortonWide = 1u << 18;
+// up to here every block reads all positions for the bounds (16 loads a thread): no partials launch
+constexpr uint32_t kMortonAlone = 4096;
 
 void launch_morton(hipStream_t s, const float* xs, const float* ys, const float* ms,
                    const uint32_t* ids, uint32_t n, float4* partials, BuildParams* prm,
                    uint32_t tree_mode, const double* caller, uint32_t* status, int B, void* keys,
                    uint32_t* vals, bool wide, float4* pk, uint32_t have_partials) {
-    const uint32_t nb = have_partials ? have_partials : bounds_grid(n);
-    if (!have_partials) k_bounds_partial<<<nb, kBlock, 0, s>>>(xs, ys, n, partials);
+    const uint32_t nb = n <= kMortonAlone ? 0u : have_partials ? have_partials : bounds_grid(n);
+    if (nb && !have_partials) k_bounds_partial<<<nb, kBlock, 0, s>>>(xs, ys, n, partials);
     const CallerBounds cb = caller_bounds(caller);
 #define BH_MORTON(K, I)                                                                           \
     k_morton<K, I><<<div_up(n, kBlock * I), kBlock, 0, s>>>(                                      \
@@ -2013,34 +2013,33 @@ void launch_sort(hipStream_t s, void* keys_a, uint32_t* vals_a, void* keys_b, ui
     *result_in_b = (passes & 1) != 0;
 }
 
-void launch_gather(hipStream_t s, const uint32_t* perm, uint32_t n, const float4* pk,
-                   const float* vx, const float* vy, float* xo, float* yo, float* mo, float* vxo,
-                   float* vyo, uint32_t* ido, float4* pos4, const uint32_t* sort_err, void* codes,
-                   bool wide) {
-    k_gather<<<div_up(n, kBlock), kBlock, 0, s>>>(perm, n, pk, vx, vy, xo, yo, mo, vxo, vyo, ido,
-                                                  pos4, sort_err, codes, wide ? 1 : 0);
-}
-
 uint32_t tree_tiles(uint32_t n) { return div_up(n, kTreeTile); }
 
-void launch_tree(hipStream_t s, const void* codes, bool wide, uint32_t n, int B, int cap,
-                 int fixed_depth, int single_child_pp, uint8_t* leaf_lvl, uint8_t* lcp1,
-                 uint32_t* cnt, uint32_t* noff, uint32_t* sums, BuildParams* prm,
-                 Node* nodes, uint32_t* parent, uint32_t* child4, uint32_t cap_nodes, int R,
-                 const BuildParams* sys_prm, const uint32_t* status) {
-    const uint32_t g = div_up(n, kTreeTile), gn = div_up(cap_nodes, kTreeThreads);
+void launch_gather_levels(hipStream_t s, const uint32_t* perm, const float4* pk, const float* vx,
+                          const float* vy, float* xo, float* yo, float* mo, float* vxo, float* vyo,
+                          uint32_t* ido, float4* pos4, void* codes, bool wide, uint32_t n, int B,
+                          int cap, int fixed_depth, uint8_t* leaf_lvl, uint8_t* lcp1, uint32_t* cnt,
+                          uint32_t* sums, int R, const uint32_t* status) {
 #define BH_LEVELS(K)                                                                              \
-    k_tree_levels<K><<<g, kTreeTile, 0, s>>>((const K*)codes, n, B, R, cap, fixed_depth,          \
-                                             leaf_lvl, lcp1, cnt, sums, status)
-#define BH_NODES(K)                                                                               \
-    k_tree_emit_nodes<K><<<gn, kTreeThreads, 0, s>>>((const K*)codes, n, B, R, lcp1, noff, prm,      \
-                                                  sys_prm, single_child_pp, nodes, parent,        \
-                                                  child4, cap_nodes)
+    k_gather_levels<K><<<div_up(n, kTreeTile), kTreeTile, 0, s>>>(                                \
+        perm, pk, vx, vy, xo, yo, mo, vxo, vyo, ido, pos4, (K*)codes, n, B, R, cap, fixed_depth,  \
+        leaf_lvl, lcp1, cnt, sums, status)
     if (wide) BH_LEVELS(uint64_t); else BH_LEVELS(uint32_t);
+#undef BH_LEVELS
+}
+
+void launch_tree(hipStream_t s, const void* codes, bool wide, uint32_t n, int B,
+                 int single_child_pp, const uint8_t* lcp1, const uint32_t* cnt, uint32_t* noff,
+                 const uint32_t* sums, BuildParams* prm, Node* nodes, uint32_t* parent,
+                 uint32_t* child4, uint32_t cap_nodes, int R, const BuildParams* sys_prm) {
+    const uint32_t g = div_up(n, kTreeTile), gn = div_up(cap_nodes, kTreeThreads);
+#define BH_NODES(K)                                                                               \
+    k_tree_emit_nodes<K><<<gn, kTreeThreads, 0, s>>>((const K*)codes, n, B, R, lcp1, noff, prm,   \
+                                                     sys_prm, single_child_pp, nodes, parent,     \
+                                                     child4, cap_nodes)
     k_tree_emit_heads<<<g, kTreeTile, 0, s>>>(n, lcp1, cnt, sums, noff, prm, nodes,
                                               (uint4*)child4, cap_nodes);
     if (wide) BH_NODES(uint64_t); else BH_NODES(uint32_t);
-#undef BH_LEVELS
 #undef BH_NODES
 }
 

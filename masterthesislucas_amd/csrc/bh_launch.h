@@ -21,7 +21,7 @@ uint32_t bounds_grid(uint32_t n);
 constexpr int kStatusWords = 4;
 constexpr uint32_t kSortSpinLimit = 1u << 22;  // look-back polls before giving up
 // Bounds, root square and Morton keys of the positions, the identity in vals, and every particle's
-// state packed for launch_gather (x, y, mass, index). ms, ids: masses and indices.
+// state packed for launch_gather_levels (x, y, mass, index). ms, ids: masses and indices.
 // have_partials: partial bounds that stand in `partials` already (0: made here).
 // gpuref: keys of the reference GPU step's tree (32-bit, path in the top 2 depth bits)
 void launch_morton_gpuref(hipStream_t s, const float* xs, const float* ys, const float* ms,
@@ -38,23 +38,25 @@ uint32_t sort_blocks(uint32_t n);
 uint64_t sort_scratch_words(uint32_t n);  // uint32 words of scratch launch_sort needs
 // Stable sort of the n keys; vals_a holds 0 .. n-1 on entry.
 // err: status word set when a look-back wait exceeds spin_limit polls (the order is then not
-// valid; later passes do nothing and launch_gather falls back to the input order)
+// valid; later passes do nothing and launch_gather_levels falls back to the input order)
 void launch_sort(hipStream_t s, void* keys_a, uint32_t* vals_a, void* keys_b, uint32_t* vals_b,
                  uint32_t n, int key_bits, bool wide, uint32_t* scratch, uint32_t* err,
                  uint32_t spin_limit, bool* result_in_b);
-// codes: the sorted codes, zeroed (with the identity order) when *sort_err is set; vx, vy: null when
-// the velocities are known to be zero
-void launch_gather(hipStream_t s, const uint32_t* perm, uint32_t n, const float4* pk,
-                   const float* vx, const float* vy, float* xo, float* yo, float* mo, float* vxo,
-                   float* vyo, uint32_t* ido, float4* pos4, const uint32_t* sort_err, void* codes,
-                   bool wide);
-// R: level of the tree roots (0; batched systems: the system id occupies the levels above R)
-uint32_t tree_tiles(uint32_t n);  // words of launch_tree's sums
-void launch_tree(hipStream_t s, const void* codes, bool wide, uint32_t n, int B, int cap,
-                 int fixed_depth, int single_child_pp, uint8_t* leaf_lvl, uint8_t* lcp1,
-                 uint32_t* cnt, uint32_t* noff, uint32_t* sums, BuildParams* prm,
-                 Node* nodes, uint32_t* parent, uint32_t* child4, uint32_t cap_nodes, int R,
-                 const BuildParams* sys_prm, const uint32_t* status);
+// The state in sorted order (from the packed records) and per particle the leaf level, the level
+// it shares with its predecessor (+ 1) and the nodes it heads; sums: node counts of the tiles.
+// codes: zeroed (with the input order) when status says that the sort gave up; vx, vy: null when the
+// velocities are known to be zero. R: level of the tree roots (0; batched systems: the system id
+// occupies the levels above R).
+uint32_t tree_tiles(uint32_t n);  // words of sums
+void launch_gather_levels(hipStream_t s, const uint32_t* perm, const float4* pk, const float* vx,
+                          const float* vy, float* xo, float* yo, float* mo, float* vxo, float* vyo,
+                          uint32_t* ido, float4* pos4, void* codes, bool wide, uint32_t n, int B,
+                          int cap, int fixed_depth, uint8_t* leaf_lvl, uint8_t* lcp1, uint32_t* cnt,
+                          uint32_t* sums, int R, const uint32_t* status);
+void launch_tree(hipStream_t s, const void* codes, bool wide, uint32_t n, int B,
+                 int single_child_pp, const uint8_t* lcp1, const uint32_t* cnt, uint32_t* noff,
+                 const uint32_t* sums, BuildParams* prm, Node* nodes, uint32_t* parent,
+                 uint32_t* child4, uint32_t cap_nodes, int R, const BuildParams* sys_prm);
 void launch_bounds_batched(hipStream_t s, const float* xs, const float* ys, const uint2* blk,
                            uint32_t nblk, const uint32_t* blk_off, const uint32_t* sys_off,
                            uint32_t nsys, float4* partials, BuildParams* sys_prm,
@@ -145,8 +147,12 @@ void launch_unsort2(hipStream_t s, const uint32_t* id, uint32_t n, const float* 
 uint32_t launch_unsort2_sum(hipStream_t s, const uint32_t* id, uint32_t n, const float* a,
                             const float* b, const float* w, float* ao, float* bo,
                             double* partials);
+// partial bounds that launch_kick_drift and launch_tsne_update leave for the next build
+uint32_t update_blocks(uint32_t n);
+// close: the closing kick of the step before goes first
 void launch_kick_drift(hipStream_t s, float* x, float* y, float* vx, float* vy, const float* ax,
-                       const float* ay, uint32_t n, float hdt, float dt);
+                       const float* ay, uint32_t n, float hdt, float dt, bool close,
+                       float4* bounds);
 void launch_kick(hipStream_t s, float* vx, float* vy, const float* ax, const float* ay, uint32_t n,
                  float hdt);
 
@@ -180,8 +186,7 @@ void launch_tsne_attract(hipStream_t s, const uint32_t* row_ptr, const uint32_t*
                          const float* val, uint32_t n, const float2* xy, float exag, float* att_x,
                          float* att_y);
 // Z = sum of nz partial sums (written to z_out when not null); sx, sy, xy, bounds (null: not wanted):
-// the next iteration's particles and their partial bounds (tsne_update_blocks of them)
-uint32_t tsne_update_blocks(uint32_t n);
+// the next iteration's particles and their partial bounds (update_blocks of them)
 void launch_tsne_update(hipStream_t s, uint32_t n, const float* yx, const float* yy,
                         const float* pyx, const float* pyy, const float* rep_x, const float* rep_y,
                         const float* att_x, const float* att_y, const double* zpart, uint32_t nz,

@@ -899,21 +899,36 @@ __global__ __launch_bounds__(kBlock) void k_unsort2_sum(const uint32_t* __restri
     if (threadIdx.x == 0) partials[blockIdx.x] = s;
 }
 
-// kick-drift of kick-drift-kick leapfrog: v += a dt/2; x += v dt
+// kick-drift of kick-drift-kick leapfrog, v += a dt/2; x += v dt, and the partial bounds of the new
+// positions for the build that follows. close: the closing kick of the step before goes first (two
+// kicks, rounded as two). One launch where three stood (kick, kick-drift, bounds: 14 -> 5 us at
+// 200k particles).
 __global__ __launch_bounds__(kBlock) void k_kick_drift(float* __restrict__ x, float* __restrict__ y,
                                                        float* __restrict__ vx,
                                                        float* __restrict__ vy,
                                                        const float* __restrict__ ax,
                                                        const float* __restrict__ ay, uint32_t n,
-                                                       float hdt, float dt) {
-    const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if (i >= n) return;
-    const float nvx = fmaf(ax[i], hdt, vx[i]);
-    const float nvy = fmaf(ay[i], hdt, vy[i]);
-    vx[i] = nvx;
-    vy[i] = nvy;
-    x[i] = fmaf(nvx, dt, x[i]);
-    y[i] = fmaf(nvy, dt, y[i]);
+                                                       float hdt, float dt, int close,
+                                                       float4* __restrict__ bounds) {
+    float4 box = make_float4(INFINITY, INFINITY, -INFINITY, -INFINITY);
+    for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock) {
+        const float a = ax[i], b = ay[i];
+        float u = vx[i], v = vy[i];
+        if (close) {
+            u = fmaf(a, hdt, u);
+            v = fmaf(b, hdt, v);
+        }
+        u = fmaf(a, hdt, u);
+        v = fmaf(b, hdt, v);
+        vx[i] = u;
+        vy[i] = v;
+        const float px = fmaf(u, dt, x[i]), py = fmaf(v, dt, y[i]);
+        x[i] = px;
+        y[i] = py;
+        box = minmax4(box, bounds_item(px, py));
+    }
+    box = block_minmax4(box);
+    if (threadIdx.x == 0) bounds[blockIdx.x] = box;
 }
 
 __global__ __launch_bounds__(kBlock) void k_kick(float* __restrict__ vx, float* __restrict__ vy,
@@ -1089,9 +1104,13 @@ uint32_t launch_unsort2_sum(hipStream_t s, const uint32_t* id, uint32_t n, const
     return g;
 }
 
+uint32_t update_blocks(uint32_t n) { return min(div_up(n, kBlock), kMaxBoundsBlocks); }
+
 void launch_kick_drift(hipStream_t s, float* x, float* y, float* vx, float* vy, const float* ax,
-                       const float* ay, uint32_t n, float hdt, float dt) {
-    k_kick_drift<<<div_up(n, kBlock), kBlock, 0, s>>>(x, y, vx, vy, ax, ay, n, hdt, dt);
+                       const float* ay, uint32_t n, float hdt, float dt, bool close,
+                       float4* bounds) {
+    k_kick_drift<<<update_blocks(n), kBlock, 0, s>>>(x, y, vx, vy, ax, ay, n, hdt, dt, close ? 1 : 0,
+                                                     bounds);
 }
 
 void launch_kick(hipStream_t s, float* vx, float* vy, const float* ax, const float* ay, uint32_t n,

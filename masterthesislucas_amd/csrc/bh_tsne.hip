@@ -261,14 +261,12 @@ void launch_tsne_attract(hipStream_t s, const uint32_t* row_ptr, const uint32_t*
                                                                 att_x, att_y);
 }
 
-uint32_t tsne_update_blocks(uint32_t n) { return min(div_up(n, kBlock), kMaxBoundsBlocks); }
-
 void launch_tsne_update(hipStream_t s, uint32_t n, const float* yx, const float* yy,
                         const float* pyx, const float* pyy, const float* rep_x, const float* rep_y,
                         const float* att_x, const float* att_y, const double* zpart, uint32_t nz,
                         double* z_out, double rep_scale, float lr, float mu, float* nyx, float* nyy,
                         float* dx, float* dy, float* sx, float* sy, float2* xy, float4* bounds) {
-    k_tsne_update<<<tsne_update_blocks(n), kBlock, 0, s>>>(
+    k_tsne_update<<<update_blocks(n), kBlock, 0, s>>>(
         n, yx, yy, pyx, pyy, rep_x, rep_y, att_x, att_y, zpart, nz, z_out, rep_scale, lr, mu, nyx,
         nyy, dx, dy, sx, sy, xy, bounds);
 }

@@ -430,3 +430,30 @@ def test_fmm_edges(gpu, n, theta):
     r = rel_err(ax, ay, bx, by)
     assert np.median(r) <= 1e-6 and np.quantile(r, 0.99) <= 1e-5, (np.median(r), r.max())
     assert abs(z - bz) <= 1e-10 * abs(bz)
+
+
+@pytest.mark.parametrize("n", [1, 1000, 4096, 4097, 262_200])
+def test_leapfrog_steps_in_one_call(gpu, n):
+    """Steps in one call share a launch between the closing kick of one and the opening kick and
+    drift of the next, and hand the new positions' bounds to the build: the same state to the bit
+    as one step per call and as replayed graphs, on both sides of the sizes at which the key kernel
+    takes the bounds itself and at which the drift's blocks stop growing."""
+    rng = np.random.default_rng(n)
+    x, y, vx, vy = rng.normal(0, 1, (4, n)).astype(np.float32)
+    m = np.full(n, 1.0 / n, np.float32)
+    out = []
+    for how in ("one", "single", "graph"):
+        ctx = BHContext(n, kernel="gravity", softening=0.05)
+        ctx.set_particles(x, y, m, vx, vy)
+        if how == "one":
+            ctx.leapfrog(3, 1e-2, 0.6)
+        elif how == "single":
+            for _ in range(3):
+                ctx.leapfrog(1, 1e-2, 0.6)
+        else:
+            ctx.leapfrog_graph(3, 1e-2, 0.6)
+        out.append(ctx.get_particles())
+        ctx.close()
+    for other in out[1:]:
+        assert all(np.array_equal(a, b) for a, b in zip(out[0], other))
+    assert np.any(out[0][0] != x)
