@@ -198,16 +198,24 @@ __device__ __forceinline__ uint32_t row_first(uint32_t v) {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x150, 0xF, 0xF, false);
 }
 
+// the threshold of a row as the other column ranges' workgroups have it so far (any of them bounds
+// the k-th smallest distance over all columns; upper bounds are >= 0, so their bits order them)
+__device__ __forceinline__ float aff_thr(const uint32_t* p) {
+    return __uint_as_float(__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+}
+
 // Workgroup: 8 waves as 2 x 4 over a 128 x 256 tile of Gram products, 64 x 64 per wave (16
 // v_mfma_f32_16x16x32_f16 tiles from 4 + 4 operand reads per K step of 32). Rows and columns
 // stream through LDS in chunks of 64 halfs, double-buffered: the next chunk's global loads are
 // in flight while the current one feeds the MFMAs. Bound by the matrix cores and the LDS reads
 // that feed them (8 reads of 1 KB per 16 MFMAs; the earlier 16 x 64 tile per wave read LDS once
-// per MFMA and left the matrix cores three quarters idle). The epilogue tests a pair against the
-// row's threshold without square roots, conservatively (a few percent of the pairs pass, so in
-// nearly every wave some lane does), and appends (column, Gram value); the bounds themselves are
-// taken when a row's list is compacted, 64 entries at a time. One LDS atomic per row and 64
-// columns reserves its slots. 20,000 points in 784-D: 4.68 -> 2.45 ms.
+// per MFMA and left the matrix cores three quarters idle). The epilogue tests every pair with one
+// addition and comparison, then the few that pass against the row's threshold without square
+// roots, conservatively, and appends (column, Gram value); the bounds themselves are taken when a
+// row's list is compacted, 64 entries at a time. Workgroups of the same rows share their
+// thresholds: those that start later collect a fraction of the candidates. 20,000 points in 784-D:
+// 4.68 ms with 16 x 64 products per wave, 2.49 with 64 x 64, 1.87 with the short test and the
+// shared thresholds.
 constexpr int kAffThreads = 512;
 constexpr int kAffLd = kAffKC + kAffPad;
 constexpr int kAffLoads = (kAffRows + kAffCols) * (kAffKC / 8) / kAffThreads;  // 16 B per thread
@@ -221,6 +229,7 @@ __global__ __launch_bounds__(kAffThreads) void k_aff_candidates(const _Float16* 
                                                                 uint32_t k,
                                                                 uint2* __restrict__ cand,
                                                                 uint32_t* __restrict__ ccount,
+                                                                uint32_t* thr,
                                                                 uint32_t* __restrict__ overflow) {
     __shared__ __attribute__((aligned(16))) _Float16 s_t[2][(kAffRows + kAffCols) * kAffLd];
     __shared__ uint32_t s_cnt[kAffRows], s_over[kAffRows];
@@ -241,7 +250,7 @@ __global__ __launch_bounds__(kAffThreads) void k_aff_candidates(const _Float16* 
         const uint32_t i = row0 + tid;
         s_cnt[tid] = 0u;
         s_over[tid] = 0u;
-        s_T[tid] = __uint_as_float(0x7F800000u);
+        s_T[tid] = i < n ? aff_thr(thr + i) : INFINITY;
         s_nh[tid] = i < n ? nh[i] : 0.f;
         s_ka[tid] = i < n ? aff_kdelta(dp) * ah[i] * kUp : 0.f;
         s_eb[tid] = i < n ? eb[i] * kUp : 0.f;
@@ -274,7 +283,7 @@ __global__ __launch_bounds__(kAffThreads) void k_aff_candidates(const _Float16* 
     for (uint32_t t = t0; t < t1; ++t) {
         // the epilogue's column constants, in flight during the products
         const uint32_t c0 = t * kAffCols;
-        float nj[4], aj[4], ej[4];
+        f32x4 nj, aj, ej;
         bool jv[4];
 #pragma unroll
         for (int b = 0; b < 4; ++b) {
@@ -284,6 +293,7 @@ __global__ __launch_bounds__(kAffThreads) void k_aff_candidates(const _Float16* 
             aj[b] = jv[b] ? ah[j] : 0.f;
             ej[b] = jv[b] ? eb[j] * kUp : 0.f;
         }
+        const float theirs = tid < kAffRows && row0 + tid < n ? aff_thr(thr + row0 + tid) : INFINITY;
         f32x4 acc[4][4];
 #pragma unroll
         for (int a = 0; a < 4; ++a)
@@ -313,52 +323,56 @@ __global__ __launch_bounds__(kAffThreads) void k_aff_candidates(const _Float16* 
             if (more) stage(buf ^ 1);
             __syncthreads();
         }
-        // acc[a][b][e] = x^_i . x^_j, i = row0 + 64 wr + 16 a + 4 q4 + e, j = c0 + 64 wc + 16 b + r16
-        // tiles off the diagonal and inside both ranges need no per-pair checks
-        const bool edge = (c0 < row0 + kAffRows && row0 < c0 + kAffCols) || c0 + kAffCols > n ||
-                          row0 + kAffRows > n;
+        // acc[a][b][e] = x^_i . x^_j, i = row0 + 64 wr + 16 a + 4 q4 + e, j = c0 + 64 wc + 16 b + r16.
+        // A pair that passes the threshold test has g >= (its row's term) + (its column's), the
+        // terms with the largest |x^_j| and rounding bound of the wave's columns and a slack of
+        // 2^-19 |x^|^2 over their own rounding: one addition and one comparison per pair.
+        const bool edge = c0 < row0 + kAffRows && row0 < c0 + kAffCols;  // holds pairs with j = i
+        float am = 0.f, em = 0.f, hc[4];
+#pragma unroll
+        for (int b = 0; b < 4; ++b) {
+            am = fmaxf(am, aj[b]);
+            em = fmaxf(em, ej[b]);
+            hc[b] = jv[b] ? 0.5f * nj[b] * (1.0f - 0x1p-19f) : INFINITY;
+        }
+        for (int o = 8; o > 0; o >>= 1) {  // over the 16 columns of a row of lanes
+            am = fmaxf(am, __shfl_xor(am, o, kWave));
+            em = fmaxf(em, __shfl_xor(em, o, kWave));
+        }
 #pragma unroll
         for (int a = 0; a < 4; ++a) {
-            uint32_t hits[4][4], base[4];  // hits: the row's 16 lanes' ballot, per row e and block b
-            uint32_t any = 0;
+            uint32_t hits = 0;  // bit 4 e + b
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int il = 64 * wr + 16 * a + 4 * q4 + e;
-                const float ni = s_nh[il], kai = s_ka[il], Te = fmaf(s_T[il], kUp, s_eb[il]);
-                uint32_t tot = 0;
+                const float te = fmaf(s_T[il], kUp, s_eb[il]) + em;
+                const float hr = row0 + il < n
+                                     ? 0.5f * fmaf(-te * (1.0f + 0x1p-19f), te,
+                                                   s_nh[il] * (1.0f - 0x1p-19f) - s_ka[il] * am * kUp)
+                                     : INFINITY;
 #pragma unroll
-                for (int b = 0; b < 4; ++b) {
-                    const float sn = ni + nj[b];
-                    const float d = sn - 2.0f * acc[a][b][e];
-                    const float te = Te + ej[b];
-                    const float dm = fmaf(-kai, aj[b], fmaf(-0x1p-21f, sn, d));
-                    bool hit = !(dm > te * te);
-                    if (edge) {
-                        const uint32_t i = row0 + il, j = c0 + 64 * wc + 16 * b + r16;
-                        hit = hit && jv[b] && i < n && j != i;
-                    }
-                    const uint64_t m = __ballot(hit);
-                    const uint32_t half = lane & 32 ? (uint32_t)(m >> 32) : (uint32_t)m;
-                    hits[e][b] = (half >> (lane & 16)) & 0xFFFFu;
-                    tot += (uint32_t)__popc(hits[e][b]);
-                }
-                base[e] = 0;
-                if (r16 == 0 && tot) base[e] = atomicAdd(&s_cnt[il], tot);
-                any |= tot;
+                for (int b = 0; b < 4; ++b) hits |= acc[a][b][e] >= hr + hc[b] ? 1u << (4 * e + b) : 0u;
             }
-            if (!__ballot(any != 0u)) continue;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const uint32_t i = row0 + 64 * wr + 16 * a + 4 * q4 + e;
-                uint32_t at = row_first(base[e]);  // < kAffCap with the ranks below: kAffHold
-                uint2* list = cand + (lists + i) * kAffCap;
-#pragma unroll
-                for (int b = 0; b < 4; ++b) {
-                    if ((hits[e][b] >> r16) & 1u)
-                        list[at + (uint32_t)__popc(hits[e][b] & ((1u << r16) - 1u))] = make_uint2(
-                            c0 + 64 * wc + 16 * b + r16, __float_as_uint(acc[a][b][e]));
-                    at += (uint32_t)__popc(hits[e][b]);
-                }
+            // a lane's few hits, tested as the bounds have them and appended one at a time
+            while (hits) {
+                const uint32_t x = (uint32_t)__builtin_ctz(hits);
+                hits &= hits - 1;
+                const uint32_t e = x >> 2, b = x & 3u;
+                auto pick = [](f32x4 c, uint32_t x) {  // no memory: selects
+                    const float p = x & 1u ? c[1] : c[0], q = x & 1u ? c[3] : c[2];
+                    return x & 2u ? q : p;
+                };
+                const f32x4 v = {pick(acc[a][0], e), pick(acc[a][1], e), pick(acc[a][2], e),
+                                 pick(acc[a][3], e)};
+                const float gv = pick(v, b);
+                const uint32_t il = 64 * wr + 16 * a + 4 * q4 + e;
+                const uint32_t i = row0 + il, j = c0 + 64 * wc + 16 * b + r16;
+                const float sn = s_nh[il] + pick(nj, b);
+                const float te = fmaf(s_T[il], kUp, s_eb[il]) + pick(ej, b);
+                const float dm = fmaf(-s_ka[il], pick(aj, b), fmaf(-0x1p-21f, sn, sn - 2.0f * gv));
+                if (dm > te * te || (edge && j == i)) continue;
+                const uint32_t at = atomicAdd(&s_cnt[il], 1u);  // < kAffCap: at most kAffHold before
+                cand[(lists + i) * kAffCap + at] = make_uint2(j, __float_as_uint(gv));
             }
         }
         __syncthreads();
@@ -374,11 +388,13 @@ __global__ __launch_bounds__(kAffThreads) void k_aff_candidates(const _Float16* 
                 aff_load(cand + (lists + row0 + rn) * kAffCap, s_cnt[rn], row0 + rn, nx);
             aff_compact(cand + (lists + row0 + r) * kAffCap, P, dp, row0 + r, en, &s_cnt[r],
                         &s_T[r], &s_over[r], k);
+            if (lane == 0) atomicMin(thr + row0 + r, __float_as_uint(s_T[r]));
             r = rn;
 #pragma unroll
             for (int u = 0; u < kAffPer; ++u) en[u] = nx[u];
         }
         __syncthreads();
+        if (tid < kAffRows) s_T[tid] = fminf(s_T[tid], theirs);  // seen after the next barrier
     }
     // the lists as they stand (at most kAffHold entries each): the refinement merges and thins them
     if (tid < kAffRows && row0 + tid < n) {
@@ -627,10 +643,10 @@ void launch_aff_pack(hipStream_t s, const float* X, uint32_t n, uint32_t dim, fl
 }
 void launch_aff_candidates(hipStream_t s, const _Float16* Xh, const float* nh, const float* ah,
                            const float* eb, uint32_t n, uint32_t dim, uint32_t k, uint32_t splits,
-                           uint2* cand, uint32_t* ccount, uint32_t* overflow) {
+                           uint2* cand, uint32_t* ccount, uint32_t* thr, uint32_t* overflow) {
     const dim3 g(div_up_a(n, kAffRows), splits);
     k_aff_candidates<<<g, kAffThreads, 0, s>>>(Xh, nh, ah, eb, n, aff_dim_padded(dim), k, cand,
-                                               ccount, overflow);
+                                               ccount, thr, overflow);
 }
 void launch_aff_refine(hipStream_t s, const float* X, const float* nh, const float* ah,
                        const float* eb, uint32_t n, uint32_t dim, uint32_t k, uint32_t splits,

@@ -1274,7 +1274,7 @@ bh_status bh_tsne_affinities(bh_ctx* c, const float* X, uint32_t n, uint32_t dim
     uint2* cand = nullptr;
     float* dval = nullptr;
     _Float16* Xh = nullptr;
-    uint32_t *ccount = nullptr, *flags = nullptr, *idx = nullptr, *vals_a = nullptr,
+    uint32_t *ccount = nullptr, *thr = nullptr, *flags = nullptr, *idx = nullptr, *vals_a = nullptr,
              *vals_b = nullptr, *head = nullptr, *pos = nullptr, *spart = nullptr,
              *scratch = nullptr, *dcol = nullptr, *drp = nullptr;
     uint64_t *keys_a = nullptr, *keys_b = nullptr;
@@ -1296,6 +1296,7 @@ bh_status bh_tsne_affinities(bh_ctx* c, const float* X, uint32_t n, uint32_t dim
     part((void**)&eb, (size_t)n * 4);
     part((void**)&cand, (size_t)splits * n * cap * 8);
     part((void**)&ccount, (size_t)splits * n * 4);
+    part((void**)&thr, (size_t)n * 4);
     part((void**)&flags, 4 * 4);  // [0] rows over capacity, [1] sort error, [2] nnz, [3] max |x|
     part((void**)&idx, nk * 4);
     part((void**)&d2, nk * 8);
@@ -1351,7 +1352,8 @@ bh_status bh_tsne_affinities(bh_ctx* c, const float* X, uint32_t n, uint32_t dim
         if (st == BH_OK) {
             launch_fill_u32(s, flags, 4, 0u);
             launch_aff_pack(s, dX, n, dim, scale, Xh, nh, ah, eb);
-            launch_aff_candidates(s, Xh, nh, ah, eb, n, dim, k, splits, cand, ccount, flags);
+            launch_fill_u32(s, thr, n, 0x7F800000u);
+            launch_aff_candidates(s, Xh, nh, ah, eb, n, dim, k, splits, cand, ccount, thr, flags);
             launch_aff_refine(s, dX, nh, ah, eb, n, dim, k, splits, cand, ccount, idx, d2, flags);
             launch_aff_bandwidth(s, d2, n, k, std::log(perplexity), 1e-5, 200, P, dbeta);
             st = hip_check(c, hipMemcpyAsync(h_flags, flags, 4, hipMemcpyDeviceToHost, s), "flags");

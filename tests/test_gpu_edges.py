@@ -457,3 +457,25 @@ def test_leapfrog_steps_in_one_call(gpu, n):
     for other in out[1:]:
         assert all(np.array_equal(a, b) for a, b in zip(out[0], other))
     assert np.any(out[0][0] != x)
+
+
+@pytest.mark.parametrize("order", ["far_first", "near_first"])
+@pytest.mark.parametrize("n,dim,k", [(700, 64, 20), (3000, 33, 90)])
+def test_affinity_thresholds_edges(gpu, n, dim, k, order):
+    """Columns in order of distance, so that the first thresholds keep all or almost none of the
+    later ones, and one point of a thousand times the others' norm, which loosens the short test of
+    its columns: the exact neighbours against FP64 brute force, distances to 1e-12."""
+    rng = np.random.default_rng(n)
+    r = np.sort(rng.uniform(0.01, 1.0, n))[:, None]
+    if order == "far_first":
+        r = r[::-1]
+    X = (r * rng.normal(0, 1, (n, dim))).astype(np.float32)
+    X[n // 2] *= 1000.0
+    a = tsne.affinities(X, perplexity=k / 3.0, k=k)
+    d = X.astype(np.float64)
+    d2 = np.stack([((d - row) ** 2).sum(1) for row in d])
+    np.fill_diagonal(d2, np.inf)
+    want = np.sort(d2, axis=1)[:, :k]
+    assert np.allclose(a["d2"], want, rtol=1e-12, atol=0)
+    got = np.take_along_axis(d2, a["idx"].astype(np.int64), 1)
+    assert np.allclose(got, want, rtol=1e-12, atol=0)
