@@ -948,7 +948,9 @@ static inline uint32_t div_up(uint64_t a, uint64_t b) { return (uint32_t)((a + b
 //   uniform disk, 20,000 sinks (313 groups)    130 / 107 /  91 us
 //   t-SNE, 70,000 points (1,094 groups)        162 / 139 / 141 us compact, 141 / 117 / 111 spread
 //   two disks, 200,003 sinks (3,126 groups)    200 / 209 / 285 us; 1,048,576: 695 / 806 / 1215 us
-// so four waves while the groups alone leave SIMDs idle, two up to two groups per SIMD.
+// and beside the attraction of a t-SNE iteration, two or four waves, five iterations: 1470 / 1448 us
+// compact, 1500 / 1475 spread. So four waves while the groups alone leave SIMDs idle, and for an
+// eighth more, two up to two groups per SIMD.
 static uint32_t walk_waves_per_group(uint64_t groups) {
     static const uint64_t simds = [] {
         int dev = 0, cus = 0;
@@ -957,7 +959,7 @@ static uint32_t walk_waves_per_group(uint64_t groups) {
             cus = 0;
         return (uint64_t)cus * 4u;
     }();
-    return groups <= simds ? 4u : groups <= 2 * simds ? 2u : 1u;
+    return groups <= simds + simds / 8 ? 4u : groups <= 2 * simds ? 2u : 1u;
 }
 
 struct WalkCall {
