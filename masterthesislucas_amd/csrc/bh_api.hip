@@ -384,7 +384,13 @@ TraverseBatch batch_of(const bh_ctx* c) {
     return b;
 }
 
-bh_status do_fmm(bh_ctx* c, double theta, bool sum_later) {
+static void unsort_out(bh_ctx* c, CallerOut out) {
+    if (out.id)
+        launch_unsort2(c->stream, out.id, c->n, c->ax, c->ay, out.x ? out.x : c->out_a,
+                       out.y ? out.y : c->out_b);
+}
+
+bh_status do_fmm(bh_ctx* c, double theta, bool sum_later, CallerOut out) {
     if (!(theta > 0.0)) return fail(c, BH_ERR_ARG, "the FMM solver needs theta > 0");
     hipStream_t s = c->stream;
     phase_begin(c, 5);
@@ -394,6 +400,7 @@ bh_status do_fmm(bh_ctx* c, double theta, bool sum_later) {
     c->zpart = launch_fmm(s, c->pos4, keys, c->slot_b, c->slot_c, c->depth, c->slot_cap, c->n,
                           c->cfg.n_max, c->prm, theta, c->fmm_buf, c->ax, c->ay,
                           sum_later ? nullptr : c->dsum, &c->nzpart);
+    unsort_out(c, out);
     phase_end(c, 5);
     c->trav_blocks = 0;  // interaction counters are those of the tree walk only
     c->have_acc = true;
@@ -402,12 +409,12 @@ bh_status do_fmm(bh_ctx* c, double theta, bool sum_later) {
 
 // plugin: the call is bh_forces / bh_forces_device, whose t-SNE sums keep the pre-order walk's
 // summation order. sum_later: with want_total, the per-point terms in tot (FMM solver: the nzpart
-// partial sums at zpart) are left to the caller to add up
+// partial sums at zpart) are left to the caller to add up. out: the forces in the caller's order too
 bh_status do_forces(bh_ctx* c, double theta, bool want_total, bool plugin = false,
-                    bool sum_later = false) {
+                    bool sum_later = false, CallerOut out = CallerOut{}) {
     if (!c->built) return fail(c, BH_ERR_STATE, "forces requested before a tree was built");
     if (!(theta >= 0.0)) return fail(c, BH_ERR_ARG, "theta must be >= 0");
-    if (c->solver == BH_SOLVER_FMM_SYM) return do_fmm(c, theta, sum_later);
+    if (c->solver == BH_SOLVER_FMM_SYM) return do_fmm(c, theta, sum_later, out);
     bh_status mst = ensure_moments(c);
     if (mst != BH_OK) return mst;
     hipStream_t s = c->stream;
@@ -415,19 +422,21 @@ bh_status do_forces(bh_ctx* c, double theta, bool want_total, bool plugin = fals
     const float eps = c->cfg.softening;
     const bool grav = c->cfg.kernel == BH_KERNEL_GRAVITY;
     phase_begin(c, 5);
-    if (plugin && !grav && !c->nsys && c->split == 1 && c->n <= kPreorderMax)
+    if (plugin && !grav && !c->nsys && c->split == 1 && c->n <= kPreorderMax) {
         c->trav_blocks = launch_traverse_preorder(s, c->pos4, c->nodes, c->prm, c->n, inv_theta2,
                                                   c->ax, c->ay, want_total ? c->tot : nullptr,
                                                   c->counters);
-    else
+        unsort_out(c, out);
+    } else {
         c->trav_blocks = launch_traverse(s, grav ? kKernelGravity : kKernelTsne, c->pos4,
                                          c->nodes, c->child4, c->prm, c->n, inv_theta2, eps * eps,
                                          grav ? c->cfg.G : 1.0f, c->ax, c->ay,
                                          want_total ? c->tot : nullptr, c->counters, batch_of(c),
-                                         c->split);
+                                         c->split, out);
+    }
     if (c->nsys)
         launch_sum_heavy(s, c->side, c->side_cap, c->heavy, c->nheavy, c->ax, c->ay,
-                         want_total ? c->tot : nullptr);
+                         want_total ? c->tot : nullptr, out);
     phase_end(c, 5);
     if (want_total && !sum_later) launch_reduce_f64(s, c->tot, nullptr, c->n, c->red_part, c->dsum);
     c->have_acc = true;
@@ -801,22 +810,21 @@ bh_status bh_build(bh_ctx* c, const double* bounds) {
 static bh_status forces_out(bh_ctx* c, double theta, float* ax, float* ay, double* total,
                             bool device) {
     if (!c) return BH_ERR_ARG;
-    bh_status st = do_forces(c, theta, total != nullptr, true);
+    CallerOut out;
+    if (ax || ay) {
+        out.id = c->id[c->cur];
+        out.x = !ax ? nullptr : device ? ax : c->out_a;
+        out.y = !ay ? nullptr : device ? ay : c->out_b;
+    }
+    bh_status st = do_forces(c, theta, total != nullptr, true, false, out);
     if (st != BH_OK) return st;
     hipStream_t s = c->stream;
-    const uint32_t n = c->n;
-    const int cur = c->cur;
-    const size_t b = (size_t)n * sizeof(float);
-    if (ax || ay) {
-        if (device) {
-            launch_unsort2(s, c->id[cur], n, c->ax, c->ay, ax ? ax : c->out_a, ay ? ay : c->out_b);
-        } else {
-            launch_unsort2(s, c->id[cur], n, c->ax, c->ay, c->out_a, c->out_b);
-            if (ax) st = hip_check(c, hipMemcpyAsync(ax, c->out_a, b, hipMemcpyDeviceToHost, s), "ax");
-            if (st == BH_OK && ay)
-                st = hip_check(c, hipMemcpyAsync(ay, c->out_b, b, hipMemcpyDeviceToHost, s), "ay");
-            if (st != BH_OK) return st;
-        }
+    const size_t b = (size_t)c->n * sizeof(float);
+    if (!device) {
+        if (ax) st = hip_check(c, hipMemcpyAsync(ax, c->out_a, b, hipMemcpyDeviceToHost, s), "ax");
+        if (st == BH_OK && ay)
+            st = hip_check(c, hipMemcpyAsync(ay, c->out_b, b, hipMemcpyDeviceToHost, s), "ay");
+        if (st != BH_OK) return st;
     }
     if (total) {
         st = hip_check(c, hipMemcpyAsync(c->h_dsum, c->dsum, sizeof(double), hipMemcpyDeviceToHost, s),
@@ -2221,11 +2229,18 @@ bh_status bh_forces_learned(bh_ctx* c, const bh_mlp* m, double theta, double ban
     const float inv_t2 = (float)(1.0 / (theta * theta));
     const float inv_b2 = band > 0.0 ? (float)(1.0 / (band * band)) : 0.f;
     const float eps = c->cfg.softening;
+    CallerOut out;
+    if (ax || ay) {
+        out.id = c->id[c->cur];
+        out.x = ax ? c->out_a : nullptr;
+        out.y = ay ? c->out_b : nullptr;
+    }
     phase_begin(c, 5);  // the per-cell inference is part of the learned force evaluation
     launch_cell_coefs(s, c->lfeat, c->nodes, c->prm, c->cap_nodes, m->wbf, c->lcoef);
     c->trav_blocks = launch_traverse_learned(s, c->pos4, c->nodes, c->child4, c->lcoef, c->prm,
                                              c->n, inv_t2, inv_b2, eps * eps, c->cfg.G, m->terms,
-                                             c->ax, c->ay, total ? c->tot : nullptr, c->counters);
+                                             c->ax, c->ay, total ? c->tot : nullptr, c->counters,
+                                             out);
     phase_end(c, 5);
     if (total) launch_reduce_f64(s, c->tot, nullptr, c->n, c->red_part, c->dsum);
     c->have_acc = true;
@@ -2233,7 +2248,6 @@ bh_status bh_forces_learned(bh_ctx* c, const bh_mlp* m, double theta, double ban
     if (st != BH_OK) return st;
     const uint32_t n = c->n;
     if (ax || ay) {
-        launch_unsort2(s, c->id[c->cur], n, c->ax, c->ay, c->out_a, c->out_b);
         if (ax) st = hip_check(c, hipMemcpyAsync(ax, c->out_a, (size_t)n * 4, hipMemcpyDeviceToHost, s), "ax");
         if (st == BH_OK && ay) st = hip_check(c, hipMemcpyAsync(ay, c->out_b, (size_t)n * 4, hipMemcpyDeviceToHost, s), "ay");
     }

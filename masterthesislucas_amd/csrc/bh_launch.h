@@ -103,9 +103,15 @@ struct TraverseBatch {
     float* side = nullptr;    // 3 planes of side_slots x kHeavySlices x kHeavySinks
     uint32_t side_slots = 0;  // heavy slots `side` holds room for
 };
+// a second copy of a walk's forces in the caller's order (id: caller index of each sorted slot; null:
+// none; either array may be null)
+struct CallerOut {
+    const uint32_t* id = nullptr;
+    float *x = nullptr, *y = nullptr;
+};
 // sums the slices of each heavy entry (heavy: (first sink, count, F, -) per slot) into the outputs
 void launch_sum_heavy(hipStream_t s, const float* side, uint32_t side_slots, const uint4* heavy,
-                      uint32_t nheavy, float* ax, float* ay, float* tot);
+                      uint32_t nheavy, float* ax, float* ay, float* tot, CallerOut out);
 // Returns the number of blocks launched (a pair of interaction counts per wave). split: waves per
 // sink group (2: two, more: four; 1: chosen from the number of groups, one for batched systems);
 // results do not depend on it.
@@ -114,7 +120,7 @@ uint32_t launch_traverse(hipStream_t s, int kernel, const float4* pos4, const No
                          const uint32_t* child4, const BuildParams* prm, uint32_t n,
                          float inv_theta2, float eps2, float scale, float* ax, float* ay,
                          float* tot, unsigned long long* counters, TraverseBatch batch,
-                         uint32_t split);
+                         uint32_t split, CallerOut out);
 // the t-SNE solver plug-in's walk in its own summation order (one system of at most kPreorderMax
 // points)
 constexpr uint32_t kPreorderMax = 1u << 17;
@@ -230,7 +236,8 @@ uint32_t launch_traverse_learned(hipStream_t s, const float4* pos4, const Node* 
                                  const uint32_t* child4, const float4* coef,
                                  const BuildParams* prm, uint32_t n, float inv_theta2,
                                  float inv_band2, float eps2, float scale, int terms, float* ax,
-                                 float* ay, float* tot, unsigned long long* counters);
+                                 float* ay, float* tot, unsigned long long* counters,
+                                 CallerOut out);
 void launch_label_pairs(hipStream_t s, const float4* pos4, const Node* nodes, const float* feat,
                         const BuildParams* prm, const uint32_t* sinks, const uint32_t* pairs, const uint32_t* counts,
                         const uint32_t* offsets, uint32_t ns, uint32_t cap, double eps2, float* X,

@@ -77,6 +77,10 @@ __device__ __forceinline__ NodeBits load_node(const Node* __restrict__ nodes, ui
 // stays what it has always been. Telling such cells apart costs 0.5% of a walk without them; a
 // walk over one with 524,288 points 331 -> 258 ms.
 //
+// Results go to sorted order and, where the call returns them, to the caller's order too: the
+// scattered stores cost nothing beside the sums, a launch of their own 4 us at 2,000 sinks, 24 at
+// 1M and 168 at 4M.
+//
 // Bound by VALU issue (13 slots per interaction, the reciprocal square root counting as four)
 // where the waves fill the device, by the latency of the steps where they do not. Measured
 // against the former walk (one node per visit for 128 sinks, fetched with scalar loads one visit
@@ -169,7 +173,8 @@ __global__ __launch_bounds__(kBlock) void k_walk(const float4* __restrict__ pos4
                                                  float* __restrict__ ay_out,
                                                  float* __restrict__ tot_out,
                                                  unsigned long long* __restrict__ counters,
-                                                 TraverseBatch batch, LearnArgs la) {
+                                                 TraverseBatch batch, LearnArgs la,
+                                                 CallerOut out) {
     constexpr int kGroupWaves = kWalkParts / NP;  // waves per sink group
     static_assert(kWavesPerBlock % kGroupWaves == 0, "whole groups per block");
     __shared__ WalkLds lds[kWavesPerBlock];
@@ -578,9 +583,15 @@ __global__ __launch_bounds__(kBlock) void k_walk(const float4* __restrict__ pos4
             batch.side[plane + o] = scale * oy;
             if (TOT) batch.side[2 * plane + o] = scale * ot;
         } else {
-            ax_out[idx] = scale * ox;
-            ay_out[idx] = scale * oy;
+            const float sx = scale * ox, sy = scale * oy;
+            ax_out[idx] = sx;
+            ay_out[idx] = sy;
             if (TOT) tot_out[idx] = scale * ot;
+            if (out.id) {  // also in the caller's order, beside other waves' sums
+                const uint32_t o = out.id[idx];
+                if (out.x) out.x[o] = sx;
+                if (out.y) out.y[o] = sy;
+            }
         }
     }
     // one pair per wave (no same-address device atomics): the group's first wave counts for it,
@@ -975,6 +986,7 @@ struct WalkCall {
     TraverseBatch batch;
     LearnArgs la;
     uint32_t waves;  // per sink group: 1, 2 or 4
+    CallerOut out;
 };
 
 template <int KERNEL, bool TOT, bool BATCHED, int LTERMS>
@@ -984,7 +996,7 @@ static uint32_t walk_launch(const WalkCall& c) {
 #define BH_WALK(NP)                                                                               \
     k_walk<KERNEL, TOT, NP, BATCHED, LTERMS><<<g, kBlock, 0, c.s>>>(                              \
         c.pos4, c.nodes, c.child4, c.prm, c.n, c.inv_theta2, c.eps2, c.scale, c.ax, c.ay, c.tot,  \
-        c.counters, c.batch, c.la)
+        c.counters, c.batch, c.la, c.out)
     if (c.waves == 4) BH_WALK(1);
     else if (c.waves == 2) BH_WALK(2);
     else BH_WALK(4);
@@ -996,9 +1008,9 @@ uint32_t launch_traverse(hipStream_t s, int kernel, const float4* pos4, const No
                          const uint32_t* child4, const BuildParams* prm, uint32_t n,
                          float inv_theta2, float eps2, float scale, float* ax, float* ay,
                          float* tot, unsigned long long* counters, TraverseBatch batch,
-                         uint32_t split) {
+                         uint32_t split, CallerOut out) {
     WalkCall c{s, pos4, nodes, child4, prm, n, inv_theta2, eps2, scale, ax, ay, tot, counters,
-               batch, LearnArgs{}, 1u};
+               batch, LearnArgs{}, 1u, out};
     if (split > 1) c.waves = split == 2 ? 2u : 4u;
     else if (!batch.work) c.waves = walk_waves_per_group(div_up(n, kWave));
     const bool grav = kernel == kKernelGravity;
@@ -1031,9 +1043,10 @@ uint32_t launch_traverse_learned(hipStream_t s, const float4* pos4, const Node* 
                                  const uint32_t* child4, const float4* coef,
                                  const BuildParams* prm, uint32_t n, float inv_theta2,
                                  float inv_band2, float eps2, float scale, int terms, float* ax,
-                                 float* ay, float* tot, unsigned long long* counters) {
+                                 float* ay, float* tot, unsigned long long* counters,
+                                 CallerOut out) {
     WalkCall c{s, pos4, nodes, child4, prm, n, inv_theta2, eps2, scale, ax, ay, tot, counters,
-               TraverseBatch{}, LearnArgs{coef, inv_band2}, walk_waves_per_group(div_up(n, kWave))};
+               TraverseBatch{}, LearnArgs{coef, inv_band2}, walk_waves_per_group(div_up(n, kWave)), out};
     if (terms == 3)
         return tot ? walk_launch<kKernelGravity, true, false, 3>(c)
                    : walk_launch<kKernelGravity, false, false, 3>(c);
@@ -1048,7 +1061,7 @@ __global__ __launch_bounds__(kBlock) void k_sum_heavy(const float* __restrict__ 
                                                       const uint4* __restrict__ heavy,
                                                       float* __restrict__ ax,
                                                       float* __restrict__ ay,
-                                                      float* __restrict__ tot) {
+                                                      float* __restrict__ tot, CallerOut out) {
     const uint4 h = heavy[blockIdx.x];  // first sink, count, F
     const size_t plane = (size_t)side_slots * kHeavySlices * kHeavySinks;
     for (uint32_t i = threadIdx.x; i < h.y; i += kBlock) {
@@ -1062,12 +1075,17 @@ __global__ __launch_bounds__(kBlock) void k_sum_heavy(const float* __restrict__ 
         ax[h.x + i] = sx;
         ay[h.x + i] = sy;
         if (tot) tot[h.x + i] = st;
+        if (out.id) {
+            const uint32_t o = out.id[h.x + i];
+            if (out.x) out.x[o] = sx;
+            if (out.y) out.y[o] = sy;
+        }
     }
 }
 
 void launch_sum_heavy(hipStream_t s, const float* side, uint32_t side_slots, const uint4* heavy,
-                      uint32_t nheavy, float* ax, float* ay, float* tot) {
-    if (nheavy) k_sum_heavy<<<nheavy, kBlock, 0, s>>>(side, side_slots, heavy, ax, ay, tot);
+                      uint32_t nheavy, float* ax, float* ay, float* tot, CallerOut out) {
+    if (nheavy) k_sum_heavy<<<nheavy, kBlock, 0, s>>>(side, side_slots, heavy, ax, ay, tot, out);
 }
 
 uint32_t reduce_grid(uint32_t n) {

@@ -479,3 +479,32 @@ def test_affinity_thresholds_edges(gpu, n, dim, k, order):
     assert np.allclose(a["d2"], want, rtol=1e-12, atol=0)
     got = np.take_along_axis(d2, a["idx"].astype(np.int64), 1)
     assert np.allclose(got, want, rtol=1e-12, atol=0)
+
+
+@pytest.mark.parametrize("kernel,n", [("gravity", 1), ("gravity", 64), ("gravity", 65),
+                                      ("gravity", 20_001), ("gravity", 150_001), ("tsne", 300),
+                                      ("tsne", 140_001)])
+def test_forces_in_callers_order(gpu, kernel, n):
+    """The walk (1, 2 and 4 parts per wave) and the pre-order walk store the forces in the caller's
+    order: host and device outputs, both or one of them, are the same to the bit."""
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(n)
+    x, y = rng.normal(0, 1, (2, n)).astype(np.float32)
+    ctx = BHContext(n, kernel=kernel, softening=0.01)
+    ctx.set_particles(x, y)
+    ctx.build()
+    ax, ay, _ = ctx.forces(0.5)
+    _, perm = ctx.morton()
+    for gx, gy in ((True, True), (True, False), (False, True)):
+        dx, dy = (torch.full((n,), 7.0, device="cuda") for _ in range(2))
+        torch.cuda.synchronize()
+        ctx.forces_device(0.5, dx if gx else None, dy if gy else None)
+        torch.cuda.synchronize()
+        assert np.array_equal(dx.cpu().numpy(), ax if gx else np.full(n, 7.0, np.float32))
+        assert np.array_equal(dy.cpu().numpy(), ay if gy else np.full(n, 7.0, np.float32))
+    # another input order, the same tree: the same forces at the same points
+    ctx.set_particles(x[perm], y[perm])
+    ctx.build()
+    bx, by, _ = ctx.forces(0.5)
+    ctx.close()
+    assert np.array_equal(bx, ax[perm]) and np.array_equal(by, ay[perm])
