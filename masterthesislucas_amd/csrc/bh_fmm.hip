@@ -377,7 +377,7 @@ __device__ __forceinline__ uint32_t wave_sum_u32(uint32_t v) {
 }
 
 // The last leaf lo with unit_off[lo] <= u: 64 entries per step, one per lane (3 dependent loads
-// for 65,536 leaves instead of 16).
+// for 16,384 leaves instead of 16).
 __device__ __forceinline__ uint32_t fmm_unit_leaf(const uint32_t* __restrict__ unit_off, uint32_t L,
                                                   uint32_t u) {
     const uint32_t lane = threadIdx.x & 63;
@@ -556,7 +556,7 @@ __device__ __forceinline__ void fmm_partners_meta(const uint32_t* __restrict__ f
 
 // exclusive scans of the per-leaf unit counts of the three unit classes (light, heavy,
 // expansion: units + c * unit_stride, unit_stride a multiple of 4) in place; entry L of each =
-// its total (one block per class: one block for all three took 15 us for 65,536 leaves, now 6). Each thread sums a contiguous run of entries (a multiple of 16, read
+// its total (one block per class: one block for all three took 15 us for 16,384 leaves, now 6). Each thread sums a contiguous run of entries (a multiple of 16, read
 // as uint4, four loads in flight), the run totals are scanned over the block, and the runs are
 // rewritten with their offsets.
 constexpr int kFmmScanArrays = 3;
