@@ -508,3 +508,32 @@ def test_forces_in_callers_order(gpu, kernel, n):
     bx, by, _ = ctx.forces(0.5)
     ctx.close()
     assert np.array_equal(bx, ax[perm]) and np.array_equal(by, ay[perm])
+
+
+@pytest.mark.parametrize("sizes", [[1] * 256, [255, 1, 256, 257, 1, 1, 510, 2, 3],
+                                   [300] + [2] * 120 + [1, 5, 1000, 31], [1024, 256, 256, 1]])
+def test_batched_system_boundaries(gpu, sizes):
+    """Many systems in one block of 256 particles, systems that start and end at a block's edge:
+    every particle is in its own system. theta = 0 sums every pair: FP32 sums of at most 1000
+    terms, a few times 6e-8 each, against FP64 direct sums."""
+    rng = np.random.default_rng(len(sizes))
+    n = sum(sizes)
+    x, y = rng.normal(0, 1, (2, n)).astype(np.float32)
+    m = rng.uniform(0.5, 1.5, n).astype(np.float32)
+    ctx = BHContext(n, kernel="gravity", softening=0.01, sizes=sizes)
+    ctx.set_particles(x, y, m)
+    ctx.build()
+    ax, ay, _ = ctx.forces(0.0)
+    ctx.close()
+    wx, wy, scale = np.zeros(n), np.zeros(n), np.zeros(n)
+    o = 0
+    for k in sizes:
+        s = slice(o, o + k)
+        dx = x[s].astype(np.float64)[None, :] - x[s].astype(np.float64)[:, None]
+        dy = y[s].astype(np.float64)[None, :] - y[s].astype(np.float64)[:, None]
+        w = m[s].astype(np.float64) / (dx * dx + dy * dy + float(np.float32(0.01)) ** 2) ** 1.5
+        wx[s], wy[s] = (w * dx).sum(1), (w * dy).sum(1)
+        scale[s] = (w * np.hypot(dx, dy)).sum(1)
+        o += k
+    assert np.all(np.abs(ax - wx) <= 2e-5 * scale)
+    assert np.all(np.abs(ay - wy) <= 2e-5 * scale)
