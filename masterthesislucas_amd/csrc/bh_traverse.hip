@@ -85,11 +85,11 @@ __device__ __forceinline__ NodeBits load_node(const Node* __restrict__ nodes, ui
 // where the waves fill the device, by the latency of the steps where they do not. Measured
 // against the former walk (one node per visit for 128 sinks, fetched with scalar loads one visit
 // ahead; every lane tested every node):
-//   two disks, theta 0.5, 1,048,576 sinks    851 -> 695 us (VALU issue 92% busy in both)
+//   two disks, theta 0.5, 1,048,576 sinks    851 -> 654 us
 //                            200,003 sinks   424 -> 200 us
 //   uniform disk, 2,000 sinks                125 ->  55 us
 //   t-SNE, 70,000 points                     268 (spread) / 325 (compact) -> 110 / 140 us
-//   128 systems of 1,024 to 65,536           1080 -> 830 us
+//   128 systems of 1,024 to 65,536           1080 -> 778 us
 // ------------------------------------------------------------------------------------------
 constexpr int kWalkParts = 4;
 constexpr int kWalkStack = 192;              // opened cells
@@ -163,8 +163,9 @@ struct LearnArgs {
     float inv_band2 = 0.f;
 };
 
-template <int KERNEL, bool TOT, int NP, bool BATCHED, int LTERMS = 0>
-__global__ __launch_bounds__(kBlock) void k_walk(const float4* __restrict__ pos4,
+// RES: waves per SIMD that the registers must allow (walk_resident)
+template <int KERNEL, bool TOT, int NP, bool BATCHED, int LTERMS, int RES>
+__global__ __launch_bounds__(kBlock, RES) void k_walk(const float4* __restrict__ pos4,
                                                  const Node* __restrict__ nodes,
                                                  const uint32_t* __restrict__ child4,
                                                  const BuildParams* __restrict__ prm, uint32_t n,
@@ -958,11 +959,11 @@ static inline uint32_t div_up(uint64_t a, uint64_t b) { return (uint32_t)((a + b
 // Waves per sink group, results do not depend on it. Measured with 1 / 2 / 4 waves:
 //   uniform disk, 20,000 sinks (313 groups)    130 / 107 /  91 us
 //   t-SNE, 70,000 points (1,094 groups)        162 / 139 / 141 us compact, 141 / 117 / 111 spread
-//   two disks, 200,003 sinks (3,126 groups)    200 / 209 / 285 us; 1,048,576: 695 / 806 / 1215 us
+//   two disks, 200,003 sinks (3,126 groups)    200 / 209 / 285 us; 1,048,576: 654 / 806 / 1215 us
 // and beside the attraction of a t-SNE iteration, two or four waves, five iterations: 1470 / 1448 us
 // compact, 1500 / 1475 spread. So four waves while the groups alone leave SIMDs idle, and for an
 // eighth more, two up to two groups per SIMD.
-static uint32_t walk_waves_per_group(uint64_t groups) {
+static uint64_t walk_simds() {
     static const uint64_t simds = [] {
         int dev = 0, cus = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
@@ -970,7 +971,28 @@ static uint32_t walk_waves_per_group(uint64_t groups) {
             cus = 0;
         return (uint64_t)cus * 4u;
     }();
+    return simds;
+}
+
+static uint32_t walk_waves_per_group(uint64_t groups) {
+    const uint64_t simds = walk_simds();
     return groups <= simds + simds / 8 ? 4u : groups <= 2 * simds ? 2u : 1u;
+}
+
+// One wave per group: left to itself the compiler takes 88 to 105 registers, five (gravity with
+// totals: four) waves per SIMD. Launches that bring more groups than that run a build held to the
+// registers of six or seven resident waves: a few values go through scratch, and the added waves
+// hide the loads and LDS reads. Where fewer groups come, the spills cost and nothing is gained.
+// Compiler's own / six / seven / eight, theta 0.5, us:
+//   two disks,   200,000 sinks  217 /  221 /  232 /  283      with totals  237 /  261 /  357
+//              1,048,576        663 /  627 /  635 /  746                   790 /  728 / 1000
+//              4,194,304       2381 / 2212 / 2195 / 2634
+//   t-SNE,       400,000        284 /  265 /  248 /  263                   321 /  314 /  293
+//   64 systems (2.9M sinks)    1242 / 1156 / 1099 / 1675                  1511 / 1344 / 1870
+//   learned,   4,194,304       2636 / 2524 / 2522 / 2735
+constexpr uint64_t kWalkResident = 5;
+static constexpr int walk_resident(int kernel, bool tot, bool batched) {
+    return kernel == kKernelTsne || (batched && !tot) ? 7 : 6;
 }
 
 struct WalkCall {
@@ -993,13 +1015,14 @@ template <int KERNEL, bool TOT, bool BATCHED, int LTERMS>
 static uint32_t walk_launch(const WalkCall& c) {
     const uint64_t groups = BATCHED ? c.batch.n_work : div_up(c.n, kWave);
     const uint32_t g = div_up(groups * c.waves, kWavesPerBlock);
-#define BH_WALK(NP)                                                                               \
-    k_walk<KERNEL, TOT, NP, BATCHED, LTERMS><<<g, kBlock, 0, c.s>>>(                              \
+#define BH_WALK(NP, RES)                                                                          \
+    k_walk<KERNEL, TOT, NP, BATCHED, LTERMS, RES><<<g, kBlock, 0, c.s>>>(                         \
         c.pos4, c.nodes, c.child4, c.prm, c.n, c.inv_theta2, c.eps2, c.scale, c.ax, c.ay, c.tot,  \
         c.counters, c.batch, c.la, c.out)
-    if (c.waves == 4) BH_WALK(1);
-    else if (c.waves == 2) BH_WALK(2);
-    else BH_WALK(4);
+    if (c.waves == 4) BH_WALK(1, 1);
+    else if (c.waves == 2) BH_WALK(2, 1);
+    else if (groups <= kWalkResident * walk_simds()) BH_WALK(4, 1);
+    else BH_WALK(4, walk_resident(KERNEL, TOT, BATCHED));
 #undef BH_WALK
     return g;
 }

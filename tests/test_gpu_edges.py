@@ -537,3 +537,28 @@ def test_batched_system_boundaries(gpu, sizes):
         o += k
     assert np.all(np.abs(ax - wx) <= 2e-5 * scale)
     assert np.all(np.abs(ay - wy) <= 2e-5 * scale)
+
+
+@pytest.mark.parametrize("n", [5 * 1024 * 64, 5 * 1024 * 64 + 1, 400_003])
+@pytest.mark.parametrize("kernel,batched", [("gravity", False), ("gravity", True), ("tsne", False),
+                                            ("tsne", True)])
+def test_walk_resident_builds(gpu, kernel, batched, n):
+    """Up to and past five sink groups per SIMD, where launches change to the walk held to fewer
+    registers: the parts of a sink's sum are fixed, so forces, totals and counts equal those of two and
+    four waves per group (always the other build) to the bit."""
+    rng = np.random.default_rng(n)
+    x, y = rng.normal(0, 1, (2, n)).astype(np.float32)
+    kw = dict(sizes=[n // 3, 1, n - n // 3 - 1]) if batched else {}
+    ctx = BHContext(n, kernel=kernel, softening=0.01, **kw)
+    ctx.set_particles(x, y)
+    ctx.build()
+    for total in (False, True):
+        got = []
+        for split in (1, 2, 4):
+            ctx.set_split(split)
+            ax, ay, tot = ctx.forces(0.8, want_total=total)
+            got.append((ax, ay, (tot, ctx.counters())))
+        for ax, ay, rest in got[1:]:
+            assert rest == got[0][2]
+            assert np.array_equal(ax, got[0][0]) and np.array_equal(ay, got[0][1])
+    ctx.close()
