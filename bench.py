@@ -4,7 +4,7 @@
 Workload: two Plummer disks (scale radius 0.1, 524,288 particles each) centred at (+-0.5, 0) on
 counter-rotating circular orbits, N = 1,048,576 FP32 particles, G = 1, Plummer softening 1e-3,
 QuadTree tree (leaf capacity 16), theta = 0.5, kick-drift-kick leapfrog with dt = 1e-4. One
-step = bounds, Morton codes, radix sort, gather, tree build, upward pass, traversal and the
+step = bounds, Morton codes, sort, gather, tree build, upward pass, traversal and the
 leapfrog update, with the particle state resident in HBM. Metric: force evaluations per second
 (particles x steps / wall time).
 
@@ -813,7 +813,7 @@ def main():
         "walk_priority": ctx.priority,
         "autotune_ms": tuning,
         "phase_ms_per_step": {k: v[0] / args.steps for k, v in phases.items()},
-        "roofline": {"bound": "valu", "pipe": "FP32 VALU (traversal)", "kernel": "k_traverse",
+        "roofline": {"bound": "valu", "pipe": "FP32 VALU (traversal)", "kernel": "k_walk",
                      "achieved": achieved, "peak": PEAK_FP32_TFLOPS, "unit": "TFLOP/s",
                      "frac": achieved / PEAK_FP32_TFLOPS, "traffic": None,
                      # packed FP32 is off in this build: the issue-limited VALU peak is half

@@ -1,5 +1,5 @@
 // Tree build of the Barnes-Hut force step on gfx950:
-//   bounds -> Morton codes -> LDS-staged LSD radix sort -> gather into sorted SoA ->
+//   bounds -> Morton codes -> sort -> gather into sorted SoA ->
 //   leaf levels -> node count scan -> pre-order node emission -> upward mass/COM/M2 pass.
 //
 // The tree is laid out in pre-order over Morton-sorted particles: every node covers a

@@ -556,9 +556,9 @@ __device__ __forceinline__ void fmm_partners_meta(const uint32_t* __restrict__ f
 
 // exclusive scans of the per-leaf unit counts of the three unit classes (light, heavy,
 // expansion: units + c * unit_stride, unit_stride a multiple of 4) in place; entry L of each =
-// its total (one block per class: one block for all three took 15 us for 16,384 leaves, now 6). Each thread sums a contiguous run of entries (a multiple of 16, read
-// as uint4, four loads in flight), the run totals are scanned over the block, and the runs are
-// rewritten with their offsets.
+// its total (one block per class: one block for all three took 15 us for 16,384 leaves, now 6).
+// Each thread sums a contiguous run of entries (a multiple of 16, read as uint4, four loads in
+// flight), the run totals are scanned over the block, and the runs are rewritten with their offsets.
 constexpr int kFmmScanArrays = 3;
 
 __device__ __forceinline__ uint4 fmm_load4(const uint32_t* __restrict__ u, uint32_t i, uint32_t L) {
