@@ -648,11 +648,14 @@ struct FmmFlat {
             on &= on - 1;
             const uint32_t o = (uint32_t)__builtin_amdgcn_readlane((int)off, (int)e);
             const uint32_t last = (uint32_t)__builtin_amdgcn_readlane((int)m, (int)e) - 1u;
-            if (blk + lane >= o) {
-                src = (uint32_t)__builtin_amdgcn_readlane((int)a, (int)e) +
-                      F * min(blk + lane - o, last);
-                who = e;
-            }
+            // read and computed for every lane, then selected: a lane outside a branch need not hold
+            // its value inside, and an expression inside the selection is hoisted by the compiler
+            // with the selection's condition taken for granted
+            const uint32_t point = (uint32_t)__builtin_amdgcn_readlane((int)a, (int)e) +
+                                   F * min(blk + lane - o, last);
+            const bool in = blk + lane >= o;
+            src = in ? point : src;
+            who = in ? e : who;
         }
         return src;
     }

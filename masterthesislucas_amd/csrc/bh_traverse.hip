@@ -107,6 +107,9 @@ struct __attribute__((aligned(16))) WalkLds {  // per wave
     uint2 mask[kWalkStack];
     uint32_t node[kWalkStack];
 };
+struct WalkLdsLearned : WalkLds {
+    uint2 slot[kWave];  // the step's cells: node, l2 / band2
+};
 
 __device__ __forceinline__ void wave_lds_sync() {  // LDS of this wave only: order, no wait
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -178,13 +181,14 @@ __global__ __launch_bounds__(kBlock, RES) void k_walk(const float4* __restrict__
                                                  CallerOut out) {
     constexpr int kGroupWaves = kWalkParts / NP;  // waves per sink group
     static_assert(kWavesPerBlock % kGroupWaves == 0, "whole groups per block");
-    __shared__ WalkLds lds[kWavesPerBlock];
+    using Lds = std::conditional_t<LTERMS != 0, WalkLdsLearned, WalkLds>;
+    __shared__ Lds lds[kWavesPerBlock];
     const uint32_t lane = threadIdx.x & 63;
     // wave-uniform (the compiler cannot tell that threadIdx.x / 64 is)
     const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t p0 = (w % kGroupWaves) * NP;  // first part of this wave
     const uint32_t group = blockIdx.x * (kWavesPerBlock / kGroupWaves) + w / kGroupWaves;
-    WalkLds& L = lds[w];
+    Lds& L = lds[w];
     const uint64_t lt = lane_mask_lt();
 
     uint32_t base = group * kWave, count, k0 = 0, slice = 0;
@@ -272,9 +276,11 @@ __global__ __launch_bounds__(kBlock, RES) void k_walk(const float4* __restrict__
                         const uint32_t e = (uint32_t)__builtin_ctzll(m);
                         m &= m - 1;
                         const uint32_t o = lane_read(off, e);
-                        if (blk + lane >= o)
-                            src = lane_read(cell.x, e) +
-                                  min(blk + lane - o, lane_read(cell.y, e) - 1u);
+                        // (computed for every lane: an expression inside the selection is hoisted
+                        // by the compiler with the selection's condition taken for granted)
+                        const uint32_t at = lane_read(cell.x, e) +
+                                            min(blk + lane - o, lane_read(cell.y, e) - 1u);
+                        src = blk + lane >= o ? at : src;
                     }
                     return pos4[src];
                 };
@@ -383,18 +389,21 @@ __global__ __launch_bounds__(kBlock, RES) void k_walk(const float4* __restrict__
         nc = 0;
     };
 
-    // one accepted cell (staged at slot e) for the calling lanes
     uint32_t id = kNone;
-    float l2 = 0.f;
+    // one accepted cell (staged at slot e) for the calling lanes. Its index and limit come from LDS
+    // like its record: the slot's own lane need not be among the callers, and a value read from a
+    // lane outside a branch survives a spill or a copy made inside it only by chance. (Both read
+    // by v_readlane before the branch: 2.55 -> 2.67 ms for the walk of 4,194,304 sinks.)
     auto cell_pair = [&](WalkSum<TOT>& s, const float4 q, uint32_t e) {
         const float dx = q.x - px, dy = q.y - py;
-        walk_pair<KERNEL, TOT>(s, dx, dy, q.z, eps2);
-        if constexpr (LTERMS != 0) {
+        if constexpr (LTERMS == 0) {
+            walk_pair<KERNEL, TOT>(s, dx, dy, q.z, eps2);
+        } else {
+            const uint2 sn = L.slot[e];
+            walk_pair<KERNEL, TOT>(s, dx, dy, q.z, eps2);
             const float d2 = fmaf(dx, dx, dy * dy);
-            const bool corr = la.inv_band2 == 0.f ||
-                              !(d2 > __uint_as_float(lane_read(__float_as_uint(l2), e)) *
-                                         la.inv_band2);
-            const float4* cr = la.coef + (size_t)lane_read(id, e) * (kCoefStride / 4);
+            const bool corr = la.inv_band2 == 0.f || !(d2 > __uint_as_float(sn.y));
+            const float4* cr = la.coef + (size_t)uniform_u32(sn.x) * (kCoefStride / 4);
             const float4 c0 = cr[0], c1 = cr[1], c2 = cr[2], c3 = cr[3];
             if (corr) {
                 const float rec[kCoefStride] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w,
@@ -426,6 +435,8 @@ __global__ __launch_bounds__(kBlock, RES) void k_walk(const float4* __restrict__
         const bool open_all = live && !acc_all && fmaf(fx, fx, fy * fy) <= lim;
         wave_lds_sync();
         L.rec[lane] = make_float4(nd.cx(), nd.cy(), nd.mass(), lim);
+        if constexpr (LTERMS != 0)
+            L.slot[lane] = make_uint2(id, __float_as_uint(nd.l2() * la.inv_band2));
         wave_lds_sync();
         uint32_t olo = open_all ? mlo : 0u, ohi = open_all ? mhi : 0u;  // lanes that open it
         uint64_t xm = __ballot(live && !acc_all && !open_all);
@@ -445,7 +456,6 @@ __global__ __launch_bounds__(kBlock, RES) void k_walk(const float4* __restrict__
         const bool all = live && alo == (uint32_t)full && ahi == (uint32_t)(full >> 32);
         uint64_t am = __ballot(all), mm = __ballot(live && !all && (alo | ahi) != 0u);
         n_pn += (uint32_t)__popc(alo) + (uint32_t)__popc(ahi);
-        if constexpr (LTERMS != 0) l2 = nd.l2();
         // particle-particle cells wait, opened cells go on the stack
         const uint64_t cm = __ballot(opened && is_pp), pm = __ballot(opened && !is_pp);
         if (opened && is_pp) {
