@@ -1976,7 +1976,7 @@ bh_status bh_mlp_forward(bh_mlp* m, const float* X, uint32_t n, float* Y, int bf
 static bh_status mlp_grad_device(bh_mlp* m, const float* dX, const float* dT, const uint32_t* order,
                                  uint32_t B) {
     bh_status st = ensure_m(m, &m->partials, &m->part_cap, (size_t)mlp_grad_chunks(B) * kMlpParams);
-    if (st == BH_OK) st = ensure_m(m, &m->loss_part, &m->loss_cap, mlp_loss_blocks(B));
+    if (st == BH_OK) st = ensure_m(m, &m->loss_part, &m->loss_cap, mlp_grad_chunks(B));
     if (st != BH_OK) return st;
     launch_mlp_grad(m->stream, dX, dT, order, B, m->params, m->loss_part, m->partials, m->terms);
     return mcheck(m, hipGetLastError(), "gradient");

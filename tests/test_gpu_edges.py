@@ -562,3 +562,29 @@ def test_walk_resident_builds(gpu, kernel, batched, n):
             assert rest == got[0][2]
             assert np.array_equal(ax, got[0][0]) and np.array_equal(ay, got[0][1])
     ctx.close()
+
+
+def test_training_gradient_of_many_samples(gpu):
+    """The gradient of a batch of 4 million: a block's sums stay at 1,024 samples however many there
+    are. All samples equal, so that a sum's roundings add up: a plain sum of m equal terms is off by at
+    most m / 2 x 2^-24, so 1,024 samples, 4,096 / 16 partials and 16 sums of those by 3.9e-5; 1e-6 for
+    the FP32 terms themselves."""
+    n = 1 << 22
+    rng = np.random.default_rng(5)
+    p = {"W1": rng.normal(0, 0.4, (10, 64)), "b1": rng.normal(0, 0.1, 64),
+         "W2": rng.normal(0, 0.15, (64, 64)), "b2": rng.normal(0, 0.1, 64),
+         "W3": rng.normal(0, 0.15, (64, N_OUT)), "b3": rng.normal(0, 0.1, N_OUT)}
+    p = {k: v.astype(np.float32) for k, v in p.items()}
+    X = rng.normal(0, 1, (1, 13)).astype(np.float32)
+    X[:, 10:] = (0.6, 0.8, 0.5)
+    T = rng.normal(0, 0.5, (1, 2)).astype(np.float32)
+    net = FarFieldMLP(max_samples=16)
+    net.set_params(flatten(p))
+    loss, g = net.loss_grad(np.tile(X, (n, 1)), np.tile(T, (n, 1)))
+    net.close()
+    ref_loss, ref = O.learned_loss_grad(X.astype(np.float64), T.astype(np.float64),
+                                        {k: v.astype(np.float64) for k, v in p.items()}, terms=7)
+    assert abs(loss - ref_loss) < 1e-5 * ref_loss
+    g = unflatten(g)
+    for k in ref:
+        assert np.abs(g[k] - ref[k]).max() <= 4e-5 * np.abs(ref[k]).max(), k
