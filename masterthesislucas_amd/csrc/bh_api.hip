@@ -13,6 +13,7 @@
 #include "bh_common.h"
 #include "bh_launch.h"
 #include "bh_mlp.h"
+#include "bh_order.h"
 
 using namespace bh;
 
@@ -136,6 +137,7 @@ struct bh_ctx {
     uint4* work = nullptr;          // traversal work table, one entry per wave
     uint32_t n_work = 0;
     std::vector<uint4> h_work0;     // the table as built (system order, no heavy slices)
+    std::vector<uint32_t> h_entry;  // per wave of `work`: its entry in h_work0
     uint4* heavy = nullptr;         // (first sink, count, slices) of its heavy slots
     uint32_t nheavy = 0;
     float* side = nullptr;          // partial results of heavy slices (TraverseBatch::side)
@@ -725,6 +727,8 @@ bh_status bh_create_batched(bh_ctx** out, const bh_config* cfg, const uint32_t* 
                                      hipMemcpyHostToDevice, s), "work"));
     TRYB(hip_check(c, hipStreamSynchronize(s), "work"));
     c->h_work0 = std::move(wk);
+    c->h_entry.resize(c->n_work);
+    for (uint32_t e = 0; e < c->n_work; ++e) c->h_entry[e] = e;
 #undef TRYB
     return hip_check(c, hipStreamSynchronize(s), "batched init");
 }
@@ -1669,14 +1673,18 @@ static bh_status upload_work(bh_ctx* c, const std::vector<uint32_t>& order, uint
         c->side_cap = nh;
     }
     std::vector<uint4> out, hv(nh);
+    std::vector<uint32_t> entry;
     out.reserve(w0.size() + (size_t)nh * (kHeavySlices - 1));
+    entry.reserve(out.capacity());
     for (uint32_t h = 0; h < nh; ++h) {
         const uint4 e = w0[order[h]];
         hv[h] = make_uint4(e.x, e.y, kHeavySlices, 0u);
         for (uint32_t f = 0; f < kHeavySlices; ++f)
             out.push_back(make_uint4(e.x, e.y, e.z, (h << 8) | (kHeavySlices << 4) | f));
+        entry.insert(entry.end(), kHeavySlices, order[h]);
     }
     for (size_t i = nh; i < order.size(); ++i) out.push_back(w0[order[i]]);
+    entry.insert(entry.end(), order.begin() + nh, order.end());
     bh_status st = hip_check(c, hipMemcpyAsync(c->work, out.data(), out.size() * sizeof(uint4),
                                                hipMemcpyHostToDevice, c->stream), "work");
     if (st == BH_OK && nh)
@@ -1685,6 +1693,7 @@ static bh_status upload_work(bh_ctx* c, const std::vector<uint32_t>& order, uint
     if (st == BH_OK) st = hip_check(c, hipStreamSynchronize(c->stream), "work table");
     if (st != BH_OK) return st;
     c->n_work = (uint32_t)out.size();
+    c->h_entry = std::move(entry);
     c->nheavy = nh;
     c->g_valid = false;  // captured steps hold the old grid
     return BH_OK;
@@ -1698,40 +1707,17 @@ bh_status bh_batch_order_by_cost(bh_ctx* c) {
     const uint32_t nw = c->n_work, nb = (nw + kWavesPerBlock - 1) / kWavesPerBlock;
     if (c->trav_blocks != nb)
         return fail(c, BH_ERR_STATE, "the last walk used another work table");
-    std::vector<unsigned long long> cnt(2ull * nw);  // per wave: entry e's pair
-    std::vector<uint4> wk(nw);
-    bh_status st = hip_check(c, hipMemcpyAsync(cnt.data(), c->counters, cnt.size() * 8,
+    bh_status st = hip_check(c, hipMemcpyAsync(c->h_counters, c->counters, 16ull * nw,
                                                hipMemcpyDeviceToHost, c->stream), "counters");
-    if (st == BH_OK)
-        st = hip_check(c, hipMemcpyAsync(wk.data(), c->work, (size_t)nw * sizeof(uint4),
-                                         hipMemcpyDeviceToHost, c->stream), "work");
     if (st == BH_OK) st = hip_check(c, hipStreamSynchronize(c->stream), "order by cost");
     if (st != BH_OK) return st;
-    // cost of each original entry: its wave's interactions in the last walk (a heavy entry's
-    // slices add up; entries are identified by their first sink) per sink: the wave's walk is
-    // shared by its lanes, so its time does not follow the entry's sink count
     const std::vector<uint4>& w0 = c->h_work0;
-    std::vector<std::pair<uint32_t, uint32_t>> by_first(w0.size());
-    for (uint32_t i = 0; i < w0.size(); ++i) by_first[i] = {w0[i].x, i};
-    std::sort(by_first.begin(), by_first.end());
-    std::vector<unsigned long long> cost(w0.size(), 0ull);
-    for (uint32_t e = 0; e < nw; ++e) {
-        const auto it = std::lower_bound(by_first.begin(), by_first.end(),
-                                         std::make_pair(wk[e].x, 0u));
-        if (it == by_first.end() || it->first != wk[e].x) continue;
-        cost[it->second] += cnt[2 * e] + cnt[2 * e + 1];
-    }
-    for (uint32_t i = 0; i < w0.size(); ++i)
-        if (w0[i].y) cost[i] /= w0[i].y;
-    std::vector<std::pair<unsigned long long, uint32_t>> ord(w0.size());  // (~cost, entry)
+    std::vector<unsigned long long> cost;
+    std::vector<uint32_t> order;
+    order_by_cost(c->h_counters, c->h_entry.data(), nw, w0.size(),
+                  [&](size_t e) { return w0[e].y; }, cost, order);
     unsigned long long total = 0;
-    for (uint32_t i = 0; i < w0.size(); ++i) {
-        ord[i] = {~cost[i], i};
-        total += cost[i];
-    }
-    std::sort(ord.begin(), ord.end());  // descending cost, ties by entry
-    std::vector<uint32_t> order(w0.size());
-    for (uint32_t i = 0; i < w0.size(); ++i) order[i] = ord[i].second;
+    for (unsigned long long v : cost) total += v;
     // heavy: the costliest entries, at least kHeavyFactor times the mean, at most kHeavyMax of
     // them (the 256-system workload: a few thousand entries whose sinks sit under one-child
     // chains of thousands of occupants, 15-50 times the mean cost, 4-17 ms each of a 17 ms walk
