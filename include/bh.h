@@ -212,7 +212,10 @@ bh_status bh_tsne_run(bh_ctx* ctx, const bh_tsne_params* p, int32_t first, int32
  * Matrix Market file (tsne.h:94-98, setupEfficientPmatrix tsne.h:462-520). Optional outputs:
  * knn_idx[n x k], knn_d2[n x k] (ascending), beta[n]. 1 <= k <= 128, k < n. Returns
  * BH_ERR_CAPACITY when some point has more than 192 candidates within the FP16 error bound of
- * its k-th neighbour (hundreds of exact or near duplicates). */
+ * its k-th neighbour (hundreds of exact or near duplicates).
+ * The call's workspace (about 6 bytes per coordinate, 4 to 16 KB per point for candidates and 108
+ * bytes per neighbour) stays with the context for the next call if it is at most 1 GiB, until
+ * bh_tsne_set_p or bh_destroy gives it back; a larger one is freed before the call returns. */
 bh_status bh_tsne_affinities(bh_ctx* ctx, const float* X, uint32_t n, uint32_t dim,
                              double perplexity, uint32_t k, uint32_t* row_ptr, uint32_t* col,
                              float* val, uint32_t* nnz, uint32_t* knn_idx, double* knn_d2,

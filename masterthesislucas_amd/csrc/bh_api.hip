@@ -112,7 +112,7 @@ struct bh_ctx {
     hipEvent_t ev_staged = nullptr, ev_att = nullptr;
     double* tz = nullptr;
     double* kl_part = nullptr;
-    void* aff_buf = nullptr;   // workspace of bh_tsne_affinities (grow-only until bh_tsne_set_p)
+    void* aff_buf = nullptr;   // workspace of bh_tsne_affinities (kept up to kAffKeepBytes)
     size_t aff_bytes = 0;
     double* kl_out = nullptr;
 
@@ -1260,6 +1260,9 @@ bh_status bh_tsne_run(bh_ctx* c, const bh_tsne_params* p, int32_t first, int32_t
     return finish_build_call(c, "t-SNE run");
 }
 
+// The largest workspace of bh_tsne_affinities that a context keeps between calls
+constexpr size_t kAffKeepBytes = (size_t)1 << 30;
+
 static void aff_release(bh_ctx* c) {
     if (c->aff_buf) (void)hipFree(c->aff_buf);
     c->aff_buf = nullptr;
@@ -1292,8 +1295,10 @@ bh_status bh_tsne_affinities(bh_ctx* c, const float* X, uint32_t n, uint32_t dim
     uint64_t *keys_a = nullptr, *keys_b = nullptr;
     double *d2 = nullptr, *P = nullptr, *dbeta = nullptr;
     const size_t nsp = scan_partials_size(m);
-    // one workspace, kept by the context until bh_tsne_set_p starts a descent (25 allocations and
-    // frees a call took 4.7 ms of a 20,000-point call)
+    // One workspace. Up to kAffKeepBytes of it stay with the context until bh_tsne_set_p starts a
+    // descent (25 allocations and frees a call took 4.7 ms of a 20,000-point call, whose workspace in
+    // 784-D is 0.54 GB); a larger one is given back at the end of the call, which takes tens of
+    // milliseconds at such sizes.
     size_t need = 0;
     std::pair<void**, size_t> parts[32];
     int np = 0;
@@ -1409,6 +1414,7 @@ bh_status bh_tsne_affinities(bh_ctx* c, const float* X, uint32_t n, uint32_t dim
     }
     (void)hipStreamSynchronize(s);
     (void)hipEventDestroy(ready);
+    if (c->aff_bytes > kAffKeepBytes) aff_release(c);
     return st;
 }
 

@@ -588,3 +588,34 @@ def test_training_gradient_of_many_samples(gpu):
     g = unflatten(g)
     for k in ref:
         assert np.abs(g[k] - ref[k]).max() <= 4e-5 * np.abs(ref[k]).max(), k
+
+
+@pytest.mark.parametrize("n,dim,k,kept", [(3000, 100, 30, True), (52_000, 1024, 128, False)])
+def test_affinity_workspace_is_given_back(gpu, n, dim, k, kept):
+    """The workspace of a call stays with the context up to 1 GiB and goes back with bh_tsne_set_p;
+    a larger one (1.25 GB here) goes back with the call. Device memory as the driver counts it, to 64
+    MiB (a context's own buffers do not change)."""
+    torch = pytest.importorskip("torch")
+    import ctypes as C
+
+    from masterthesislucas_amd import _lib
+    rng = np.random.default_rng(n)
+    X = rng.standard_normal((n, dim), dtype=np.float32)
+    ctx = BHContext(n, kernel="tsne")
+    rp, col, val = (np.empty(m, t) for m, t in ((n + 1, np.uint32), (2 * n * k, np.uint32),
+                                                (2 * n * k, np.float32)))
+    ptr = lambda a: a.ctypes.data_as(C.c_void_p)  # noqa: E731
+    nnz = C.c_uint32(0)
+    before = torch.cuda.mem_get_info()[0]
+    ctx._c(_lib.load().bh_tsne_affinities(ctx.handle, ptr(X), n, dim, k / 3.0, k, ptr(rp), ptr(col),
+                                          ptr(val), C.byref(nnz), None, None, None))
+    held = before - torch.cuda.mem_get_info()[0]
+    print(f"held {held} bytes", flush=True)
+    small = np.array([0, 1, 2], np.uint32)
+    ctx._c(_lib.load().bh_tsne_set_p(ctx.handle, 2, ptr(small), ptr(np.array([1, 0], np.uint32)),
+                                     ptr(np.full(2, 0.5, np.float32)), 2))
+    after = before - torch.cuda.mem_get_info()[0]
+    ctx.close()
+    assert held < (1 << 30) + (64 << 20) if kept else held < 64 << 20
+    assert after < 64 << 20
+    assert rp[n] == nnz.value and np.all(np.diff(rp.astype(np.int64)) >= k)
