@@ -592,7 +592,7 @@ static bh_status create_impl(bh_ctx** out, const bh_config* cfg, uint32_t extra_
     TRY(dalloc(c, &c->vals_a, N));
     TRY(dalloc(c, &c->vals_b, N));
     TRY(dalloc(c, &c->sort_scratch, sort_scratch_words(N)));
-    TRY(dalloc(c, &c->tree_sums, tree_tiles(N)));
+    TRY(dalloc(c, &c->tree_sums, tree_sums_words(N)));
     TRY(dalloc(c, &c->leaf_lvl, N));
     TRY(dalloc(c, &c->lcp1, N));
     TRY(dalloc(c, &c->cnt, N));

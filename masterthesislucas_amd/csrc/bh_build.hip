@@ -1177,11 +1177,13 @@ struct CodeSearch {
     }
 };
 
-// nodes of particle i: k = noff[i] + t at level lcp1[i] + t, t < cnt[i]
+// nodes of particle i: k = noff[i] + t at level lcp1[i] + t, t < cnt[i]. sums: the node counts of the
+// tiles or, scanned, the nodes before each tile
 __global__ __launch_bounds__(kTreeTile) void k_tree_emit_heads(uint32_t n,
                                                                const uint8_t* __restrict__ lcp1,
                                                                const uint32_t* __restrict__ cnt,
                                                                const uint32_t* __restrict__ sums,
+                                                               int scanned,
                                                                uint32_t* __restrict__ noff,
                                                                BuildParams* __restrict__ prm,
                                                                Node* __restrict__ nodes,
@@ -1191,8 +1193,12 @@ __global__ __launch_bounds__(kTreeTile) void k_tree_emit_heads(uint32_t n,
     const uint32_t c = i < n ? cnt[i] : 0u;
     const uint32_t l0 = i < n ? lcp1[i] : 0u;
     uint32_t before = 0, all, tot;
-    for (uint32_t b = threadIdx.x; b < blockIdx.x; b += kTreeTile) before += sums[b];
-    block_exclusive_scan_t<kTreeTile>(before, &all);
+    if (scanned) {
+        all = sums[blockIdx.x];
+    } else {
+        for (uint32_t b = threadIdx.x; b < blockIdx.x; b += kTreeTile) before += sums[b];
+        block_exclusive_scan_t<kTreeTile>(before, &all);
+    }
     const uint32_t base = all + block_exclusive_scan_t<kTreeTile>(c, &tot);
     if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) prm->n_nodes = all + tot;
     if (i >= n) return;
@@ -2024,7 +2030,17 @@ void launch_sort(hipStream_t s, void* keys_a, uint32_t* vals_a, void* keys_b, ui
     *result_in_b = (passes & 1) != 0;
 }
 
-uint32_t tree_tiles(uint32_t n) { return div_up(n, kTreeTile); }
+// Up to here (8,388,608 particles) every block of k_tree_emit_heads adds up the counts of the tiles
+// before its own, which spares a build three launches; those reads grow with the square of the tiles,
+// so larger builds scan the counts first. The tree's launches, adding / scanning, us: 1M particles
+// 30 / 37, 4M 93 / 97, 8M 200 / 196, 17M 473 / 439, 67M 2,373 / 1,895, 134M 5,877 / 4,073, 268M
+// 16,135 / 9,199.
+constexpr uint32_t kTreeSumsAlone = 8192;
+
+uint32_t tree_sums_words(uint32_t n) {  // counts; then the nodes before each tile, scan partials
+    const uint32_t t = div_up(n, kTreeTile);
+    return t <= kTreeSumsAlone ? t : 2 * t + scan_partials_size(t);
+}
 
 void launch_gather_levels(hipStream_t s, const uint32_t* perm, const float4* pk, const float* vx,
                           const float* vy, float* xo, float* yo, float* mo, float* vxo, float* vyo,
@@ -2041,15 +2057,17 @@ void launch_gather_levels(hipStream_t s, const uint32_t* perm, const float4* pk,
 
 void launch_tree(hipStream_t s, const void* codes, bool wide, uint32_t n, int B,
                  int single_child_pp, const uint8_t* lcp1, const uint32_t* cnt, uint32_t* noff,
-                 const uint32_t* sums, BuildParams* prm, Node* nodes, uint32_t* parent,
+                 uint32_t* sums, BuildParams* prm, Node* nodes, uint32_t* parent,
                  uint32_t* child4, uint32_t cap_nodes, int R, const BuildParams* sys_prm) {
     const uint32_t g = div_up(n, kTreeTile), gn = div_up(cap_nodes, kTreeThreads);
 #define BH_NODES(K)                                                                               \
     k_tree_emit_nodes<K><<<gn, kTreeThreads, 0, s>>>((const K*)codes, n, B, R, lcp1, noff, prm,   \
                                                      sys_prm, single_child_pp, nodes, parent,     \
                                                      child4, cap_nodes)
-    k_tree_emit_heads<<<g, kTreeTile, 0, s>>>(n, lcp1, cnt, sums, noff, prm, nodes,
-                                              (uint4*)child4, cap_nodes);
+    const bool scan = g > kTreeSumsAlone;
+    if (scan) launch_exclusive_scan(s, sums, sums + g, g, sums + 2 * (size_t)g, nullptr);
+    k_tree_emit_heads<<<g, kTreeTile, 0, s>>>(n, lcp1, cnt, scan ? sums + g : sums, scan ? 1 : 0,
+                                              noff, prm, nodes, (uint4*)child4, cap_nodes);
     if (wide) BH_NODES(uint64_t); else BH_NODES(uint32_t);
 #undef BH_NODES
 }
