@@ -226,8 +226,8 @@ def batched_comparison(args, eps, theta, dt, rmax=0.0, variant=None, split=None)
     """Batched systems: `args.batched_systems` independent systems with N log-uniform in
     [1,024, 262,144] (even: uniform disks, odd: Plummer a = 0.1, untruncated unless rmax > 0),
     all in one context (one set of build launches, one traversal launch per step). Leapfrog
-    steps timed eagerly and replayed from captured HIP graphs; the traversal variant is
-    autotuned on the batched tree unless given."""
+    steps timed eagerly and replayed from captured HIP graphs; the waves per work entry are
+    tuned on the batched tree unless a variant is given."""
     from masterthesislucas_amd import BHContext
     from masterthesislucas_amd.autotune import tune
     from masterthesislucas_amd.workloads import batched_systems
@@ -244,18 +244,14 @@ def batched_comparison(args, eps, theta, dt, rmax=0.0, variant=None, split=None)
     if variant is None:
         from masterthesislucas_amd.autotune import time_variant
 
-        # the variants are timed on cost-ordered work tables, as the steps will run: one walk
-        # and bh_batch_order_by_cost per table (variants 0, 4, 8: 1, 2, 4 sinks per lane)
-        for v0 in (0, 4, 8):
-            ctx.set_variant(v0)
-            ctx.forces_device_only(theta)
-            ctx.order_by_cost()
+        # the walk is timed on the cost-ordered work table, as the steps will run
+        ctx.forces_device_only(theta)
+        ctx.order_by_cost()
         variant, times = tune(ctx, theta)
-        # then the split (each work entry walked by F waves, each taking a slice of every
-        # particle-particle cell) for the chosen variant
-        best_ms = min(times[variant], times.get(f"{variant}:no-priority", times[variant]))
+        # then the split (the F waves of a work entry share its parts of the sums)
+        best_ms = times[variant]
         split = 1
-        for F in (2, 4, 8):
+        for F in (2, 4):
             ctx.set_split(F)
             ms = time_variant(ctx, variant, theta)
             times[f"{variant}/split{F}"] = ms
@@ -347,7 +343,7 @@ def tsne_run(args):
     y0 = T.initial_embedding(n, seed=SEED_TSNE, std=1e-2)
     run = T.TSNE(rp, col, val, y0, min_theta=0.5, max_theta=0.5, exaggeration=(48.0, 4.0))
     kl0, _ = run.costFunction()
-    # warm, then tune the walk variant and split per phase of the run: on the trees of two
+    # warm, then tune the waves per sink group per phase of the run: on the trees of two
     # snapshots inside the early-exaggeration phase (iterations 60 and 180: compact clusters,
     # crowded leaves) for the first `switch` iterations, and of three later ones (260, mid-run,
     # end) for the rest; the walks change with the embedding's spread, so each choice minimises
