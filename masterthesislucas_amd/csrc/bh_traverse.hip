@@ -136,6 +136,8 @@ struct WalkSum {  // one part: plain sums (b) and compensated ones (a with terms
 
 // gravity: a += m (q - p) / (|q - p|^2 + eps^2)^(3/2); potential -= m / sqrt(...)
 // t-SNE:   w = 1 / (1 + |p - q|^2); total += m w; derivative += m w^2 (p - q)
+// Every multiply-add is written as one: left to the compiler, the potential's was fused in the plain walk
+// and not in the learned one, and their potentials differed by 1e-10.
 template <int KERNEL, bool TOT>
 __device__ __forceinline__ void walk_pair(WalkSum<TOT>& s, float dx, float dy, float m,
                                           float eps2) {
@@ -145,14 +147,14 @@ __device__ __forceinline__ void walk_pair(WalkSum<TOT>& s, float dx, float dy, f
         const float f = mi * inv * inv;
         s.bx = fmaf(f, dx, s.bx);
         s.by = fmaf(f, dy, s.by);
-        if (TOT) s.bt -= mi;
+        if (TOT) s.bt = fmaf(-m, inv, s.bt);
     } else {
         const float w = __builtin_amdgcn_rcpf(fmaf(dx, dx, fmaf(dy, dy, 1.0f)));
         const float mw = m * w;
         const float f = mw * w;
         s.bx = fmaf(-f, dx, s.bx);
         s.by = fmaf(-f, dy, s.by);
-        if (TOT) s.bt += mw;
+        if (TOT) s.bt = fmaf(m, w, s.bt);
     }
 }
 
