@@ -1,16 +1,77 @@
 """Calls whose path depends on their size or input, on each path that the other tests leave out: the
-learned walk with one, two and four waves per group and with totals."""
+radix sort's give-up, the affinity call that is repeated with one column range, and the learned walk
+with one, two and four waves per group and with totals."""
 import numpy as np
 import pytest
 
+from masterthesislucas_amd import BHContext, _lib, tsne
+from masterthesislucas_amd._lib import BHError
 from masterthesislucas_amd.learned import N_OUT, FarFieldMLP, flatten
+from masterthesislucas_amd.workloads import two_plummer_disks
 from oracle import oracle as O
-from tests.helpers import WALK_TOL, exact_walk
+from tests.helpers import WALK_TOL, exact_walk, oracle_tree
 from tests.test_gpu_learned import _gpu_tree, _params, _plummer_ctx
 
 pytestmark = pytest.mark.gpu
 
 EPS = float(np.float32(1e-3))
+
+
+@pytest.mark.parametrize("n", [20_000, 1 << 21, (1 << 21) + 1])
+def test_sort_give_up_of_each_sort(gpu, n):
+    """The bucket sort (up to 2^21 keys) and the radix sort (above) with a wait bound of 0 polls,
+    set from the host: a build that gave up is reported and leaves no tree, one that did not is
+    right, and with the default bound the order is bit-exact again."""
+    p = two_plummer_disks(n, seed=33)
+    ctx = BHContext(n, kernel="gravity", softening=EPS)
+    ctx.set_particles(p.x, p.y, p.m)
+    ctx.set_sort_spin_limit(0)
+    raised = 0
+    for _ in range(3):
+        try:
+            ctx.build()
+        except BHError as e:
+            assert e.status == _lib.BH_ERR_HIP and "look-back" in str(e)
+            raised += 1
+            with pytest.raises(BHError) as f:
+                ctx.forces(0.5)
+            assert f.value.status == _lib.BH_ERR_STATE
+    # hundreds of tiles start together and some finds its predecessor unpublished; 10 tiles may not
+    assert raised >= 1 or n == 20_000
+    ctx.set_sort_spin_limit(1 << 22)
+    ctx.build()
+    codes, perm = ctx.morton()
+    ctx.close()
+    t = oracle_tree(p.x, p.y, p.m, mode="quadtree")
+    assert np.array_equal(perm, t["perm"])
+    assert np.array_equal(codes, t["codes_sorted"])
+
+
+def test_affinities_repeated_with_one_range(gpu):
+    """1,024 points are two column ranges of 512. The first 512 lie on a line along the first axis, the
+    others on a ring around that axis, so that a point of the line has all of them at one distance:
+    more than its list of the second range can hold beside each other, while one list over all
+    columns has the near points of the line first and drops the ring. Neighbours exact, distances to
+    1e-12."""
+    rng = np.random.default_rng(5)
+    n, dim, k = 1024, 64, 60
+    X = np.zeros((n, dim))
+    X[:512, 0] = np.linspace(-0.3, 0.3, 512)
+    z = rng.normal(0, 1, (512, dim - 1))
+    X[512:, 1:] = 0.5 * z / np.linalg.norm(z, axis=1, keepdims=True)
+    X[512:, 0] = np.sqrt(0.75)
+    X = X.astype(np.float32)
+    a = tsne.affinities(X, perplexity=20.0, k=k)
+    d = X.astype(np.float64)
+    d2 = np.stack([((d - row) ** 2).sum(1) for row in d])
+    np.fill_diagonal(d2, np.inf)
+    want = np.sort(d2, axis=1)[:, :k]
+    assert np.allclose(a["d2"], want, rtol=1e-12, atol=0)
+    got = np.take_along_axis(d2, a["idx"].astype(np.int64), 1)
+    assert np.allclose(got, want, rtol=1e-12, atol=0)
+    # far points of the line from the ring: their distance agrees to 2^-11 of it and less
+    ring = np.sqrt(d2[:512, 512:])
+    assert np.all(np.ptp(ring, axis=1) < 2.0 ** -11 * ring.mean(axis=1))
 
 
 @pytest.mark.parametrize("total", [False, True])
