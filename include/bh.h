@@ -131,7 +131,8 @@ bh_status bh_forces_device(bh_ctx* ctx, double theta, float* d_ax, float* d_ay, 
 bh_status bh_leapfrog(bh_ctx* ctx, int steps, float dt, double theta);
 /* bh_leapfrog with each step (kick-drift, build, traversal, kick) captured once in a HIP graph
  * and replayed: same kernels and results, without per-launch host overhead. The graphs are
- * re-captured when dt, theta or a traversal setting change. */
+ * re-captured when dt, theta, the particle count, the split, the solver, the work table or the
+ * learned correction's switch change. */
 bh_status bh_leapfrog_graph(bh_ctx* ctx, int steps, float dt, double theta);
 
 /* Conserved quantities of a gravity context in FP64 (no counterpart in the reference, whose

@@ -149,7 +149,8 @@ struct bh_ctx {
     bool g_valid = false;
     float g_dt = 0.f;
     double g_theta = 0.0;
-    int g_variant = -1;
+    uint32_t g_n = 0, g_spin = 0;
+    bool g_learned = false;
 
     int variant = 4;        // selected variant id and issue priority: kept for the caller, the
     bool walk_prio = true;  // walk does not depend on them
@@ -917,7 +918,8 @@ bh_status bh_leapfrog_graph(bh_ctx* c, int steps, float dt, double theta) {
         if (st == BH_OK) st = do_forces(c, theta, false);
         if (st != BH_OK) return st;
     }
-    if (!c->g_valid || c->g_dt != dt || c->g_theta != theta || c->g_variant != c->variant) {
+    if (!c->g_valid || c->g_dt != dt || c->g_theta != theta || c->g_n != c->n ||
+        c->g_learned != c->learned || c->g_spin != c->sort_spin) {
         graph_reset(c);
         // capture one step from each ping-pong parity; the host-side state the build updates
         // (current buffer, sort parity) is the same on replay, so it is restored afterwards
@@ -951,7 +953,9 @@ bh_status bh_leapfrog_graph(bh_ctx* c, int steps, float dt, double theta) {
         c->g_valid = true;
         c->g_dt = dt;
         c->g_theta = theta;
-        c->g_variant = c->variant;
+        c->g_n = c->n;
+        c->g_learned = c->learned;
+        c->g_spin = c->sort_spin;
     }
     for (int k = 0; k < steps; ++k) {
         st = hip_check(c, hipGraphLaunch(c->gexec[c->cur], c->stream), "graph launch");

@@ -1,6 +1,7 @@
 """Calls whose path depends on their size or input, on each path that the other tests leave out: the
-radix sort's give-up, the affinity call that is repeated with one column range, and the learned walk
-with one, two and four waves per group and with totals."""
+radix sort's give-up, the affinity call that is repeated with one column range, the learned walk
+with one, two and four waves per group and with totals, and captured steps after a change of what
+they were captured with."""
 import numpy as np
 import pytest
 
@@ -108,3 +109,44 @@ def test_learned_walk_of_each_launch(gpu, n, total):
         assert pot == ctx.forces(theta, want_total=True)[2]
     net.close()
     ctx.close()
+
+
+@pytest.mark.parametrize("n1,n2", [(3000, 9001), (20_011, 700), (5000, 5000)])
+def test_captured_steps_follow_the_particles(gpu, n1, n2):
+    """Steps captured for one particle set and replayed after another was set, larger, smaller or of
+    the same size: the state of eager steps to the bit, several replays long."""
+    rng = np.random.default_rng(n1 + n2)
+    ctx = BHContext(max(n1, n2), kernel="gravity", softening=0.05)
+    for n in (n1, n2, n1):
+        x, y, vx, vy = rng.normal(0, 1, (4, n)).astype(np.float32)
+        m = np.full(n, 1.0 / n, np.float32)
+        ctx.set_particles(x, y, m, vx, vy)
+        ctx.leapfrog_graph(2, 1e-2, 0.6)
+        ctx.leapfrog_graph(3, 1e-2, 0.6)
+        got = ctx.get_particles()
+        eager = BHContext(n, kernel="gravity", softening=0.05)
+        eager.set_particles(x, y, m, vx, vy)
+        eager.leapfrog(5, 1e-2, 0.6)
+        want = eager.get_particles()
+        eager.close()
+        assert all(np.array_equal(a, b) for a, b in zip(got, want))
+    ctx.close()
+
+
+def test_captured_steps_follow_the_learned_switch(gpu):
+    """Steps captured before the learned correction was switched on build no second moments; replayed
+    after it they are captured anew: the cell features are those of eager steps."""
+    n = 4000
+    rng = np.random.default_rng(1)
+    x, y, vx, vy = rng.normal(0, 1, (4, n)).astype(np.float32)
+    m = np.full(n, 1.0 / n, np.float32)
+    out = []
+    for graph in (False, True):
+        ctx = BHContext(n, kernel="gravity", softening=0.05)
+        for on in (False, True):
+            ctx.learned_enable(on)
+            ctx.set_particles(x, y, m, vx, vy)
+            (ctx.leapfrog_graph if graph else ctx.leapfrog)(3, 1e-2, 0.6)
+        out.append(ctx.learned_export()[0])
+        ctx.close()
+    assert np.any(out[0]) and np.array_equal(out[0], out[1])
