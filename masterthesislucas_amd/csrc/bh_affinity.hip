@@ -35,6 +35,7 @@ constexpr uint32_t kAffCap = 512;             // candidate slots per row and col
 constexpr uint32_t kAffHold = kAffCap - kAffCols;  // compact above this many (a tile adds <= 256)
 constexpr uint32_t kAffKeep = 192;            // most candidates of a row over all columns
 constexpr uint32_t kAffMaxSplits = 4;         // most column ranges
+constexpr uint32_t kAffOver = 1u << 31;       // flag of a list's count: its window outgrew the buffer
 
 // largest magnitude bits of the inputs (order = |x|; infinities and NaN above every finite one),
 // into *out (cleared by the caller); one integer atomic per block
@@ -229,8 +230,7 @@ __global__ __launch_bounds__(kAffThreads) void k_aff_candidates(const _Float16* 
                                                                 uint32_t k,
                                                                 uint2* __restrict__ cand,
                                                                 uint32_t* __restrict__ ccount,
-                                                                uint32_t* thr,
-                                                                uint32_t* __restrict__ overflow) {
+                                                                uint32_t* thr) {
     __shared__ __attribute__((aligned(16))) _Float16 s_t[2][(kAffRows + kAffCols) * kAffLd];
     __shared__ uint32_t s_cnt[kAffRows], s_over[kAffRows];
     __shared__ float s_T[kAffRows], s_nh[kAffRows], s_ka[kAffRows], s_eb[kAffRows];
@@ -398,8 +398,7 @@ __global__ __launch_bounds__(kAffThreads) void k_aff_candidates(const _Float16* 
     }
     // the lists as they stand (at most kAffHold entries each): the refinement merges and thins them
     if (tid < kAffRows && row0 + tid < n) {
-        ccount[lists + row0 + tid] = s_cnt[tid];
-        if (s_over[tid]) atomicAdd(overflow, 1u);
+        ccount[lists + row0 + tid] = s_cnt[tid] | (s_over[tid] ? kAffOver : 0u);
     }
 }
 
@@ -432,9 +431,12 @@ __global__ __launch_bounds__(kBlock) void k_aff_refine(const float* __restrict__
         uint32_t j[kAffMaxSplits * kPer], hb[kAffMaxSplits * kPer];
         float lo[kAffMaxSplits * kPer];
         bool v[kAffMaxSplits * kPer];
+        uint32_t over = 0;
 #pragma unroll
         for (int s = 0; s < (int)kAffMaxSplits; ++s) {
-            const uint32_t cs = s < (int)splits ? ccount[(size_t)s * n + i] : 0u;
+            const uint32_t cf = s < (int)splits ? ccount[(size_t)s * n + i] : 0u;
+            const uint32_t cs = cf & ~kAffOver;
+            over |= cf & kAffOver;
 #pragma unroll
             for (int u = 0; u < kPer; ++u) {
                 const size_t o = ((size_t)s * n + i) * kAffCap + lane + 64 * u;
@@ -457,7 +459,7 @@ __global__ __launch_bounds__(kBlock) void k_aff_refine(const float* __restrict__
             if (keep && p < kAffKeep) s_j[w][p] = j[x];
             c += (uint32_t)__popcll(bm);
         }
-        if (lane == 0 && (c > kAffKeep || c < k)) atomicAdd(overflow, 1u);
+        if (lane == 0 && (over || c > kAffKeep || c < k)) atomicAdd(overflow, 1u);  // once a row
         c = min(c, kAffKeep);
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -643,10 +645,10 @@ void launch_aff_pack(hipStream_t s, const float* X, uint32_t n, uint32_t dim, fl
 }
 void launch_aff_candidates(hipStream_t s, const _Float16* Xh, const float* nh, const float* ah,
                            const float* eb, uint32_t n, uint32_t dim, uint32_t k, uint32_t splits,
-                           uint2* cand, uint32_t* ccount, uint32_t* thr, uint32_t* overflow) {
+                           uint2* cand, uint32_t* ccount, uint32_t* thr) {
     const dim3 g(div_up_a(n, kAffRows), splits);
     k_aff_candidates<<<g, kAffThreads, 0, s>>>(Xh, nh, ah, eb, n, aff_dim_padded(dim), k, cand,
-                                               ccount, thr, overflow);
+                                               ccount, thr);
 }
 void launch_aff_refine(hipStream_t s, const float* X, const float* nh, const float* ah,
                        const float* eb, uint32_t n, uint32_t dim, uint32_t k, uint32_t splits,

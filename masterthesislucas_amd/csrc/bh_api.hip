@@ -1374,7 +1374,7 @@ bh_status bh_tsne_affinities(bh_ctx* c, const float* X, uint32_t n, uint32_t dim
             launch_fill_u32(s, flags, 4, 0u);
             launch_aff_pack(s, dX, n, dim, scale, Xh, nh, ah, eb);
             launch_fill_u32(s, thr, n, 0x7F800000u);
-            launch_aff_candidates(s, Xh, nh, ah, eb, n, dim, k, splits, cand, ccount, thr, flags);
+            launch_aff_candidates(s, Xh, nh, ah, eb, n, dim, k, splits, cand, ccount, thr);
             launch_aff_refine(s, dX, nh, ah, eb, n, dim, k, splits, cand, ccount, idx, d2, flags);
             launch_aff_bandwidth(s, d2, n, k, std::log(perplexity), 1e-5, 200, P, dbeta);
             st = hip_check(c, hipMemcpyAsync(h_flags, flags, 4, hipMemcpyDeviceToHost, s), "flags");

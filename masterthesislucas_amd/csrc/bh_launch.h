@@ -268,7 +268,7 @@ void launch_aff_pack(hipStream_t s, const float* X, uint32_t n, uint32_t dim, fl
 // thr: a threshold per row that its column ranges share, set to infinity by the caller
 void launch_aff_candidates(hipStream_t s, const _Float16* Xh, const float* nh, const float* ah,
                            const float* eb, uint32_t n, uint32_t dim, uint32_t k, uint32_t splits,
-                           uint2* cand, uint32_t* ccount, uint32_t* thr, uint32_t* overflow);
+                           uint2* cand, uint32_t* ccount, uint32_t* thr);
 void launch_aff_refine(hipStream_t s, const float* X, const float* nh, const float* ah,
                        const float* eb, uint32_t n, uint32_t dim, uint32_t k, uint32_t splits,
                        const uint2* cand, const uint32_t* ccount, uint32_t* idx, double* d2,

@@ -1,7 +1,7 @@
 """Calls whose path depends on their size or input, on each path that the other tests leave out: the
 radix sort's give-up, the affinity call that is repeated with one column range, the learned walk
 with one, two and four waves per group and with totals, and captured steps after a change of what
-they were captured with."""
+they were captured with, and the affinity call that is refused."""
 import numpy as np
 import pytest
 
@@ -150,3 +150,16 @@ def test_captured_steps_follow_the_learned_switch(gpu):
         out.append(ctx.learned_export()[0])
         ctx.close()
     assert np.any(out[0]) and np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("n,near", [(300, 300), (900, 280), (1500, 1500)])
+def test_refused_affinities_name_the_points(gpu, n, near):
+    """Hundreds of near duplicates: refused, and the message counts each point with too many
+    candidates once, whatever the number of column ranges (two for 1,500 points)."""
+    rng = np.random.default_rng(n)
+    X = rng.normal(0, 1, (n, 32))
+    X[n - near:] = 5.0 + 1e-5 * rng.normal(0, 1, (near, 32))
+    with pytest.raises(BHError) as e:
+        tsne.affinities(X.astype(np.float32), perplexity=10.0, k=30)
+    assert e.value.status == _lib.BH_ERR_CAPACITY
+    assert f"{near} points have" in str(e.value)
