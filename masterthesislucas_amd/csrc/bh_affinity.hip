@@ -59,7 +59,7 @@ __global__ __launch_bounds__(kBlock) void k_aff_maxbits(const uint32_t* __restri
 // scaled FP16 copy, squared norms and rounding bounds (one wave per point)
 // ---------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(kBlock) void k_aff_pack(const float* __restrict__ X, uint32_t n,
-                                                     uint32_t dim, uint32_t dp, float scale,
+                                                     uint32_t dim, uint32_t dp, float2 scale,
                                                      _Float16* __restrict__ Xh,
                                                      float* __restrict__ nh,
                                                      float* __restrict__ ah,
@@ -69,7 +69,8 @@ __global__ __launch_bounds__(kBlock) void k_aff_pack(const float* __restrict__ X
     if (i >= n) return;
     double sh = 0.0, sx = 0.0;
     for (uint32_t e = lane; e < dp; e += kWave) {
-        const float v = e < dim ? X[(size_t)i * dim + e] * scale : 0.f;  // scale = 2^m
+        // 2^m in two factors: for the smallest inputs m exceeds a float's exponent
+        const float v = e < dim ? X[(size_t)i * dim + e] * scale.x * scale.y : 0.f;
         const _Float16 h = (_Float16)v;
         Xh[(size_t)i * dp + e] = h;
         const double hd = (double)h;
@@ -510,6 +511,11 @@ __global__ __launch_bounds__(kBlock) void k_aff_refine(const float* __restrict__
             d2[(size_t)i * k + rank] = dq;
         }
     }
+    // a row with fewer candidates than neighbours is reported; what follows still reads whole rows
+    for (uint32_t q = c + lane; q < k; q += kWave) {
+        idx[(size_t)i * k + q] = i;
+        d2[(size_t)i * k + q] = 0.0;
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -611,7 +617,9 @@ __global__ __launch_bounds__(kBlock) void k_sym_reduce(const uint64_t* __restric
     double s = P[vals[u] % nk] / two_n;
     if (u + 1 < m && keys[u + 1] == key) s += P[vals[u + 1] % nk] / two_n;
     const uint32_t q = pos[u];
-    const uint32_t r = (uint32_t)(key / n);
+    const uint64_t r64 = key / n;
+    if (r64 >= n) return;  // no key of an entry: left behind by a sort that gave up (reported)
+    const uint32_t r = (uint32_t)r64;
     col[q] = (uint32_t)(key % n);
     val[q] = (float)s;
     if (u == 0 || (uint32_t)(keys[u - 1] / n) != r) row_ptr[r] = q;  // every row has entries
@@ -638,7 +646,7 @@ void launch_aff_maxbits(hipStream_t s, const float* x, uint64_t n, uint32_t* out
     const uint32_t g = div_up_a(n, 8 * kBlock);
     k_aff_maxbits<<<g < 2048 ? g : 2048, kBlock, 0, s>>>((const uint32_t*)x, n, out);
 }
-void launch_aff_pack(hipStream_t s, const float* X, uint32_t n, uint32_t dim, float scale,
+void launch_aff_pack(hipStream_t s, const float* X, uint32_t n, uint32_t dim, float2 scale,
                      _Float16* Xh, float* nh, float* ah, float* eb) {
     k_aff_pack<<<div_up_a(n, kWavesPerBlock), kBlock, 0, s>>>(X, n, dim, aff_dim_padded(dim),
                                                               scale, Xh, nh, ah, eb);

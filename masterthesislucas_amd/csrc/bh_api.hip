@@ -1348,7 +1348,7 @@ bh_status bh_tsne_affinities(bh_ctx* c, const float* X, uint32_t n, uint32_t dim
     bh_status st = hip_check(c, hipEventCreateWithFlags(&ready, hipEventDisableTiming), "event");
     if (st != BH_OK) return st;
     uint32_t* h_flags = reinterpret_cast<uint32_t*>(c->h_counters);  // pinned
-    float scale = 1.0f;
+    float2 scale = make_float2(1.0f, 1.0f);
     st = hip_check(c, hipMemcpyAsync(dX, X, (size_t)n * dim * 4, hipMemcpyHostToDevice, s), "X");
     if (st == BH_OK) {
         // scale by a power of two so that the largest |x| lands in [2^13, 2^14): no FP16 overflow.
@@ -1365,7 +1365,10 @@ bh_status bh_tsne_affinities(bh_ctx* c, const float* X, uint32_t n, uint32_t dim
         std::memcpy(&maxf, h_flags, 4);
         int ex = 0;
         if (maxf > 0.0f) (void)std::frexp((double)maxf, &ex);
-        scale = maxf > 0.0f ? std::ldexp(1.0f, 14 - ex) : 1.0f;
+        if (maxf > 0.0f) {
+            const int m = 14 - ex, m1 = std::min(m, 127);
+            scale = make_float2(std::ldexp(1.0f, m1), std::ldexp(1.0f, m - m1));
+        }
     }
     // Column ranges keep thresholds of their own, so a range's list can overflow where one list
     // over all columns would not: such a call is repeated with one range.

@@ -263,7 +263,7 @@ uint32_t aff_keep();  // most candidates of a row after the merge (more: counted
 uint32_t aff_splits(uint32_t n);  // column ranges (lists per row) of the candidate search
 // out (cleared) = the largest magnitude bits of n values
 void launch_aff_maxbits(hipStream_t s, const float* x, uint64_t n, uint32_t* out);
-void launch_aff_pack(hipStream_t s, const float* X, uint32_t n, uint32_t dim, float scale,
+void launch_aff_pack(hipStream_t s, const float* X, uint32_t n, uint32_t dim, float2 scale,
                      _Float16* Xh, float* nh, float* ah, float* eb);
 // thr: a threshold per row that its column ranges share, set to infinity by the caller
 void launch_aff_candidates(hipStream_t s, const _Float16* Xh, const float* nh, const float* ah,

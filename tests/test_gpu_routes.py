@@ -1,7 +1,7 @@
 """Calls whose path depends on their size or input, on each path that the other tests leave out: the
 radix sort's give-up, the affinity call that is repeated with one column range, the learned walk
 with one, two and four waves per group and with totals, and captured steps after a change of what
-they were captured with, and the affinity call that is refused."""
+they were captured with, and affinity calls that are refused or have the smallest inputs."""
 import numpy as np
 import pytest
 
@@ -163,3 +163,23 @@ def test_refused_affinities_name_the_points(gpu, n, near):
         tsne.affinities(X.astype(np.float32), perplexity=10.0, k=30)
     assert e.value.status == _lib.BH_ERR_CAPACITY
     assert f"{near} points have" in str(e.value)
+
+
+@pytest.mark.parametrize("n", [50, 700])
+@pytest.mark.parametrize("scale", [1e-38, 3e-42, 3e37])
+def test_affinities_of_the_smallest_and_largest_inputs(gpu, n, scale):
+    """Inputs whose scaling to FP16 takes a factor beyond a float's exponent (1e-38 and subnormal ones),
+    and near the largest floats: the exact neighbours, distances to 1e-12."""
+    rng = np.random.default_rng(n)
+    k = 20
+    X = (np.clip(rng.normal(0, 1, (n, 8)), -4, 4) * scale).astype(np.float32)
+    assert np.all(np.isfinite(X))
+    a = tsne.affinities(X, perplexity=6.0, k=k)
+    d = X.astype(np.float64) / scale  # (the squares of 1e-42 in FP64 are exact enough; keep them near 1)
+    d2 = ((d[:, None, :] - d[None, :, :]) ** 2).sum(2)
+    np.fill_diagonal(d2, np.inf)
+    want = np.sort(d2, axis=1)[:, :k]
+    assert np.allclose(a["d2"] / scale / scale, want, rtol=1e-12, atol=0)
+    got = np.take_along_axis(d2, a["idx"].astype(np.int64), 1)
+    assert np.allclose(got, want, rtol=1e-12, atol=0)
+    assert a["row_ptr"][n] == a["val"].size and np.all(a["col"] < n)
