@@ -69,10 +69,10 @@ struct bh_ctx {
     uint32_t *vals_a = nullptr, *vals_b = nullptr;
     uint32_t* sort_scratch = nullptr;  // sort counts, look-back words, totals, tickets
     uint32_t* tree_sums = nullptr;
-    uint8_t *leaf_lvl = nullptr, *lcp1 = nullptr;
+    uint8_t* lcp1 = nullptr;
     uint32_t *cnt = nullptr, *noff = nullptr;
     Node* nodes = nullptr;
-    uint32_t *parent = nullptr, *child4 = nullptr, *deferred = nullptr, *bylevel = nullptr;
+    uint32_t *child4 = nullptr, *deferred = nullptr, *bylevel = nullptr;
     float4* m2 = nullptr;
     BuildParams* prm = nullptr;
     float4* bounds_part = nullptr;
@@ -335,7 +335,7 @@ bh_status do_build(bh_ctx* c, const double* bounds, uint32_t have_partials = 0) 
     const float *vx = c->v_zero ? nullptr : c->vx[cur], *vy = c->v_zero ? nullptr : c->vy[cur];
     launch_gather_levels(s, perm, c->packed, vx, vy, c->x[nxt], c->y[nxt], c->m[nxt], c->vx[nxt],
                          c->vy[nxt], c->id[nxt], c->pos4, codes, c->wide, n, c->B,
-                         c->cfg.max_children, fixed, c->leaf_lvl, c->lcp1, c->cnt, c->tree_sums,
+                         c->cfg.max_children, fixed, c->lcp1, c->cnt, c->tree_sums,
                          c->R, c->dstatus);
     phase_end(c, 2);
     c->cur = nxt;
@@ -343,7 +343,7 @@ bh_status do_build(bh_ctx* c, const double* bounds, uint32_t have_partials = 0) 
     if (!quadtree) c->depth = fixed;
     phase_begin(c, 3);
     launch_tree(s, codes, c->wide, n, c->B, quadtree ? 1 : 0, c->lcp1, c->cnt, c->noff, c->tree_sums,
-                c->prm, c->nodes, c->parent, c->child4, c->cap_nodes, c->R,
+                c->prm, c->nodes, c->child4, c->cap_nodes, c->R,
                 c->nsys ? c->sys_prm : nullptr);
     if (c->nsys) launch_batch_roots(s, c->sys_off, c->nsys, c->noff, c->prm, c->roots);
     phase_end(c, 3);
@@ -594,12 +594,10 @@ static bh_status create_impl(bh_ctx** out, const bh_config* cfg, uint32_t extra_
     TRY(dalloc(c, &c->vals_b, N));
     TRY(dalloc(c, &c->sort_scratch, sort_scratch_words(N)));
     TRY(dalloc(c, &c->tree_sums, tree_sums_words(N)));
-    TRY(dalloc(c, &c->leaf_lvl, N));
     TRY(dalloc(c, &c->lcp1, N));
     TRY(dalloc(c, &c->cnt, N));
     TRY(dalloc(c, &c->noff, N));
     TRY(dalloc(c, &c->nodes, c->cap_nodes));
-    TRY(dalloc(c, &c->parent, c->cap_nodes));
     TRY(dalloc(c, &c->deferred, (size_t)up_chunks(c->cap_nodes) * kDeferStride));
     TRY(dalloc(c, &c->bylevel, (size_t)up_chunks(c->cap_nodes) * kDeferStride));
     TRY(dalloc(c, &c->stats_part, kStatsBlocks));

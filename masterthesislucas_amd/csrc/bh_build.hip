@@ -1069,7 +1069,6 @@ __global__ __launch_bounds__(kTreeTile) void k_gather_levels(const uint32_t* __r
                                                         float4* __restrict__ pos4,
                                                         K* codes, uint32_t n,
                                                         int B, int R, int cap, int fixed_depth,
-                                                        uint8_t* __restrict__ leaf_lvl,
                                                         uint8_t* __restrict__ lcp1,
                                                         uint32_t* __restrict__ cnt,
                                                         uint32_t* __restrict__ sums,
@@ -1127,7 +1126,6 @@ __global__ __launch_bounds__(kTreeTile) void k_gather_levels(const uint32_t* __r
         }
         // levels below R only separate batched systems: every system's tree starts at level R
         const int lp = max((i == 0) ? -1 : lcp_level(codes[i - 1], codes[i], B), R - 1);
-        leaf_lvl[i] = (uint8_t)leaf;
         lcp1[i] = (uint8_t)(lp + 1);
         c = (!failed && leaf > lp) ? (uint32_t)(leaf - lp) : 0u;
         cnt[i] = c;
@@ -1212,7 +1210,7 @@ __global__ __launch_bounds__(kTreeTile) void k_tree_emit_heads(uint32_t n,
     }
 }
 
-// one thread per node: subtree extent, flags, side, parent and the parent's child slot
+// one thread per node: subtree extent, flags, side and the parent's child slot
 template <typename K>
 __global__ __launch_bounds__(kTreeThreads) void k_tree_emit_nodes(const K* __restrict__ codes,
                                                             uint32_t n, int B, int R,
@@ -1222,7 +1220,6 @@ __global__ __launch_bounds__(kTreeThreads) void k_tree_emit_nodes(const K* __res
                                                             const BuildParams* __restrict__ sys_prm,
                                                             int single_child_pp,
                                                             Node* __restrict__ nodes,
-                                                            uint32_t* __restrict__ parent,
                                                             uint32_t* __restrict__ child4,
                                                             uint32_t cap_nodes) {
     __shared__ K s_key[kTreeKeys];
@@ -1306,12 +1303,10 @@ __global__ __launch_bounds__(kTreeThreads) void k_tree_emit_nodes(const K* __res
     nd->skip = skip;
     nd->count = end - i;
     nd->meta = meta;
-    uint32_t par = kNone;
     if (l > R) {
-        par = !(meta & kMetaHead) ? k - 1 : pk;
+        const uint32_t par = !(meta & kMetaHead) ? k - 1 : pk;
         child4[4ull * par + ((uint32_t)(ci >> (2 * (B - l))) & 3u)] = k;
     }
-    parent[k] = par;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -2045,25 +2040,25 @@ uint32_t tree_sums_words(uint32_t n) {  // counts; then the nodes before each ti
 void launch_gather_levels(hipStream_t s, const uint32_t* perm, const float4* pk, const float* vx,
                           const float* vy, float* xo, float* yo, float* mo, float* vxo, float* vyo,
                           uint32_t* ido, float4* pos4, void* codes, bool wide, uint32_t n, int B,
-                          int cap, int fixed_depth, uint8_t* leaf_lvl, uint8_t* lcp1, uint32_t* cnt,
+                          int cap, int fixed_depth, uint8_t* lcp1, uint32_t* cnt,
                           uint32_t* sums, int R, const uint32_t* status) {
 #define BH_LEVELS(K)                                                                              \
     k_gather_levels<K><<<div_up(n, kTreeTile), kTreeTile, 0, s>>>(                                \
         perm, pk, vx, vy, xo, yo, mo, vxo, vyo, ido, pos4, (K*)codes, n, B, R, cap, fixed_depth,  \
-        leaf_lvl, lcp1, cnt, sums, status)
+        lcp1, cnt, sums, status)
     if (wide) BH_LEVELS(uint64_t); else BH_LEVELS(uint32_t);
 #undef BH_LEVELS
 }
 
 void launch_tree(hipStream_t s, const void* codes, bool wide, uint32_t n, int B,
                  int single_child_pp, const uint8_t* lcp1, const uint32_t* cnt, uint32_t* noff,
-                 uint32_t* sums, BuildParams* prm, Node* nodes, uint32_t* parent,
-                 uint32_t* child4, uint32_t cap_nodes, int R, const BuildParams* sys_prm) {
+                 uint32_t* sums, BuildParams* prm, Node* nodes, uint32_t* child4,
+                 uint32_t cap_nodes, int R, const BuildParams* sys_prm) {
     const uint32_t g = div_up(n, kTreeTile), gn = div_up(cap_nodes, kTreeThreads);
 #define BH_NODES(K)                                                                               \
     k_tree_emit_nodes<K><<<gn, kTreeThreads, 0, s>>>((const K*)codes, n, B, R, lcp1, noff, prm,   \
-                                                     sys_prm, single_child_pp, nodes, parent,     \
-                                                     child4, cap_nodes)
+                                                     sys_prm, single_child_pp, nodes, child4,     \
+                                                     cap_nodes)
     const bool scan = g > kTreeSumsAlone;
     if (scan) launch_exclusive_scan(s, sums, sums + g, g, sums + 2 * (size_t)g, nullptr);
     k_tree_emit_heads<<<g, kTreeTile, 0, s>>>(n, lcp1, cnt, scan ? sums + g : sums, scan ? 1 : 0,

@@ -52,7 +52,7 @@ struct BuildParams {
     uint32_t pad[3];
 };
 
-// Traversal record, 32 bytes: read once per visit by the whole wave (scalar loads).
+// Traversal record, 32 bytes: one lane of a step reads it with two 16-byte loads.
 struct __attribute__((aligned(16))) Node {
     float cx, cy;   // centre of mass
     float mass;     // total mass
@@ -74,14 +74,6 @@ __device__ __forceinline__ int lcp_level(uint64_t a, uint64_t b, int B) {
     if (!x) return B;
     const int lz = __builtin_clzll(x) - (64 - 2 * B);
     return lz >> 1;
-}
-
-// blockIdx -> work block such that each XCD (blocks are dealt round-robin over 8 XCDs) gets a
-// contiguous range of work blocks, which keeps neighbouring tree cells in one L2.
-__device__ __forceinline__ uint32_t xcd_block(uint32_t b, uint32_t nb) {
-    const uint32_t q = nb >> 3, r = nb & 7u;
-    const uint32_t x = b & 7u, k = b >> 3;
-    return x * q + (x < r ? x : r) + k;
 }
 
 __device__ __forceinline__ float wave_sum_f(float v) {

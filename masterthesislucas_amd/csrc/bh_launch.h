@@ -42,8 +42,8 @@ uint64_t sort_scratch_words(uint32_t n);  // uint32 words of scratch launch_sort
 void launch_sort(hipStream_t s, void* keys_a, uint32_t* vals_a, void* keys_b, uint32_t* vals_b,
                  uint32_t n, int key_bits, bool wide, uint32_t* scratch, uint32_t* err,
                  uint32_t spin_limit, bool* result_in_b);
-// The state in sorted order (from the packed records) and per particle the leaf level, the level
-// it shares with its predecessor (+ 1) and the nodes it heads; sums: node counts of the tiles.
+// The state in sorted order (from the packed records) and per particle the level it shares with its
+// predecessor (+ 1) and the nodes it heads; sums: node counts of the tiles.
 // codes: zeroed (with the input order) when status says that the sort gave up; vx, vy: null when the
 // velocities are known to be zero. R: level of the tree roots (0; batched systems: the system id
 // occupies the levels above R).
@@ -51,12 +51,12 @@ uint32_t tree_sums_words(uint32_t n);
 void launch_gather_levels(hipStream_t s, const uint32_t* perm, const float4* pk, const float* vx,
                           const float* vy, float* xo, float* yo, float* mo, float* vxo, float* vyo,
                           uint32_t* ido, float4* pos4, void* codes, bool wide, uint32_t n, int B,
-                          int cap, int fixed_depth, uint8_t* leaf_lvl, uint8_t* lcp1, uint32_t* cnt,
+                          int cap, int fixed_depth, uint8_t* lcp1, uint32_t* cnt,
                           uint32_t* sums, int R, const uint32_t* status);
 void launch_tree(hipStream_t s, const void* codes, bool wide, uint32_t n, int B,
                  int single_child_pp, const uint8_t* lcp1, const uint32_t* cnt, uint32_t* noff,
-                 uint32_t* sums, BuildParams* prm, Node* nodes, uint32_t* parent,
-                 uint32_t* child4, uint32_t cap_nodes, int R, const BuildParams* sys_prm);
+                 uint32_t* sums, BuildParams* prm, Node* nodes, uint32_t* child4,
+                 uint32_t cap_nodes, int R, const BuildParams* sys_prm);
 void launch_bounds_batched(hipStream_t s, const float* xs, const float* ys, const uint2* blk,
                            uint32_t nblk, const uint32_t* blk_off, const uint32_t* sys_off,
                            uint32_t nsys, float4* partials, BuildParams* sys_prm,
