@@ -577,7 +577,8 @@ __global__ __launch_bounds__(kBlock) void k_aff_bandwidth(const double* __restri
 
 // ---------------------------------------------------------------------------------------------
 // symmetrisation: entries (i, j, p_{j|i}) and (j, i, p_{j|i}) keyed by row * n + column, sorted
-// by the project's radix sort (stable), equal keys (at most two) summed in FP64 in sorted order
+// by the project's sort (launch_sort: stable), equal keys (at most two) summed in FP64 in sorted
+// order
 // ---------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(kBlock) void k_sym_entries(const uint32_t* __restrict__ idx,
                                                         uint32_t n, uint32_t k,

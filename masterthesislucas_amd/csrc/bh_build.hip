@@ -7,9 +7,11 @@
 // its subtree. Nodes starting at sorted index i are the cells of levels
 // lcp(i-1, i)+1 .. leaf_level(i) whose first particle is i, so the layout follows from one scan.
 //
-// No kernel here uses device-scope fences or same-address device atomics: on a multi-XCD
-// part both are expensive (a device-scope fence writes back or invalidates the XCD's L2).
-// Results pass between kernels, and within a kernel only through LDS.
+// No kernel here uses device-scope fences, and same-address device atomics only to hand out the tiles
+// of a sort: on a multi-XCD part both are expensive (a device-scope fence writes back or invalidates
+// the XCD's L2). Results pass between kernels, and within a kernel through LDS; the exception are the
+// sorts' look-back words, each a state and a count in one relaxed device-scope word that needs no
+// fence.
 #include "bh_common.h"
 #include "bh_launch.h"
 

@@ -121,8 +121,10 @@ uint32_t launch_traverse(hipStream_t s, int kernel, const float4* pos4, const No
                          float inv_theta2, float eps2, float scale, float* ax, float* ay,
                          float* tot, unsigned long long* counters, TraverseBatch batch,
                          uint32_t split, CallerOut out);
-// the t-SNE solver plug-in's walk in its own summation order (one system of at most kPreorderMax
-// points)
+// The t-SNE solver plug-in's walk in its own summation order, one system of at most kPreorderMax
+// points: the sizes (the reference's 70,000 with room) whose sums a caller's doubles have kept to the
+// bit. It is no faster anywhere (131,072 points, spread: 329 us, the common walk 149), and its plain
+// sums are less accurate: larger calls take the common walk.
 constexpr uint32_t kPreorderMax = 1u << 17;
 uint32_t launch_traverse_preorder(hipStream_t s, const float4* pos4, const Node* nodes,
                                   const BuildParams* prm, uint32_t n, float inv_theta2, float* ax,

@@ -972,9 +972,17 @@ static inline uint32_t div_up(uint64_t a, uint64_t b) { return (uint32_t)((a + b
 //   uniform disk, 20,000 sinks (313 groups)    130 / 107 /  91 us
 //   t-SNE, 70,000 points (1,094 groups)        162 / 139 / 141 us compact, 141 / 117 / 111 spread
 //   two disks, 200,003 sinks (3,126 groups)    200 / 209 / 285 us; 1,048,576: 654 / 806 / 1215 us
-// and beside the attraction of a t-SNE iteration, two or four waves, five iterations: 1470 / 1448 us
-// compact, 1500 / 1475 spread. So four waves while the groups alone leave SIMDs idle, and for an
-// eighth more, two up to two groups per SIMD.
+// So four waves while the groups alone leave SIMDs idle, two up to two groups per SIMD. Around one
+// group per SIMD (1,024), the time with four waves over the time with two, theta 0.4 to 1.1 on two
+// disks, a uniform and a Plummer disk (t-SNE: spread and compact):
+//   groups            969         1,025-1,047  1,079-1,110  1,152       1,204       1,563
+//   gravity           0.93-1.02   0.95-1.02    0.96-1.06    0.98-1.08   0.98-1.04   1.15-1.26
+//   with the total    0.92-1.01   0.92-1.02    0.95-1.06    0.95-1.06   0.95-1.02   1.09-1.12
+//   learned           0.95        0.85-0.92    0.87-0.95    0.90-0.95   0.91-0.95   0.92-1.09
+//   t-SNE             0.72-0.97   0.83-0.98    0.68-0.95    0.79-0.95   0.66-0.98   0.80-1.08
+// Gravity is even there (the smaller angles gain what the larger ones lose), the learned walk and
+// t-SNE gain (beside the attraction 1470 -> 1448 us for five iterations, compact, 1500 -> 1475
+// spread): four waves for an eighth of a group per SIMD more.
 static uint64_t walk_simds() {
     static const uint64_t simds = [] {
         int dev = 0, cus = 0;
@@ -991,8 +999,8 @@ static uint32_t walk_waves_per_group(uint64_t groups) {
     return groups <= simds + simds / 8 ? 4u : groups <= 2 * simds ? 2u : 1u;
 }
 
-// One wave per group: left to itself the compiler takes 88 to 105 registers, five (gravity with
-// totals: four) waves per SIMD. Launches that bring more groups than that run a build held to the
+// One wave per group: left to itself the compiler takes 88 to 106 registers, five (with totals four)
+// waves per SIMD. Launches that bring more groups than that run a build held to the
 // registers of six or seven resident waves: a few values go through scratch, and the added waves
 // hide the loads and LDS reads. Where fewer groups come, the spills cost and nothing is gained.
 // Compiler's own / six / seven / eight, theta 0.5, us:

@@ -1,11 +1,12 @@
 // t-SNE gradient step on gfx950 (the TSNE driver of the reference, tsne.h:179-233, 272-301,
 // 356-460), built on the Barnes-Hut repulsion of this library.
 //
-// The embedding lives in the caller's point order (P is indexed that way). Per iteration:
-// stage the embedding as the solver's particles, build the tree, traverse with the t-SNE kernel
-// (repulsion and per-point Z terms in sorted order), reduce Z in FP64, bring the repulsion
-// back to the caller's order, then one kernel per row adds the CSR attraction and applies the
-// momentum update y' = y + lr d + mu (y - y_prev).
+// The embedding lives in the caller's point order (P is indexed that way). Per iteration: the
+// embedding as the solver's particles (staged by the first iteration of a call, then left by the
+// update before), the tree, the walk with the t-SNE kernel (repulsion and per-point Z terms in sorted
+// order) beside the CSR attraction on a stream of its own, the repulsion back in the caller's order
+// with partial sums of Z in FP64, and one kernel that finishes Z and applies the momentum update
+// y' = y + lr d + mu (y - y_prev).
 #include "bh_common.h"
 #include "bh_launch.h"
 
@@ -39,7 +40,7 @@ __global__ __launch_bounds__(kBlock) void k_tsne_stage(const float* __restrict__
 
 // One wave per row i: attraction exag * sum_j P_ij w_ij (y_j - y_i) with w = 1/(1+|y_j-y_i|^2)
 // (updateAttractive, tsne.h:356-381). It needs only the current embedding, so it runs on a
-// stream of its own while the tree is built and walked. The neighbours' positions are gathered
+// stream of its own beside the walk. The neighbours' positions are gathered
 // from the interleaved copy xy (one 8-byte load per non-zero instead of two 4-byte ones: the
 // gathers, not the bytes, bound this kernel).
 __global__ __launch_bounds__(kBlock) void k_tsne_attract(const uint32_t* __restrict__ row_ptr,
